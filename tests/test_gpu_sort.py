@@ -56,3 +56,21 @@ def test_keys_differing_in_high_bytes_only(ctx):
     assert np.array_equal(ctx.sort_by_keys(k, 1), stable_order(k, 1))
     same = np.full(n, 12345, dtype=np.int64)
     assert np.array_equal(ctx.sort_by_keys(same, 1), np.arange(n, dtype=np.int32))
+
+
+@pytest.mark.parametrize("bits", [(20, 20, 24), (20, 21, 24), (52, 52, 52), (64, 1, 64)])
+@pytest.mark.parametrize("ties", [False, True])
+def test_wide_tuples_in_one_or_several_packed_keys(ctx, bits, ties):
+    """Components whose differing bits fit 64 bits together are sorted as one
+    key, others group by group; leading keys without ties decide alone."""
+    rng = np.random.default_rng(sum(bits) + ties)
+    n = 9001
+    k = np.stack([rng.integers(-2**(b - 1), 2**(b - 1), size=n, endpoint=False) for b in bits],
+                 axis=1).astype(np.int64)
+    if ties:
+        k[:, 0] = k[rng.integers(0, 40, size=n), 0]
+        k[::3, 1] = k[0, 1]
+    else:
+        k[:, 0] = np.unique(rng.integers(-2**(bits[0] - 1), 2**(bits[0] - 1), size=3 * n,
+                                         endpoint=False))[rng.permutation(n)]
+    assert np.array_equal(ctx.sort_by_keys(k.ravel(), 3), stable_order(k.ravel(), 3))
