@@ -295,6 +295,19 @@ __device__ __forceinline__ LO xcd_thread_index() {
   return LO(start + k) * LO(blockDim.x) + LO(threadIdx.x);
 }
 
+// the row of item p: the last row whose items start at or before p
+__device__ __forceinline__ LO row_of(LO p, LO nrows, LO const* offsets) {
+  LO lo = 0, hi = nrows - 1;
+  while (lo < hi) {
+    LO mid = lo + (hi - lo + 1) / 2;
+    if (offsets[mid] <= p)
+      lo = mid;
+    else
+      hi = mid - 1;
+  }
+  return lo;
+}
+
 // ---- primitives (osh_prims.hip) ----
 // exclusive scans (n + 1 outputs, out[0] = 0) of LO values, I8 values or I8
 // nonzero flags; several share one launch through offset_scans

@@ -164,3 +164,25 @@ def test_constant_density_stays_constant(ctx):
     opts.verbosity = 0
     g.adapt(opts)
     np.testing.assert_allclose(g.elem_tag("rho"), 2.5, rtol=1e-13)
+
+
+@pytest.mark.parametrize("ncomps", [1, 17, 64, 65])
+def test_intersection_densities_of_many_components(ctx, ncomps):
+    """Each lane of a product's group sums its share of the components: in
+    registers up to four a lane, in place beyond.  An infinite value spoils
+    the products of its cavities, apart from it or not, as in the oracle."""
+    g = A.Mesh.box(ctx, 3, 5)
+    g.set_metric(g.implied_isos() * (1.0 / 1.6 ** 2), 1)
+    o = O.Mesh.copy_of(g)
+    rho = np.random.default_rng(ncomps).uniform(0.5, 2.0, size=(g.nents(3), ncomps))
+    rho[::50, 0] = np.inf
+    for m in (o, g):
+        m.add_elem_tag("rho", ncomps, rho.ravel())
+        m.set_elem_transfer("rho", m.DENSITY)
+    oo, go = O.default_opts(3), ctx.default_opts(3)
+    oo.verbosity = go.verbosity = 0
+    assert o.coarsen_by_size(oo) == g.coarsen_by_size(go) == 1
+    a, b = o.elem_tag("rho"), g.elem_tag("rho")
+    assert np.array_equal(np.isnan(a), np.isnan(b))
+    assert_same(a[~np.isnan(a)], b[~np.isnan(a)], "rho")
+    assert not np.all(np.isfinite(b)) and np.isfinite(b).sum() > len(b) // 4
