@@ -75,6 +75,7 @@ Ctx::Ctx() : pool(std::make_shared<Pool>()) {
   std::memset(pinned, 0, 8 * kSlots + 64);
   OSH_HIP(hipMalloc(&partials, 1024 * sizeof(double)));
   OSH_HIP(hipMalloc((void**)&tile_counter, sizeof(unsigned)));
+  OSH_HIP(hipMalloc((void**)&tile_sums, sizeof(LO) * kScanTiles * kMaxScanJobs));
   unsigned zero = 0;
   OSH_HIP(hipMemcpy(tile_counter, &zero, sizeof(zero), hipMemcpyHostToDevice));
   noalloc_setup(device);
@@ -93,6 +94,7 @@ Ctx::~Ctx() {
   }
   if (scan_status) (void)hipFree(scan_status);
   if (tile_counter) (void)hipFree(tile_counter);
+  if (tile_sums) (void)hipFree(tile_sums);
   if (pool) pool->close();
   if (partials) (void)hipFree(partials);
   if (pinned) (void)hipHostFree(pinned);
@@ -338,6 +340,172 @@ __global__ void __launch_bounds__(kBlock) scan_lookback(ScanBatch b,
   }
 }
 
+// Scans of moderate jobs take two launches instead: one sums each tile, the
+// next scans each tile behind the sum of its job's earlier tile sums, which
+// every workgroup adds up for itself.  A look-back has to carry the prefix
+// from workgroup to workgroup across the XCDs, a device-scope round trip at
+// a time: 10 us from two tiles on, 21 us at 542, against 11 us for the two
+// launches.  Jobs of one tile of 16384 values need only the second launch,
+// and in moderate jobs (kOwnTiles) each workgroup adds up the values in front
+// of its tile itself, from L2, which costs less than the first launch.
+//
+// A thread takes four consecutive values per round (one 16-byte load, or one
+// 4-byte load of byte values, where the array is so aligned) and writes the
+// four offsets in front of them, so loads and stores are wide and coalesced
+// without a pass through LDS.
+template <int BLOCK, int ROUNDS>
+struct TileScan {
+  static constexpr int kWaves = BLOCK / kWave;
+  static constexpr int kParts = ROUNDS * kWaves;
+  static constexpr int kTile = BLOCK * ROUNDS * 4;
+  static_assert(kParts <= kWave, "one wave scans the partial sums");
+};
+
+__device__ __forceinline__ void load_four(void const* in, int kind, LO i, LO n, bool wide,
+    LO* v) {
+  if (wide && i + 4 <= n) {
+    if (kind == kScanLO) {
+      int4 q = *reinterpret_cast<int4 const*>(static_cast<LO const*>(in) + i);
+      v[0] = q.x;
+      v[1] = q.y;
+      v[2] = q.z;
+      v[3] = q.w;
+    } else {
+      char4 q = *reinterpret_cast<char4 const*>(static_cast<I8 const*>(in) + i);
+      bool b = kind == kScanBytes;
+      v[0] = b ? LO(q.x) : LO(q.x != 0);
+      v[1] = b ? LO(q.y) : LO(q.y != 0);
+      v[2] = b ? LO(q.z) : LO(q.z != 0);
+      v[3] = b ? LO(q.w) : LO(q.w != 0);
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = (i + k < n) ? scan_input(in, kind, i + k) : 0;
+  }
+}
+
+__device__ __forceinline__ bool wide_input(void const* in, int kind) {
+  return (reinterpret_cast<std::uintptr_t>(in) & (kind == kScanLO ? 15u : 3u)) == 0;
+}
+
+__device__ __forceinline__ int job_of(ScanBatch const& b, unsigned t) {
+  int job = 0;
+  while (job + 1 < b.count && t >= b.first[job + 1]) ++job;
+  return job;
+}
+
+constexpr int kSumBlock = 256;
+constexpr int kSumRounds = 2;
+constexpr int kSumTile = TileScan<kSumBlock, kSumRounds>::kTile;
+constexpr int kOneBlock = 1024;
+constexpr int kOneRounds = 4;
+constexpr int kOneTile = TileScan<kOneBlock, kOneRounds>::kTile;
+// every workgroup reads its job's earlier tile sums: up to this many tiles
+// (16.7 M values) that costs less than the look-back's chain
+constexpr unsigned kMaxSumTiles = Ctx::kScanTiles;
+// a workgroup of the one-launch form reads at most this many tiles of 4096
+// values, and all of a launch at most kOwnBytes: at up to 16 tiles it takes 6
+// us against 8.5 us for the two launches and 10 us for the look-back, at 32
+// tiles 10 us
+constexpr int kOwnTile = TileScan<kOneBlock, 1>::kTile;
+constexpr unsigned kOwnTiles = 16;
+constexpr double kOwnBytes = 8e6;
+
+__global__ void __launch_bounds__(kSumBlock) sum_tiles(ScanBatch b, LO* sums) {
+  unsigned t = blockIdx.x;
+  int job = job_of(b, t);
+  LO base = LO(t - b.first[job]) * kSumTile;
+  bool wide = wide_input(b.in[job], b.kind[job]);
+  LO acc = 0;
+#pragma unroll
+  for (int r = 0; r < kSumRounds; ++r) {
+    LO v[4];
+    load_four(b.in[job], b.kind[job], base + (r * kSumBlock + LO(threadIdx.x)) * 4, b.n[job],
+        wide, v);
+    acc += (v[0] + v[1]) + (v[2] + v[3]);
+  }
+  __shared__ LO part[kSumBlock / kWave];
+  acc = wave_sum(acc);
+  if ((threadIdx.x & (kWave - 1)) == 0) part[threadIdx.x / kWave] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    LO s = 0;
+    for (int w = 0; w < kSumBlock / kWave; ++w) s += part[w];
+    sums[t] = s;
+  }
+}
+
+// with OWN each workgroup sums its job's earlier values instead of reading
+// their tile sums
+template <int BLOCK, int ROUNDS, bool OWN>
+__global__ void __launch_bounds__(BLOCK) scan_tiles(ScanBatch b, LO const* sums) {
+  using T = TileScan<BLOCK, ROUNDS>;
+  __shared__ LO part[T::kParts];
+  __shared__ LO before[T::kWaves];
+  unsigned t = blockIdx.x;
+  int job = job_of(b, t);
+  unsigned tile = t - b.first[job];
+  unsigned ntiles = b.first[job + 1] - b.first[job];
+  LO n = b.n[job];
+  int lane = int(threadIdx.x) & (kWave - 1);
+  int wave = int(threadIdx.x) / kWave;
+  LO base = LO(tile) * T::kTile;
+  bool wide = wide_input(b.in[job], b.kind[job]);
+  LO v[ROUNDS][4];
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r)
+    load_four(b.in[job], b.kind[job], base + (r * BLOCK + LO(threadIdx.x)) * 4, n, wide, v[r]);
+  LO earlier = 0;
+  if constexpr (OWN) {
+    // whole tiles, all in range
+#pragma unroll 4
+    for (LO i = LO(threadIdx.x) * 4; i < base; i += BLOCK * 4) {
+      LO u[4];
+      load_four(b.in[job], b.kind[job], i, n, wide, u);
+      earlier += (u[0] + u[1]) + (u[2] + u[3]);
+    }
+  } else {
+    for (unsigned j = threadIdx.x; j < tile; j += BLOCK) earlier += sums[b.first[job] + j];
+  }
+  if (tile) earlier = wave_sum(earlier);
+  if (lane == 0) before[wave] = earlier;
+  LO inc[ROUNDS];
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    inc[r] = wave_inclusive_scan((v[r][0] + v[r][1]) + (v[r][2] + v[r][3]));
+    if (lane == kWave - 1) part[r * T::kWaves + wave] = inc[r];
+  }
+  __syncthreads();
+  if (wave == 0) {
+    LO p = lane < T::kParts ? part[lane] : 0;
+    LO s = lane < T::kWaves ? before[lane] : 0;
+    LO prefix = wave_sum(s);
+    LO i = wave_inclusive_scan(p);
+    if (lane < T::kParts) part[lane] = prefix + i - p;
+    if (lane == kWave - 1 && tile == ntiles - 1) {
+      b.out[job][n] = prefix + i;
+      if (b.total[job]) *b.total[job] = prefix + i;
+    }
+  }
+  __syncthreads();
+  LO* out = b.out[job];
+  bool wide_out = (reinterpret_cast<std::uintptr_t>(out) & 15u) == 0;
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    LO i = base + (r * BLOCK + LO(threadIdx.x)) * 4;
+    LO o0 = part[r * T::kWaves + wave] + inc[r] - ((v[r][0] + v[r][1]) + (v[r][2] + v[r][3]));
+    LO o1 = o0 + v[r][0], o2 = o1 + v[r][1], o3 = o2 + v[r][2];
+    if (wide_out && i + 4 <= n) {
+      *reinterpret_cast<int4*>(out + i) = make_int4(o0, o1, o2, o3);
+    } else {
+      if (i < n) out[i] = o0;
+      if (i + 1 < n) out[i + 1] = o1;
+      if (i + 2 < n) out[i + 2] = o2;
+      if (i + 3 < n) out[i + 3] = o3;
+    }
+  }
+}
+
 __global__ void zero_u64(LO n, unsigned long long* a) {
   LO i = thread_index();
   if (i < n) a[i] = 0ull;
@@ -368,11 +536,13 @@ unsigned long long* scan_status_words(Ctx& c, LO ntiles, unsigned* epoch) {
 
 }  // namespace
 
-void offset_scans(Ctx& c, ScanJob const* jobs, int njobs) {
-  OSH_CHECK(njobs >= 1 && njobs <= kMaxScanJobs, "offset_scans: 1 to 12 jobs per launch");
-  ScanBatch b{};
+namespace {
+
+// the jobs as a batch in tiles of `tile` values; returns the tile count and
+// the largest job's in *most
+unsigned batch_jobs(ScanJob const* jobs, int njobs, int tile, ScanBatch& b, unsigned* most) {
   unsigned tiles = 0;
-  bool multi = false;
+  *most = 0;
   for (int j = 0; j < njobs; ++j) {
     OSH_CHECK(jobs[j].n >= 0 && jobs[j].out, "offset_scans: bad job");
     b.in[j] = jobs[j].in;
@@ -382,21 +552,59 @@ void offset_scans(Ctx& c, ScanJob const* jobs, int njobs) {
     b.kind[j] = jobs[j].kind;
     b.first[j] = tiles;
     // an empty job still takes one tile, which writes its 0 and its total
-    unsigned nt = jobs[j].n == 0 ? 1u : unsigned((std::int64_t(jobs[j].n) + kScanTile - 1) / kScanTile);
-    multi = multi || nt > 1;
+    unsigned nt = jobs[j].n == 0 ? 1u : unsigned((std::int64_t(jobs[j].n) + tile - 1) / tile);
+    *most = nt > *most ? nt : *most;
     tiles += nt;
   }
   b.first[njobs] = tiles;
   b.count = njobs;
-  unsigned epoch = 0;
-  unsigned long long* status = nullptr;
-  unsigned ticket_base = c.tile_tickets;
-  if (multi) {
-    status = scan_status_words(c, LO(tiles), &epoch);
-    c.tile_tickets += tiles;
+  return tiles;
+}
+
+}  // namespace
+
+void offset_scans(Ctx& c, ScanJob const* jobs, int njobs) {
+  OSH_CHECK(njobs >= 1 && njobs <= kMaxScanJobs, "offset_scans: 1 to 12 jobs per launch");
+  ScanBatch b{};
+  unsigned most = 0;
+  unsigned tiles = batch_jobs(jobs, njobs, kOneTile, b, &most);
+  if (most <= 1) {
+    hipLaunchKernelGGL((scan_tiles<kOneBlock, kOneRounds, false>), dim3(tiles), dim3(kOneBlock),
+        0, c.stream, b, (LO const*)nullptr);
+    OSH_HIP(hipGetLastError());
+    return;
   }
+  tiles = batch_jobs(jobs, njobs, kOwnTile, b, &most);
+  if (most <= kOwnTiles) {
+    double read = 0.0;
+    for (int j = 0; j < njobs; ++j) {
+      double nt = double(b.first[j + 1] - b.first[j]);
+      read += 0.5 * nt * nt * kOwnTile * (jobs[j].kind == kScanLO ? 4.0 : 1.0);
+    }
+    if (read <= kOwnBytes) {
+      hipLaunchKernelGGL((scan_tiles<kOneBlock, 1, true>), dim3(tiles), dim3(kOneBlock), 0,
+          c.stream, b, (LO const*)nullptr);
+      OSH_HIP(hipGetLastError());
+      return;
+    }
+  }
+  tiles = batch_jobs(jobs, njobs, kSumTile, b, &most);
+  if (most <= kMaxSumTiles) {
+    LO* sums = c.tile_sums;
+    hipLaunchKernelGGL(sum_tiles, dim3(tiles), dim3(kSumBlock), 0, c.stream, b, sums);
+    OSH_HIP(hipGetLastError());
+    hipLaunchKernelGGL((scan_tiles<kSumBlock, kSumRounds, false>), dim3(tiles), dim3(kSumBlock), 0,
+        c.stream, b, static_cast<LO const*>(sums));
+    OSH_HIP(hipGetLastError());
+    return;
+  }
+  tiles = batch_jobs(jobs, njobs, kScanTile, b, &most);
+  unsigned epoch = 0;
+  unsigned ticket_base = c.tile_tickets;
+  unsigned long long* status = scan_status_words(c, LO(tiles), &epoch);
+  c.tile_tickets += tiles;
   hipLaunchKernelGGL(scan_lookback, dim3(tiles), dim3(kBlock), 0, c.stream, b, status,
-      c.tile_counter, ticket_base, multi ? 1 : 0, epoch, c.error_word());
+      c.tile_counter, ticket_base, 1, epoch, c.error_word());
   OSH_HIP(hipGetLastError());
 }
 

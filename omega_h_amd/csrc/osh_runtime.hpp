@@ -122,6 +122,10 @@ struct Ctx {
   static constexpr unsigned kMaxScanEpoch = (1u << 24) - 1;
   unsigned* tile_counter = nullptr;
   unsigned tile_tickets = 0;
+  // tile sums of the two-launch scans: up to kScanTiles tiles for each job of
+  // a call
+  static constexpr unsigned kScanTiles = 8192;
+  LO* tile_sums = nullptr;
   Tuning tuning;
   // when set (by the batched driver), each pass marks here the parts of a
   // joined mesh that it changes

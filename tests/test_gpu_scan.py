@@ -41,6 +41,33 @@ def test_single_scan(ctx, n):
     assert np.array_equal(got, expected(a)), n
 
 
+@pytest.mark.parametrize("n", [16383, 16384, 16385, 20479, 20480, 16 * 4096,
+                               16 * 4096 + 1, 8192 * 2048, 8192 * 2048 + 1])
+def test_sizes_at_the_edges_of_tiles_and_launch_forms(ctx, n):
+    """One 16384-value tile, the 4096-value tiles of the one-launch form and
+    its largest job, and the largest job of the two-launch form."""
+    a = np.random.default_rng(n).integers(0, 8, size=n, dtype=np.int32)
+    (got,) = run_scans(ctx, [a])
+    assert np.array_equal(got, expected(a)), n
+
+
+@pytest.mark.parametrize("shift", [1, 2, 3])
+@pytest.mark.parametrize("n", [5, 16384, 40_001, 300_001])
+def test_arrays_at_any_word(ctx, n, shift):
+    """Arrays that don't start at a 16-byte boundary."""
+    from omega_h_amd.hip import DeviceArray
+    a = np.random.default_rng(n).integers(0, 8, size=n + shift, dtype=np.int32)
+    d = DeviceArray(a)
+    for in_shift, out_shift in ((shift, 0), (0, shift), (shift, shift)):
+        o = DeviceArray(np.full(n + 1 + shift, -7, dtype=np.int32))
+        ctx.offset_scans([d.ptr + 4 * in_shift], [n], [o.ptr + 4 * out_shift])
+        ctx.synchronize()
+        got = o.numpy()
+        assert np.array_equal(got[out_shift:out_shift + n + 1],
+                              expected(a[in_shift:in_shift + n]))
+        assert np.all(got[:out_shift] == -7) and np.all(got[out_shift + n + 1:] == -7)
+
+
 def test_batched_scans_in_one_launch(ctx):
     rng = np.random.default_rng(7)
     for sizes in ([5, 0, 4096, 1], [300_000, 17, 1_000_000, 4097], [2_500_000, 2_500_000],
