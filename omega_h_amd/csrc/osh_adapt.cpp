@@ -114,7 +114,7 @@ bool run_pass(Ctx& c, DMesh& m, AdaptOptions const& o, int kind,
   else
     r = coarsen_slivers(c, m, o);
   min_real_async(c, ask_qualities(c, m), kQminSlot);
-  c.sync();
+  c.wait();
   double t1 = now();
   range.end();
   *qmin = read_slot<Real>(c, kQminSlot);

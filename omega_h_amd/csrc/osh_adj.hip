@@ -175,7 +175,7 @@ Adj invert_adj(Ctx& c, LO nhigh, int deg, LO nlow, LOs const& hl2l, Bytes const*
     ScanJob jobs[2] = {{counts.data(), kScanLO, nlow, a.a2ab.data(), nullptr},
         {mk, kScanNonzero, nlow, marked_offsets.data(), slot_ptr<LO>(c, 1)}};
     offset_scans(c, jobs, 2);
-    c.sync();
+    c.wait();
     *marked = LOs(c, read_slot<LO>(c, 1));
     scatter_marked_list(c, *marks, marked_offsets, *marked);
     if (marked_index) *marked_index = marked_offsets;

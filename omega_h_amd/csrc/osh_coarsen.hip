@@ -886,7 +886,7 @@ bool coarsen(Ctx& c, DMesh& m, AdaptOptions const& o, Bytes& codes, bool oversho
     }
     OSH_LAUNCH(live_counts, dim * nkeys * kLanes, c, nkeys, keys2verts.data(), rows);
     offset_scans(c, jobs, dim);
-    c.sync();
+    c.wait();
     for (int d = 1; d <= dim; ++d) nprods[d] = read_slot<LO>(c, d);
   }
   // every dimension's new numbering by one more scan launch

@@ -801,7 +801,7 @@ void modify_scan(Ctx& c, ModPlan* plans, int nplans) {
   ScanJob jobs[kMaxScanJobs];
   int njobs = modify_scan_jobs(c, plans, nplans, jobs, 1);
   offset_scans(c, jobs, njobs);
-  c.sync();
+  c.wait();
   modify_scan_totals(c, plans, nplans, 1);
 }
 

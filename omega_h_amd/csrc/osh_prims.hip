@@ -71,8 +71,8 @@ void Pool::release_all() {
 Ctx::Ctx() : pool(std::make_shared<Pool>()) {
   OSH_HIP(hipGetDevice(&device));
   OSH_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-  OSH_HIP(hipHostMalloc(&pinned, 8 * kSlots + 64, hipHostMallocDefault));
-  std::memset(pinned, 0, 8 * kSlots + 64);
+  OSH_HIP(hipHostMalloc(&pinned, 8 * kSlots + 128, hipHostMallocDefault));
+  std::memset(pinned, 0, 8 * kSlots + 128);
   OSH_HIP(hipMalloc(&partials, 1024 * sizeof(double)));
   OSH_HIP(hipMalloc((void**)&tile_counter, sizeof(unsigned)));
   OSH_HIP(hipMalloc((void**)&tile_sums, sizeof(LO) * kScanTiles * kMaxScanJobs));
@@ -115,6 +115,48 @@ void range_end(Ctx& c) {
 
 void Ctx::sync() {
   OSH_HIP(hipStreamSynchronize(stream));
+  raise_device_error();
+}
+
+namespace {
+
+// stores made by the stream's earlier kernels happen before this release
+__global__ void signal_kernel(unsigned* word, unsigned value) {
+  __hip_atomic_store(word, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// how long wait() polls before it leaves the core to other threads
+constexpr double kPollSeconds = 200e-6;
+
+}  // namespace
+
+// A pass waits for its counts four to six times, each wait with the device
+// idle until the host has seen it and launched again.  hipStreamSynchronize
+// adds 8 to 30 us to the kernels it waits for (a system-scope barrier packet
+// and often an interrupt); a one-thread kernel that stores into pinned memory
+// with the host polling that word adds 6 to 8 us.
+void Ctx::wait() {
+  unsigned value = ++signal_value;
+  unsigned* word = signal_word();
+  hipLaunchKernelGGL(signal_kernel, dim3(1), dim3(1), 0, stream, word, value);
+  OSH_HIP(hipGetLastError());
+  double limit = 0.0;
+  for (unsigned polls = 1;; ++polls) {
+    if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == value) {
+      raise_device_error();
+      return;
+    }
+    __builtin_ia32_pause();
+    if (polls % 64 == 0) {
+      double t = profile_now();
+      if (limit == 0.0) limit = t + kPollSeconds;
+      if (t > limit) break;
+    }
+  }
+  sync();
+}
+
+void Ctx::raise_device_error() {
   int* err = error_word();
   if (*err != kNoError) {
     int code = *err;

@@ -268,7 +268,7 @@ bool refine_by_size(Ctx& c, DMesh& m, AdaptOptions const& o) {
       jobs[d - 1] = {counts[d].data(), kScanLO, nkeys, k2p[d].data(), slot_ptr<LO>(c, d)};
     }
     offset_scans(c, jobs, dim);
-    c.sync();
+    c.wait();
     for (int d = 1; d <= dim; ++d) nprods[d] = read_slot<LO>(c, d);
   }
   // every dimension's new numbering by one more scan launch

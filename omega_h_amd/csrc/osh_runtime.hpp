@@ -107,7 +107,7 @@ struct Ctx {
   int device = 0;
   // pinned host words that kernels write results into: 8-byte slots
   // 0..kSlots-1 (totals, reductions) and one error word that kernels set
-  // when they find a broken invariant; sync() raises it
+  // when they find a broken invariant; sync() and wait() raise it
   static constexpr int kSlots = 16;
   void* pinned = nullptr;
   int* error_word() const { return reinterpret_cast<int*>(static_cast<char*>(pinned) + 8 * kSlots); }
@@ -139,7 +139,18 @@ struct Ctx {
   ~Ctx();
   Ctx(Ctx const&) = delete;
   Ctx& operator=(Ctx const&) = delete;
+  // drains the stream and raises what kernels left in the error word
   void sync();
+  // the same for callers that go on to read pinned words the kernels wrote
+  // (not for copies into host memory, which only sync() completes)
+  void wait();
+
+ private:
+  unsigned signal_value = 0;
+  unsigned* signal_word() const {
+    return reinterpret_cast<unsigned*>(static_cast<char*>(pinned) + 8 * kSlots + 64);
+  }
+  void raise_device_error();
 };
 
 void range_begin(Ctx& c, char const* name);
@@ -218,8 +229,8 @@ inline std::vector<T> to_host(Ctx& c, DArray<T> const& d) {
   return h;
 }
 
-// a value that a kernel wrote into a pinned slot; read_slot assumes the
-// stream has been drained, pinned_value drains it first
+// a value that a kernel wrote into a pinned slot; read_slot assumes that the
+// caller has waited for the stream, pinned_value waits first
 template <class T>
 inline T read_slot(Ctx& c, int slot) {
   T v;
@@ -228,7 +239,7 @@ inline T read_slot(Ctx& c, int slot) {
 }
 template <class T>
 inline T pinned_value(Ctx& c, int slot = 0) {
-  c.sync();
+  c.wait();
   return read_slot<T>(c, slot);
 }
 template <class T>

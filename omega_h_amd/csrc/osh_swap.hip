@@ -987,7 +987,7 @@ bool swap_edges_3d(Ctx& c, DMesh& m, AdaptOptions const& o, SwapCache* cache) {
   modify_plans_masked(c, m, 1, 3, keys, pc, plans, rep_of);
   int njobs = 4 + modify_scan_jobs(c, plans, 3, jobs + 4, 4);
   offset_scans(c, jobs, njobs);
-  c.sync();
+  c.wait();
   modify_scan_totals(c, plans, 3, 4);
   LO nkeys = read_slot<LO>(c, 0);
   if (o.verbosity >= 2) std::printf("swapping %d 3D edges\n", int(nkeys));
