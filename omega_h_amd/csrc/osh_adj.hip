@@ -11,6 +11,7 @@
 //                           src/Omega_h_adj.cpp:591-657
 //   find_unique             src/Omega_h_adj.cpp:55-153
 #include "osh_mesh.hpp"
+#include "osh_passes.hpp"
 
 namespace osh {
 
@@ -213,99 +214,156 @@ __device__ __forceinline__ LO min_vertex(LO const* v) {
   return m;
 }
 
-// counts[v] = 1 marks v; a marked row's final slot stays unused; each use's
-// match count starts at zero
+// The four sweeps below take the products of faces and of tets together (a
+// job each, owning the workgroups [first[w], first[w + 1])), since neither
+// needs the other's result: half the launches, which for the small product
+// lists of late passes are the cost.
+struct SideDim {
+  LO nuses;
+  LO const* pverts;
+  LO const* prods2new;  // null: products keep their numbers
+  LO nl;                // the lower entities and their vertices
+  LO const* lv2v;
+  LO* counts;
+  LO* slot;
+  LO const* a2ab;
+  int4* rows;
+  LO* out;
+  I8* codes;
+};
+
+struct SideJobs {
+  int n;
+  int high[2];
+  unsigned first[3];
+  SideDim d[2];
+};
+
+__device__ __forceinline__ int side_job(SideJobs const& j) {
+  return (j.n > 1 && blockIdx.x >= j.first[1]) ? 1 : 0;
+}
+__device__ __forceinline__ LO job_thread(SideJobs const& j, int w) {
+  return LO(blockIdx.x - j.first[w]) * kBlock + LO(threadIdx.x);
+}
+
+// counts[v] = 1 marks v; a marked row's final slot stays unused
 template <int HIGH>
-__global__ void mark_use_min_verts(LO nuses, LO const* prod_verts, LO* counts, LO* found) {
-  LO u = thread_index();
-  if (u >= nuses) return;
-  found[u] = 0;
+__device__ __forceinline__ void mark_use_min_vert(LO u, SideDim const& a) {
+  if (u >= a.nuses) return;
   constexpr int LOW = HIGH - 1;
   LO h = u / (HIGH + 1);
   int which = u % (HIGH + 1);
   LO av[3];
 #pragma unroll
   for (int k = 0; k < LOW + 1; ++k)
-    av[k] = prod_verts[h * (HIGH + 1) + down_template(HIGH, LOW, which, k)];
-  counts[min_vertex<LOW + 1>(av)] = 1;
+    av[k] = a.pverts[h * (HIGH + 1) + down_template(HIGH, LOW, which, k)];
+  a.counts[min_vertex<LOW + 1>(av)] = 1;
+}
+
+__global__ void mark_use_min_verts(SideJobs j) {
+  int w = side_job(j);
+  if (j.high[w] == 2)
+    mark_use_min_vert<2>(job_thread(j, w), j.d[w]);
+  else
+    mark_use_min_vert<3>(job_thread(j, w), j.d[w]);
 }
 
 template <int NVL>
-__global__ void count_min_rows(LO nl, LO const* lv2v, LO* counts, LO* slot) {
-  LO l = thread_index();
-  if (l >= nl) return;
-  LO vm = min_vertex<NVL>(lv2v + l * NVL);
+__device__ __forceinline__ void count_min_row(LO l, SideDim const& a) {
+  if (l >= a.nl) return;
+  LO vm = min_vertex<NVL>(a.lv2v + std::size_t(l) * NVL);
   // unmarked counts stay 0 throughout this kernel, marked ones are >= 1
-  slot[l] = counts[vm] ? atomicAdd(&counts[vm], 1) - 1 : -1;
+  a.slot[l] = a.counts[vm] ? atomicAdd(&a.counts[vm], 1) - 1 : -1;
+}
+
+__global__ void count_min_rows(SideJobs j) {
+  int w = side_job(j);
+  if (j.high[w] == 2)
+    count_min_row<2>(job_thread(j, w), j.d[w]);
+  else
+    count_min_row<3>(job_thread(j, w), j.d[w]);
 }
 
 // a row entry is {entity, its vertices}, so the match reads no other array
 template <int NVL>
-__global__ void fill_min_rows(LO nl, LO const* lv2v, LO const* a2ab, LO const* slot, int4* rows) {
-  LO l = thread_index();
-  if (l >= nl) return;
-  LO s = slot[l];
+__device__ __forceinline__ void fill_min_row(LO l, SideDim const& a) {
+  if (l >= a.nl) return;
+  LO s = a.slot[l];
   if (s < 0) return;
   LO v[3] = {0, 0, 0};
 #pragma unroll
-  for (int k = 0; k < NVL; ++k) v[k] = lv2v[l * NVL + k];
-  rows[a2ab[min_vertex<NVL>(v)] + s] = make_int4(l, v[0], v[1], v[2]);
+  for (int k = 0; k < NVL; ++k) v[k] = a.lv2v[std::size_t(l) * NVL + k];
+  a.rows[a.a2ab[min_vertex<NVL>(v)] + s] = make_int4(l, v[0], v[1], v[2]);
 }
 
-// kMatchLanes threads per use share its row; a lane that finds a match
-// writes it and counts it in found[u], which the consumer checks (a use needs
-// exactly one match)
+__global__ void fill_min_rows(SideJobs j) {
+  int w = side_job(j);
+  if (j.high[w] == 2)
+    fill_min_row<2>(job_thread(j, w), j.d[w]);
+  else
+    fill_min_row<3>(job_thread(j, w), j.d[w]);
+}
+
+// kMatchLanes threads per use share its row; the lane that finds the match
+// writes it at the product's new number.  A use without exactly one match
+// sets the error word and gets entity 0, which keeps every index in range.
 constexpr int kMatchLanes = 4;
 
 template <int HIGH>
-__global__ void match_uses(LO nt, LO const* __restrict__ prod_verts,
-    LO const* __restrict__ a2ab, int4 const* __restrict__ rows, LO* __restrict__ out,
-    I8* __restrict__ out_codes, LO* __restrict__ found) {
-  LO t = thread_index();
-  if (t >= nt) return;
+__device__ __forceinline__ void match_use(LO t, SideDim const& a, int* error) {
   LO u = t / kMatchLanes;
   int lane = t % kMatchLanes;
   constexpr int LOW = HIGH - 1;
   constexpr int nvh = HIGH + 1;
   constexpr int nvl = LOW + 1;
-  LO h = u / (HIGH + 1);
-  int which = u % (HIGH + 1);
-  LO av[3];
+  int found = 0;
+  LO at = 0;
+  if (u < a.nuses) {
+    LO h = u / (HIGH + 1);
+    int which = u % (HIGH + 1);
+    at = (a.prods2new ? a.prods2new[h] : h) * nvh + which;
+    LO av[3];
 #pragma unroll
-  for (int k = 0; k < nvl; ++k) av[k] = prod_verts[h * nvh + down_template(HIGH, LOW, which, k)];
-  LO vm = min_vertex<nvl>(av);
-  LO k0 = a2ab[vm], k1 = a2ab[vm + 1] - 1;
-  for (LO k = k0 + lane; k < k1; k += kMatchLanes) {
-    int4 r = rows[k];
-    LO bv[3] = {r.y, r.z, r.w};
-    // wd: the position of the use's first vertex in the candidate
-    int wd = (bv[0] == av[0]) ? 0 : (bv[1] == av[0]) ? 1 : (nvl == 3 && bv[2] == av[0]) ? 2 : -1;
-    if (wd < 0) continue;
-    I8 code;
-    if (nvl == 2) {
-      if (av[1] != bv[1 - wd]) continue;
-      code = make_code(0, wd, 0);
-    } else if (av[1] == bv[(wd + 1) % 3] && av[2] == bv[(wd + 2) % 3]) {
-      code = make_code(0, (3 - wd) % 3, 0);
-    } else if (av[1] == bv[(wd + 2) % 3] && av[2] == bv[(wd + 1) % 3]) {
-      code = make_code(1, (3 - wd) % 3, 0);
-    } else {
-      continue;
+    for (int k = 0; k < nvl; ++k) av[k] = a.pverts[h * nvh + down_template(HIGH, LOW, which, k)];
+    LO vm = min_vertex<nvl>(av);
+    LO k0 = a.a2ab[vm], k1 = a.a2ab[vm + 1] - 1;
+    for (LO k = k0 + lane; k < k1; k += kMatchLanes) {
+      int4 r = a.rows[k];
+      LO bv[3] = {r.y, r.z, r.w};
+      // wd: the position of the use's first vertex in the candidate
+      int wd =
+          (bv[0] == av[0]) ? 0 : (bv[1] == av[0]) ? 1 : (nvl == 3 && bv[2] == av[0]) ? 2 : -1;
+      if (wd < 0) continue;
+      I8 code;
+      if (nvl == 2) {
+        if (av[1] != bv[1 - wd]) continue;
+        code = make_code(0, wd, 0);
+      } else if (av[1] == bv[(wd + 1) % 3] && av[2] == bv[(wd + 2) % 3]) {
+        code = make_code(0, (3 - wd) % 3, 0);
+      } else if (av[1] == bv[(wd + 2) % 3] && av[2] == bv[(wd + 1) % 3]) {
+        code = make_code(1, (3 - wd) % 3, 0);
+      } else {
+        continue;
+      }
+      a.out[at] = r.x;
+      a.codes[at] = code;
+      ++found;
     }
-    out[u] = r.x;
-    out_codes[u] = code;
-    atomicAdd(&found[u], 1);
+  }
+  for (int d = kMatchLanes / 2; d > 0; d >>= 1) found += __shfl_xor(found, d, 64);
+  if (u < a.nuses && lane == 0 && found != 1) {
+    a.out[at] = 0;
+    a.codes[at] = 0;
+    *error = kReflectDownNoMatch;
   }
 }
 
-// for callers that use the matches directly: a use without exactly one match
-// sets the error word and gets entity 0, which keeps every index in range
-__global__ void check_matches(LO nuses, LO const* found, LO* out, I8* out_codes, int* error) {
-  LO u = thread_index();
-  if (u >= nuses || found[u] == 1) return;
-  out[u] = 0;
-  out_codes[u] = 0;
-  *error = kReflectDownNoMatch;
+__global__ void __launch_bounds__(kBlock) match_uses(SideJobs j, int* error) {
+  int w = side_job(j);
+  if (j.high[w] == 2)
+    match_use<2>(job_thread(j, w), j.d[w], error);
+  else
+    match_use<3>(job_thread(j, w), j.d[w], error);
 }
 
 // per side, the number of elements on it (high 32 bits) and the sum of their
@@ -452,45 +510,93 @@ Adj const& ask_up(Ctx& c, DMesh& m, int low, int high) {
   return m.up[low][high];
 }
 
+namespace {
+
+// sets the jobs' workgroups for a sweep with n[w] threads in job w; returns
+// their number
+unsigned side_blocks(SideJobs& j, std::int64_t const* n) {
+  unsigned b = 0;
+  for (int w = 0; w < j.n; ++w) {
+    j.first[w] = b;
+    OSH_CHECK(n[w] <= std::int64_t(0x7fffffff), "reflect_down: too many uses");
+    b += unsigned((n[w] + kBlock - 1) / kBlock);
+    j.first[w + 1] = b;
+  }
+  return b;
+}
+
+void run_sides(Ctx& c, DMesh& m, SideJobs& j) {
+  LO nv = m.nents[0];
+  LOs counts = fill_lo(c, nv * j.n, 0);
+  LOs slot[2], a2ab[2];
+  DArray<int4> rows[2];
+  ScanJob scans[2];
+  std::int64_t uses[2], lows[2], lanes[2];
+  for (int w = 0; w < j.n; ++w) {
+    SideDim& a = j.d[w];
+    a.counts = counts.data() + std::size_t(w) * nv;
+    slot[w] = LOs(c, a.nl);
+    a.slot = slot[w].data();
+    a2ab[w] = LOs(c, nv + 1);
+    a.a2ab = a2ab[w].data();
+    // every lower entity in at most one row plus one spare slot per marked row
+    rows[w] = DArray<int4>(c, a.nl + nv);
+    a.rows = rows[w].data();
+    scans[w] = {a.counts, kScanLO, nv, a2ab[w].data(), nullptr};
+    uses[w] = a.nuses;
+    lows[w] = a.nl;
+    lanes[w] = std::int64_t(a.nuses) * kMatchLanes;
+  }
+  auto launch = [&](auto kernel, std::int64_t const* n, auto... args) {
+    unsigned b = side_blocks(j, n);
+    if (b == 0) return;
+    hipLaunchKernelGGL(kernel, dim3(b), dim3(kBlock), 0, c.stream, j, args...);
+    OSH_HIP(hipGetLastError());
+  };
+  launch(mark_use_min_verts, uses);
+  launch(count_min_rows, lows);
+  offset_scans(c, scans, j.n);
+  launch(fill_min_rows, lows);
+  launch(match_uses, lanes, c.error_word());
+}
+
+}  // namespace
+
 void reflect_down(Ctx& c, DMesh& m, int high_dim, LO nprods, LOs const& prod_verts,
-    LOs& down, Bytes& codes, LOs* found_out) {
+    LOs& down, Bytes& codes) {
   int low_dim = high_dim - 1;
   LO nuses = nprods * (high_dim + 1);
   down = LOs(c, nuses);
   codes = Bytes(c, nuses);
-  LOs found(c, nuses);
-  if (found_out) *found_out = found;
   if (nuses == 0) return;
-  LOs const& lv2v = verts_of(c, m, low_dim);
-  LO nv = m.nents[0];
-  LO nl = m.nents[low_dim];
-  LOs counts = fill_lo(c, nv, 0);
-  LOs slot(c, nl);
-  if (high_dim == 2) {
-    OSH_LAUNCH(mark_use_min_verts<2>, nuses, c, prod_verts.data(), counts.data(), found.data());
-    OSH_LAUNCH(count_min_rows<2>, nl, c, lv2v.data(), counts.data(), slot.data());
-  } else {
-    OSH_LAUNCH(mark_use_min_verts<3>, nuses, c, prod_verts.data(), counts.data(), found.data());
-    OSH_LAUNCH(count_min_rows<3>, nl, c, lv2v.data(), counts.data(), slot.data());
+  SideJobs j{};
+  j.n = 1;
+  j.high[0] = high_dim;
+  SideDim& a = j.d[0];
+  a.nuses = nuses;
+  a.pverts = prod_verts.data();
+  a.nl = m.nents[low_dim];
+  a.lv2v = verts_of(c, m, low_dim).data();
+  a.out = down.data();
+  a.codes = codes.data();
+  run_sides(c, m, j);
+}
+
+void match_sides(Ctx& c, DMesh& nw, Products const* prods, ModOut const* mo) {
+  SideJobs j{};
+  for (int d = 2; d <= nw.dim; ++d) {
+    if (prods[d].n == 0) continue;
+    j.high[j.n] = d;
+    SideDim& a = j.d[j.n++];
+    a.nuses = prods[d].n * (d + 1);
+    a.pverts = prods[d].verts.data();
+    a.prods2new = mo[d].prods2new.data();
+    a.nl = nw.nents[d - 1];
+    a.lv2v = verts_of(c, nw, d - 1).data();
+    a.out = nw.down[d].data();
+    a.codes = nw.down_codes[d].data();
   }
-  LOs a2ab = offset_scan(c, counts);
-  // every lower entity in at most one row plus one spare slot per marked row
-  DArray<int4> rows(c, nl + nv);
-  if (high_dim == 2) {
-    OSH_LAUNCH(fill_min_rows<2>, nl, c, lv2v.data(), a2ab.data(), slot.data(), rows.data());
-    OSH_LAUNCH(match_uses<2>, nuses * kMatchLanes, c, prod_verts.data(), a2ab.data(),
-        rows.data(), down.data(), codes.data(), found.data());
-  } else {
-    OSH_LAUNCH(fill_min_rows<3>, nl, c, lv2v.data(), a2ab.data(), slot.data(), rows.data());
-    OSH_LAUNCH(match_uses<3>, nuses * kMatchLanes, c, prod_verts.data(), a2ab.data(),
-        rows.data(), down.data(), codes.data(), found.data());
-  }
-  // a use without a unique match sets the context's error word, which the
-  // next stream sync raises; a caller that takes the match counts checks
-  // them where it reads the matches
-  if (!found_out)
-    OSH_LAUNCH(check_matches, nuses, c, found.data(), down.data(), codes.data(),
-        c.error_word());
+  if (j.n) run_sides(c, nw, j);
 }
 
 Adj const& ask_star(Ctx& c, DMesh& m, int d) {

@@ -1394,11 +1394,16 @@ int osh_reflect_down(osh_mesh* mesh, int high_dim, int nprods, const int* prod_v
     auto& c = mesh->owner->ctx;
     std::vector<int> h = host_copy(c, prod_verts, std::size_t(nprods) * (high_dim + 1));
     for (int v : h) OSH_CHECK(v >= 0 && v < mesh->m.nents[0], "vertex out of range");
-    osh::LOs d, found;
+    osh::LOs d;
     osh::Bytes cd;
-    osh::reflect_down(c, mesh->m, high_dim, nprods, osh::to_device(c, h), d, cd, &found);
-    std::vector<int> hf = osh::to_host(c, found);
-    for (int f : hf) OSH_CHECK(f == 1, "a side of a given simplex is not in the mesh");
+    osh::reflect_down(c, mesh->m, high_dim, nprods, osh::to_device(c, h), d, cd);
+    try {
+      c.sync();
+    } catch (osh::Error const& e) {
+      OSH_CHECK(std::string(e.what()) != osh::kNoMatchMessage,
+          "a side of a given simplex is not in the mesh");
+      throw;
+    }
     download(c, d, down);
     download(c, cd, reinterpret_cast<osh::I8*>(codes));
   });

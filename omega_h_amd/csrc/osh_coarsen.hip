@@ -439,26 +439,50 @@ __global__ void live_counts(LO nt, LO nkeys, LO const* keys2verts, LiveRows r) {
   if (n) atomicAdd(&r.counts[d][k], n);
 }
 
-__global__ void coarsen_products(LO nt, int nvd, LO const* keys2verts, LO const* keys2onto,
-    LO const* a2ab, LO const* ab2b, I8 const* codes, I8 const* dead, LO const* dv2v,
-    LO const* o2n, LO const* keys2prods, LO* pv, LO* psrc) {
+// the products of every dimension in one launch: a round of kLanes row entries
+// at a time, whose live ones take the next products in row order (a ballot
+// gives each its rank; counting the live entries before each one in the row
+// cost 28 us a launch on the 64^3 workload)
+struct CoarsenRows {
+  LO const* a2ab[3];
+  LO const* ab2b[3];
+  I8 const* codes[3];
+  I8 const* dead[3];
+  LO const* verts[3];
+  LO const* keys2prods[3];
+  LO* pv[3];
+  LO* psrc[3];
+};
+
+__global__ void coarsen_products(LO nt, LO nkeys, LO const* keys2verts, LO const* keys2onto,
+    LO const* vert_offsets, CoarsenRows r) {
   LO t = thread_index();
   if (t >= nt) return;
-  LO k = t / kLanes;
+  LO per = nkeys * kLanes;
+  int d = t / per;
+  LO k = (t % per) / kLanes;
   int lane = t % kLanes;
+  int base = int(threadIdx.x % 64) & ~(kLanes - 1);
+  int nvd = d + 2;
   LO v = keys2verts[k];
-  LO b = a2ab[v], e = a2ab[v + 1];
-  for (LO j = b + lane; j < e; j += kLanes) {
-    LO cell = ab2b[j];
-    if (dead[cell]) continue;
-    LO prod = keys2prods[k];
-    for (LO i = b; i < j; ++i) prod += !dead[ab2b[i]];
-    int ccv_col = code_which_down(codes[j]);
-    for (int ccv = 0; ccv < nvd; ++ccv) {
-      LO ov = (ccv == ccv_col) ? keys2onto[k] : dv2v[cell * nvd + ccv];
-      pv[prod * nvd + ccv] = o2n[ov];
+  LO onto = keys2onto[k];
+  LO e = r.a2ab[d][v + 1];
+  LO prod = r.keys2prods[d][k];
+  for (LO b = r.a2ab[d][v]; b < e; b += kLanes) {
+    LO j = b + lane;
+    LO cell = j < e ? r.ab2b[d][j] : 0;
+    bool live = j < e && !r.dead[d][cell];
+    unsigned mask = unsigned(__ballot(live) >> base) & ((1u << kLanes) - 1u);
+    if (live) {
+      LO p = prod + __popc(mask & ((1u << lane) - 1u));
+      int ccv_col = code_which_down(r.codes[d][j]);
+      for (int ccv = 0; ccv < nvd; ++ccv) {
+        LO ov = (ccv == ccv_col) ? onto : r.verts[d][std::size_t(cell) * nvd + ccv];
+        r.pv[d][std::size_t(p) * nvd + ccv] = vert_offsets[ov];
+      }
+      r.psrc[d][p] = cell;
     }
-    psrc[prod] = cell;
+    prod += __popc(mask);
   }
 }
 
@@ -867,11 +891,10 @@ bool coarsen(Ctx& c, DMesh& m, AdaptOptions const& o, Bytes& codes, bool oversho
   DMesh nw;
   nw.dim = dim;
   nw.metric_ncomps = nc;
-  LOs o2n, old_lows2new_lows;
   // products per key of every dimension, numbered by one scan launch
   LOs k2p[4];
   LO nprods[4] = {0, 0, 0, 0};
-  k2p[0] = fill_lo(c, nkeys + 1, 0);
+  k2p[0] = fill_lo(c, nkeys + 1, 0);  // no key vertex has a product vertex
   {
     LOs counts = fill_lo(c, dim * nkeys, 0);
     LiveRows rows{};
@@ -893,40 +916,38 @@ bool coarsen(Ctx& c, DMesh& m, AdaptOptions const& o, Bytes& codes, bool oversho
   ModPlan plans[4];
   modify_plans(c, m, 0, 0, dim, keys2verts, k2p, plans);
   modify_scan(c, plans, dim + 1);
-  for (int d = 0; d <= dim; ++d) {
-    LOs pv, psrc;
-    if (d > 0) {
-      pv = LOs(c, nprods[d] * (d + 1));
-      psrc = LOs(c, nprods[d]);
-      LOs const& dv2v = verts_of(c, m, d);
-      OSH_LAUNCH(coarsen_products, nkeys * kLanes, c, d + 1, keys2verts.data(), keys2onto.data(),
-          v2d[d].a2ab.data(), v2d[d].ab2b.data(), v2d[d].codes.data(), dead[d].data(),
-          dv2v.data(), o2n.data(), k2p[d].data(), pv.data(), psrc.data());
-    }
-    ModOut mo;
-    modify_build(c, m, nw, plans[d], keys2verts, k2p[d], nprods[d], pv, old_lows2new_lows, mo,
-        d > 0 ? &o2n : nullptr);
-    if (d == 0) {
-      o2n = mo.old2new;
-      nw.coords = transfer<Real>(c, mo, dim, m.coords, nullptr);
-      nw.metric = transfer<Real>(c, mo, nc, m.metric, nullptr);
-      for (auto const& t : m.vtags)
-        nw.vtags.push_back(t.with_data(transfer<Real>(c, mo, t.ncomps, t.data, nullptr)));
-      nw.itags = m.itags;
-      for (std::size_t t = 0; t < m.itags.size(); ++t)
-        nw.itags[t].data[0] = transfer<Real>(c, mo, m.itags[t].ncomps, m.itags[t].data[0], nullptr);
-      nw.class_id[0] = transfer<LO>(c, mo, 1, m.class_id[0], nullptr);
-      nw.class_dim[0] = transfer<I8>(c, mo, 1, m.class_dim[0], nullptr);
-    } else {
-      transfer_class(c, m, nw, d, mo, psrc, d, nullptr);
-      if (d == dim) {
-        transfer_pointwise(c, m, nw, mo, 0, keys2verts, k2p[d], pv);
-        conserve_pass(c, m, nw, 1, 0, keys2verts, k2p[d], mo);
-      }
-      transfer_measures(c, m, nw, d, mo);
-    }
-    old_lows2new_lows = mo.old2new;
+  ModOut mo[4];
+  rebuild_same(c, m, nw, 0, plans, mo);
+  Products prods[4];
+  CoarsenRows rows{};
+  for (int d = 1; d <= dim; ++d) {
+    Products& p = prods[d];
+    p.n = nprods[d];
+    p.keys2prods = k2p[d];
+    p.verts = LOs(c, p.n * (d + 1));
+    p.src = LOs(c, p.n);
+    p.src_dim = d;
+    rows.a2ab[d - 1] = v2d[d].a2ab.data();
+    rows.ab2b[d - 1] = v2d[d].ab2b.data();
+    rows.codes[d - 1] = v2d[d].codes.data();
+    rows.dead[d - 1] = dead[d].data();
+    rows.verts[d - 1] = verts_of(c, m, d).data();
+    rows.keys2prods[d - 1] = k2p[d].data();
+    rows.pv[d - 1] = p.verts.data();
+    rows.psrc[d - 1] = p.src.data();
   }
+  OSH_LAUNCH(coarsen_products, dim * nkeys * kLanes, c, nkeys, keys2verts.data(),
+      keys2onto.data(), plans[0].offsets.data(), rows);
+  place_products(c, m, nw, 1, dim, 0, plans, keys2verts, prods, mo);
+  match_sides(c, nw, prods, mo);
+  measure_products(c, nw, mo);
+  for (auto const& t : m.vtags)
+    nw.vtags.push_back(t.with_data(transfer<Real>(c, mo[0], t.ncomps, t.data, nullptr)));
+  for (std::size_t t = 0; t < m.itags.size(); ++t)
+    nw.itags[t].data[0] =
+        transfer<Real>(c, mo[0], m.itags[t].ncomps, m.itags[t].data[0], nullptr);
+  transfer_pointwise(c, m, nw, mo[dim], 0, keys2verts, k2p[dim], prods[dim].verts);
+  conserve_pass(c, m, nw, 1, 0, keys2verts, k2p[dim], mo[dim]);
   m = nw;
   return true;
 }

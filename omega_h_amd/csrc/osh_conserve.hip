@@ -608,18 +608,16 @@ __global__ void cavity_errors(LO nkeys, LO const* keys2kds, LO const* up_a2ab,
         new_cls, false, intro, carry, oq, nq, oerr, osize, nsize, nc, err, error);
 }
 
-// the new mesh's error array: same elements keep theirs, products start at 0
-__global__ void errors_start(LO n, LO nsame, int nc, LO const* same2old, LO const* same2new,
-    LO nprods, LO const* prods2new, Real const* oerr, Real* err) {
+// the new mesh's error array: surviving elements keep theirs, products start
+// at 0
+__global__ void errors_start(LO n, LO nold, int nc, LO const* old2new, LO const* prods2new,
+    Real const* oerr, Real* err) {
   LO i = thread_index();
   if (i >= n) return;
-  if (i < nsame) {
-    for (int q = 0; q < nc; ++q)
-      err[std::size_t(same2new[i]) * nc + q] = oerr[std::size_t(same2old[i]) * nc + q];
-  } else {
-    LO ne = prods2new[i - nsame];
-    for (int q = 0; q < nc; ++q) err[std::size_t(ne) * nc + q] = 0.0;
-  }
+  LO ne = i < nold ? old2new[i] : prods2new[i - nold];
+  if (ne < 0) return;
+  for (int q = 0; q < nc; ++q)
+    err[std::size_t(ne) * nc + q] = i < nold ? oerr[std::size_t(i) * nc + q] : 0.0;
 }
 
 // ------------------------------------------------------------- correction
@@ -776,8 +774,6 @@ Quantity<D, false> density_quantity(Real const* data, int nc) {
 template <int D>
 void pass_errors(Ctx& c, DMesh& old, DMesh& nw, LO nkeys, LOs const& keys2kds, Adj const& up,
     LOs const& k2p, ModOut const& mo, Bytes const& kinds, int op) {
-  LO nsame = mo.same2old.size();
-  LO nprods = mo.prods2new.size();
   Reals const& osize = ask_sizes(c, old);
   Reals const& nsize = ask_sizes(c, nw);
   // OpConservation (src/Omega_h_conserve.cpp:294-305): a density is always
@@ -794,8 +790,8 @@ void pass_errors(Ctx& c, DMesh& old, DMesh& nw, LO nkeys, LOs const& keys2kds, A
     auto& b = nw.etags[t];
     int nc = a.ncomps;
     Reals err(c, nw.nents[D] * nc);
-    OSH_LAUNCH(errors_start, nsame + nprods, c, nsame, nc, mo.same2old.data(),
-        mo.same2new.data(), nprods, mo.prods2new.data(), a.err.data(), err.data());
+    OSH_LAUNCH(errors_start, mo.nold + mo.nprods, c, mo.nold, nc, mo.old2new.data(),
+        mo.prods2new.data(), a.err.data(), err.data());
     OSH_LAUNCH((cavity_errors<D, false>), nkeys, c, keys2kds.data(), up.a2ab.data(),
         up.ab2b.data(), k2p.data(), mo.prods2new.data(), kinds.data(), old.class_id[D].data(),
         nw.class_id[D].data(), d_intro, d_carry, density_quantity<D>(a.data.data(), nc),
@@ -815,8 +811,8 @@ void pass_errors(Ctx& c, DMesh& old, DMesh& nw, LO nkeys, LOs const& keys2kds, A
     OSH_CHECK(orho && nrho, "momentum velocity without its density");
     int nc = a.ncomps;
     Reals err(c, nw.nents[D] * nc);
-    OSH_LAUNCH(errors_start, nsame + nprods, c, nsame, nc, mo.same2old.data(),
-        mo.same2new.data(), nprods, mo.prods2new.data(), a.err.data(), err.data());
+    OSH_LAUNCH(errors_start, mo.nold + mo.nprods, c, mo.nold, nc, mo.old2new.data(),
+        mo.prods2new.data(), a.err.data(), err.data());
     Quantity<D, true> oq{a.data.data(), orho->data.data(), oev2v.data(), nc};
     Quantity<D, true> nq{b.data.data(), nrho->data.data(), nev2v.data(), nc};
     OSH_LAUNCH((cavity_errors<D, true>), nkeys, c, keys2kds.data(), up.a2ab.data(),
@@ -831,7 +827,7 @@ template <int D>
 void pass_tmpl(Ctx& c, DMesh& old, DMesh& nw, int op, int key_dim, LOs const& keys2kds,
     LOs const& k2p, ModOut const& mo) {
   LO nkeys = keys2kds.size();
-  LO nprods = mo.prods2new.size();
+  LO nprods = mo.nprods;
   Adj const& up = ask_up(c, old, key_dim, D);
   LOs const& oev2v = verts_of(c, old, D);
   Bytes kinds(c, nkeys);

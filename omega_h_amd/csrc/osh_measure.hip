@@ -6,6 +6,7 @@
 //   get_mident_metrics    src/Omega_h_metric.cpp:56-104
 #include "osh_math.hpp"
 #include "osh_mesh.hpp"
+#include "osh_passes.hpp"
 
 namespace osh {
 
@@ -121,24 +122,21 @@ __global__ void elem_qualities32_kernel(LO n, LO const* ev2v, Real const* coords
   unsure[e] = u ? 1 : 0;
 }
 
-// the length (WHICH 1) or quality (WHICH 0) tag of a rebuilt mesh in one
-// launch: threads [0, nsame) copy the old value of a same entity, the rest
-// measure a product on the new mesh
-template <int WHICH, int D, int M>
-__global__ void __launch_bounds__(kBlock) measure_transfer_kernel(LO n, LO nsame,
-    LO const* same2old, LO const* same2new, Real const* old_vals, LO const* prods2new,
-    LO const* ev2v, Real const* coords, Real const* metric, Real* out) {
+// the lengths of new edges (threads [0, nl)) and the qualities of new elements
+// (the rest) of a rebuilt mesh in one launch
+template <int D, int M>
+__global__ void __launch_bounds__(kBlock) measure_products_kernel(LO n, LO nl, LO const* edges,
+    LO const* edge_verts, LO const* elems, LO const* elem_verts, Real const* coords,
+    Real const* metric, Real* lengths, Real* quals) {
   LO i = thread_index();
   if (i >= n) return;
-  if (i < nsame) {
-    out[same2new[i]] = old_vals[same2old[i]];
-    return;
+  if (i < nl) {
+    LO e = edges[i];
+    lengths[e] = length_of<D, M>(e, edge_verts, coords, metric);
+  } else {
+    LO e = elems[i - nl];
+    quals[e] = quality_of<D, M>(e, elem_verts, coords, metric);
   }
-  LO e = prods2new[i - nsame];
-  if constexpr (WHICH == 1)
-    out[e] = length_of<D, M>(e, ev2v, coords, metric);
-  else
-    out[e] = quality_of<D, M>(e, ev2v, coords, metric);
 }
 
 template <int M>
@@ -287,30 +285,26 @@ Reals const& ask_qualities(Ctx& c, DMesh& m) {
   return m.quality;
 }
 
-Reals measure_transfer(Ctx& c, DMesh& nw, int d, LO nsame, LO const* same2old,
-    LO const* same2new, Real const* old_vals, LO nprods, LO const* prods2new) {
-  OSH_CHECK(d == 1 || d == nw.dim, "lengths of edges or qualities of elements only");
-  Reals out(c, nw.nents[d]);
-  int md = metric_dim(nw);
-  LO const* ev2v = (d == 1) ? nw.down[1].data() : verts_of(c, nw, d).data();
-  check_alignment(nw.dim, md, d + 1, ev2v, nw.metric.data());
-  LO n = nsame + nprods;
-#define OSH_MT(W, D, M)                                                                    \
-  OSH_LAUNCH((measure_transfer_kernel<W, D, M>), n, c, nsame, same2old, same2new, old_vals, \
-      prods2new, ev2v, nw.coords.data(), nw.metric.data(), out.data())
-  if (d == 1) {
-    if (nw.dim == 3 && md == 3) OSH_MT(1, 3, 3);
-    else if (nw.dim == 3) OSH_MT(1, 3, 1);
-    else if (md == 2) OSH_MT(1, 2, 2);
-    else OSH_MT(1, 2, 1);
-  } else {
-    if (nw.dim == 3 && md == 3) OSH_MT(0, 3, 3);
-    else if (nw.dim == 3) OSH_MT(0, 3, 1);
-    else if (md == 2) OSH_MT(0, 2, 2);
-    else OSH_MT(0, 2, 1);
-  }
-#undef OSH_MT
-  return out;
+void measure_products(Ctx& c, DMesh& nw, ModOut const* mo) {
+  int md = metric_dim(nw), dim = nw.dim;
+  LO const* ev = nw.down[1].data();
+  LO const* tv = verts_of(c, nw, dim).data();
+  check_alignment(dim, md, 2, ev, nw.metric.data());
+  check_alignment(dim, md, dim + 1, tv, nw.metric.data());
+  LO nl = mo[1].nprods, n = nl + mo[dim].nprods;
+#define OSH_MP(D, M)                                                                        \
+  OSH_LAUNCH((measure_products_kernel<D, M>), n, c, nl, mo[1].prods2new.data(), ev,           \
+      mo[dim].prods2new.data(), tv, nw.coords.data(), nw.metric.data(), nw.length.data(),     \
+      nw.quality.data())
+  if (dim == 3 && md == 3)
+    OSH_MP(3, 3);
+  else if (dim == 3)
+    OSH_MP(3, 1);
+  else if (md == 2)
+    OSH_MP(2, 2);
+  else
+    OSH_MP(2, 1);
+#undef OSH_MP
 }
 
 void mident_values(Ctx& c, DMesh& m, LO n, LO const* edges, Real const* data, int ncomps,

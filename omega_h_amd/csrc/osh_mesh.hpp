@@ -137,11 +137,11 @@ Adj const& ask_dual(Ctx& c, DMesh& m);
 // volumes (measure_elements_real, src/Omega_h_shape.cpp:55-89)
 Reals const& ask_sizes(Ctx& c, DMesh& m);
 // vertex lists of new entities of dimension high_dim >= 2 matched against the
-// already-built dimension high_dim-1 of m (src/Omega_h_adj.cpp:424-441)
-// With found_out, the per-use match counts come back unchecked and the caller
-// must treat a use whose count is not 1 as an error (and not read its match).
+// already-built dimension high_dim-1 of m (src/Omega_h_adj.cpp:424-441); a use
+// without a unique match sets the context's error word, which the next wait
+// for the stream raises
 void reflect_down(Ctx& c, DMesh& m, int high_dim, LO nprods, LOs const& prod_verts,
-    LOs& down, Bytes& codes, LOs* found_out = nullptr);
+    LOs& down, Bytes& codes);
 // invert_adj (src/Omega_h_adj.cpp:231-263) of any high -> low map with deg
 // entries per high entity: rows sorted by high index, codes carrying the
 // down codes' flip and rotation and the use's position
@@ -173,10 +173,6 @@ void measure_edges(Ctx& c, DMesh& m, LO n, LO const* edges, Real* out);
 // metric was not clear marked in `unsure`
 void screen_estimates(Ctx& c, DMesh& m, Reals& lengths32, Reals& quals32, Bytes& unsure);
 void measure_elems(Ctx& c, DMesh& m, LO n, LO const* elems, Real* out);
-// the length (d = 1) or quality (d = dim) tag of a rebuilt mesh: same
-// entities copy old values, products are measured on the new mesh
-Reals measure_transfer(Ctx& c, DMesh& nw, int d, LO nsame, LO const* same2old,
-    LO const* same2new, Real const* old_vals, LO nprods, LO const* prods2new);
 Reals const& ask_lengths(Ctx& c, DMesh& m);
 Reals const& ask_qualities(Ctx& c, DMesh& m);
 void mident_metrics(Ctx& c, DMesh& m, LO n, LO const* edges, Real* out);

@@ -53,55 +53,6 @@ __global__ void mark_same_up_kernel(LO nt, I8 const* low_marks, SameUpJobs j) {
   j.counts[w][h] = r;
 }
 
-// new numbers of the old entities in one sweep: same entities take their
-// offset, the rest -1 (src/Omega_h_modify.cpp:141-161); the same entities
-// are also listed in order (collect_same) and, when `down` is given, write
-// their connectivity renumbered (modify_conn, :446-466; a null
-// old_lows2new_lows keeps the lower numbers) and, when `verts` is given,
-// their vertex list renumbered
-struct SameNumbering {
-  I8 const* same;
-  LO const* same_offsets;
-  LO const* offsets;
-  LO* same2old;
-  LO* same2new;
-  LO* old2new;
-  int deg;
-  LO const* old_down;
-  I8 const* old_codes;
-  LO const* old_lows2new_lows;
-  LO* down;
-  I8* codes;
-  int nvpe;
-  LO const* old_verts;
-  LO const* verts_old2new;
-  LO* verts;
-};
-
-__device__ __forceinline__ void number_same(LO o, SameNumbering const& a) {
-  if (a.same && !a.same[o]) {
-    a.old2new[o] = -1;
-    return;
-  }
-  LO s = a.same ? a.same_offsets[o] : o;
-  LO w = a.offsets[o];
-  a.same2old[s] = o;
-  a.same2new[s] = w;
-  a.old2new[o] = w;
-  int deg = a.deg;
-  if (a.down)
-    for (int j = 0; j < deg; ++j) {
-      LO l = a.old_down[o * deg + j];
-      a.down[w * deg + j] = a.old_lows2new_lows ? a.old_lows2new_lows[l] : l;
-      if (a.codes) a.codes[w * deg + j] = a.old_codes[o * deg + j];
-    }
-  if (a.verts)
-    for (int k = 0; k < a.nvpe; ++k) {
-      LO v = a.old_verts[o * a.nvpe + k];
-      a.verts[w * a.nvpe + k] = a.verts_old2new ? a.verts_old2new[v] : v;
-    }
-}
-
 // One sweep over the key-dimension entities starts the plans of every
 // dimension of a pass: no key marked, no entity above found yet, and (when
 // the key dimension itself is rebuilt) every entity the same, counting one.
@@ -204,6 +155,126 @@ __global__ void reps_masked(LO nt, LO nkd, I8 const* key_mask, MaskedReps j, int
   atomicAdd(&j.counts[w][r], j.prod_counts[w][kd]);
 }
 
+// a same entity's new number is its offset (assign_new_numbering,
+// src/Omega_h_modify.cpp:141-161), whatever its dimension, so one launch moves
+// the same entities of every dimension with all they carry: a lower entity's
+// or vertex's new number is read from its own dimension's offsets (a same
+// entity's lower entities are same entities).  Bound by memory: about 45 bytes
+// in and out per edge, 80 per face, 110 per tet; numbering, classification,
+// measures and swap choices in launches of their own, through lists of the
+// same entities, took 48 us where this takes 16 us (200,000 edges, 338,000
+// faces, 167,000 tets).
+struct SameDim {
+  int dim;
+  LO n;
+  I8 const* same;  // null: all are
+  LO const* offsets;
+  LO* old2new;
+  LO const* old_down;
+  I8 const* old_codes;
+  LO const* low_offsets;  // null: lower entities keep their numbers
+  LO* down;
+  I8* codes;
+  LO const* old_verts;
+  LO const* vert_offsets;
+  LO* verts;
+  LO const* old_ids;
+  I8 const* old_dims;
+  LO* ids;
+  I8* dims;
+  Real const* old_measure;
+  Real* measure;
+  // rows of reals (dimension 0: coordinates and metric)
+  Real const* old_rows[2];
+  Real* rows[2];
+  int ncomps[2];
+};
+
+struct SameCache {
+  I8 const* dirty;
+  I8 const* valid;
+  I8 const* cfg;
+  I8 const* keep;
+  Real const* q;
+  I8* n_valid;
+  I8* n_cfg;
+  I8* n_keep;
+  Real* n_q;
+};
+
+// job w owns the workgroups [first[w], first[w + 1]), so that every branch on
+// the dimension is uniform
+struct SameJobs {
+  int n;
+  unsigned first[5];
+  SameDim d[4];
+  SameCache cache;  // of the edges, when cache.valid
+};
+
+__device__ __forceinline__ LO renumber(LO const* offsets, LO l) {
+  return offsets ? offsets[l] : l;
+}
+
+__global__ void __launch_bounds__(kBlock) rebuild_same_kernel(SameJobs j) {
+  int w = 0;
+  while (w + 1 < j.n && blockIdx.x >= j.first[w + 1]) ++w;
+  SameDim const& a = j.d[w];
+  LO o = LO(blockIdx.x - j.first[w]) * kBlock + LO(threadIdx.x);
+  if (o >= a.n) return;
+  bool keep = !a.same || a.same[o];
+  LO x = a.offsets[o];
+  if (a.old2new) a.old2new[o] = keep ? x : -1;
+  if (!keep) return;
+  a.ids[x] = a.old_ids[o];
+  a.dims[x] = a.old_dims[o];
+  if (a.measure) a.measure[x] = a.old_measure[o];
+  if (a.dim == 0) {
+    for (int r = 0; r < 2; ++r)
+      for (int k = 0; k < a.ncomps[r]; ++k)
+        a.rows[r][std::size_t(x) * a.ncomps[r] + k] = a.old_rows[r][std::size_t(o) * a.ncomps[r] + k];
+  } else if (a.dim == 1) {
+    int2 v = reinterpret_cast<int2 const*>(a.old_down)[o];
+    reinterpret_cast<int2*>(a.down)[x] =
+        make_int2(renumber(a.low_offsets, v.x), renumber(a.low_offsets, v.y));
+    if (j.cache.valid) {
+      bool ok = j.cache.valid[o] && !j.cache.dirty[o];
+      j.cache.n_valid[x] = I8(ok);
+      if (ok) {
+        j.cache.n_cfg[x] = j.cache.cfg[o];
+        j.cache.n_keep[x] = j.cache.keep[o];
+        j.cache.n_q[x] = j.cache.q[o];
+      }
+    }
+  } else if (a.dim == 2) {
+    std::size_t so = std::size_t(o) * 3, sx = std::size_t(x) * 3;
+    LO l[3], v[3];
+    I8 c[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      l[k] = a.old_down[so + k];
+      v[k] = a.old_verts[so + k];
+      c[k] = a.old_codes[so + k];
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      a.down[sx + k] = renumber(a.low_offsets, l[k]);
+      a.verts[sx + k] = renumber(a.vert_offsets, v[k]);
+      a.codes[sx + k] = c[k];
+    }
+  } else {
+    int4 l = reinterpret_cast<int4 const*>(a.old_down)[o];
+    int4 v = reinterpret_cast<int4 const*>(a.old_verts)[o];
+    reinterpret_cast<int4*>(a.down)[x] =
+        make_int4(renumber(a.low_offsets, l.x), renumber(a.low_offsets, l.y),
+            renumber(a.low_offsets, l.z), renumber(a.low_offsets, l.w));
+    reinterpret_cast<int4*>(a.verts)[x] =
+        make_int4(renumber(a.vert_offsets, v.x), renumber(a.vert_offsets, v.y),
+            renumber(a.vert_offsets, v.z), renumber(a.vert_offsets, v.w));
+    // the four codes are one word
+    reinterpret_cast<int*>(a.codes)[x] = reinterpret_cast<int const*>(a.old_codes)[o];
+  }
+}
+
 __global__ void scatter_index(LO n, LO const* a2b, LO* b2a) {
   LO i = thread_index();
   if (i < n) b2a[a2b[i]] = i;
@@ -225,107 +296,80 @@ __global__ void rep2md_order_kernel(LO nreps, LO const* a2ab, LO const* ab2b, I8
 }
 
 // the products' new numbers, following their representative
-// (src/Omega_h_modify.cpp:141-161), with their connectivity (modify_conn),
-// their vertex lists and the entity each came from when those are asked for.
-// A key's products take consecutive numbers, so kProdLanes threads per key
-// share its products without talking to each other.
+// (src/Omega_h_modify.cpp:141-161), with their vertex lists and their
+// classification, inherited from the entity each came from
+// (src/Omega_h_transfer.cpp:20-34,212-267).  A key's products take
+// consecutive numbers, so kProdLanes threads per key and dimension share them
+// without talking to each other.
 constexpr int kProdLanes = 8;
 
-struct ProdNumbering {
+struct PlaceDim {
   LO const* reps;
-  LO const* keys2kds;
   LO const* offsets;
-  LO const* order;
+  LO const* order;  // products sit after their representative, in this order
   LO const* keys2prods;
   LO* prods2new;
-  int deg;
-  LO const* pdown;
-  I8 const* pcodes;
-  LO const* found;
-  LO* down;
-  I8* codes;
-  int nvpe;
+  int nverts;  // 0 for vertices
   LO const* pverts;
   LO* verts;
-  LO const* key_src;
-  LO* src;
-  int* error;
+  LO const* src;  // null: the key
+  int src_dim;
+  I8 const* src_dims;
+  LO const* ids_a;
+  I8 const* dims_a;
+  LO const* ids_b;
+  I8 const* dims_b;
+  LO* ids;
+  I8* dims;
+  LO* src_out;
+  I8* zeroed;
 };
 
-__device__ __forceinline__ void number_prods(LO t, ProdNumbering const& a) {
-  LO k = t / kProdLanes;
+struct PlaceJobs {
+  LO const* keys2kds;
+  PlaceDim d[4];
+};
+
+__global__ void __launch_bounds__(kBlock) place_products_kernel(LO nt, LO nkeys, PlaceJobs j) {
+  LO t = thread_index();
+  if (t >= nt) return;
+  LO per = nkeys * kProdLanes;
+  PlaceDim const& a = j.d[t / per];
+  LO k = (t % per) / kProdLanes;
   int lane = t % kProdLanes;
   LO first = a.keys2prods[k];
+  LO end = a.keys2prods[k + 1];
+  LO key = j.keys2kds[k];
   LO base = a.offsets[a.reps[k]];
-  if (a.order) base += a.order[a.keys2kds[k]] + 1;
-  int deg = a.deg;
-  for (LO p = first + lane; p < a.keys2prods[k + 1]; p += kProdLanes) {
+  if (a.order) base += a.order[key] + 1;
+  for (LO p = first + lane; p < end; p += kProdLanes) {
     LO w = base + (p - first);
     a.prods2new[p] = w;
-    if (a.down)
-      for (int j = 0; j < deg; ++j) {
-        // a side matched by reflect_down must have matched exactly once; an
-        // error keeps the index in range until the host sees it
-        bool ok = !a.found || a.found[p * deg + j] == 1;
-        if (!ok) *a.error = kReflectDownNoMatch;
-        a.down[w * deg + j] = ok ? a.pdown[p * deg + j] : 0;
-        if (a.codes) a.codes[w * deg + j] = ok ? a.pcodes[p * deg + j] : I8(0);
-      }
-    if (a.verts)
-      for (int j = 0; j < a.nvpe; ++j) a.verts[w * a.nvpe + j] = a.pverts[p * a.nvpe + j];
-    if (a.src) a.src[p] = a.key_src[k];
+    for (int v = 0; v < a.nverts; ++v)
+      a.verts[std::size_t(w) * a.nverts + v] = a.pverts[std::size_t(p) * a.nverts + v];
+    LO s = a.src ? a.src[p] : key;
+    bool second = a.src_dims && a.src_dims[p] != a.src_dim;
+    a.ids[w] = second ? a.ids_b[s] : a.ids_a[s];
+    a.dims[w] = second ? a.dims_b[s] : a.dims_a[s];
+    if (a.src_out) a.src_out[p] = s;
+    if (a.zeroed) a.zeroed[w] = 0;
   }
 }
 
-// the new numbers of one dimension in one launch: threads [0, nold) number
-// the old entities (same ones keep their order), the rest (kProdLanes per
-// key) the products; the two halves write disjoint entries
-__global__ void number_entities(LO n, LO nold, SameNumbering same, ProdNumbering prods) {
-  LO t = thread_index();
-  if (t >= n) return;
-  if (t < nold)
-    number_same(t, same);
-  else
-    number_prods(t - nold, prods);
-}
-
-// one launch for a transferred tag: threads [0, nsame) copy same entities,
-// the rest place the products' values (src/Omega_h_transfer.cpp:631-653)
+// one launch for a transferred tag: threads [0, nold) copy the old entities
+// that survive, the rest place the products' values
+// (src/Omega_h_transfer.cpp:631-653)
 template <class T>
-__global__ void scatter_data(LO n, LO nsame, int nc, LO const* same2old, LO const* same2new,
-    T const* old_data, LO const* prods2new, T const* pdata, T* data) {
+__global__ void scatter_data(LO n, LO nold, int nc, LO const* old2new, T const* old_data,
+    LO const* prods2new, T const* pdata, T* data) {
   LO i = thread_index();
   if (i >= n) return;
-  if (i < nsame) {
-    for (int k = 0; k < nc; ++k) data[same2new[i] * nc + k] = old_data[same2old[i] * nc + k];
-  } else {
-    LO p = i - nsame;
-    for (int k = 0; k < nc; ++k) data[prods2new[p] * nc + k] = pdata[p * nc + k];
-  }
-}
-
-// class_id and class_dim of the new entities in one launch: same entities
-// copy theirs, products inherit from their source entity of dimension
-// src_dims[p] (or src_dim), src/Omega_h_transfer.cpp:20-34,212-267
-__global__ void transfer_class_kernel(LO n, LO nsame, LO const* same2old, LO const* same2new,
-    LO const* old_ids, I8 const* old_dims, LO const* prods2new, LO const* src, int src_dim,
-    I8 const* src_dims, LO const* ids_a, I8 const* dims_a, LO const* ids_b, I8 const* dims_b,
-    LO* ids, I8* dims) {
-  LO i = thread_index();
-  if (i >= n) return;
-  if (i < nsame) {
-    LO o = same2old[i], w = same2new[i];
-    ids[w] = old_ids[o];
-    dims[w] = old_dims[o];
-    return;
-  }
-  LO p = i - nsame;
-  int sd = src_dims ? src_dims[p] : src_dim;
-  bool second = (sd != src_dim);
-  LO s = src[p];
-  LO w = prods2new[p];
-  ids[w] = second ? ids_b[s] : ids_a[s];
-  dims[w] = second ? dims_b[s] : dims_a[s];
+  bool prod = i >= nold;
+  LO p = i - nold;
+  LO w = prod ? prods2new[p] : old2new[i];
+  if (w < 0) return;
+  T const* from = prod ? pdata + std::size_t(p) * nc : old_data + std::size_t(i) * nc;
+  for (int k = 0; k < nc; ++k) data[std::size_t(w) * nc + k] = from[k];
 }
 
 // row p of out = row src[p] of in
@@ -405,23 +449,26 @@ __global__ void pointwise_kernel(LO nt, int lshift, LO nkeys, LO const* keys2kds
     best[p] = row < end ? up_ab2b[(nan || pos == 0x7fffffff) ? row : pos] : -1;
 }
 
-// an inheritance tag of the new entities, by the same sources as
-// transfer_class_kernel
-__global__ void inherit_kernel(LO n, LO nsame, int nc, LO const* same2old, LO const* same2new,
-    Real const* old_vals, LO const* prods2new, LO const* src, int src_dim, I8 const* src_dims,
-    Real const* vals_a, Real const* vals_b, Real* out) {
+// an inheritance tag of the new entities: survivors keep theirs, products
+// inherit as they do their classification
+__global__ void inherit_kernel(LO n, LO nold, int nc, LO const* old2new, Real const* old_vals,
+    LO const* prods2new, LO const* src, int src_dim, I8 const* src_dims, Real const* vals_a,
+    Real const* vals_b, Real* out) {
   LO i = thread_index();
   if (i >= n) return;
-  if (i < nsame) {
-    for (int k = 0; k < nc; ++k) out[same2new[i] * nc + k] = old_vals[same2old[i] * nc + k];
+  if (i < nold) {
+    LO w = old2new[i];
+    if (w < 0) return;
+    for (int k = 0; k < nc; ++k)
+      out[std::size_t(w) * nc + k] = old_vals[std::size_t(i) * nc + k];
     return;
   }
-  LO p = i - nsame;
+  LO p = i - nold;
   int sd = src_dims ? src_dims[p] : src_dim;
   Real const* from = (sd != src_dim) ? vals_b : vals_a;
   LO s = src[p];
   LO w = prods2new[p];
-  for (int k = 0; k < nc; ++k) out[w * nc + k] = from[s * nc + k];
+  for (int k = 0; k < nc; ++k) out[std::size_t(w) * nc + k] = from[std::size_t(s) * nc + k];
 }
 
 // one round of indset::find (src/Omega_h_indset.cpp:5-35).  In the first
@@ -772,32 +819,21 @@ void modify_plans_masked(Ctx& c, DMesh& old, int key_dim, int d1, Bytes const& k
 }
 
 int modify_scan_jobs(Ctx& c, ModPlan* plans, int nplans, ScanJob* jobs, int first_slot) {
-  int njobs = 0;
   for (int i = 0; i < nplans; ++i) {
     ModPlan& p = plans[i];
     p.offsets = LOs(c, p.nold + 1);
-    jobs[njobs++] = {p.counts.data(), kScanLO, p.nold, p.offsets.data(),
-        slot_ptr<LO>(c, first_slot + 2 * i)};
-    if (p.same.exists()) {
-      p.same_offsets = LOs(c, p.nold + 1);
-      jobs[njobs++] = {p.same.data(), kScanNonzero, p.nold, p.same_offsets.data(),
-          slot_ptr<LO>(c, first_slot + 2 * i + 1)};
-    }
+    jobs[i] = {p.counts.data(), kScanLO, p.nold, p.offsets.data(),
+        slot_ptr<LO>(c, first_slot + i)};
   }
-  return njobs;
+  return nplans;
 }
 
 void modify_scan_totals(Ctx& c, ModPlan* plans, int nplans, int first_slot) {
-  for (int i = 0; i < nplans; ++i) {
-    plans[i].nnew = read_slot<LO>(c, first_slot + 2 * i);
-    plans[i].nsame = plans[i].same.exists() ? read_slot<LO>(c, first_slot + 2 * i + 1)
-                                             : plans[i].nold;
-  }
+  for (int i = 0; i < nplans; ++i) plans[i].nnew = read_slot<LO>(c, first_slot + i);
 }
 
 void modify_scan(Ctx& c, ModPlan* plans, int nplans) {
-  OSH_CHECK(nplans >= 1 && 2 * nplans <= kMaxScanJobs && 2 * nplans < Ctx::kSlots,
-      "modify_scan: too many dimensions");
+  OSH_CHECK(nplans >= 1 && nplans <= 4, "modify_scan: too many dimensions");
   ScanJob jobs[kMaxScanJobs];
   int njobs = modify_scan_jobs(c, plans, nplans, jobs, 1);
   offset_scans(c, jobs, njobs);
@@ -805,113 +841,173 @@ void modify_scan(Ctx& c, ModPlan* plans, int nplans) {
   modify_scan_totals(c, plans, nplans, 1);
 }
 
-void modify_build(Ctx& c, DMesh& old, DMesh& nw, ModPlan const& plan, LOs const& keys2kds,
-    LOs const& keys2prods, LO nprods, LOs const& prod_verts, LOs const& old_lows2new_lows,
-    ModOut& out, LOs const* verts_old2new, LOs* prod_src, LOs const* given_down,
-    Bytes const* given_codes) {
-  int ent_dim = plan.ent_dim, key_dim = plan.key_dim;
-  LO nkeys = keys2kds.size();
-  LO nold = plan.nold;
-  LO nsame = plan.nsame;
-  Bytes const& same = plan.same;
-  out.nnew = plan.nnew;
-  LO nnew = out.nnew;
-  out.same2old = LOs(c, nsame);
-  out.same2new = LOs(c, nsame);
-  out.old2new = LOs(c, nold);
-  out.prods2new = LOs(c, nprods);
-  LOs order;
-  if (key_dim > ent_dim) {
-    LO nkd = old.nents[key_dim];
-    order = fill_lo(c, nkd, -1);
-    LOs md2mod = fill_lo(c, nkd, -1);
-    OSH_LAUNCH(scatter_index, nkeys, c, keys2kds.data(), md2mod.data());
-    Adj const& up = ask_up(c, old, ent_dim, key_dim);
-    OSH_LAUNCH(rep2md_order_kernel, nold, c, up.a2ab.data(), up.ab2b.data(), up.codes.data(),
-        md2mod.data(), keys2prods.data(), order.data());
-  }
-  int deg = ent_dim + 1;
-  bool with_codes = ent_dim >= 2;
-  LOs down;
-  Bytes codes;
-  LOs pdown, found;
-  Bytes pcodes;
-  // the vertex lists of new faces and elements come with the numbering
-  // (those of same entities renumbered, those of products as built), so the
-  // new mesh does not derive them again
-  LOs verts;
-  LO const* old_verts = nullptr;
-  if (ent_dim >= 1) {
-    down = LOs(c, nnew * deg);
-    if (with_codes) {
-      codes = Bytes(c, nnew * deg);
-      // a caller that knows where the products' sides are hands them over
-      if (given_down) {
-        pdown = *given_down;
-        pcodes = *given_codes;
-      } else {
-        reflect_down(c, nw, ent_dim, nprods, prod_verts, pdown, pcodes, &found);
-      }
-      verts = LOs(c, nnew * deg);
-      old_verts = verts_of(c, old, ent_dim).data();
+bool has_tags(DMesh const& m) {
+  return !m.vtags.empty() || !m.itags.empty() || !m.etags.empty();
+}
+
+void rebuild_same(Ctx& c, DMesh& old, DMesh& nw, int d0, ModPlan const* plans, ModOut* mo,
+    CacheMove const* cache) {
+  int dim = old.dim;
+  bool tags = has_tags(old);
+  SameJobs j{};
+  unsigned blocks = 0;
+  for (int d = d0; d <= dim; ++d) {
+    ModPlan const& p = plans[d - d0];
+    LO nnew = p.nnew;
+    int deg = d + 1;
+    mo[d].nold = p.nold;
+    mo[d].nnew = nnew;
+    nw.nents[d] = nnew;
+    SameDim& a = j.d[j.n];
+    a.dim = d;
+    a.n = p.nold;
+    a.same = p.same.exists() ? p.same.data() : nullptr;
+    a.offsets = p.offsets.data();
+    if (tags) {
+      mo[d].old2new = LOs(c, p.nold);
+      a.old2new = mo[d].old2new.data();
+    }
+    nw.class_id[d] = LOs(c, nnew);
+    nw.class_dim[d] = Bytes(c, nnew);
+    a.old_ids = old.class_id[d].data();
+    a.old_dims = old.class_dim[d].data();
+    a.ids = nw.class_id[d].data();
+    a.dims = nw.class_dim[d].data();
+    if (d == 0) {
+      nw.coords = Reals(c, nnew * dim);
+      nw.metric = Reals(c, nnew * old.metric_ncomps);
+      a.old_rows[0] = old.coords.data();
+      a.old_rows[1] = old.metric.data();
+      a.rows[0] = nw.coords.data();
+      a.rows[1] = nw.metric.data();
+      a.ncomps[0] = dim;
+      a.ncomps[1] = old.metric_ncomps;
     } else {
-      pdown = prod_verts;
+      nw.down[d] = LOs(c, nnew * deg);
+      a.old_down = old.down[d].data();
+      a.down = nw.down[d].data();
+      a.low_offsets = d > d0 ? plans[d - 1 - d0].offsets.data() : nullptr;
+    }
+    if (d >= 2) {
+      nw.down_codes[d] = Bytes(c, nnew * deg);
+      nw.verts[d] = LOs(c, nnew * deg);
+      a.old_codes = old.down_codes[d].data();
+      a.codes = nw.down_codes[d].data();
+      a.old_verts = verts_of(c, old, d).data();
+      a.verts = nw.verts[d].data();
+      a.vert_offsets = d0 == 0 ? plans[0].offsets.data() : nullptr;
+    }
+    if (d == 1) {
+      nw.length = Reals(c, nnew);
+      a.old_measure = ask_lengths(c, old).data();
+      a.measure = nw.length.data();
+    }
+    if (d == dim) {
+      nw.quality = Reals(c, nnew);
+      a.old_measure = ask_qualities(c, old).data();
+      a.measure = nw.quality.data();
+    }
+    j.first[j.n] = blocks;
+    blocks += nblocks(p.nold);
+    ++j.n;
+    j.first[j.n] = blocks;
+  }
+  if (cache) {
+    LO nnew = nw.nents[1];
+    cache->to->valid = Bytes(c, nnew);
+    cache->to->cfg = Bytes(c, nnew);
+    cache->to->keep = Bytes(c, nnew);
+    cache->to->q = Reals(c, nnew);
+    j.cache = SameCache{cache->dirty->data(), cache->from->valid.data(),
+        cache->from->cfg.data(), cache->from->keep.data(), cache->from->q.data(),
+        cache->to->valid.data(), cache->to->cfg.data(), cache->to->keep.data(),
+        cache->to->q.data()};
+  }
+  if (blocks == 0) return;
+  hipLaunchKernelGGL(rebuild_same_kernel, dim3(blocks), dim3(kBlock), 0, c.stream, j);
+  OSH_HIP(hipGetLastError());
+}
+
+void place_products(Ctx& c, DMesh& old, DMesh& nw, int d0, int d1, int plan0,
+    ModPlan const* plans, LOs const& keys2kds, Products const* prods, ModOut* mo,
+    I8* new_edges_valid) {
+  LO nkeys = keys2kds.size();
+  PlaceJobs j{};
+  j.keys2kds = keys2kds.data();
+  LOs src[4];
+  LOs order;
+  for (int d = d0; d <= d1; ++d) {
+    ModPlan const& plan = plans[d - plan0];
+    Products const& p = prods[d];
+    PlaceDim& a = j.d[d - d0];
+    mo[d].nprods = p.n;
+    mo[d].prods2new = LOs(c, p.n);
+    if (plan.key_dim > d) {
+      OSH_CHECK(!order.exists(), "one dimension below the keys");
+      LO nkd = old.nents[plan.key_dim];
+      order = fill_lo(c, nkd, -1);
+      LOs md2mod = fill_lo(c, nkd, -1);
+      OSH_LAUNCH(scatter_index, nkeys, c, keys2kds.data(), md2mod.data());
+      Adj const& up = ask_up(c, old, d, plan.key_dim);
+      OSH_LAUNCH(rep2md_order_kernel, plan.nold, c, up.a2ab.data(), up.ab2b.data(),
+          up.codes.data(), md2mod.data(), p.keys2prods.data(), order.data());
+      a.order = order.data();
+    }
+    a.reps = plan.reps.data();
+    a.offsets = plan.offsets.data();
+    a.keys2prods = p.keys2prods.data();
+    a.prods2new = mo[d].prods2new.data();
+    if (d >= 1) {
+      a.nverts = d + 1;
+      a.pverts = p.verts.data();
+      a.verts = d == 1 ? nw.down[1].data() : nw.verts[d].data();
+    }
+    int sd = p.src_dim;
+    int other = (p.src_dims.exists() && sd + 1 <= old.dim) ? sd + 1 : sd;
+    a.src = p.src.exists() ? p.src.data() : nullptr;
+    a.src_dim = sd;
+    a.src_dims = p.src_dims.exists() ? p.src_dims.data() : nullptr;
+    a.ids_a = old.class_id[sd].data();
+    a.dims_a = old.class_dim[sd].data();
+    a.ids_b = old.class_id[other].data();
+    a.dims_b = old.class_dim[other].data();
+    a.ids = nw.class_id[d].data();
+    a.dims = nw.class_dim[d].data();
+    if (!old.itags.empty()) {
+      src[d] = LOs(c, p.n);
+      a.src_out = src[d].data();
+    }
+    if (d == 1) a.zeroed = new_edges_valid;
+  }
+  int nd = d1 - d0 + 1;
+  OSH_CHECK(std::int64_t(nkeys) * kProdLanes * nd <= std::int64_t(0x7fffffff),
+      "place_products: too many keys");
+  OSH_LAUNCH(place_products_kernel, nkeys * kProdLanes * nd, c, nkeys, j);
+  if (nw.itags.size() != old.itags.size()) nw.itags = old.itags;
+  for (int d = d0; d <= d1; ++d) {
+    Products const& p = prods[d];
+    int sd = p.src_dim;
+    int other = (p.src_dims.exists() && sd + 1 <= old.dim) ? sd + 1 : sd;
+    for (std::size_t t = 0; t < old.itags.size(); ++t) {
+      auto const& a = old.itags[t];
+      Reals out(c, mo[d].nnew * a.ncomps);
+      OSH_LAUNCH(inherit_kernel, mo[d].nold + p.n, c, mo[d].nold, a.ncomps,
+          mo[d].old2new.data(), a.data[d].data(), mo[d].prods2new.data(), src[d].data(), sd,
+          p.src_dims.exists() ? p.src_dims.data() : (I8 const*)nullptr, a.data[sd].data(),
+          a.data[other].data(), out.data());
+      nw.itags[t].data[d] = out;
     }
   }
-  if (prod_src) *prod_src = LOs(c, nprods);
-  SameNumbering sn;
-  sn.same = same.exists() ? same.data() : (I8 const*)nullptr;
-  sn.same_offsets = same.exists() ? plan.same_offsets.data() : (LO const*)nullptr;
-  sn.offsets = plan.offsets.data();
-  sn.same2old = out.same2old.data();
-  sn.same2new = out.same2new.data();
-  sn.old2new = out.old2new.data();
-  sn.deg = deg;
-  sn.old_down = ent_dim >= 1 ? old.down[ent_dim].data() : (LO const*)nullptr;
-  sn.old_codes = with_codes ? old.down_codes[ent_dim].data() : (I8 const*)nullptr;
-  sn.old_lows2new_lows = ent_dim >= 1 ? old_lows2new_lows.data() : (LO const*)nullptr;
-  sn.down = ent_dim >= 1 ? down.data() : (LO*)nullptr;
-  sn.codes = with_codes ? codes.data() : (I8*)nullptr;
-  sn.nvpe = deg;
-  sn.old_verts = old_verts;
-  sn.verts_old2new = verts_old2new ? verts_old2new->data() : (LO const*)nullptr;
-  sn.verts = verts.exists() ? verts.data() : (LO*)nullptr;
-  ProdNumbering pn;
-  pn.reps = plan.reps.data();
-  pn.keys2kds = keys2kds.data();
-  pn.offsets = plan.offsets.data();
-  pn.order = order.exists() ? order.data() : (LO const*)nullptr;
-  pn.keys2prods = keys2prods.data();
-  pn.prods2new = out.prods2new.data();
-  pn.deg = deg;
-  pn.pdown = ent_dim >= 1 ? pdown.data() : (LO const*)nullptr;
-  pn.pcodes = with_codes ? pcodes.data() : (I8 const*)nullptr;
-  pn.found = with_codes ? found.data() : (LO const*)nullptr;
-  pn.down = ent_dim >= 1 ? down.data() : (LO*)nullptr;
-  pn.codes = with_codes ? codes.data() : (I8*)nullptr;
-  pn.nvpe = deg;
-  pn.pverts = verts.exists() ? prod_verts.data() : (LO const*)nullptr;
-  pn.verts = verts.exists() ? verts.data() : (LO*)nullptr;
-  pn.key_src = keys2kds.data();
-  pn.src = prod_src ? prod_src->data() : (LO*)nullptr;
-  pn.error = c.error_word();
-  OSH_LAUNCH(number_entities, nold + nkeys * kProdLanes, c, nold, sn, pn);
-  nw.nents[ent_dim] = nnew;
-  if (ent_dim == 0) return;
-  nw.down[ent_dim] = down;
-  nw.down_codes[ent_dim] = codes;
-  if (verts.exists()) nw.verts[ent_dim] = verts;
 }
 
 template <class T>
 DArray<T> transfer(Ctx& c, ModOut const& mo, int nc, DArray<T> const& old_data,
     DArray<T> const* prod_data) {
   DArray<T> d(c, mo.nnew * nc);
-  LO nsame = mo.same2old.size();
-  LO nprods = prod_data ? mo.prods2new.size() : 0;
-  OSH_LAUNCH(scatter_data<T>, nsame + nprods, c, nsame, nc, mo.same2old.data(),
-      mo.same2new.data(), old_data.data(), mo.prods2new.data(),
-      prod_data ? prod_data->data() : (T const*)nullptr, d.data());
+  LO nprods = prod_data ? mo.nprods : 0;
+  OSH_LAUNCH(scatter_data<T>, mo.nold + nprods, c, mo.nold, nc, mo.old2new.data(),
+      old_data.data(), mo.prods2new.data(), prod_data ? prod_data->data() : (T const*)nullptr,
+      d.data());
   return d;
 }
 
@@ -919,37 +1015,10 @@ template DArray<LO> transfer(Ctx&, ModOut const&, int, DArray<LO> const&, DArray
 template DArray<I8> transfer(Ctx&, ModOut const&, int, DArray<I8> const&, DArray<I8> const*);
 template DArray<Real> transfer(Ctx&, ModOut const&, int, DArray<Real> const&, DArray<Real> const*);
 
-void transfer_class(Ctx& c, DMesh& old, DMesh& nw, int d, ModOut const& mo,
-    LOs const& prod_src, int src_dim, Bytes const* src_dims) {
-  LO nprods = mo.prods2new.size();
-  LO nsame = mo.same2old.size();
-  int other = (src_dims && src_dim + 1 <= old.dim) ? src_dim + 1 : src_dim;
-  LOs ids(c, mo.nnew);
-  Bytes dims(c, mo.nnew);
-  OSH_LAUNCH(transfer_class_kernel, nsame + nprods, c, nsame, mo.same2old.data(),
-      mo.same2new.data(), old.class_id[d].data(), old.class_dim[d].data(),
-      mo.prods2new.data(), prod_src.data(), src_dim,
-      src_dims ? src_dims->data() : (I8 const*)nullptr, old.class_id[src_dim].data(),
-      old.class_dim[src_dim].data(), old.class_id[other].data(), old.class_dim[other].data(),
-      ids.data(), dims.data());
-  nw.class_id[d] = ids;
-  nw.class_dim[d] = dims;
-  if (nw.itags.size() != old.itags.size()) nw.itags = old.itags;
-  for (std::size_t t = 0; t < old.itags.size(); ++t) {
-    auto const& a = old.itags[t];
-    Reals out(c, mo.nnew * a.ncomps);
-    OSH_LAUNCH(inherit_kernel, nsame + nprods, c, nsame, a.ncomps, mo.same2old.data(),
-        mo.same2new.data(), a.data[d].data(), mo.prods2new.data(), prod_src.data(), src_dim,
-        src_dims ? src_dims->data() : (I8 const*)nullptr, a.data[src_dim].data(),
-        a.data[other].data(), out.data());
-    nw.itags[t].data[d] = out;
-  }
-}
-
 void transfer_elem_tags(Ctx& c, DMesh const& old, DMesh& nw, ModOut const& mo,
     LOs const* prod_src) {
   nw.etags.clear();
-  LO nprods = mo.prods2new.size();
+  LO nprods = mo.nprods;
   for (auto const& t : old.etags) {
     Reals pd;
     if (prod_src) {
@@ -968,7 +1037,7 @@ void transfer_pointwise(Ctx& c, DMesh& old, DMesh& nw, ModOut const& mo, int key
   LO nkeys = keys2kds.size();
   Adj const& up = ask_up(c, old, key_dim, dim);
   LOs const& ev2v = verts_of(c, old, dim);
-  LO nprods = mo.prods2new.size();
+  LO nprods = mo.nprods;
   int lanes = fit_lanes(nprods, kPointLanes);
   int lshift = lanes_shift(lanes);
   LOs best(c, nprods);
@@ -983,17 +1052,6 @@ void transfer_pointwise(Ctx& c, DMesh& old, DMesh& nw, ModOut const& mo, int key
         up.a2ab.data(), up.ab2b.data(), ev2v.data(), old.coords.data(), prod_verts.data(),
         nw.coords.data(), best.data());
   transfer_elem_tags(c, old, nw, mo, &best);
-}
-
-void transfer_measures(Ctx& c, DMesh& old, DMesh& nw, int d, ModOut const& mo) {
-  LO nprods = mo.prods2new.size();
-  LO nsame = mo.same2old.size();
-  if (d == 1)
-    nw.length = measure_transfer(c, nw, 1, nsame, mo.same2old.data(), mo.same2new.data(),
-        ask_lengths(c, old).data(), nprods, mo.prods2new.data());
-  if (d == old.dim)
-    nw.quality = measure_transfer(c, nw, d, nsame, mo.same2old.data(), mo.same2new.data(),
-        ask_qualities(c, old).data(), nprods, mo.prods2new.data());
 }
 
 Bytes find_indset(Ctx& c, DMesh& m, int d, Reals const& quality, Bytes const& cands,

@@ -32,26 +32,28 @@ struct AdaptOptions {
 
 void default_options(int dim, AdaptOptions& o);
 
-// result of modify_ents for one dimension (src/Omega_h_modify.cpp:468-517)
+// the new numbers of one dimension's entities after modify_ents: old2new
+// (-1 for entities that do not survive; built only for meshes that carry
+// tags) and, per product, prods2new
 struct ModOut {
+  LO nold = 0;
   LO nnew = 0;
-  LOs same2old;
-  LOs same2new;
-  LOs prods2new;
+  LO nprods = 0;
   LOs old2new;
+  LOs prods2new;
 };
 
-// modify_ents_adapt (src/Omega_h_modify.cpp:468-517) in three steps, so
-// that a pass numbers all its dimensions with one scan launch and one sync:
-// modify_plans marks the same entities, counts the new entities each old one
-// stands for and finds the representatives (no sync); modify_scan scans the
-// plans of up to four dimensions together; modify_build numbers and connects
-// one dimension
+// modify_ents_adapt (src/Omega_h_modify.cpp:468-517) in steps that each cover
+// every dimension of a pass in one launch: modify_plans marks the same
+// entities, counts the new entities each old one stands for and finds the
+// representatives (no sync); modify_scan scans the counts of up to four
+// dimensions together; rebuild_same moves the same entities with all they
+// carry; place_products numbers the products; match_sides connects them
 struct ModPlan {
   int ent_dim = 0, key_dim = 0;
-  LO nold = 0, nnew = 0, nsame = 0;
+  LO nold = 0, nnew = 0;
   Bytes same;
-  LOs counts, reps, offsets, same_offsets;
+  LOs counts, reps, offsets;
 };
 // the plans of dimensions d0..d1 (keys2prods indexed by dimension)
 void modify_plans(Ctx& c, DMesh& old, int key_dim, int d0, int d1, LOs const& keys2kds,
@@ -66,26 +68,55 @@ void modify_plans_masked(Ctx& c, DMesh& old, int key_dim, int d1, Bytes const& k
     LO const* const* prod_counts, ModPlan* plans, LOs* rep_of);
 // modify_scan in two halves, for callers that add the plans' scans to a
 // launch of their own: the jobs (totals in pinned slots first_slot...), then,
-// after the caller's sync, the totals
+// after the caller's wait, the totals
 int modify_scan_jobs(Ctx& c, ModPlan* plans, int nplans, ScanJob* jobs, int first_slot);
 void modify_scan_totals(Ctx& c, ModPlan* plans, int nplans, int first_slot);
-// verts_old2new: the vertex renumbering (null when vertices keep their
-// numbers); prod_src, when given, receives each product's key entity
-void modify_build(Ctx& c, DMesh& old, DMesh& nw, ModPlan const& plan, LOs const& keys2kds,
-    LOs const& keys2prods, LO nprods, LOs const& prod_verts, LOs const& old_lows2new_lows,
-    ModOut& out, LOs const* verts_old2new, LOs* prod_src = nullptr,
-    LOs const* given_down = nullptr, Bytes const* given_codes = nullptr);
+
+// the swap choices carried along with the edges (see SwapCache)
+struct SwapCache;
+struct CacheMove {
+  SwapCache const* from;
+  SwapCache* to;
+  Bytes const* dirty;
+};
+// the new mesh's arrays of dimensions d0..dim with the same entities in
+// place: connectivity, codes and vertex lists renumbered, classification,
+// lengths and qualities, and for dimension 0 coordinates and metric, in one
+// launch (transfer_common's same part, src/Omega_h_transfer.cpp:149-180, and
+// modify_conn, src/Omega_h_modify.cpp:446-466).  plans[d - d0] and mo[d] are
+// dimension d's; dimensions below d0 must be set in nw and keep their numbers.
+void rebuild_same(Ctx& c, DMesh& old, DMesh& nw, int d0, ModPlan const* plans, ModOut* mo,
+    CacheMove const* cache = nullptr);
+// the products of one dimension: vertex lists in the new numbering (absent
+// for vertices) and the entity each comes from: src[p] of dimension src_dim,
+// or src_dims[p]; without src the key itself, of dimension src_dim
+struct Products {
+  LO n = 0;
+  LOs keys2prods;
+  LOs verts;
+  LOs src;
+  int src_dim = 0;
+  Bytes src_dims;
+};
+// numbers the products of dimensions d0..d1 (prods[d], mo[d], plans[d -
+// plan0]) and writes their vertex lists and classification, in one launch;
+// inheritance tags of those dimensions follow.  new_edges_valid, when given,
+// is zeroed at new edges.
+void place_products(Ctx& c, DMesh& old, DMesh& nw, int d0, int d1, int plan0,
+    ModPlan const* plans, LOs const& keys2kds, Products const* prods, ModOut* mo,
+    I8* new_edges_valid = nullptr);
+// the sides and codes of the placed products of dimensions 2..dim, by their
+// vertices among the new mesh's entities (reflect_down)
+void match_sides(Ctx& c, DMesh& nw, Products const* prods, ModOut const* mo);
+// lengths of new edges and qualities of new elements, in one launch
+void measure_products(Ctx& c, DMesh& nw, ModOut const* mo);
+// every tag of a rebuilt mesh but the vertex tags' and refinement's own
+bool has_tags(DMesh const& m);
 
 // new tag data: same entities copy old values, products take prod values
 template <class T>
 DArray<T> transfer(Ctx& c, ModOut const& mo, int ncomps, DArray<T> const& old_data,
     DArray<T> const* prod_data);
-// class_id/class_dim of products from one old entity each, of dimension
-// src_dims[p] (or src_dim when src_dims is null)
-void transfer_class(Ctx& c, DMesh& old, DMesh& nw, int d, ModOut const& mo,
-    LOs const& prod_src, int src_dim, Bytes const* src_dims);
-// lengths (d == 1) and qualities (d == dim) of products on the new mesh
-void transfer_measures(Ctx& c, DMesh& old, DMesh& nw, int d, ModOut const& mo);
 // element tags of the new elements: products take the value of old element
 // prod_src[p] (no products when prod_src is null)
 void transfer_elem_tags(Ctx& c, DMesh const& old, DMesh& nw, ModOut const& mo,
@@ -149,7 +180,8 @@ void swap3d_choices(Ctx& c, DMesh& m, AdaptOptions const& o, LOs const& edges,
     LOs& configs_out, Reals& quals_out);
 
 // known-answer hooks used by the tests
-Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands);
+Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands,
+    Reals* midpoint_metrics = nullptr);
 // coarsen_qualities (src/Omega_h_coarsen_qualities.cpp:65-88) on device
 // arrays, stream-ordered: out[2 i + col] is the quality after collapsing
 // candidate i's edge in direction col (-1 where cand_codes[i] does not

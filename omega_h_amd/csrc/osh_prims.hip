@@ -161,8 +161,7 @@ void Ctx::raise_device_error() {
   if (*err != kNoError) {
     int code = *err;
     *err = kNoError;
-    if (code == kReflectDownNoMatch)
-      throw Error("reflect_down: entity without a unique match");
+    if (code == kReflectDownNoMatch) throw Error(kNoMatchMessage);
     if (code == kScanTimeout) throw Error("scan: a tile waited too long for its predecessor");
     if (code == kScanTicket) throw Error("scan: tile tickets out of step");
     if (code == kKeyWithoutUp) throw Error("modify: a key entity has no adjacent entity above it");

@@ -100,81 +100,148 @@ __global__ void seed_keys(LO ncands, LO const* cands, Real const* quals, Real qm
   edge_quals[cands[c]] = quals[c];
 }
 
-__global__ void prod_counts(LO nkeys, LO const* keys2edges, LO const* pairs_a2ab,
-    LO const* cuts_a2ab, LO* counts) {
-  LO k = thread_index();
-  if (k >= nkeys) return;
+// the rows that refinement products of dimensions 1..3 come from: pairs (the
+// entities of the dimension around the key edge, two products each; the edge
+// itself in dimension 1) and cuts (the entities one dimension up, one product
+// each)
+struct RefineRows {
+  LO const* pairs_a2ab[3];  // null: none
+  LO const* pairs_ab2b[3];
+  I8 const* pairs_codes[3];
+  LO const* pair_verts[3];
+  LO const* cuts_a2ab[3];
+  LO const* cuts_ab2b[3];
+  I8 const* cuts_codes[3];
+  LO const* cut_verts[3];
+  LO const* keys2prods[3];
+  LO* counts[3];
+  LO* pv[3];
+  LO* psrc[3];
+  I8* psrc_dim[3];
+};
+
+__global__ void prod_counts(LO nt, LO nkeys, LO const* keys2edges, RefineRows r) {
+  LO t = thread_index();
+  if (t >= nt) return;
+  int d = t / nkeys;
+  LO k = t % nkeys;
   LO e = keys2edges[k];
-  LO n = pairs_a2ab ? 2 * (pairs_a2ab[e + 1] - pairs_a2ab[e]) : 2;
-  if (cuts_a2ab) n += cuts_a2ab[e + 1] - cuts_a2ab[e];
-  counts[k] = n;
+  LO n = r.pairs_a2ab[d] ? 2 * (r.pairs_a2ab[d][e + 1] - r.pairs_a2ab[d][e]) : 2;
+  if (r.cuts_a2ab[d]) n += r.cuts_a2ab[d][e + 1] - r.cuts_a2ab[d][e];
+  r.counts[d][k] = n;
 }
+
+// every product's position follows from its row entry, so kRowLanes threads
+// per key and dimension share the rows; one thread per key and a launch per
+// dimension was a chain of dependent gathers (12 to 24 us a launch)
+constexpr int kRowLanes = 8;
 
 template <int ED>
-__global__ void refine_products_kernel(LO nkeys, LO const* keys2edges, LO const* keys2mid,
-    LO const* o2n, LO const* ev2v, LO const* keys2prods, LO const* pairs_a2ab,
-    LO const* pairs_ab2b, I8 const* pairs_codes, LO const* pair_dom_verts, LO const* cuts_a2ab,
-    LO const* cuts_ab2b, I8 const* cuts_codes, LO const* cut_dom_verts, LO* pv, LO* psrc,
-    I8* psrc_dim) {
-  LO k = thread_index();
-  if (k >= nkeys) return;
+__device__ __forceinline__ void refine_products_of(int lane, LO e, LO mid, LO prod0,
+    LO const* ev2v, LO const* vert_offsets, RefineRows const& r) {
   constexpr int nv = ED + 1;
-  LO e = keys2edges[k];
-  LO mid = keys2mid[k];
-  LO prod = keys2prods[k];
+  constexpr int d = ED - 1;
+  LO* pv = r.pv[d];
+  LO npairs = 1;
   if (ED == 1) {
-    pv[prod * 2 + 0] = o2n[ev2v[e * 2 + 0]];
-    pv[prod * 2 + 1] = mid;
-    psrc[prod] = e;
-    psrc_dim[prod] = 1;
-    ++prod;
-    pv[prod * 2 + 0] = mid;
-    pv[prod * 2 + 1] = o2n[ev2v[e * 2 + 1]];
-    psrc[prod] = e;
-    psrc_dim[prod] = 1;
-    ++prod;
+    if (lane < 2) {
+      LO p = prod0 + lane;
+      LO end = vert_offsets[ev2v[e * 2 + lane]];
+      pv[std::size_t(p) * 2 + lane] = end;
+      pv[std::size_t(p) * 2 + 1 - lane] = mid;
+      r.psrc[d][p] = e;
+      r.psrc_dim[d][p] = 1;
+    }
   } else {
-    for (LO ed = pairs_a2ab[e]; ed < pairs_a2ab[e + 1]; ++ed) {
-      LO dom = pairs_ab2b[ed];
-      I8 code = pairs_codes[ed];
+    LO row = r.pairs_a2ab[d][e];
+    npairs = r.pairs_a2ab[d][e + 1] - row;
+    for (LO i = lane; i < 2 * npairs; i += kRowLanes) {
+      LO ed = row + i / 2;
+      int eev = i % 2;
+      LO dom = r.pairs_ab2b[d][ed];
+      I8 code = r.pairs_codes[d][ed];
       int dde = code_which_down(code);
-      int rot = code_rotation(code);
-      for (int eev = 0; eev < 2; ++eev) {
-        int dev = eev ^ rot;
-        int ddv = down_template(ED, 1, dde, dev);
-        int dds = opposite_template(ED, 0, ddv);
-        LO* ppv = pv + prod * nv;
-        for (int dsv = 0; dsv < ED; ++dsv)
-          ppv[dsv] = o2n[pair_dom_verts[dom * (ED + 1) + down_template(ED, ED - 1, dds, dsv)]];
-        ppv[ED] = mid;
-        if (ED == 3) {
-          LO t = ppv[1];
-          ppv[1] = ppv[2];
-          ppv[2] = t;
-        }
-        psrc[prod] = dom;
-        psrc_dim[prod] = ED;
-        ++prod;
+      int dev = eev ^ code_rotation(code);
+      int ddv = down_template(ED, 1, dde, dev);
+      int dds = opposite_template(ED, 0, ddv);
+      LO v[nv];
+#pragma unroll
+      for (int dsv = 0; dsv < ED; ++dsv)
+        v[dsv] = vert_offsets[r.pair_verts[d][std::size_t(dom) * nv +
+                                              down_template(ED, ED - 1, dds, dsv)]];
+      v[ED] = mid;
+      if (ED == 3) {
+        LO t = v[1];
+        v[1] = v[2];
+        v[2] = t;
       }
+      LO p = prod0 + i;
+#pragma unroll
+      for (int k = 0; k < nv; ++k) pv[std::size_t(p) * nv + k] = v[k];
+      r.psrc[d][p] = dom;
+      r.psrc_dim[d][p] = ED;
     }
   }
-  if (cuts_a2ab) {
-    constexpr int CD = ED + 1;
-    for (LO ed = cuts_a2ab[e]; ed < cuts_a2ab[e + 1]; ++ed) {
-      LO dom = cuts_ab2b[ed];
-      int dde = code_which_down(cuts_codes[ed]);
+  if (ED < 3 && r.cuts_a2ab[d]) {
+    constexpr int CD = ED < 3 ? ED + 1 : 3;
+    LO row = r.cuts_a2ab[d][e], end = r.cuts_a2ab[d][e + 1];
+    for (LO ed = row + lane; ed < end; ed += kRowLanes) {
+      LO dom = r.cuts_ab2b[d][ed];
+      int dde = code_which_down(r.cuts_codes[d][ed]);
       int ddt = opposite_template(CD, 1, dde);
-      LO* ccv = pv + prod * nv;
+      LO p = prod0 + 2 * npairs + (ed - row);
       for (int dtv = 0; dtv < CD - 1; ++dtv)
-        ccv[dtv] = o2n[cut_dom_verts[dom * (CD + 1) + down_template(CD, CD - 2, ddt, dtv)]];
-      ccv[CD - 1] = mid;
-      psrc[prod] = dom;
-      psrc_dim[prod] = CD;
-      ++prod;
+        pv[std::size_t(p) * nv + dtv] =
+            vert_offsets[r.cut_verts[d][std::size_t(dom) * (CD + 1) +
+                                        down_template(CD, CD - 2, ddt, dtv)]];
+      pv[std::size_t(p) * nv + CD - 1] = mid;
+      r.psrc[d][p] = dom;
+      r.psrc_dim[d][p] = CD;
     }
   }
 }
 
+__global__ void refine_products(LO nt, LO nkeys, LO const* keys2edges, LO const* keys2mid,
+    LO const* ev2v, LO const* vert_offsets, RefineRows r) {
+  LO t = thread_index();
+  if (t >= nt) return;
+  LO per = nkeys * kRowLanes;
+  int d = t / per;
+  LO k = (t % per) / kRowLanes;
+  int lane = t % kRowLanes;
+  LO e = keys2edges[k];
+  LO mid = keys2mid[k];
+  LO prod0 = r.keys2prods[d][k];
+  if (d == 0)
+    refine_products_of<1>(lane, e, mid, prod0, ev2v, vert_offsets, r);
+  else if (d == 1)
+    refine_products_of<2>(lane, e, mid, prod0, ev2v, vert_offsets, r);
+  else
+    refine_products_of<3>(lane, e, mid, prod0, ev2v, vert_offsets, r);
+}
+
+// the midpoint vertices' coordinates (the mean of the ends) and metrics (the
+// ones their candidates' qualities were measured with)
+__global__ void place_midpoints(LO nkeys, int dim, int nc, LO const* keys2edges,
+    LO const* keys2mid, LO const* ev2v, Real const* old_coords, LO const* cand_of_edge,
+    Real const* midpt_metrics, Real* coords, Real* metric) {
+  LO k = thread_index();
+  if (k >= nkeys) return;
+  LO e = keys2edges[k];
+  LO w = keys2mid[k];
+  LO cand = cand_of_edge[e];
+  for (int j = 0; j < dim; ++j) {
+    double comp = 0;
+    comp += old_coords[ev2v[e * 2] * dim + j];
+    comp += old_coords[ev2v[e * 2 + 1] * dim + j];
+    comp /= 2;
+    coords[w * dim + j] = comp;
+  }
+  for (int j = 0; j < nc; ++j)
+    metric[std::size_t(w) * nc + j] = midpt_metrics[std::size_t(cand) * nc + j];
+}
+
+// the mean of a vertex tag over each key edge's ends
 __global__ void midpoint_coords(LO nkeys, int dim, LO const* keys2edges, LO const* ev2v,
     Real const* coords, Real* out) {
   LO k = thread_index();
@@ -191,13 +258,14 @@ __global__ void midpoint_coords(LO nkeys, int dim, LO const* keys2edges, LO cons
 
 }  // namespace
 
-Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands) {
+Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands, Reals* midpoint_metrics) {
   Range range(c, "refine_qualities");
   LO n = cands.size();
   int dim = m.dim;
   int nc = m.metric_ncomps;
   int md = (nc == 1) ? 1 : dim;
   Reals mm(c, n * nc);
+  if (midpoint_metrics) *midpoint_metrics = mm;
   mident_metrics(c, m, n, cands.data(), mm.data());
   Reals out(c, n);
   LOs const& cv2v = verts_of(c, m, dim);
@@ -228,9 +296,11 @@ bool refine_by_size(Ctx& c, DMesh& m, AdaptOptions const& o) {
   ask_qualities(c, m);
   Bytes cand(c, ne);
   OSH_LAUNCH(gt_kernel, ne, c, lengths.data(), o.max_length_desired, cand.data());
-  LOs cands = collect_marked(c, cand);
+  LOs cand_of_edge;
+  LOs cands = collect_marked(c, cand, &cand_of_edge);
   if (cands.size() == 0) return false;
-  Reals quals = refine_qualities(c, m, cands);
+  Reals cand_metrics;
+  Reals quals = refine_qualities(c, m, cands, &cand_metrics);
   Bytes initial = fill_i8(c, ne, 0);
   Reals edge_quals = fill_real(c, ne, 0.0);
   OSH_LAUNCH(seed_keys, cands.size(), c, cands.data(), quals.data(), o.min_quality_allowed,
@@ -247,26 +317,35 @@ bool refine_by_size(Ctx& c, DMesh& m, AdaptOptions const& o) {
   DMesh nw;
   nw.dim = dim;
   nw.metric_ncomps = nc;
-  LOs keys2mid, o2n, old_lows2new_lows;
   // products per key of every dimension, numbered by one scan launch
   LOs k2p[4];
   LO nprods[4] = {nkeys, 0, 0, 0};
-  Adj const* pairs[4] = {nullptr, nullptr, nullptr, nullptr};
-  Adj const* cuts[4] = {nullptr, nullptr, nullptr, nullptr};
+  RefineRows rows{};
   k2p[0] = iota(c, nkeys + 1);
   {
-    LOs counts[4];
+    LOs counts(c, dim * nkeys);
     ScanJob jobs[3];
     for (int d = 1; d <= dim; ++d) {
-      pairs[d] = (d > 1) ? &ask_up(c, m, 1, d) : nullptr;
-      cuts[d] = (d < dim) ? &ask_up(c, m, 1, d + 1) : nullptr;
-      counts[d] = LOs(c, nkeys);
-      OSH_LAUNCH(prod_counts, nkeys, c, keys2edges.data(),
-          pairs[d] ? pairs[d]->a2ab.data() : (LO const*)nullptr,
-          cuts[d] ? cuts[d]->a2ab.data() : (LO const*)nullptr, counts[d].data());
+      if (d > 1) {
+        Adj const& pr = ask_up(c, m, 1, d);
+        rows.pairs_a2ab[d - 1] = pr.a2ab.data();
+        rows.pairs_ab2b[d - 1] = pr.ab2b.data();
+        rows.pairs_codes[d - 1] = pr.codes.data();
+        rows.pair_verts[d - 1] = verts_of(c, m, d).data();
+      }
+      if (d < dim) {
+        Adj const& ct = ask_up(c, m, 1, d + 1);
+        rows.cuts_a2ab[d - 1] = ct.a2ab.data();
+        rows.cuts_ab2b[d - 1] = ct.ab2b.data();
+        rows.cuts_codes[d - 1] = ct.codes.data();
+        rows.cut_verts[d - 1] = verts_of(c, m, d + 1).data();
+      }
+      rows.counts[d - 1] = counts.data() + std::size_t(d - 1) * nkeys;
       k2p[d] = LOs(c, nkeys + 1);
-      jobs[d - 1] = {counts[d].data(), kScanLO, nkeys, k2p[d].data(), slot_ptr<LO>(c, d)};
+      rows.keys2prods[d - 1] = k2p[d].data();
+      jobs[d - 1] = {rows.counts[d - 1], kScanLO, nkeys, k2p[d].data(), slot_ptr<LO>(c, d)};
     }
+    OSH_LAUNCH(prod_counts, dim * nkeys, c, nkeys, keys2edges.data(), rows);
     offset_scans(c, jobs, dim);
     c.wait();
     for (int d = 1; d <= dim; ++d) nprods[d] = read_slot<LO>(c, d);
@@ -275,64 +354,45 @@ bool refine_by_size(Ctx& c, DMesh& m, AdaptOptions const& o) {
   ModPlan plans[4];
   modify_plans(c, m, 1, 0, dim, keys2edges, k2p, plans);
   modify_scan(c, plans, dim + 1);
-  for (int d = 0; d <= dim; ++d) {
-    LOs pv, psrc;
-    Bytes psrc_dim;
-    if (d > 0) {
-      Adj const* pr = pairs[d];
-      Adj const* ct = cuts[d];
-      pv = LOs(c, nprods[d] * (d + 1));
-      psrc = LOs(c, nprods[d]);
-      psrc_dim = Bytes(c, nprods[d]);
-      LO const* pdv = (d > 1) ? verts_of(c, m, d).data() : nullptr;
-      LO const* cdv = ct ? verts_of(c, m, d + 1).data() : nullptr;
-#define OSH_RP(ED)                                                                        \
-  OSH_LAUNCH(refine_products_kernel<ED>, nkeys, c, keys2edges.data(), keys2mid.data(),       \
-      o2n.data(), m.down[1].data(), k2p[d].data(), pr ? pr->a2ab.data() : (LO const*)nullptr, \
-      pr ? pr->ab2b.data() : (LO const*)nullptr, pr ? pr->codes.data() : (I8 const*)nullptr,  \
-      pdv, ct ? ct->a2ab.data() : (LO const*)nullptr, ct ? ct->ab2b.data() : (LO const*)nullptr, \
-      ct ? ct->codes.data() : (I8 const*)nullptr, cdv, pv.data(), psrc.data(), psrc_dim.data())
-      if (d == 1)
-        OSH_RP(1);
-      else if (d == 2)
-        OSH_RP(2);
-      else
-        OSH_RP(3);
-#undef OSH_RP
-    }
-    ModOut mo;
-    modify_build(c, m, nw, plans[d], keys2edges, k2p[d], nprods[d], pv, old_lows2new_lows, mo,
-        d > 0 ? &o2n : nullptr);
-    if (d == 0) {
-      keys2mid = mo.prods2new;
-      o2n = mo.old2new;
-      Reals pc(c, nkeys * dim);
-      OSH_LAUNCH(midpoint_coords, nkeys, c, dim, keys2edges.data(), m.down[1].data(),
-          m.coords.data(), pc.data());
-      nw.coords = transfer<Real>(c, mo, dim, m.coords, &pc);
-      Reals pm(c, nkeys * nc);
-      mident_metrics(c, m, nkeys, keys2edges.data(), pm.data());
-      nw.metric = transfer<Real>(c, mo, nc, m.metric, &pm);
-      for (auto const& t : m.vtags) {
-        Reals pt(c, nkeys * t.ncomps);
-        if (t.kind == 1)
-          mident_values(c, m, nkeys, keys2edges.data(), t.data.data(), t.ncomps, pt.data());
-        else
-          OSH_LAUNCH(midpoint_coords, nkeys, c, t.ncomps, keys2edges.data(), m.down[1].data(),
-              t.data.data(), pt.data());
-        nw.vtags.push_back(t.with_data(transfer<Real>(c, mo, t.ncomps, t.data, &pt)));
-      }
-      transfer_class(c, m, nw, 0, mo, keys2edges, 1, nullptr);
-    } else {
-      transfer_class(c, m, nw, d, mo, psrc, d, &psrc_dim);
-      if (d == dim) {
-        transfer_elem_tags(c, m, nw, mo, &psrc);
-        conserve_pass(c, m, nw, 0, 1, keys2edges, k2p[d], mo);
-      }
-      transfer_measures(c, m, nw, d, mo);
-    }
-    old_lows2new_lows = mo.old2new;
+  ModOut mo[4];
+  rebuild_same(c, m, nw, 0, plans, mo);
+  Products prods[4];
+  prods[0].n = nkeys;
+  prods[0].keys2prods = k2p[0];
+  prods[0].src_dim = 1;
+  place_products(c, m, nw, 0, 0, 0, plans, keys2edges, prods, mo);
+  LO const* keys2mid = mo[0].prods2new.data();
+  OSH_LAUNCH(place_midpoints, nkeys, c, dim, nc, keys2edges.data(), keys2mid,
+      m.down[1].data(), m.coords.data(), cand_of_edge.data(), cand_metrics.data(),
+      nw.coords.data(), nw.metric.data());
+  for (int d = 1; d <= dim; ++d) {
+    Products& p = prods[d];
+    p.n = nprods[d];
+    p.keys2prods = k2p[d];
+    p.verts = LOs(c, p.n * (d + 1));
+    p.src = LOs(c, p.n);
+    p.src_dims = Bytes(c, p.n);
+    p.src_dim = d;
+    rows.pv[d - 1] = p.verts.data();
+    rows.psrc[d - 1] = p.src.data();
+    rows.psrc_dim[d - 1] = p.src_dims.data();
   }
+  OSH_LAUNCH(refine_products, dim * nkeys * kRowLanes, c, nkeys, keys2edges.data(), keys2mid,
+      m.down[1].data(), plans[0].offsets.data(), rows);
+  place_products(c, m, nw, 1, dim, 0, plans, keys2edges, prods, mo);
+  match_sides(c, nw, prods, mo);
+  measure_products(c, nw, mo);
+  for (auto const& t : m.vtags) {
+    Reals pt(c, nkeys * t.ncomps);
+    if (t.kind == 1)
+      mident_values(c, m, nkeys, keys2edges.data(), t.data.data(), t.ncomps, pt.data());
+    else
+      OSH_LAUNCH(midpoint_coords, nkeys, c, t.ncomps, keys2edges.data(), m.down[1].data(),
+          t.data.data(), pt.data());
+    nw.vtags.push_back(t.with_data(transfer<Real>(c, mo[0], t.ncomps, t.data, &pt)));
+  }
+  transfer_elem_tags(c, m, nw, mo[dim], &prods[dim].src);
+  conserve_pass(c, m, nw, 0, 1, keys2edges, k2p[dim], mo[dim]);
   m = nw;
   return true;
 }

@@ -263,6 +263,9 @@ enum DeviceError {
   kPolytopeOverflow = 11
 };
 
+// what a raised kReflectDownNoMatch says
+constexpr char const* kNoMatchMessage = "reflect_down: entity without a unique match";
+
 template <class T>
 inline T get_value(Ctx& c, T const* dptr) {
   OSH_HIP(hipMemcpyAsync(c.pinned, dptr, sizeof(T), hipMemcpyDeviceToHost, c.stream));

@@ -463,73 +463,102 @@ __global__ void swap3d_choose(LO nt, int lanes, LO const* cands, LO const* lsize
 // around the key edge, so those are the only candidates (vertices keep their
 // numbers in a swap).  `lanes` threads (a power of two up to 64,
 // Tuning::side_lanes) share one side's candidates; the one that matches
-// writes the side and the code match_uses would compute.
+// writes the side, at the product's new number, and the code match_uses would
+// compute.  Faces and tets are one launch: job 0 owns the first workgroups.
+struct LocalSides {
+  LO nuses;
+  LO const* prod_key;
+  LO const* k2p_low;
+  LO const* pv_high;
+  LO const* pv_low;
+  LO const* low_prods2new;
+  LO const* prods2new;
+  LO const* t2low;
+  LO const* old_low_verts;
+  I8 const* low_same;
+  LO const* low_offsets;
+  LO* out;
+  I8* out_codes;
+};
+
 template <int HIGH>
-__global__ void swap3d_local_down(LO nt, int lanes, LO const* prod_key, LO const* keys2edges,
-    LO const* k2p_low, LO const* pv_high, LO const* pv_low, LO const* low_prods2new,
-    LO const* e2t_a2ab, LO const* e2t_ab2b, LO const* t2low, LO const* old_low_verts,
-    LO const* low_old2new, LO* out, I8* out_codes, int* error) {
-  LO t = thread_index();
-  if (t >= nt) return;
+__device__ __forceinline__ void local_side(LO t, int lanes, LO const* keys2edges,
+    LO const* e2t_a2ab, LO const* e2t_ab2b, LocalSides const& a, int* error) {
   LO u = t / lanes;
   int lane = t % lanes;
   constexpr int LOW = HIGH - 1;
   constexpr int nvh = HIGH + 1;
   constexpr int nvl = LOW + 1;
   constexpr int nlpt = (HIGH == 3) ? 4 : 6;  // faces or edges of an old tet
-  LO p = u / nvh;
-  int which = u % nvh;
-  LO key = prod_key[p];
-  LO av[3];
-#pragma unroll
-  for (int k = 0; k < nvl; ++k) av[k] = pv_high[p * nvh + down_template(HIGH, LOW, which, k)];
-  LO q0 = k2p_low[key];
-  LO nq = k2p_low[key + 1] - q0;
-  LO e = keys2edges[key];
-  LO r0 = e2t_a2ab[e];
-  LO ncand = nq + (e2t_a2ab[e + 1] - r0) * nlpt;
   bool found = false;
-  for (LO cnd = lane; cnd < ncand; cnd += lanes) {
-    LO id;
-    LO bv[3];
-    if (cnd < nq) {
-      id = low_prods2new[q0 + cnd];
+  LO at = 0;
+  if (u < a.nuses) {
+    LO p = u / nvh;
+    int which = u % nvh;
+    at = a.prods2new[p] * nvh + which;
+    LO key = a.prod_key[p];
+    LO av[3];
 #pragma unroll
-      for (int k = 0; k < nvl; ++k) bv[k] = pv_low[(q0 + cnd) * nvl + k];
-    } else {
-      LO r = cnd - nq;
-      LO o = t2low[e2t_ab2b[r0 + r / nlpt] * nlpt + r % nlpt];
-      id = low_old2new[o];
-      if (id < 0) continue;
+    for (int k = 0; k < nvl; ++k) av[k] = a.pv_high[p * nvh + down_template(HIGH, LOW, which, k)];
+    LO q0 = a.k2p_low[key];
+    LO nq = a.k2p_low[key + 1] - q0;
+    LO e = keys2edges[key];
+    LO r0 = e2t_a2ab[e];
+    LO ncand = nq + (e2t_a2ab[e + 1] - r0) * nlpt;
+    for (LO cnd = lane; cnd < ncand; cnd += lanes) {
+      LO id;
+      LO bv[3];
+      if (cnd < nq) {
+        id = a.low_prods2new[q0 + cnd];
 #pragma unroll
-      for (int k = 0; k < nvl; ++k) bv[k] = old_low_verts[o * nvl + k];
+        for (int k = 0; k < nvl; ++k) bv[k] = a.pv_low[(q0 + cnd) * nvl + k];
+      } else {
+        LO r = cnd - nq;
+        LO o = a.t2low[e2t_ab2b[r0 + r / nlpt] * nlpt + r % nlpt];
+        if (!a.low_same[o]) continue;
+        id = a.low_offsets[o];
+#pragma unroll
+        for (int k = 0; k < nvl; ++k) bv[k] = a.old_low_verts[o * nvl + k];
+      }
+      int wd =
+          (bv[0] == av[0]) ? 0 : (bv[1] == av[0]) ? 1 : (nvl == 3 && bv[2] == av[0]) ? 2 : -1;
+      if (wd < 0) continue;
+      I8 code;
+      if (nvl == 2) {
+        if (av[1] != bv[1 - wd]) continue;
+        code = make_code(0, wd, 0);
+      } else if (av[1] == bv[(wd + 1) % 3] && av[2] == bv[(wd + 2) % 3]) {
+        code = make_code(0, (3 - wd) % 3, 0);
+      } else if (av[1] == bv[(wd + 2) % 3] && av[2] == bv[(wd + 1) % 3]) {
+        code = make_code(1, (3 - wd) % 3, 0);
+      } else {
+        continue;
+      }
+      a.out[at] = id;
+      a.out_codes[at] = code;
+      found = true;
     }
-    int wd = (bv[0] == av[0]) ? 0 : (bv[1] == av[0]) ? 1 : (nvl == 3 && bv[2] == av[0]) ? 2 : -1;
-    if (wd < 0) continue;
-    I8 code;
-    if (nvl == 2) {
-      if (av[1] != bv[1 - wd]) continue;
-      code = make_code(0, wd, 0);
-    } else if (av[1] == bv[(wd + 1) % 3] && av[2] == bv[(wd + 2) % 3]) {
-      code = make_code(0, (3 - wd) % 3, 0);
-    } else if (av[1] == bv[(wd + 2) % 3] && av[2] == bv[(wd + 1) % 3]) {
-      code = make_code(1, (3 - wd) % 3, 0);
-    } else {
-      continue;
-    }
-    out[u] = id;
-    out_codes[u] = code;
-    found = true;
   }
   // the side's lanes are `lanes` consecutive lanes of one wave
   unsigned long long any = __ballot(found);
   int base = int(threadIdx.x % 64) & ~(lanes - 1);
   unsigned long long group = (lanes >= 64) ? ~0ull : ((1ull << lanes) - 1);
-  if (lane == 0 && ((any >> base) & group) == 0ull) {
+  if (u < a.nuses && lane == 0 && ((any >> base) & group) == 0ull) {
     *error = kReflectDownNoMatch;
-    out[u] = 0;
-    out_codes[u] = 0;
+    a.out[at] = 0;
+    a.out_codes[at] = 0;
   }
+}
+
+__global__ void __launch_bounds__(kBlock) swap3d_local_down(int lanes, unsigned face_blocks,
+    LO const* keys2edges, LO const* e2t_a2ab, LO const* e2t_ab2b, LocalSides faces,
+    LocalSides tets, int* error) {
+  if (blockIdx.x < face_blocks)
+    local_side<2>(LO(blockIdx.x) * kBlock + LO(threadIdx.x), lanes, keys2edges, e2t_a2ab,
+        e2t_ab2b, faces, error);
+  else
+    local_side<3>(LO(blockIdx.x - face_blocks) * kBlock + LO(threadIdx.x), lanes, keys2edges,
+        e2t_a2ab, e2t_ab2b, tets, error);
 }
 
 // the edges of the tets the pass replaces: their tet rings change
@@ -537,28 +566,6 @@ __global__ void swap3d_mark_dirty(LO ntets, I8 const* tet_same, LO const* t2e, I
   LO t = thread_index();
   if (t >= ntets || tet_same[t]) return;
   for (int i = 0; i < 6; ++i) dirty[t2e[t * 6 + i]] = 1;
-}
-
-// the carried-over choices of the same edges whose tets did not change
-// threads [0, nsame) carry the same edges' choices; the rest mark the new
-// edges (products) as having none
-__global__ void swap3d_cache_transfer(LO n, LO nsame, LO const* same2old, LO const* same2new,
-    LO const* prods2new, I8 const* dirty, I8 const* valid, I8 const* cfg, I8 const* keep,
-    Real const* q, I8* n_valid, I8* n_cfg, I8* n_keep, Real* n_q) {
-  LO i = thread_index();
-  if (i >= n) return;
-  if (i >= nsame) {
-    n_valid[prods2new[i - nsame]] = 0;
-    return;
-  }
-  LO o = same2old[i], w = same2new[i];
-  bool ok = valid[o] && !dirty[o];
-  n_valid[w] = I8(ok);
-  if (ok) {
-    n_cfg[w] = cfg[o];
-    n_keep[w] = keep[o];
-    n_q[w] = q[o];
-  }
 }
 
 // the interior edges among the marked ones (mark_by_class_dim), and the
@@ -776,76 +783,71 @@ void swap_rebuild(Ctx& c, DMesh& m, LOs const& keys2edges, LOs const* k2p, LO co
     Bytes const* dirty = nullptr, Adj const* key_tets = nullptr,
     LOs const* prod_keys = nullptr) {
   int dim = m.dim;
-  LO nv = m.nents[0];
   DMesh nw;
   nw.dim = dim;
   nw.metric_ncomps = m.metric_ncomps;
-  nw.nents[0] = nv;
+  nw.nents[0] = m.nents[0];
   nw.coords = m.coords;
   nw.metric = m.metric;
   nw.vtags = m.vtags;
   nw.itags = m.itags;
   nw.class_id[0] = m.class_id[0];
   nw.class_dim[0] = m.class_dim[0];
-  LOs old_lows2new_lows;  // vertices keep their numbers
   ModPlan own[3];
   if (!plans) {
     plans = own;
     modify_plans(c, m, 1, 1, dim, keys2edges, k2p, plans);
     modify_scan(c, plans, dim);
   }
-  ModOut low_mo;  // the previous dimension's numbering
+  ModOut mo[4];
+  SwapCache next;
+  CacheMove move{cache, &next, dirty};
+  rebuild_same(c, m, nw, 1, plans, mo, cache ? &move : nullptr);
+  Products prods[4];
   for (int d = 1; d <= dim; ++d) {
-    ModOut mo;
-    LOs src;  // each product's key edge
-    // in 3D the products' sides come from a search around each key
-    LOs gdown;
-    Bytes gcodes;
-    if (key_tets && prod_keys && d >= 2) {
-      LO nuses = nprods[d] * (d + 1);
-      int side_lanes = fit_lanes(nuses, c.tuning.side_lanes);
-      gdown = LOs(c, nuses);
-      gcodes = Bytes(c, nuses);
-      LO const* t2low = (d == 3) ? m.down[3].data() : ask_down(c, m, 3, 1, nullptr).data();
-      if (d == 3)
-        OSH_LAUNCH(swap3d_local_down<3>, nuses * side_lanes, c, side_lanes, prod_keys[3].data(),
-            keys2edges.data(), k2p[2].data(), pv[3].data(), pv[2].data(),
-            low_mo.prods2new.data(), key_tets->a2ab.data(), key_tets->ab2b.data(), t2low,
-            verts_of(c, m, 2).data(), low_mo.old2new.data(), gdown.data(), gcodes.data(),
-            c.error_word());
-      else
-        OSH_LAUNCH(swap3d_local_down<2>, nuses * side_lanes, c, side_lanes, prod_keys[2].data(),
-            keys2edges.data(), k2p[1].data(), pv[2].data(), pv[1].data(),
-            low_mo.prods2new.data(), key_tets->a2ab.data(), key_tets->ab2b.data(), t2low,
-            verts_of(c, m, 1).data(), low_mo.old2new.data(), gdown.data(), gcodes.data(),
-            c.error_word());
-    }
-    modify_build(c, m, nw, plans[d - 1], keys2edges, k2p[d], nprods[d], pv[d],
-        old_lows2new_lows, mo, nullptr, &src, gdown.exists() ? &gdown : nullptr,
-        gcodes.exists() ? &gcodes : nullptr);
-    transfer_class(c, m, nw, d, mo, src, 1, nullptr);
-    if (d == 1 && cache) {
-      SwapCache next;
-      next.valid = Bytes(c, mo.nnew);
-      next.cfg = Bytes(c, mo.nnew);
-      next.keep = Bytes(c, mo.nnew);
-      next.q = Reals(c, mo.nnew);
-      LO nsame = mo.same2old.size();
-      OSH_CHECK(nsame + mo.prods2new.size() == mo.nnew, "swap cache: same + new edges");
-      OSH_LAUNCH(swap3d_cache_transfer, mo.nnew, c, nsame, mo.same2old.data(),
-          mo.same2new.data(), mo.prods2new.data(), dirty->data(), cache->valid.data(),
-          cache->cfg.data(), cache->keep.data(), cache->q.data(), next.valid.data(),
-          next.cfg.data(), next.keep.data(), next.q.data());
-      *cache = next;
-    }
-    if (d == dim) {
-      transfer_pointwise(c, m, nw, mo, 1, keys2edges, k2p[d], pv[d]);
-      conserve_pass(c, m, nw, 2, 1, keys2edges, k2p[d], mo);
-    }
-    transfer_measures(c, m, nw, d, mo);
-    old_lows2new_lows = mo.old2new;
-    low_mo = mo;
+    prods[d].n = nprods[d];
+    prods[d].keys2prods = k2p[d];
+    prods[d].verts = pv[d];
+    prods[d].src_dim = 1;  // products come from their key edge
   }
+  place_products(c, m, nw, 1, dim, 1, plans, keys2edges, prods, mo,
+      cache ? next.valid.data() : nullptr);
+  if (cache) *cache = next;
+  if (key_tets && prod_keys) {
+    // in 3D the products' sides come from a search around each key
+    LO most = nprods[2] * 3 > nprods[3] * 4 ? nprods[2] * 3 : nprods[3] * 4;
+    int lanes = fit_lanes(most, c.tuning.side_lanes);
+    LocalSides s[2];
+    unsigned blocks[2];
+    for (int d = 2; d <= 3; ++d) {
+      LocalSides& a = s[d - 2];
+      a.nuses = nprods[d] * (d + 1);
+      a.prod_key = prod_keys[d].data();
+      a.k2p_low = k2p[d - 1].data();
+      a.pv_high = pv[d].data();
+      a.pv_low = pv[d - 1].data();
+      a.low_prods2new = mo[d - 1].prods2new.data();
+      a.prods2new = mo[d].prods2new.data();
+      a.t2low = d == 3 ? m.down[3].data() : ask_down(c, m, 3, 1, nullptr).data();
+      a.old_low_verts = verts_of(c, m, d - 1).data();
+      a.low_same = plans[d - 2].same.data();
+      a.low_offsets = plans[d - 2].offsets.data();
+      a.out = nw.down[d].data();
+      a.out_codes = nw.down_codes[d].data();
+      blocks[d - 2] = unsigned((std::int64_t(a.nuses) * lanes + kBlock - 1) / kBlock);
+    }
+    if (blocks[0] + blocks[1]) {
+      hipLaunchKernelGGL(swap3d_local_down, dim3(blocks[0] + blocks[1]), dim3(kBlock), 0,
+          c.stream, lanes, blocks[0], keys2edges.data(), key_tets->a2ab.data(),
+          key_tets->ab2b.data(), s[0], s[1], c.error_word());
+      OSH_HIP(hipGetLastError());
+    }
+  } else {
+    match_sides(c, nw, prods, mo);
+  }
+  measure_products(c, nw, mo);
+  transfer_pointwise(c, m, nw, mo[dim], 1, keys2edges, k2p[dim], pv[dim]);
+  conserve_pass(c, m, nw, 2, 1, keys2edges, k2p[dim], mo[dim]);
   m = nw;
 }
 
