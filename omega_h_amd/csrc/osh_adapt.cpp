@@ -79,15 +79,13 @@ void print_histograms(Ctx& c, DMesh& m, AdaptOptions const& o) {
   std::fflush(stdout);
 }
 
-constexpr int kQminSlot = Ctx::kSlots - 1;
-
 double now() {
   return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch())
       .count();
 }
 
-// *qmin receives the minimum element quality after the pass, reduced before
-// the pass's closing sync so that it costs no sync of its own
+// *qmin receives the minimum element quality after the pass, whose reduction is
+// also the pass's closing wait
 // the most passes one adapt() records: a guard on the log, far above real
 // runs (the reference's loops have no limit; one 1.3M-tet box of the serving
 // workload under a constant anisotropic metric takes 4,639 swap and 283
@@ -113,11 +111,9 @@ bool run_pass(Ctx& c, DMesh& m, AdaptOptions const& o, int kind,
     r = swap_edges(c, m, o, cache);
   else
     r = coarsen_slivers(c, m, o);
-  min_real_async(c, ask_qualities(c, m), kQminSlot);
-  c.wait();
+  *qmin = min_real_wait(c, ask_qualities(c, m));
   double t1 = now();
   range.end();
-  *qmin = read_slot<Real>(c, kQminSlot);
   if (r && log) log->push_back({kind, nin, m.nents[m.dim], t1 - t0});
   if (r && hook && *hook) (*hook)(m);
   // post_rebuild, src/Omega_h_adapt.cpp:169-171

@@ -172,13 +172,15 @@ Adj invert_adj(Ctx& c, LO nhigh, int deg, LO nlow, LOs const& hl2l, Bytes const*
   Adj a;
   a.a2ab = LOs(c, nlow + 1);
   if (marked) {
-    LOs marked_offsets(c, nlow + 1);
+    LOs marked_offsets;
+    if (marked_index) marked_offsets = LOs(c, nlow + 1);
+    *marked = LOs(c, nlow);
     ScanJob jobs[2] = {{counts.data(), kScanLO, nlow, a.a2ab.data(), nullptr},
-        {mk, kScanNonzero, nlow, marked_offsets.data(), slot_ptr<LO>(c, 1)}};
-    offset_scans(c, jobs, 2);
+        {mk, kScanNonzero, nlow, marked_index ? marked_offsets.data() : nullptr,
+            slot_ptr<LO>(c, 1), marked->data()}};
+    offset_scans(c, jobs, nlow ? 2 : 1);
     c.wait();
-    *marked = LOs(c, read_slot<LO>(c, 1));
-    scatter_marked_list(c, *marks, marked_offsets, *marked);
+    marked->shrink(nlow ? read_slot<LO>(c, 1) : 0);
     if (marked_index) *marked_index = marked_offsets;
   } else {
     ScanJob job{counts.data(), kScanLO, nlow, a.a2ab.data(), nullptr};

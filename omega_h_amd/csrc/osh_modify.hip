@@ -490,14 +490,35 @@ __device__ __forceinline__ I8 indset_state(I8 const* old_state, LO x) {
 // read whole every round.
 constexpr int kDomBits = 64;
 
+// Each batch of rounds ends with a wait for two words: kUndecidedWord, set by
+// the last round's nodes that stay undecided, and kCandWord, set by the first
+// round's candidates, so that no reduction over the states is needed.
+constexpr int kUndecidedWord = 0;
+constexpr int kCandWord = 1;
+
+// one lane a wave stores, and only where the word does not hold the tag yet
+__device__ __forceinline__ void tell(bool is, unsigned* word, unsigned tag) {
+  unsigned long long b = __ballot(is);
+  if (b == 0ull || int(threadIdx.x & 63) != __ffsll(static_cast<long long>(b)) - 1) return;
+  if (__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != tag)
+    __hip_atomic_store(word, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+struct IndsetWords {
+  unsigned* words;
+  unsigned cand_tag;  // 0: not the first round
+  unsigned last_tag;  // 0: not the last round of its batch
+};
+
+__device__ __forceinline__ void tell_round(I8 before, I8 after, IndsetWords w) {
+  if (w.cand_tag) tell(before == 2, w.words + kCandWord, w.cand_tag);
+  if (w.last_tag) tell(after == 2, w.words + kUndecidedWord, w.last_tag);
+}
+
+// an undecided node's next state
 template <bool FIRST>
-__global__ void indset_iteration(LO n, LO const* a2ab, LO const* ab2b, Real const* q,
-    I8 const* old_state, I8* new_state, unsigned long long* dom) {
-  LO v = thread_index();
-  if (v >= n) return;
-  I8 s = indset_state<FIRST>(old_state, v);
-  new_state[v] = s;
-  if (s != 2) return;
+__device__ __forceinline__ I8 indset_node(LO v, LO const* a2ab, LO const* ab2b, Real const* q,
+    I8 const* old_state, unsigned long long* dom) {
   LO b = a2ab[v], e = a2ab[v + 1];
   bool undecided = false;
   if (!FIRST && e - b <= kDomBits) {
@@ -506,10 +527,7 @@ __global__ void indset_iteration(LO n, LO const* a2ab, LO const* ab2b, Real cons
       int j = __ffsll(static_cast<long long>(mask)) - 1;
       mask &= mask - 1;
       I8 su = old_state[ab2b[b + j]];
-      if (su == 1) {
-        new_state[v] = 0;
-        return;
-      }
+      if (su == 1) return 0;
       if (su == 2) undecided = true;
     }
   } else {
@@ -522,16 +540,24 @@ __global__ void indset_iteration(LO n, LO const* a2ab, LO const* ab2b, Real cons
       Real qu = q[u];
       bool beaten = (qu != qv) ? (qu < qv) : (u < v);
       if (beaten) continue;
-      if (su == 1) {
-        new_state[v] = 0;
-        return;
-      }
+      if (su == 1) return 0;
       undecided = true;
       if (FIRST && j - b < kDomBits) mask |= 1ull << (j - b);
     }
     if (FIRST) dom[v] = mask;
   }
-  if (!undecided) new_state[v] = 1;
+  return undecided ? 2 : 1;
+}
+
+template <bool FIRST>
+__global__ void indset_iteration(LO n, LO const* a2ab, LO const* ab2b, Real const* q,
+    I8 const* old_state, I8* new_state, unsigned long long* dom, IndsetWords w) {
+  LO v = thread_index();
+  if (v >= n) return;
+  I8 s = indset_state<FIRST>(old_state, v);
+  I8 r = s == 2 ? indset_node<FIRST>(v, a2ab, ab2b, q, old_state, dom) : s;
+  new_state[v] = r;
+  tell_round(s, r, w);
 }
 
 // the first round for edges with `lanes` threads per edge (a power of two,
@@ -540,7 +566,8 @@ __global__ void indset_iteration(LO n, LO const* a2ab, LO const* ab2b, Real cons
 // one after another
 template <int NEPC>
 __global__ void indset_first_edges(LO nt, int lanes, LO const* e2c_a2ab, LO const* e2c_ab2b,
-    LO const* c2e, Real const* q, I8 const* cands, I8* new_state, unsigned long long* dom) {
+    LO const* c2e, Real const* q, I8 const* cands, I8* new_state, unsigned long long* dom,
+    IndsetWords w) {
   LO t = thread_index();
   if (t >= nt) return;
   LO v = t / lanes;
@@ -567,39 +594,32 @@ __global__ void indset_first_edges(LO nt, int lanes, LO const* e2c_a2ab, LO cons
     undecided |= __shfl_xor(undecided, d, 64);
   }
   if (lane != 0) return;
-  new_state[v] = (s == 2 && !undecided) ? I8(1) : s;
+  I8 r = (s == 2 && !undecided) ? I8(1) : s;
+  new_state[v] = r;
   if (s == 2) dom[v] = mask;
+  tell_round(s, r, w);
 }
 
 // the same round for edges, whose star (edges_across_tris/tets,
 // src/Omega_h_adj.cpp:532-589) is the set of other edges of the elements
 // around the edge: read through the edge -> element adjacency instead of a
 // built star (an edge met twice is checked twice, which changes nothing);
-// row position (j, k) is bit j * NEPC + k of `dom`
-template <int NEPC, bool FIRST>
-__global__ void indset_iteration_edges(LO n, LO const* e2c_a2ab, LO const* e2c_ab2b,
-    LO const* c2e, Real const* q, I8 const* old_state, I8* new_state, unsigned long long* dom) {
-  LO v = thread_index();
-  if (v >= n) return;
-  I8 s = indset_state<FIRST>(old_state, v);
-  new_state[v] = s;
-  if (s != 2) return;
+// row position (j, k) is bit j * NEPC + k of `dom`.  Rounds after the first.
+template <int NEPC>
+__device__ __forceinline__ I8 indset_edge(LO v, LO const* e2c_a2ab, LO const* e2c_ab2b,
+    LO const* c2e, Real const* q, I8 const* old_state, unsigned long long const* dom) {
   LO b = e2c_a2ab[v], e = e2c_a2ab[v + 1];
   bool undecided = false;
-  if (!FIRST && (e - b) * NEPC <= kDomBits) {
+  if ((e - b) * NEPC <= kDomBits) {
     unsigned long long mask = dom[v];
     while (mask) {
       int p = __ffsll(static_cast<long long>(mask)) - 1;
       mask &= mask - 1;
       I8 su = old_state[c2e[e2c_ab2b[b + p / NEPC] * NEPC + p % NEPC]];
-      if (su == 1) {
-        new_state[v] = 0;
-        return;
-      }
+      if (su == 1) return 0;
       if (su == 2) undecided = true;
     }
   } else {
-    unsigned long long mask = 0;
     Real qv = q[v];
     for (LO j = b; j < e; ++j) {
       LO const* ce = c2e + e2c_ab2b[j] * NEPC;
@@ -607,23 +627,29 @@ __global__ void indset_iteration_edges(LO n, LO const* e2c_a2ab, LO const* e2c_a
       for (int k = 0; k < NEPC; ++k) {
         LO u = ce[k];
         if (u == v) continue;
-        I8 su = indset_state<FIRST>(old_state, u);
+        I8 su = old_state[u];
         if (su == 0) continue;
         Real qu = q[u];
         bool beaten = (qu != qv) ? (qu < qv) : (u < v);
         if (beaten) continue;
-        if (su == 1) {
-          new_state[v] = 0;
-          return;
-        }
+        if (su == 1) return 0;
         undecided = true;
-        int p = (j - b) * NEPC + k;
-        if (FIRST && p < kDomBits) mask |= 1ull << p;
       }
     }
-    if (FIRST) dom[v] = mask;
   }
-  if (!undecided) new_state[v] = 1;
+  return undecided ? 2 : 1;
+}
+
+template <int NEPC>
+__global__ void indset_iteration_edges(LO n, LO const* e2c_a2ab, LO const* e2c_ab2b,
+    LO const* c2e, Real const* q, I8 const* old_state, I8* new_state,
+    unsigned long long const* dom, IndsetWords w) {
+  LO v = thread_index();
+  if (v >= n) return;
+  I8 s = old_state[v];
+  I8 r = s == 2 ? indset_edge<NEPC>(v, e2c_a2ab, e2c_ab2b, c2e, q, old_state, dom) : s;
+  new_state[v] = r;
+  tell_round(s, r, w);
 }
 
 __global__ void mark_down_kernel(LO nl, LO const* a2ab, LO const* ab2b, I8 const* marks, I8* out) {
@@ -1077,45 +1103,39 @@ Bytes find_indset(Ctx& c, DMesh& m, int d, Reals const& quality, Bytes const& ca
   // extra rounds after convergence change nothing: run two rounds before each
   // of the first four checks, then 4, 8 and 16 (long chains of decreasing
   // quality, as on the first coarsening passes of a large smooth mesh, take
-  // some 200 rounds and would otherwise spend a sync every two); after the
-  // first check a state of 2 means undecided nodes remain, and a state of 1
-  // or 2 that there was a candidate (the best candidate joins the set in the
-  // first round)
+  // some 200 rounds and would otherwise spend a wait every two)
   int first_lanes = fit_lanes(n, c.tuning.first_lanes);
   for (LO round = 0;;) {
     OSH_CHECK(round <= n + 1, "independent set does not converge");
     int batch = round < 8 ? 2 : (round < 16 ? 4 : (round < 32 ? 8 : 16));
+    unsigned tag = c.wait_tag();
     for (int k = 0; k < batch; ++k, ++round) {
       bool first = round == 0;
+      IndsetWords w{c.words, first ? tag : 0u, k == batch - 1 ? tag : 0u};
       I8 const* in = first ? cands.data() : a.data();
-#define OSH_IS(F)                                                                         \
-  do {                                                                                    \
-    if (g)                                                                                \
-      OSH_LAUNCH(indset_iteration<F>, n, c, g->a2ab.data(), g->ab2b.data(), quality.data(), \
-          in, b.data(), dom.data());                                                      \
-    else if (m.dim == 3)                                                                  \
-      OSH_LAUNCH((indset_iteration_edges<6, F>), n, c, e2c->a2ab.data(), e2c->ab2b.data(),  \
-          c2e, quality.data(), in, b.data(), dom.data());                                 \
-    else                                                                                  \
-      OSH_LAUNCH((indset_iteration_edges<3, F>), n, c, e2c->a2ab.data(), e2c->ab2b.data(),  \
-          c2e, quality.data(), in, b.data(), dom.data());                                 \
-  } while (0)
-      if (first && !g && m.dim == 3)
+      if (g && first)
+        OSH_LAUNCH(indset_iteration<true>, n, c, g->a2ab.data(), g->ab2b.data(),
+            quality.data(), in, b.data(), dom.data(), w);
+      else if (g)
+        OSH_LAUNCH(indset_iteration<false>, n, c, g->a2ab.data(), g->ab2b.data(),
+            quality.data(), in, b.data(), dom.data(), w);
+      else if (first && m.dim == 3)
         OSH_LAUNCH((indset_first_edges<6>), n * first_lanes, c, first_lanes, e2c->a2ab.data(),
-            e2c->ab2b.data(), c2e, quality.data(), cands.data(), b.data(), dom.data());
-      else if (first && !g)
-        OSH_LAUNCH((indset_first_edges<3>), n * first_lanes, c, first_lanes, e2c->a2ab.data(),
-            e2c->ab2b.data(), c2e, quality.data(), cands.data(), b.data(), dom.data());
+            e2c->ab2b.data(), c2e, quality.data(), in, b.data(), dom.data(), w);
       else if (first)
-        OSH_IS(true);
+        OSH_LAUNCH((indset_first_edges<3>), n * first_lanes, c, first_lanes, e2c->a2ab.data(),
+            e2c->ab2b.data(), c2e, quality.data(), in, b.data(), dom.data(), w);
+      else if (m.dim == 3)
+        OSH_LAUNCH(indset_iteration_edges<6>, n, c, e2c->a2ab.data(), e2c->ab2b.data(), c2e,
+            quality.data(), in, b.data(), dom.data(), w);
       else
-        OSH_IS(false);
-#undef OSH_IS
+        OSH_LAUNCH(indset_iteration_edges<3>, n, c, e2c->a2ab.data(), e2c->ab2b.data(), c2e,
+            quality.data(), in, b.data(), dom.data(), w);
       std::swap(a, b);
     }
-    I8 top = max_i8(c, a);
-    if (any_cands && round == 2) *any_cands = top >= 1;
-    if (top != 2) break;
+    c.wait();
+    if (any_cands && round == 2) *any_cands = c.word_set(kCandWord, tag);
+    if (!c.word_set(kUndecidedWord, tag)) break;
   }
   return a;
 }

@@ -71,8 +71,11 @@ void Pool::release_all() {
 Ctx::Ctx() : pool(std::make_shared<Pool>()) {
   OSH_HIP(hipGetDevice(&device));
   OSH_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-  OSH_HIP(hipHostMalloc(&pinned, 8 * kSlots + 128, hipHostMallocDefault));
-  std::memset(pinned, 0, 8 * kSlots + 128);
+  OSH_HIP(hipHostMalloc(&pinned, 8 * kSlots + 192, hipHostMallocDefault));
+  std::memset(pinned, 0, 8 * kSlots + 192);
+  OSH_HIP(hipMalloc((void**)&words, sizeof(unsigned) * kWords));
+  unsigned none[kWords] = {0};
+  OSH_HIP(hipMemcpy(words, none, sizeof(none), hipMemcpyHostToDevice));
   OSH_HIP(hipMalloc(&partials, 1024 * sizeof(double)));
   OSH_HIP(hipMalloc((void**)&tile_counter, sizeof(unsigned)));
   OSH_HIP(hipMalloc((void**)&tile_sums, sizeof(LO) * kScanTiles * kMaxScanJobs));
@@ -95,6 +98,7 @@ Ctx::~Ctx() {
   if (scan_status) (void)hipFree(scan_status);
   if (tile_counter) (void)hipFree(tile_counter);
   if (tile_sums) (void)hipFree(tile_sums);
+  if (words) (void)hipFree(words);
   if (pool) pool->close();
   if (partials) (void)hipFree(partials);
   if (pinned) (void)hipHostFree(pinned);
@@ -121,7 +125,9 @@ void Ctx::sync() {
 namespace {
 
 // stores made by the stream's earlier kernels happen before this release
-__global__ void signal_kernel(unsigned* word, unsigned value) {
+__global__ void signal_kernel(unsigned const* words, unsigned* host_words, unsigned* word,
+    unsigned value) {
+  for (int i = 0; i < Ctx::kWords; ++i) host_words[i] = words[i];
   __hip_atomic_store(word, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
@@ -136,10 +142,15 @@ constexpr double kPollSeconds = 200e-6;
 // and often an interrupt); a one-thread kernel that stores into pinned memory
 // with the host polling that word adds 6 to 8 us.
 void Ctx::wait() {
+  hipLaunchKernelGGL(signal_kernel, dim3(1), dim3(1), 0, stream,
+      static_cast<unsigned const*>(words), host_words(), signal_word(), wait_tag());
+  OSH_HIP(hipGetLastError());
+  wait_signalled();
+}
+
+void Ctx::wait_signalled() {
   unsigned value = ++signal_value;
   unsigned* word = signal_word();
-  hipLaunchKernelGGL(signal_kernel, dim3(1), dim3(1), 0, stream, word, value);
-  OSH_HIP(hipGetLastError());
   double limit = 0.0;
   for (unsigned polls = 1;; ++polls) {
     if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == value) {
@@ -295,6 +306,7 @@ __device__ __forceinline__ LO look_back(unsigned long long* status, unsigned til
 struct ScanBatch {
   void const* in[kMaxScanJobs];
   LO* out[kMaxScanJobs];
+  LO* list[kMaxScanJobs];
   LO* total[kMaxScanJobs];
   LO n[kMaxScanJobs];
   int kind[kMaxScanJobs];
@@ -332,6 +344,7 @@ __global__ void __launch_bounds__(kBlock) scan_lookback(ScanBatch b,
   int kind = b.kind[job];
   void const* in = b.in[job];
   LO* out = b.out[job];
+  LO* list = b.list[job];
   unsigned long long* st = status + b.first[job];
   LO tile_base = LO(tile) * kScanTile;
 #pragma unroll
@@ -364,7 +377,7 @@ __global__ void __launch_bounds__(kBlock) scan_lookback(ScanBatch b,
         __hip_atomic_store(&st[tile], status_word(epoch, kFlagInclusive, prefix + total),
             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       s_prefix = prefix;
-      if (tile == 0) out[0] = 0;
+      if (tile == 0 && out) out[0] = 0;
       if (b.total[job] && tile == ntiles - 1) *b.total[job] = prefix + total;
     }
   }
@@ -377,7 +390,11 @@ __global__ void __launch_bounds__(kBlock) scan_lookback(ScanBatch b,
   for (int k = 0; k < kScanItems; ++k) {
     int j = k * kBlock + int(threadIdx.x);
     LO i = tile_base + j;
-    if (i < n) out[1 + i] = s_vals[j + (j >> 4)];
+    if (i < n) {
+      LO inc = s_vals[j + (j >> 4)];
+      if (out) out[1 + i] = inc;
+      if (list && scan_input(in, kind, i)) list[inc - 1] = i;
+    }
   }
 }
 
@@ -524,7 +541,7 @@ __global__ void __launch_bounds__(BLOCK) scan_tiles(ScanBatch b, LO const* sums)
     LO i = wave_inclusive_scan(p);
     if (lane < T::kParts) part[lane] = prefix + i - p;
     if (lane == kWave - 1 && tile == ntiles - 1) {
-      b.out[job][n] = prefix + i;
+      if (b.out[job]) b.out[job][n] = prefix + i;
       if (b.total[job]) *b.total[job] = prefix + i;
     }
   }
@@ -536,6 +553,14 @@ __global__ void __launch_bounds__(BLOCK) scan_tiles(ScanBatch b, LO const* sums)
     LO i = base + (r * BLOCK + LO(threadIdx.x)) * 4;
     LO o0 = part[r * T::kWaves + wave] + inc[r] - ((v[r][0] + v[r][1]) + (v[r][2] + v[r][3]));
     LO o1 = o0 + v[r][0], o2 = o1 + v[r][1], o3 = o2 + v[r][2];
+    if (LO* list = b.list[job]) {
+      // values past the end are 0
+      if (v[r][0]) list[o0] = i;
+      if (v[r][1]) list[o1] = i + 1;
+      if (v[r][2]) list[o2] = i + 2;
+      if (v[r][3]) list[o3] = i + 3;
+    }
+    if (!out) continue;
     if (wide_out && i + 4 <= n) {
       *reinterpret_cast<int4*>(out + i) = make_int4(o0, o1, o2, o3);
     } else {
@@ -585,9 +610,10 @@ unsigned batch_jobs(ScanJob const* jobs, int njobs, int tile, ScanBatch& b, unsi
   unsigned tiles = 0;
   *most = 0;
   for (int j = 0; j < njobs; ++j) {
-    OSH_CHECK(jobs[j].n >= 0 && jobs[j].out, "offset_scans: bad job");
+    OSH_CHECK(jobs[j].n >= 0 && (jobs[j].out || jobs[j].list), "offset_scans: bad job");
     b.in[j] = jobs[j].in;
     b.out[j] = jobs[j].out;
+    b.list[j] = jobs[j].list;
     b.total[j] = jobs[j].total;
     b.n[j] = jobs[j].n;
     b.kind[j] = jobs[j].kind;
@@ -739,11 +765,6 @@ LOs offset_scan_t(Ctx& c, DArray<T> const& counts, LO* total_out) {
   return out;
 }
 
-__global__ void scatter_marked(LO n, I8 const* marks, LO const* offsets, LO* out) {
-  LO i = thread_index();
-  if (i < n && marks[i]) out[offsets[i]] = i;
-}
-
 __global__ void iota_kernel(LO n, LO* out, LO start, LO stride) {
   LO i = thread_index();
   if (i < n) out[i] = start + i * stride;
@@ -762,7 +783,8 @@ __device__ __forceinline__ T combine(T a, T b) {
 // over the partials then writes the result into host-visible memory (the
 // kernel boundary orders the two, so no device-wide fences are needed)
 template <class T, int Op>
-__global__ void __launch_bounds__(kBlock) reduce_blocks(LO n, T const* in, T* out, T init) {
+__global__ void __launch_bounds__(kBlock) reduce_blocks(LO n, T const* in, T* out, T init,
+    unsigned* signal, unsigned value) {
   __shared__ T buf[kBlock];
   T acc = init;
   for (LO i = LO(blockIdx.x) * kBlock + LO(threadIdx.x); i < n; i += LO(gridDim.x) * kBlock)
@@ -773,39 +795,37 @@ __global__ void __launch_bounds__(kBlock) reduce_blocks(LO n, T const* in, T* ou
     if (int(threadIdx.x) < s) buf[threadIdx.x] = combine<T, Op>(buf[threadIdx.x], buf[threadIdx.x + s]);
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[blockIdx.x] = buf[0];
+  if (threadIdx.x == 0) {
+    out[blockIdx.x] = buf[0];
+    // the one-block launch that ends a reduction can end the wait for it
+    if (signal) __hip_atomic_store(signal, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
-// the result lands in `result` (device-visible) once the stream reaches it
+// the reduction of a, waited for
 template <class T, int Op>
-void reduce_to(Ctx& c, DArray<T> const& a, T init, T* result) {
+T reduce(Ctx& c, DArray<T> const& a, T init) {
   LO n = a.size();
-  if (n == 0) {
-    hipLaunchKernelGGL((fill_kernel<T>), dim3(1), dim3(kBlock), 0, c.stream, 1, result, init);
-    OSH_HIP(hipGetLastError());
-    return;
-  }
+  if (n == 0) return init;
+  T* result = static_cast<T*>(c.pinned);
+  unsigned* signal = c.signal_word();
+  unsigned value = c.wait_tag();
   LO nb = LO(nblocks(n, kBlock * 4));
   if (nb > 1024) nb = 1024;
   if (nb == 1) {
     hipLaunchKernelGGL((reduce_blocks<T, Op>), dim3(1), dim3(kBlock), 0, c.stream, n, a.data(),
-        result, init);
+        result, init, signal, value);
   } else {
     T* part = static_cast<T*>(c.partials);
     hipLaunchKernelGGL((reduce_blocks<T, Op>), dim3(nb), dim3(kBlock), 0, c.stream, n, a.data(),
-        part, init);
+        part, init, (unsigned*)nullptr, 0u);
     OSH_HIP(hipGetLastError());
     hipLaunchKernelGGL((reduce_blocks<T, Op>), dim3(1), dim3(kBlock), 0, c.stream, nb, part,
-        result, init);
+        result, init, signal, value);
   }
   OSH_HIP(hipGetLastError());
-}
-
-template <class T, int Op>
-T reduce(Ctx& c, DArray<T> const& a, T init) {
-  if (a.size() == 0) return init;
-  reduce_to<T, Op>(c, a, init, static_cast<T*>(c.pinned));
-  return pinned_value<T>(c);
+  c.wait_signalled();
+  return read_slot<T>(c, 0);
 }
 
 }  // namespace
@@ -823,19 +843,76 @@ LOs offset_scan_bytes(Ctx& c, Bytes const& counts, LO* total) {
 
 LOs collect_marked(Ctx& c, Bytes const& marks) { return collect_marked(c, marks, nullptr); }
 
-void scatter_marked_list(Ctx& c, Bytes const& marks, LOs const& offsets, LOs& out) {
-  OSH_LAUNCH(scatter_marked, marks.size(), c, marks.data(), offsets.data(), out.data());
-}
-
 LOs collect_marked(Ctx& c, Bytes const& marks, LOs* offsets_out) {
   LO n = marks.size();
-  // the scan counts nonzero marks directly
-  LOs offsets = offset_scan_t<I8, true>(c, marks, static_cast<LO*>(c.pinned));
-  LO count = pinned_value<LO>(c);
-  LOs out(c, count);
-  OSH_LAUNCH(scatter_marked, n, c, marks.data(), offsets.data(), out.data());
-  if (offsets_out) *offsets_out = offsets;
+  // the scan counts nonzero marks directly and lists them in the same launch,
+  // in an array sized for all of them
+  LOs out(c, n);
+  if (offsets_out) *offsets_out = LOs(c, n + 1);
+  ScanJob job{marks.data(), kScanNonzero, n, offsets_out ? offsets_out->data() : nullptr,
+      slot_ptr<LO>(c, 0), out.data()};
+  if (n == 0) {
+    if (offsets_out) *offsets_out = fill_lo(c, 1, 0);
+    return out;
+  }
+  offset_scans(c, &job, 1);
+  out.shrink(pinned_value<LO>(c));
   return out;
+}
+
+namespace {
+
+struct FillJobs {
+  int n;
+  unsigned first[9];
+  void* p[8];
+  std::size_t bytes[8];
+  unsigned pattern[8];
+};
+
+// 16 bytes a thread; blocks come from the pool, so every start is aligned and
+// only the last bytes of a job need single stores
+__global__ void __launch_bounds__(kBlock) fill_jobs(FillJobs j) {
+  int w = 0;
+  while (w + 1 < j.n && blockIdx.x >= j.first[w + 1]) ++w;
+  std::size_t at = (std::size_t(blockIdx.x - j.first[w]) * kBlock + threadIdx.x) * 16;
+  std::size_t bytes = j.bytes[w];
+  char* p = static_cast<char*>(j.p[w]) + at;
+  unsigned v = j.pattern[w];
+  if (at + 16 <= bytes) {
+    *reinterpret_cast<uint4*>(p) = make_uint4(v, v, v, v);
+  } else {
+    for (int k = 0; at + k < bytes && k < 16; ++k) p[k] = char(v >> (8 * (k & 3)));
+  }
+}
+
+}  // namespace
+
+void Fills::add(void* p, std::size_t bytes, unsigned pattern) {
+  if (bytes == 0) return;
+  OSH_CHECK(n_ < kMax, "too many fills");
+  p_[n_] = p;
+  bytes_[n_] = bytes;
+  pattern_[n_] = pattern;
+  ++n_;
+}
+
+void Fills::run() {
+  FillJobs j{};
+  unsigned blocks = 0;
+  for (int i = 0; i < n_; ++i) {
+    j.p[i] = p_[i];
+    j.bytes[i] = bytes_[i];
+    j.pattern[i] = pattern_[i];
+    j.first[i] = blocks;
+    blocks += unsigned((bytes_[i] + 16 * kBlock - 1) / (16 * kBlock));
+    j.first[i + 1] = blocks;
+  }
+  j.n = n_;
+  n_ = 0;
+  if (blocks == 0) return;
+  hipLaunchKernelGGL(fill_jobs, dim3(blocks), dim3(kBlock), 0, c_.stream, j);
+  OSH_HIP(hipGetLastError());
 }
 
 LOs iota(Ctx& c, LO n, LO start, LO stride) {
@@ -864,9 +941,12 @@ Reals fill_real(Ctx& c, LO n, Real value) {
 
 I8 max_i8(Ctx& c, Bytes const& a) { return reduce<I8, kMax>(c, a, I8(-128)); }
 Real min_real(Ctx& c, Reals const& a) { return reduce<Real, kMin>(c, a, 1.79769313486231570815e+308); }
-void min_real_async(Ctx& c, Reals const& a, int slot) {
-  OSH_CHECK(slot >= 0 && slot < Ctx::kSlots, "pinned slot out of range");
-  reduce_to<Real, kMin>(c, a, 1.79769313486231570815e+308, slot_ptr<Real>(c, slot));
+Real min_real_wait(Ctx& c, Reals const& a) {
+  if (a.size() == 0) {
+    c.wait();
+    return 1.79769313486231570815e+308;
+  }
+  return min_real(c, a);
 }
 Real max_real(Ctx& c, Reals const& a) { return reduce<Real, kMax>(c, a, -1.79769313486231570815e+308); }
 LO sum_lo(Ctx& c, LOs const& a) { return reduce<LO, kSum>(c, a, 0); }

@@ -144,12 +144,25 @@ struct Ctx {
   // the same for callers that go on to read pinned words the kernels wrote
   // (not for copies into host memory, which only sync() completes)
   void wait();
-
- private:
-  unsigned signal_value = 0;
+  // Device words that kernels set to the tag of the coming wait and that the
+  // wait brings to the host: word_set(i, tag) after it.  A tag is never used
+  // twice, so nothing has to be cleared.
+  static constexpr int kWords = 4;
+  unsigned* words = nullptr;
+  unsigned wait_tag() const { return signal_value + 1; }
+  bool word_set(int i, unsigned tag) const {
+    return __atomic_load_n(host_words() + i, __ATOMIC_RELAXED) == tag;
+  }
+  // for a kernel that signals by itself, as its last store (a release at
+  // system scope of wait_tag() into signal_word()): waits for that
+  void wait_signalled();
   unsigned* signal_word() const {
     return reinterpret_cast<unsigned*>(static_cast<char*>(pinned) + 8 * kSlots + 64);
   }
+
+ private:
+  unsigned signal_value = 0;
+  unsigned* host_words() const { return signal_word() + 16; }
   void raise_device_error();
 };
 
@@ -183,6 +196,8 @@ template <class T>
 class DArray {
  public:
   DArray() = default;
+  // the array's first n entries (an array sized by an upper bound)
+  void shrink(LO n) { n_ = n < n_ ? n : n_; }
   DArray(Ctx& c, LO n) : n_(n), exists_(true) {
     OSH_CHECK(n >= 0, "negative array size");
     T* p = nullptr;
@@ -337,6 +352,7 @@ struct ScanJob {
   LO n;
   LO* out;    // n + 1 entries
   LO* total;  // device-visible grand total (a pinned slot), or nullptr
+  LO* list = nullptr;  // for nonzero flags: the indices of the nonzero ones
 };
 void offset_scans(Ctx& c, ScanJob const* jobs, int njobs);
 // the same scans with no allocation: the tile status words and ticket
@@ -350,18 +366,53 @@ void offset_scans_noalloc(Ctx& c, ScanJob const* jobs, int njobs);
 LOs offset_scan(Ctx& c, LOs const& counts, LO* total = nullptr);
 LOs offset_scan_bytes(Ctx& c, Bytes const& counts, LO* total = nullptr);
 LOs collect_marked(Ctx& c, Bytes const& marks);       // indices of nonzero
-// out[offsets[i]] = i for nonzero marks[i], with offsets from a nonzero scan
-void scatter_marked_list(Ctx& c, Bytes const& marks, LOs const& offsets, LOs& out);
 // the same, also returning the n+1 offsets of the nonzero marks
 LOs collect_marked(Ctx& c, Bytes const& marks, LOs* offsets_out);
+// fills of several arrays in one launch: add() allocates each, run() fills
+// all of them
+class Fills {
+ public:
+  explicit Fills(Ctx& c) : c_(c) {}
+  Fills(Fills const&) = delete;
+  Fills& operator=(Fills const&) = delete;
+  Bytes bytes(LO n, I8 value) {
+    Bytes a(c_, n);
+    unsigned b = static_cast<unsigned char>(value);
+    add(a.data(), std::size_t(n), b * 0x01010101u);
+    return a;
+  }
+  LOs ints(LO n, LO value) {
+    LOs a(c_, n);
+    add(a.data(), sizeof(LO) * std::size_t(n), static_cast<unsigned>(value));
+    return a;
+  }
+  // all bits zero: 0 and 0.0 of any type
+  template <class T>
+  DArray<T> zeros(LO n) {
+    DArray<T> a(c_, n);
+    add(a.data(), sizeof(T) * std::size_t(n), 0u);
+    return a;
+  }
+  void run();
+
+ private:
+  static constexpr int kMax = 8;
+  void add(void* p, std::size_t bytes, unsigned pattern);
+  Ctx& c_;
+  int n_ = 0;
+  void* p_[kMax];
+  std::size_t bytes_[kMax];
+  unsigned pattern_[kMax];
+};
 LOs iota(Ctx& c, LO n, LO start = 0, LO stride = 1);
 LOs fill_lo(Ctx& c, LO n, LO value);
 Bytes fill_i8(Ctx& c, LO n, I8 value);
 Reals fill_real(Ctx& c, LO n, Real value);
 I8 max_i8(Ctx& c, Bytes const& a);
 Real min_real(Ctx& c, Reals const& a);
-// the same without a sync: the minimum lands in pinned slot `slot`
-void min_real_async(Ctx& c, Reals const& a, int slot);
+// the same, bringing everything kernels left in pinned words with it
+// (Ctx::wait)
+Real min_real_wait(Ctx& c, Reals const& a);
 Real max_real(Ctx& c, Reals const& a);
 LO sum_lo(Ctx& c, LOs const& a);
 // stable sort of n tuples of `width` int64 keys; returns the permutation
