@@ -111,95 +111,142 @@ __global__ void transit_kernel(LO nuses, LO const* hm2m, I8 const* m2hm_codes,
 //               index (sort_by_high_index, src/Omega_h_adj.cpp:178-200)
 //               and forms the codes of separate_upward_with_codes (:202-217)
 // With `marks`, only the rows of marked lows are built (the rest are empty).
-__global__ void count_lows(LO nhl, LO const* hl2l, I8 const* marks, LO* counts, LO* slot) {
-  LO i = thread_index();
-  if (i >= nhl) return;
-  LO l = hl2l[i];
-  if (!marks || marks[l]) slot[i] = atomicAdd(&counts[l], 1);
+// Without `sorted`, rows keep the order of the atomics, for uses that do not
+// depend on it (one sweep less).  Several maps are inverted by the same
+// launches: job w owns the workgroups [first[w], first[w + 1]).
+struct UseJob {
+  LO nhl;
+  LO const* hl2l;
+  I8 const* marks;
+  LO* counts;
+  LO* slot;
+  LO const* a2ab;
+  int deg;
+  I8 const* down_codes;
+  int sorted;
+  LO* ab2hl;
+  LO* ab2b;
+  I8* codes;
+};
+constexpr int kMaxUseJobs = 3;
+struct UseJobs {
+  int n;
+  unsigned first[kMaxUseJobs + 1];
+  UseJob d[kMaxUseJobs];
+};
+
+__device__ __forceinline__ int use_job(UseJobs const& j, LO* i) {
+  int w = 0;
+  while (w + 1 < j.n && blockIdx.x >= j.first[w + 1]) ++w;
+  *i = LO(blockIdx.x - j.first[w]) * kBlock + LO(threadIdx.x);
+  return w;
 }
 
-__global__ void fill_uses(LO nhl, LO const* hl2l, I8 const* marks, LO const* a2ab,
-    LO const* slot, LO* ab2hl) {
-  LO hl = thread_index();
-  if (hl >= nhl) return;
-  LO l = hl2l[hl];
-  if (!marks || marks[l]) ab2hl[a2ab[l] + slot[hl]] = hl;
+__device__ __forceinline__ I8 use_code(UseJob const& a, LO hl) {
+  int which_down = hl % a.deg;
+  return a.down_codes ? make_code(code_is_flipped(a.down_codes[hl]),
+                            code_rotation(a.down_codes[hl]), which_down)
+                      : make_code(0, 0, which_down);
 }
 
-__global__ void rank_uses(LO nhl, LO const* hl2l, I8 const* marks, LO const* a2ab,
-    LO const* ab2hl, int deg, I8 const* down_codes, LO* ab2b, I8* codes) {
-  LO hl = thread_index();
-  if (hl >= nhl) return;
-  LO l = hl2l[hl];
-  if (marks && !marks[l]) return;
-  LO b = a2ab[l], e = a2ab[l + 1];
+__global__ void __launch_bounds__(kBlock) count_lows(UseJobs j) {
+  LO i;
+  UseJob const& a = j.d[use_job(j, &i)];
+  if (i >= a.nhl) return;
+  LO l = a.hl2l[i];
+  if (!a.marks || a.marks[l]) a.slot[i] = atomicAdd(&a.counts[l], 1);
+}
+
+__global__ void __launch_bounds__(kBlock) fill_uses(UseJobs j) {
+  LO hl;
+  UseJob const& a = j.d[use_job(j, &hl)];
+  if (hl >= a.nhl) return;
+  LO l = a.hl2l[hl];
+  if (a.marks && !a.marks[l]) return;
+  LO pos = a.a2ab[l] + a.slot[hl];
+  if (a.sorted) {
+    a.ab2hl[pos] = hl;
+  } else {
+    a.ab2b[pos] = hl / a.deg;
+    a.codes[pos] = use_code(a, hl);
+  }
+}
+
+__global__ void __launch_bounds__(kBlock) rank_uses(UseJobs j) {
+  LO hl;
+  UseJob const& a = j.d[use_job(j, &hl)];
+  if (hl >= a.nhl) return;
+  LO l = a.hl2l[hl];
+  if (a.marks && !a.marks[l]) return;
+  LO b = a.a2ab[l], e = a.a2ab[l + 1];
   LO rank = 0;
-  for (LO j = b; j < e; ++j) rank += (ab2hl[j] < hl);
-  int which_down = hl % deg;
-  I8 c = down_codes ? make_code(code_is_flipped(down_codes[hl]), code_rotation(down_codes[hl]),
-                          which_down)
-                    : make_code(0, 0, which_down);
-  ab2b[b + rank] = hl / deg;
-  codes[b + rank] = c;
+  for (LO k = b; k < e; ++k) rank += (a.ab2hl[k] < hl);
+  a.ab2b[b + rank] = hl / a.deg;
+  a.codes[b + rank] = use_code(a, hl);
 }
 
-// rows in atomic order, for uses that do not depend on the order of a row
-__global__ void fill_uses_unsorted(LO nhl, LO const* hl2l, I8 const* marks, LO const* a2ab,
-    LO const* slot, int deg, I8 const* down_codes, LO* ab2b, I8* codes) {
-  LO hl = thread_index();
-  if (hl >= nhl) return;
-  LO l = hl2l[hl];
-  if (marks && !marks[l]) return;
-  LO pos = a2ab[l] + slot[hl];
-  int which_down = hl % deg;
-  ab2b[pos] = hl / deg;
-  codes[pos] = down_codes ? make_code(code_is_flipped(down_codes[hl]),
-                                code_rotation(down_codes[hl]), which_down)
-                          : make_code(0, 0, which_down);
+struct Invert {
+  LO nhigh;
+  int deg;
+  LO nlow;
+  LOs hl2l;
+  Bytes const* down_codes;
+  Bytes const* marks;
+  bool sorted;
+};
+
+void invert_adjs(Ctx& c, int n, Invert const* in, Adj* out) {
+  OSH_CHECK(n >= 1 && n <= kMaxUseJobs, "invert_adjs: too many maps");
+  UseJobs j{};
+  LOs counts[kMaxUseJobs], slot[kMaxUseJobs], ab2hl[kMaxUseJobs];
+  ScanJob scans[kMaxUseJobs];
+  Fills fills(c);
+  unsigned blocks = 0;
+  for (int w = 0; w < n; ++w) {
+    LO nhl = in[w].nhigh * in[w].deg;
+    counts[w] = fills.ints(in[w].nlow, 0);
+    slot[w] = LOs(c, nhl);
+    out[w].a2ab = LOs(c, in[w].nlow + 1);
+    // with marks the rows hold at most nhl uses; the size stays an upper bound
+    out[w].ab2b = LOs(c, nhl);
+    out[w].codes = Bytes(c, nhl);
+    if (in[w].sorted) ab2hl[w] = LOs(c, nhl);
+    j.d[w] = UseJob{nhl, in[w].hl2l.data(), in[w].marks ? in[w].marks->data() : nullptr,
+        counts[w].data(), slot[w].data(), out[w].a2ab.data(), in[w].deg,
+        in[w].down_codes ? in[w].down_codes->data() : nullptr, in[w].sorted ? 1 : 0,
+        in[w].sorted ? ab2hl[w].data() : nullptr, out[w].ab2b.data(), out[w].codes.data()};
+    scans[w] = {counts[w].data(), kScanLO, in[w].nlow, out[w].a2ab.data(), nullptr};
+    j.first[w] = blocks;
+    blocks += nblocks(nhl);
+    j.first[w + 1] = blocks;
+  }
+  j.n = n;
+  fills.run();
+  auto launch = [&](auto kernel, UseJobs const& jobs, unsigned nb) {
+    if (nb == 0) return;
+    hipLaunchKernelGGL(kernel, dim3(nb), dim3(kBlock), 0, c.stream, jobs);
+    OSH_HIP(hipGetLastError());
+  };
+  launch(count_lows, j, blocks);
+  offset_scans(c, scans, n);
+  launch(fill_uses, j, blocks);
+  UseJobs s{};
+  blocks = 0;
+  for (int w = 0; w < n; ++w) {
+    if (!in[w].sorted) continue;
+    s.d[s.n] = j.d[w];
+    s.first[s.n++] = blocks;
+    blocks += nblocks(j.d[w].nhl);
+    s.first[s.n] = blocks;
+  }
+  launch(rank_uses, s, blocks);
 }
 
-// With `marks`, only marked lows get rows; with `marked`, the list of marked
-// lows comes from the same scan launch; without `sorted`, rows keep the
-// order of the atomics (one sweep less)
-Adj invert_adj(Ctx& c, LO nhigh, int deg, LO nlow, LOs const& hl2l, Bytes const* down_codes,
-    Bytes const* marks = nullptr, LOs* marked = nullptr, bool sorted = true,
-    LOs* marked_index = nullptr) {
-  LO nhl = nhigh * deg;
-  I8 const* mk = marks ? marks->data() : nullptr;
-  LOs counts = fill_lo(c, nlow, 0);
-  LOs slot(c, nhl);
-  OSH_LAUNCH(count_lows, nhl, c, hl2l.data(), mk, counts.data(), slot.data());
-  Adj a;
-  a.a2ab = LOs(c, nlow + 1);
-  if (marked) {
-    LOs marked_offsets;
-    if (marked_index) marked_offsets = LOs(c, nlow + 1);
-    *marked = LOs(c, nlow);
-    ScanJob jobs[2] = {{counts.data(), kScanLO, nlow, a.a2ab.data(), nullptr},
-        {mk, kScanNonzero, nlow, marked_index ? marked_offsets.data() : nullptr,
-            slot_ptr<LO>(c, 1), marked->data()}};
-    offset_scans(c, jobs, nlow ? 2 : 1);
-    c.wait();
-    marked->shrink(nlow ? read_slot<LO>(c, 1) : 0);
-    if (marked_index) *marked_index = marked_offsets;
-  } else {
-    ScanJob job{counts.data(), kScanLO, nlow, a.a2ab.data(), nullptr};
-    offset_scans(c, &job, 1);
-  }
-  // with marks the rows hold at most nhl uses; the size stays an upper bound
-  a.ab2b = LOs(c, nhl);
-  a.codes = Bytes(c, nhl);
-  I8 const* dc = down_codes ? down_codes->data() : nullptr;
-  if (sorted) {
-    LOs ab2hl(c, nhl);
-    OSH_LAUNCH(fill_uses, nhl, c, hl2l.data(), mk, a.a2ab.data(), slot.data(), ab2hl.data());
-    OSH_LAUNCH(rank_uses, nhl, c, hl2l.data(), mk, a.a2ab.data(), ab2hl.data(), deg, dc,
-        a.ab2b.data(), a.codes.data());
-  } else {
-    OSH_LAUNCH(fill_uses_unsorted, nhl, c, hl2l.data(), mk, a.a2ab.data(), slot.data(), deg, dc,
-        a.ab2b.data(), a.codes.data());
-  }
-  return a;
+Adj invert_adj(Ctx& c, LO nhigh, int deg, LO nlow, LOs const& hl2l, Bytes const* down_codes) {
+  Invert in{nhigh, deg, nlow, hl2l, down_codes, nullptr, true};
+  Adj out;
+  invert_adjs(c, 1, &in, &out);
+  return out;
 }
 
 // reflect_down: each existing lower entity is listed once, in the row of its
@@ -494,12 +541,21 @@ LOs const& ask_down(Ctx& c, DMesh& m, int high, int low, Bytes const** codes) {
   return m.t2e;
 }
 
-Adj marked_up(Ctx& c, DMesh& m, int low, int high, Bytes const& marks, LOs* marked,
-    bool sorted, LOs* marked_index) {
-  Bytes const* codes = nullptr;
-  LOs const& down = ask_down(c, m, high, low, &codes);
-  return invert_adj(c, m.nents[high], simplex_degree(high, low), m.nents[low], down, codes,
-      &marks, marked, sorted, marked_index);
+void marked_ups(Ctx& c, DMesh& m, int low, Bytes const& marks, int n, int const* highs,
+    bool const* sorted, Adj* out) {
+  Invert in[kMaxUseJobs];
+  OSH_CHECK(n <= kMaxUseJobs, "marked_ups: too many dimensions");
+  for (int w = 0; w < n; ++w) {
+    Bytes const* codes = nullptr;
+    in[w].hl2l = ask_down(c, m, highs[w], low, &codes);
+    in[w].down_codes = codes;
+    in[w].nhigh = m.nents[highs[w]];
+    in[w].deg = simplex_degree(highs[w], low);
+    in[w].nlow = m.nents[low];
+    in[w].marks = &marks;
+    in[w].sorted = sorted[w];
+  }
+  invert_adjs(c, n, in, out);
 }
 
 Adj const& ask_up(Ctx& c, DMesh& m, int low, int high) {

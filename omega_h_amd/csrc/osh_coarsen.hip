@@ -27,35 +27,35 @@ constexpr I8 kDont = 0;
 __device__ __forceinline__ bool collapses(I8 code, int col) { return (code & (1 << col)) != 0; }
 __device__ __forceinline__ I8 dont_collapse(I8 code, int col) { return I8(code & ~(1 << col)); }
 
-__global__ void lt_kernel(LO n, Real const* a, Real v, I8* out) {
-  LO i = thread_index();
-  if (i < n) out[i] = a[i] < v;
+// the vertices of edges shorter than `shortest`
+__global__ void mark_short_edges(LO ne, Real const* lengths, Real shortest, LO const* ev2v,
+    I8* vmarks) {
+  LO e = thread_index();
+  if (e >= ne || !(lengths[e] < shortest)) return;
+  vmarks[ev2v[e * 2]] = 1;
+  vmarks[ev2v[e * 2 + 1]] = 1;
 }
 
-__global__ void edge_codes_from_verts(LO ne, LO const* ev2v, I8 const* vmarks, I8* codes) {
+// the collapse directions of each edge: away from its marked ends
+// (src/Omega_h_coarsen.cpp:29-47), as far as classification allows
+// (check_collapse_class, src/Omega_h_check_collapse.cpp:10-40)
+__global__ void collapse_codes(LO ne, LO const* ev2v, I8 const* vmarks, I8 const* vdim,
+    I8 const* edim, I8* codes) {
   LO e = thread_index();
   if (e >= ne) return;
+  LO v[2] = {ev2v[e * 2], ev2v[e * 2 + 1]};
   I8 code = kDont;
   for (int eev = 0; eev < 2; ++eev)
-    if (vmarks[ev2v[e * 2 + eev]]) code = I8(code | (1 << eev));
-  codes[e] = code;
-}
-
-__global__ void check_class_kernel(LO ne, LO const* ev2v, I8 const* vdim, I8 const* edim,
-    I8* codes) {
-  LO e = thread_index();
-  if (e >= ne) return;
-  I8 code = codes[e];
-  if (code == kDont) return;
-  int cd0 = vdim[ev2v[e * 2]], cd1 = vdim[ev2v[e * 2 + 1]];
-  int ecd = edim[e];
-  I8 orig = code;
-  if (cd0 == cd1) {
-    if (cd0 != ecd) code = kDont;
-  } else {
-    int cds[2] = {cd0, cd1};
-    for (int col = 0; col < 2; ++col)
-      if (collapses(orig, col) && cds[col] != ecd) code = dont_collapse(code, col);
+    if (vmarks[v[eev]]) code = I8(code | (1 << eev));
+  if (code != kDont) {
+    int cds[2] = {vdim[v[0]], vdim[v[1]]};
+    int ecd = edim[e];
+    if (cds[0] == cds[1]) {
+      if (cds[0] != ecd) code = kDont;
+    } else {
+      for (int col = 0; col < 2; ++col)
+        if (cds[col] != ecd) code = dont_collapse(code, col);
+    }
   }
   codes[e] = code;
 }
@@ -73,223 +73,279 @@ __device__ __forceinline__ int local_vertex(LO const* cv, LO v) {
   return k;
 }
 
+// the cells (faces and tets) of a sweep that looks at each cell's edges and
+// sides: job w owns the workgroups [first[w], first[w + 1])
+struct CellSweep {
+  int n;
+  unsigned first[3];
+  int dim[2];
+  LO ncells[2];
+  LO const* c2e[2];
+  LO const* cv2v[2];
+  LO const* cs2s[2];
+  I8 const* cdim[2];
+  I8 const* sdim[2];
+  I8* dead_cells[2];
+  I8* dead_sides[2];
+};
+
 template <int CD>
-__global__ void check_exposure_cells(LO ncells, LO const* c2e, LO const* cv2v, LO const* cs2s,
-    I8 const* cdim, I8 const* sdim, LO const* ev2v, I8 const* codes, I8* veto) {
-  LO c = thread_index();
-  if (c >= ncells) return;
+__device__ __forceinline__ void check_exposure(LO c, CellSweep const& a, int w,
+    LO const* ev2v, I8 const* codes, I8* veto) {
+  if (c >= a.ncells[w]) return;
   constexpr int nepc = (CD == 3) ? 6 : 3;
-  LO const* cv = cv2v + c * (CD + 1);
+  LO const* cv = a.cv2v[w] + std::size_t(c) * (CD + 1);
   for (int j = 0; j < nepc; ++j) {
-    LO e = c2e[c * nepc + j];
+    LO e = a.c2e[w][std::size_t(c) * nepc + j];
     I8 code = codes[e];
     if (code == kDont) continue;
     for (int col = 0; col < 2; ++col) {
       if (!collapses(code, col)) continue;
       int ccv_onto = local_vertex<CD>(cv, ev2v[e * 2 + (1 - col)]);
       int ccs_opp = opposite_template(CD, 0, ccv_onto);
-      if (sdim[cs2s[c * (CD + 1) + ccs_opp]] != cdim[c]) veto[e * 2 + col] = 1;
+      if (a.sdim[w][a.cs2s[w][std::size_t(c) * (CD + 1) + ccs_opp]] != a.cdim[w][c])
+        veto[e * 2 + col] = 1;
     }
   }
 }
 
-// the vetoed sides of the candidate edges leave their codes
-__global__ void apply_edge_vetoes(LO ncands, LO const* cands, I8 const* veto, I8* codes) {
-  LO i = thread_index();
-  if (i >= ncands) return;
-  LO e = cands[i];
-  I8 code = codes[e];
-  for (int col = 0; col < 2; ++col)
-    if (veto[e * 2 + col]) code = dont_collapse(code, col);
-  codes[e] = code;
+__device__ __forceinline__ int cell_job(CellSweep const& a, LO* c) {
+  int w = (a.n > 1 && blockIdx.x >= a.first[1]) ? 1 : 0;
+  *c = LO(blockIdx.x - a.first[w]) * kBlock + LO(threadIdx.x);
+  return w;
+}
+
+__global__ void __launch_bounds__(kBlock) check_exposure_cells(CellSweep a, LO const* ev2v,
+    I8 const* codes, I8* veto) {
+  LO c;
+  int w = cell_job(a, &c);
+  if (a.dim[w] == 3)
+    check_exposure<3>(c, a, w, ev2v, codes, veto);
+  else
+    check_exposure<2>(c, a, w, ev2v, codes, veto);
 }
 
 // Each collapse side (candidate edge, direction) gets 2^lshift threads
-// (Tuning::coarsen_lanes), which split the collapsing vertex's row between
-// them, so that passes with few candidates still spread their work over the
-// device.  Minima do not depend on how a row is split, so the lane count
-// changes no result.  The product builders below use kLanes threads per key.
+// (Tuning::coarsen_lanes, at most 32 so that an edge's two sides share a
+// wave), which split the collapsing vertex's row between them, so that passes
+// with few candidates still spread their work over the device.  Minima do not
+// depend on how a row is split, so the lane count changes no result.  The two
+// sides' verdicts meet through ballots and one lane writes the edge's code.
+// The product builders below use kLanes threads per key.
 constexpr int kLanes = 8;
+constexpr int kMaxSideLanes = 32;
+
+// the lanes of a side and of its edge in the wave
+struct SideLanes {
+  int lane;
+  int base;  // the side's first lane
+  unsigned long long side;  // its lanes
+  __device__ __forceinline__ SideLanes(LO t, int lshift) {
+    int lanes = 1 << lshift;
+    lane = int(t) & (lanes - 1);
+    base = int(threadIdx.x % 64) & ~(lanes - 1);
+    side = ((1ull << lanes) - 1ull) << base;
+  }
+  __device__ __forceinline__ bool any(bool x) const { return (__ballot(x) & side) != 0ull; }
+};
+
+// writes the code of the edge whose sides' verdicts are `keep`
+__device__ __forceinline__ void write_code(SideLanes const& s, int lshift, int col, bool keep,
+    I8 code, LO e, I8* codes) {
+  unsigned long long b = __ballot(keep);
+  if (col != 0 || s.lane != 0) return;
+  I8 out = code;
+  if (!((b >> s.base) & 1ull)) out = dont_collapse(out, 0);
+  if (!((b >> (s.base + (1 << lshift))) & 1ull)) out = dont_collapse(out, 1);
+  if (out != code) codes[e] = out;
+}
 
 // prevent_coarsen_overshoot: a side is vetoed when any new edge would reach
-// max_length (the order of the row does not matter).  F32 (mixed
-// precision): the lengths are FP32 estimates; a side is vetoed when one is
-// over max_length by more than the screening band, and sides with a length
-// inside the band are marked in `need` for the FP64 sweep.  With `need`
-// given, the FP64 sweep looks only at marked sides not already vetoed.
-template <int D, int M, bool F32>
+// max_length (the order of the row does not matter); sides vetoed by exposure
+// leave their codes here too.  MIXED: FP32 estimates first; a side is vetoed
+// when one is over max_length by more than the screening band, and measured
+// in FP64 only when none is but one lies inside the band.
+template <int D, int M, bool MIXED>
 __global__ void overshoot_lanes(LO nt, int lshift, LO const* cands, LO const* ev2v,
     LO const* v2e_a2ab, LO const* v2e_ab2b, I8 const* v2e_codes, Real const* coords,
-    Real const* metric, Real max_length, I8 const* codes, I8* veto, I8* need) {
+    Real const* metric, Real max_length, I8 const* exposed, I8* codes) {
   LO t = thread_index();
   if (t >= nt) return;
   LO side = t >> lshift;
-  int lane = t & ((1 << lshift) - 1);
+  SideLanes s(t, lshift);
   LO e = cands[side / 2];
   int col = side % 2;
-  if (!collapses(codes[e], col)) return;
-  if (!F32 && need && (!need[side] || veto[side])) return;
+  I8 code = codes[e];
   constexpr int nc = (M == 1) ? 1 : (M == 2 ? 3 : 6);
   LO v_col = ev2v[e * 2 + col];
   LO v_onto = ev2v[e * 2 + (1 - col)];
-  for (LO ve = v2e_a2ab[v_col] + lane; ve < v2e_a2ab[v_col + 1]; ve += (1 << lshift)) {
+  bool open = collapses(code, col) && !exposed[e * 2 + col];
+  LO row = open ? v2e_a2ab[v_col] : 0;
+  LO end = open ? v2e_a2ab[v_col + 1] : 0;
+  // the ends of the new edge at row entry ve; false for the candidate itself
+  auto ends = [&](LO ve, double (&p0)[D], double (&p1)[D], double (&m0)[nc], double (&m1)[nc]) {
     LO e2 = v2e_ab2b[ve];
-    if (e2 == e) continue;
+    if (e2 == e) return false;
     int eev_in = code_which_down(v2e_codes[ve]);
-    int eev_out = 1 - eev_in;
-    LO nv[2];
-    nv[eev_in] = v_onto;
-    nv[eev_out] = ev2v[e2 * 2 + eev_out];
-    double p0[D], p1[D], m0[nc], m1[nc];
+    LO out = ev2v[e2 * 2 + 1 - eev_in];
+    LO a = eev_in == 0 ? v_onto : out, b = eev_in == 0 ? out : v_onto;
     for (int k = 0; k < D; ++k) {
-      p0[k] = coords[nv[0] * D + k];
-      p1[k] = coords[nv[1] * D + k];
+      p0[k] = coords[a * D + k];
+      p1[k] = coords[b * D + k];
     }
     for (int k = 0; k < nc; ++k) {
-      m0[k] = metric[nv[0] * nc + k];
-      m1[k] = metric[nv[1] * nc + k];
+      m0[k] = metric[a * nc + k];
+      m1[k] = metric[b * nc + k];
     }
-    if constexpr (F32) {
+    return true;
+  };
+  double p0[D], p1[D], m0[nc], m1[nc];
+  bool veto = false;
+  if constexpr (MIXED) {
+    bool unsure = false;
+    float lmax = float(max_length);
+    for (LO ve = row + s.lane; ve < end; ve += (1 << lshift)) {
+      if (!ends(ve, p0, p1, m0, m1)) continue;
       float l = f32::edge_length<D, M>(p0, p1, m0, m1);
-      float lmax = float(max_length);
-      if (l >= lmax * (1.0f + f32::kScreenBand)) {
-        veto[side] = 1;
-        return;
-      }
-      if (!(l < lmax * (1.0f - f32::kScreenBand))) need[side] = 1;
-    } else {
-      if (edge_length<D, M>(p0, p1, m0, m1) >= max_length) {
-        veto[side] = 1;
-        return;
-      }
+      veto = veto || l >= lmax * (1.0f + f32::kScreenBand);
+      unsure = unsure || !(l < lmax * (1.0f - f32::kScreenBand));
     }
+    veto = s.any(veto);
+    if (veto || !s.any(unsure)) end = row;
   }
+  for (LO ve = row + s.lane; ve < end && !veto; ve += (1 << lshift))
+    if (ends(ve, p0, p1, m0, m1)) veto = edge_length<D, M>(p0, p1, m0, m1) >= max_length;
+  write_code(s, lshift, col, open && !s.any(veto), code, e, codes);
 }
 
-__global__ void apply_vetoes(LO ncands, LO const* cands, I8 const* veto, I8* codes) {
-  LO i = thread_index();
-  if (i >= ncands) return;
-  LO e = cands[i];
-  I8 code = codes[e];
-  for (int col = 0; col < 2; ++col)
-    if (veto[i * 2 + col]) code = dont_collapse(code, col);
-  codes[e] = code;
+// the vertices' metric determinants, which every quality around a vertex
+// needs (24 times in a tet mesh)
+template <int M>
+__global__ void vert_dets(LO nv, Real const* metric, Real* dets) {
+  LO v = thread_index();
+  if (v >= nv) return;
+  constexpr int nc = (M == 2) ? 3 : 6;
+  double m[nc];
+  for (int k = 0; k < nc; ++k) m[k] = metric[std::size_t(v) * nc + k];
+  dets[v] = det<M>(get_symm<M>(m));
 }
 
-// coarsen_qualities: each lane folds the qualities of its share of the
-// collapsing vertex's cells (those that survive the collapse, with v_col
-// moved onto v_onto) into a partial minimum.  F32 (mixed precision): the
-// qualities are FP32 estimates, and a lane that meets an element whose
-// max-determinant metric is not clear marks its side in `unsure`.  With
-// `need` given, the FP64 sweep evaluates only the marked sides.
-template <int D, int M, bool F32>
-__global__ void __launch_bounds__(kBlock, 6) coarsen_quality_lanes(LO nt, int lshift,
-    LO const* cands, LO const* ev2v, LO const* cv2v, LO const* v2c_a2ab, LO const* v2c_ab2b,
-    I8 const* v2c_codes, Real const* coords, Real const* metric, I8 const* codes,
-    I8 const* need, I8* unsure, Real* partial) {
+// coarsen_qualities with its filters (src/Omega_h_coarsen_qualities.cpp:16-122):
+// the minimum quality of the cells that survive a collapse, with v_col moved
+// onto v_onto; a side is kept when it reaches qmin and, with `improve`, exceeds
+// the old minimum around v_col.  FILTER off: every side's minimum goes to
+// quals and nothing is kept or dropped.
+//
+// Bound by FP64 issue (166 operations a quality and its correctly rounded
+// divisions), so work is left out where it decides nothing: the determinants
+// come from vert_dets, a lane reads only the metric it uses, and a side stops
+// at the first cell below qmin unless it has to know the old minimum too.
+//
+// MIXED: FP32 estimates first; a side is rejected (quality -1) when their
+// minimum is below qmin by more than the band and every element's
+// max-determinant metric was clear, else evaluated in FP64.
+struct SideQualities {
+  LO const* cands;
+  LO const* ev2v;
+  LO const* cv2v;
+  LO const* v2c_a2ab;
+  LO const* v2c_ab2b;
+  I8 const* v2c_codes;
+  Real const* coords;
+  Real const* metric;
+  Real const* dets;
+  Real qmin;
+  Real const* old_quals;  // improve: the elements' qualities (else null)
+  I8* codes;
+  Real* quals;  // by (edge, direction); by (candidate, direction) with FILTER off
+};
+
+template <int D, int M, bool MIXED, bool FILTER>
+__global__ void __launch_bounds__(kBlock) coarsen_quality_lanes(LO nt, int lshift,
+    SideQualities a) {
   LO t = thread_index();
   if (t >= nt) return;
   LO side = t >> lshift;
-  int lane = t & ((1 << lshift) - 1);
-  LO e = cands[side / 2];
+  SideLanes s(t, lshift);
+  int lanes = 1 << lshift;
+  LO e = a.cands[side / 2];
   int col = side % 2;
-  double minqual = 1.0;
-  float minq32 = 1.0f;
-  bool unclear = false;
-  if (collapses(codes[e], col) && (F32 || !need || need[side])) {
-    constexpr int nc = (M == 1) ? 1 : (M == 2 ? 3 : 6);
-    LO v_col = ev2v[e * 2 + col];
-    LO v_onto = ev2v[e * 2 + (1 - col)];
-    for (LO vc = v2c_a2ab[v_col] + lane; vc < v2c_a2ab[v_col + 1]; vc += (1 << lshift)) {
-      LO c = v2c_ab2b[vc];
-      int ccv_col = code_which_down(v2c_codes[vc]);
+  I8 code = a.codes[e];
+  constexpr int nc = (M == 1) ? 1 : (M == 2 ? 3 : 6);
+  bool open = collapses(code, col);
+  LO v_col = a.ev2v[e * 2 + col];
+  LO v_onto = a.ev2v[e * 2 + (1 - col)];
+  LO row = open ? a.v2c_a2ab[v_col] : 0;
+  LO end = open ? a.v2c_a2ab[v_col + 1] : 0;
+  // the vertices of row entry vc's cell after the collapse; false if it dies
+  auto moved = [&](LO vc, LO (&cv)[D + 1]) {
+    LO c = a.v2c_ab2b[vc];
+    int ccv_col = code_which_down(a.v2c_codes[vc]);
+    bool lives = true;
+#pragma unroll
+    for (int k = 0; k < D + 1; ++k) {
+      cv[k] = a.cv2v[std::size_t(c) * (D + 1) + k];
+      if (k != ccv_col && cv[k] == v_onto) lives = false;
+    }
+#pragma unroll
+    for (int k = 0; k < D + 1; ++k)
+      if (k == ccv_col) cv[k] = v_onto;
+    return lives;
+  };
+  bool rejected = false;
+  double const* pp[D + 1];
+  double const* ms[D + 1];
+  if constexpr (MIXED) {
+    float minq = 1.0f;
+    bool unclear = false;
+    for (LO vc = row + s.lane; vc < end; vc += lanes) {
       LO cv[D + 1];
-      bool will_die = false;
+      if (!moved(vc, cv)) continue;
       for (int k = 0; k < D + 1; ++k) {
-        cv[k] = cv2v[c * (D + 1) + k];
-        if (k != ccv_col && cv[k] == v_onto) will_die = true;
+        pp[k] = a.coords + std::size_t(cv[k]) * D;
+        ms[k] = a.metric + std::size_t(cv[k]) * nc;
       }
-      if (will_die) continue;
-      cv[ccv_col] = v_onto;
-      // the quality reads the vertices' coordinates and metrics where they
-      // lie, so that they are loaded as they are used rather than all held
-      // at once (fewer live registers, more waves per SIMD)
-      double const* pp[D + 1];
-      double const* ms[D + 1];
-      for (int k = 0; k < D + 1; ++k) {
-        pp[k] = coords + cv[k] * D;
-        ms[k] = metric + cv[k] * nc;
-      }
-      if constexpr (F32) {
-        float q = f32::element_quality<D, M>(pp, ms, &unclear);
-        minq32 = (q < minq32) ? q : minq32;
-      } else {
-        minqual = math::min2(minqual, element_quality<D, M>(pp, ms));
+      float q = f32::element_quality<D, M>(pp, ms, &unclear);
+      minq = (q < minq) ? q : minq;
+    }
+    for (int d = lanes / 2; d > 0; d >>= 1) {
+      float o = __shfl_xor(minq, d, 64);
+      minq = (o < minq) ? o : minq;
+    }
+    rejected = open && !s.any(unclear) &&
+               double(minq) < a.qmin * (1.0 - double(f32::kScreenBand));
+    if (rejected) end = row;
+  }
+  double minq = 1.0;
+  double vold = 1.79769313486231570815e+308;
+  for (LO b = row; b < end; b += lanes) {
+    LO vc = b + s.lane;
+    LO cv[D + 1];
+    if (vc < end) {
+      if (FILTER && a.old_quals) vold = math::min2(vold, a.old_quals[a.v2c_ab2b[vc]]);
+      if (moved(vc, cv)) {
+        double dets[D + 1];
+        for (int k = 0; k < D + 1; ++k) {
+          pp[k] = a.coords + std::size_t(cv[k]) * D;
+          ms[k] = a.metric + std::size_t(cv[k]) * nc;
+          dets[k] = a.dets[cv[k]];
+        }
+        minq = math::min2(minq, element_quality<D, M>(pp, ms, dets));
       }
     }
+    if (FILTER && !a.old_quals && s.any(minq < a.qmin)) break;
   }
-  if constexpr (F32) {
-    if (unclear) unsure[side] = 1;
-    partial[t] = double(minq32);
+  for (int d = lanes / 2; d > 0; d >>= 1) {
+    minq = math::min2(minq, __shfl_xor(minq, d, 64));
+    vold = math::min2(vold, __shfl_xor(vold, d, 64));
+  }
+  if (rejected || !open) minq = -1.0;
+  if constexpr (FILTER) {
+    bool keep = open && minq >= a.qmin && (!a.old_quals || minq > vold);
+    if (keep && s.lane == 0) a.quals[std::size_t(e) * 2 + col] = minq;
+    write_code(s, lshift, col, keep, code, e, a.codes);
   } else {
-    partial[t] = minqual;
-  }
-}
-
-// the minimum over the lanes: the minimum over the row, as the reference's
-// loop computes it (min2 never takes a NaN, and a zero's sign decides
-// nothing downstream: the filters, rails and independent set compare it
-// only).  After a mixed-precision screen (`need` given) a side the screen
-// rejected gets -1, below every quality threshold.
-__global__ void combine_quality_lanes(LO ncands, int lanes, LO const* cands, I8 const* codes,
-    I8 const* need, Real const* partial, Real* quals) {
-  LO i = thread_index();
-  if (i >= ncands) return;
-  LO e = cands[i];
-  I8 code = codes[e];
-  for (int col = 0; col < 2; ++col) {
-    double q = -1.0;
-    if (collapses(code, col) && (!need || need[i * 2 + col])) {
-      q = 1.0;
-      for (int l = 0; l < lanes; ++l) q = math::min2(q, partial[(i * 2 + col) * lanes + l]);
-    }
-    quals[e * 2 + col] = q;
-  }
-}
-
-// the screen's verdict per side: FP64 is needed unless the FP32 minimum is
-// below qmin by more than the band and every element's metric was clear
-// (a NaN estimate compares false and is evaluated again)
-__global__ void screen_quality_sides(LO nsides, int lanes, LO const* cands, I8 const* codes,
-    I8 const* unsure, Real const* partial, Real qmin, I8* need) {
-  LO side = thread_index();
-  if (side >= nsides) return;
-  LO e = cands[side / 2];
-  int col = side % 2;
-  if (!collapses(codes[e], col)) {
-    need[side] = 0;
-    return;
-  }
-  double q = 1.0;
-  for (int l = 0; l < lanes; ++l) q = math::min2(q, partial[side * lanes + l]);
-  bool reject = !unsure[side] && q < qmin * (1.0 - double(f32::kScreenBand));
-  need[side] = reject ? 0 : 1;
-}
-
-// combine_quality_lanes with one output row per candidate (the layout of
-// the reference's coarsen_qualities, two values per candidate)
-__global__ void combine_to_cands(LO ncands, int lanes, LO const* cands, I8 const* codes,
-    I8 const* need, Real const* partial, Real* out) {
-  LO i = thread_index();
-  if (i >= ncands) return;
-  I8 code = codes[cands[i]];
-  for (int col = 0; col < 2; ++col) {
-    double q = -1.0;
-    if (collapses(code, col) && (!need || need[i * 2 + col])) {
-      q = 1.0;
-      for (int l = 0; l < lanes; ++l) q = math::min2(q, partial[(i * 2 + col) * lanes + l]);
-    }
-    out[i * 2 + col] = q;
+    if (s.lane == 0) a.quals[side] = minq;
   }
 }
 
@@ -309,134 +365,154 @@ __global__ void mark_collapsing_verts(LO ncands, LO const* cands, LO const* ev2v
     if (collapses(code, col)) vmarks[ev2v[e * 2 + col]] = 1;
 }
 
-// the vertex star (verts_across_edges, src/Omega_h_adj.cpp:512-530) of the
-// vertices whose vertex -> edge rows are built
-__global__ void star_from_v2e(LO nv, LO const* a2ab, LO const* ab2b, I8 const* codes,
-    LO const* ev2v, LO* out) {
-  LO v = thread_index();
-  if (v >= nv) return;
-  for (LO ve = a2ab[v]; ve < a2ab[v + 1]; ++ve)
-    out[ve] = ev2v[ab2b[ve] * 2 + (1 - code_which_down(codes[ve]))];
+// choose_rails (src/Omega_h_collapse_rail.cpp:15-60): each vertex that can
+// collapse takes the shortest of its edges that allow it, the one of higher
+// quality among equally long ones, the first one of those; and the vertex star
+// (verts_across_edges, src/Omega_h_adj.cpp:512-530) of the vertices whose rows
+// are built.  kLanes threads per vertex share its row: a chain of some 14
+// dependent gathers a vertex otherwise (41 us for the two sweeps on the 64^3
+// workload).  A length or quality that is not a number leaves the row to one
+// lane, since the choice then depends on the order of the comparisons.
+struct Rails {
+  LO const* a2ab;
+  LO const* ab2b;
+  I8 const* v2e_codes;
+  I8 const* codes;
+  LO const* ev2v;
+  Real const* lengths;
+  Real const* quals;
+};
+
+__device__ __forceinline__ bool better_rail(double len, double q, double best_len,
+    double best_q) {
+  return len < best_len || (len == best_len && q > best_q);
 }
 
-__global__ void vert_min_quality(LO nv, LO const* a2ab, LO const* ab2b, Real const* q, Real* out) {
-  LO v = thread_index();
-  if (v >= nv) return;
-  double r = 1.79769313486231570815e+308;
-  for (LO j = a2ab[v]; j < a2ab[v + 1]; ++j) r = math::min2(r, q[ab2b[j]]);
-  out[v] = r;
-}
-
-__global__ void filter_quals_kernel(LO ncands, LO const* cands, LO const* ev2v,
-    Real const* quals, Real qmin, Real const* vold, I8* codes) {
-  LO i = thread_index();
-  if (i >= ncands) return;
-  LO e = cands[i];
-  I8 code = codes[e];
-  if (code == kDont) return;
-  for (int col = 0; col < 2; ++col)
-    if (!(quals[e * 2 + col] >= qmin)) code = dont_collapse(code, col);
-  if (vold)
-    for (int col = 0; col < 2; ++col)
-      if (!(quals[e * 2 + col] > vold[ev2v[e * 2 + col]])) code = dont_collapse(code, col);
-  codes[e] = code;
-}
-
-__global__ void choose_rails_kernel(LO nv, LO const* v2e_a2ab, LO const* v2e_ab2b,
-    I8 const* v2e_codes, I8 const* codes, Real const* lengths, Real const* quals, I8* vcand,
-    Real* vqual, LO* vrail) {
-  LO v = thread_index();
-  if (v >= nv) return;
-  LO best = -1;
-  double best_len = -1, best_q = -1;
-  I8 is_cand = 0;
-  for (LO ve = v2e_a2ab[v]; ve < v2e_a2ab[v + 1]; ++ve) {
-    LO e = v2e_ab2b[ve];
-    I8 code = codes[e];
-    if (code == kDont) continue;
-    int eev = code_which_down(v2e_codes[ve]);
-    if (!collapses(code, eev)) continue;
-    double len = lengths[e];
-    double q = quals[e * 2 + eev];
-    if (best == -1 || len < best_len || (len == best_len && q > best_q)) {
-      is_cand = 1;
+__global__ void choose_rails_kernel(std::int64_t nt, Rails r, I8* vcand, Real* vqual,
+    LO* vrail, LO* star) {
+  std::int64_t t = thread_index64();
+  if (t >= nt) return;
+  LO v = LO(t / kLanes);
+  int lane = int(t % kLanes);
+  LO b = r.a2ab[v], end = r.a2ab[v + 1];
+  if (b == end) {
+    if (lane == 0) vcand[v] = 0;
+    return;
+  }
+  LO best = -1, at = 0x7fffffff;
+  double best_len = 0.0, best_q = 0.0;
+  bool nan = false;
+  auto visit = [&](LO ve) {
+    LO e = r.ab2b[ve];
+    int eev = code_which_down(r.v2e_codes[ve]);
+    if (!collapses(r.codes[e], eev)) return;
+    double len = r.lengths[e];
+    double q = r.quals[std::size_t(e) * 2 + eev];
+    nan = nan || len != len || q != q;
+    if (best == -1 || better_rail(len, q, best_len, best_q)) {
       best = e;
+      at = ve;
       best_len = len;
       best_q = q;
     }
+  };
+  for (LO ve = b + lane; ve < end; ve += kLanes) {
+    star[ve] = r.ev2v[r.ab2b[ve] * 2 + (1 - code_which_down(r.v2e_codes[ve]))];
+    visit(ve);
   }
-  vcand[v] = is_cand;
+  int base = int(threadIdx.x % 64) & ~(kLanes - 1);
+  bool any_nan = ((__ballot(nan) >> base) & ((1ull << kLanes) - 1ull)) != 0ull;
+  if (any_nan) {
+    if (lane != 0) return;
+    best = -1;
+    for (LO ve = b; ve < end; ++ve) visit(ve);
+  } else {
+    for (int d = kLanes / 2; d > 0; d >>= 1) {
+      LO ob = __shfl_xor(best, d, 64), oa = __shfl_xor(at, d, 64);
+      double ol = __shfl_xor(best_len, d, 64), oq = __shfl_xor(best_q, d, 64);
+      bool tie = ol == best_len && oq == best_q;
+      if (ob >= 0 && (best < 0 || better_rail(ol, oq, best_len, best_q) || (tie && oa < at))) {
+        best = ob;
+        at = oa;
+        best_len = ol;
+        best_q = oq;
+      }
+    }
+    if (lane != 0) return;
+  }
+  vcand[v] = best >= 0 ? 1 : 0;
   vqual[v] = best_q;
   vrail[v] = best;
 }
 
-__global__ void find_rails_kernel(LO nkeys, LO const* keys2verts, LO const* vrail,
-    LO const* v2e_a2ab, LO const* v2e_ab2b, I8 const* v2e_codes, LO const* ev2v,
-    LO* rails2edges, LO* col_dirs, LO* keys2onto) {
-  LO k = thread_index();
-  if (k >= nkeys) return;
-  LO v = keys2verts[k];
-  for (LO ve = v2e_a2ab[v]; ve < v2e_a2ab[v + 1]; ++ve) {
-    if (v2e_ab2b[ve] == vrail[v]) {
-      LO e = v2e_ab2b[ve];
-      int eev = code_which_down(v2e_codes[ve]);
-      rails2edges[k] = e;
-      col_dirs[k] = eev;
-      keys2onto[k] = ev2v[e * 2 + (1 - eev)];
-      return;
-    }
-  }
-}
-
 // mark_dead_ents (src/Omega_h_coarsen_topology.cpp:15-60): the rails die,
 // and so do the cells around a rail and each such cell's side opposite the
-// target vertex; rail_col[e] is the collapsing end of rail e (-1 elsewhere)
-__global__ void mark_rails(LO nkeys, LO const* rails2edges, LO const* col_dirs, I8* dead_edges,
-    I8* rail_col) {
-  LO k = thread_index();
-  if (k >= nkeys) return;
-  LO e = rails2edges[k];
+// target vertex; rail_col[e] is the collapsing end of rail e (-1 elsewhere),
+// onto[v] a key's target vertex
+__global__ void mark_rails(LO nv, I8 const* keys, LO const* vrail, LO const* ev2v,
+    I8* dead_edges, I8* rail_col, LO* onto) {
+  LO v = thread_index();
+  if (v >= nv || !keys[v]) return;
+  LO e = vrail[v];
+  int eev = ev2v[e * 2] == v ? 0 : 1;
   dead_edges[e] = 1;
-  rail_col[e] = I8(col_dirs[k]);
+  rail_col[e] = I8(eev);
+  onto[v] = ev2v[e * 2 + 1 - eev];
 }
 
 template <int CD>
-__global__ void mark_dead_cells(LO ncells, LO const* c2e, LO const* cv2v, LO const* cs2s,
-    LO const* ev2v, I8 const* rail_col, I8* dead_cells, I8* dead_sides) {
-  LO c = thread_index();
-  if (c >= ncells) return;
+__device__ __forceinline__ void mark_dead(LO c, CellSweep const& a, int w, LO const* ev2v,
+    I8 const* rail_col) {
+  if (c >= a.ncells[w]) return;
   constexpr int nepc = (CD == 3) ? 6 : 3;
   for (int j = 0; j < nepc; ++j) {
-    LO e = c2e[c * nepc + j];
+    LO e = a.c2e[w][std::size_t(c) * nepc + j];
     int col = rail_col[e];
     if (col < 0) continue;
-    int ccv_onto = local_vertex<CD>(cv2v + c * (CD + 1), ev2v[e * 2 + (1 - col)]);
-    dead_cells[c] = 1;
-    dead_sides[cs2s[c * (CD + 1) + opposite_template(CD, 0, ccv_onto)]] = 1;
+    int ccv_onto =
+        local_vertex<CD>(a.cv2v[w] + std::size_t(c) * (CD + 1), ev2v[e * 2 + (1 - col)]);
+    a.dead_cells[w][c] = 1;
+    a.dead_sides[w][a.cs2s[w][std::size_t(c) * (CD + 1) + opposite_template(CD, 0, ccv_onto)]] =
+        1;
   }
 }
 
+__global__ void __launch_bounds__(kBlock) mark_dead_cells(CellSweep a, LO const* ev2v,
+    I8 const* rail_col) {
+  LO c;
+  int w = cell_job(a, &c);
+  if (a.dim[w] == 3)
+    mark_dead<3>(c, a, w, ev2v, rail_col);
+  else
+    mark_dead<2>(c, a, w, ev2v, rail_col);
+}
+
 // a key's products are the live entries of its vertex's row, in row order;
-// kLanes threads per key share the row (the counts of all dimensions in one
-// launch, added into zeroed counts)
+// kLanes threads per vertex count those of every dimension (0 for vertices
+// that are no keys)
 struct LiveRows {
+  int n;
   LO const* a2ab[3];
   LO const* ab2b[3];
   I8 const* dead[3];
   LO* counts[3];
 };
 
-__global__ void live_counts(LO nt, LO nkeys, LO const* keys2verts, LiveRows r) {
-  LO t = thread_index();
+__global__ void live_counts(std::int64_t nt, I8 const* keys, LiveRows r) {
+  std::int64_t t = thread_index64();
   if (t >= nt) return;
-  LO per = nkeys * kLanes;
-  int d = t / per;
-  LO k = (t % per) / kLanes;
-  int lane = t % kLanes;
-  LO v = keys2verts[k];
-  LO n = 0;
-  for (LO j = r.a2ab[d][v] + lane; j < r.a2ab[d][v + 1]; j += kLanes) n += !r.dead[d][r.ab2b[d][j]];
-  if (n) atomicAdd(&r.counts[d][k], n);
+  LO v = LO(t / kLanes);
+  int lane = int(t % kLanes);
+  bool key = keys[v] != 0;
+  for (int d = 0; d < r.n; ++d) {
+    LO n = 0;
+    if (key) {
+      LO end = r.a2ab[d][v + 1];
+      for (LO j = r.a2ab[d][v] + lane; j < end; j += kLanes) n += !r.dead[d][r.ab2b[d][j]];
+      for (int k = kLanes / 2; k > 0; k >>= 1) n += __shfl_xor(n, k, 64);
+    }
+    if (lane == 0) r.counts[d][v] = n;
+  }
 }
 
 // the products of every dimension in one launch: a round of kLanes row entries
@@ -454,18 +530,18 @@ struct CoarsenRows {
   LO* psrc[3];
 };
 
-__global__ void coarsen_products(LO nt, LO nkeys, LO const* keys2verts, LO const* keys2onto,
-    LO const* vert_offsets, CoarsenRows r) {
-  LO t = thread_index();
+__global__ void coarsen_products(std::int64_t nt, LO nkeys, LO const* keys2verts,
+    LO const* onto_of, LO const* vert_offsets, CoarsenRows r) {
+  std::int64_t t = thread_index64();
   if (t >= nt) return;
-  LO per = nkeys * kLanes;
-  int d = t / per;
-  LO k = (t % per) / kLanes;
-  int lane = t % kLanes;
+  std::int64_t row = t / kLanes;
+  int d = int(row / nkeys);
+  LO k = LO(row % nkeys);
+  int lane = int(t % kLanes);
   int base = int(threadIdx.x % 64) & ~(kLanes - 1);
   int nvd = d + 2;
   LO v = keys2verts[k];
-  LO onto = keys2onto[k];
+  LO onto = onto_of[v];
   LO e = r.a2ab[d][v + 1];
   LO prod = r.keys2prods[d][k];
   for (LO b = r.a2ab[d][v]; b < e; b += kLanes) {
@@ -737,193 +813,198 @@ void prevent_coarsen_flip(Ctx& c, DMesh& m, LOs const& cands, Bytes& codes) {
   }
 }
 
-bool coarsen(Ctx& c, DMesh& m, AdaptOptions const& o, Bytes& codes, bool overshoot_allowed,
-    bool improve) {
+// the determinants of the vertices' metrics (a scalar metric is its own)
+Reals metric_dets(Ctx& c, DMesh& m) {
+  if (m.metric_ncomps == 1) return m.metric;
+  LO nv = m.nents[0];
+  Reals d(c, nv);
+  if (m.metric_ncomps == 6)
+    OSH_LAUNCH(vert_dets<3>, nv, c, m.metric.data(), d.data());
+  else
+    OSH_LAUNCH(vert_dets<2>, nv, c, m.metric.data(), d.data());
+  return d;
+}
+
+// the lanes of each collapse side
+int side_lanes(Ctx& c, LO ncands) {
+  int lanes = c.tuning.coarsen_lanes < kMaxSideLanes ? c.tuning.coarsen_lanes : kMaxSideLanes;
+  return fit_lanes(ncands * 2, lanes);
+}
+
+template <bool FILTER>
+void launch_side_qualities(Ctx& c, DMesh& m, LO ncands, int precision, SideQualities const& a) {
+  int dim = m.dim;
+  int md = (m.metric_ncomps == 1) ? 1 : dim;
+  int lanes = side_lanes(c, ncands);
+  int lshift = lanes_shift(lanes);
+  bool mixed = precision == 1;
+#define OSH_CQ(D, M)                                                                       \
+  do {                                                                                     \
+    if (mixed)                                                                             \
+      OSH_LAUNCH((coarsen_quality_lanes<D, M, true, FILTER>), ncands * 2 * lanes, c, lshift, a); \
+    else                                                                                   \
+      OSH_LAUNCH((coarsen_quality_lanes<D, M, false, FILTER>), ncands * 2 * lanes, c, lshift, a); \
+  } while (0)
+  if (dim == 3 && md == 3)
+    OSH_CQ(3, 3);
+  else if (dim == 3)
+    OSH_CQ(3, 1);
+  else if (md == 2)
+    OSH_CQ(2, 2);
+  else
+    OSH_CQ(2, 1);
+#undef OSH_CQ
+}
+
+bool coarsen_verts(Ctx& c, DMesh& m, AdaptOptions const& o, Bytes const& vm,
+    bool overshoot_allowed, bool improve) {
   int dim = m.dim;
   LO ne = m.nents[1];
   LO nv = m.nents[0];
   int nc = m.metric_ncomps;
   int md = (nc == 1) ? 1 : dim;
   LO const* ev2v = m.down[1].data();
-  OSH_LAUNCH(check_class_kernel, ne, c, ev2v, m.class_dim[0].data(), m.class_dim[1].data(),
-      codes.data());
+  Bytes codes(c, ne);
+  OSH_LAUNCH(collapse_codes, ne, c, ev2v, vm.data(), m.class_dim[0].data(),
+      m.class_dim[1].data(), codes.data());
   // the candidate edges: every later sweep runs over this list
   LOs cands = collect_marked(c, codes);
   LO ncands = cands.size();
   if (ncands == 0) return false;
-  // upward rows only where the candidates look: the candidate edges' cells
-  // (read by order-free tests), the collapsing vertices' edges (ordered:
-  // choose_rails keeps the first best rail) and cells (order-free minimum)
-  Bytes vmarks = fill_i8(c, nv, 0);
+  Fills fills(c);
+  Bytes vmarks = fills.bytes(nv, 0);
+  Bytes exposed = fills.bytes(2 * ne, 0);
+  fills.run();
   OSH_LAUNCH(mark_collapsing_verts, ncands, c, cands.data(), ev2v, codes.data(), vmarks.data());
-  Bytes eveto = fill_i8(c, 2 * ne, 0);
-  for (int cell_dim = 2; cell_dim <= dim; ++cell_dim) {
-    LO const* c2e = ask_down(c, m, cell_dim, 1, nullptr).data();
-    LO const* cv2v = verts_of(c, m, cell_dim).data();
-    if (cell_dim == 3)
-      OSH_LAUNCH(check_exposure_cells<3>, m.nents[3], c, c2e, cv2v, m.down[3].data(),
-          m.class_dim[3].data(), m.class_dim[2].data(), ev2v, codes.data(), eveto.data());
-    else
-      OSH_LAUNCH(check_exposure_cells<2>, m.nents[2], c, c2e, cv2v, m.down[2].data(),
-          m.class_dim[2].data(), m.class_dim[1].data(), ev2v, codes.data(), eveto.data());
+  CellSweep cells{};
+  unsigned cell_blocks = 0;
+  for (int d = dim; d > 1; --d) {
+    int w = cells.n++;
+    cells.dim[w] = d;
+    cells.ncells[w] = m.nents[d];
+    cells.c2e[w] = ask_down(c, m, d, 1, nullptr).data();
+    cells.cv2v[w] = verts_of(c, m, d).data();
+    cells.cs2s[w] = m.down[d].data();
+    cells.cdim[w] = m.class_dim[d].data();
+    cells.sdim[w] = m.class_dim[d - 1].data();
+    cells.first[w] = cell_blocks;
+    cell_blocks += nblocks(m.nents[d]);
+    cells.first[w + 1] = cell_blocks;
   }
-  OSH_LAUNCH(apply_edge_vetoes, ncands, c, cands.data(), eveto.data(), codes.data());
+  hipLaunchKernelGGL(check_exposure_cells, dim3(cell_blocks), dim3(kBlock), 0, c.stream, cells,
+      ev2v, static_cast<I8 const*>(codes.data()), exposed.data());
+  OSH_HIP(hipGetLastError());
+  // upward rows only where the candidates look: the collapsing vertices' edges
+  // (ordered: the first best rail is kept) and cells (order-free minima)
+  Adj up[2];
+  int const highs[2] = {1, dim};
+  bool const sorted[2] = {true, false};
+  marked_ups(c, m, 0, vmarks, 2, highs, sorted, up);
+  Adj const& v2e = up[0];
+  Adj const& v2c = up[1];
   Real max_length = overshoot_allowed ? o.max_length_allowed : o.max_length_desired;
-  Adj v2e = marked_up(c, m, 0, 1, vmarks);
-  int lanes = fit_lanes(ncands * 2, c.tuning.coarsen_lanes);
-  int lshift = lanes_shift(lanes);
-  LO nlanes = ncands * 2 * lanes;
-  Range overshoot_range(c, "prevent_overshoot");
-  Bytes veto = fill_i8(c, ncands * 2, 0);
-  // mixed precision: an FP32 screen first, then FP64 only for the sides it
-  // left open
   bool mixed = o.precision == 1;
-  Bytes need;
-  if (mixed) need = fill_i8(c, ncands * 2, 0);
-#define OSH_OV(D, M, F32)                                                                \
-  OSH_LAUNCH((overshoot_lanes<D, M, F32>), nlanes, c, lshift, cands.data(), ev2v,          \
+  int lanes = side_lanes(c, ncands);
+  int lshift = lanes_shift(lanes);
+  Range overshoot_range(c, "prevent_overshoot");
+#define OSH_OV(D, M, X)                                                                    \
+  OSH_LAUNCH((overshoot_lanes<D, M, X>), ncands * 2 * lanes, c, lshift, cands.data(), ev2v,  \
       v2e.a2ab.data(), v2e.ab2b.data(), v2e.codes.data(), m.coords.data(), m.metric.data(), \
-      max_length, codes.data(), veto.data(), mixed ? need.data() : (I8*)nullptr)
-#define OSH_OV_ALL(F32)      \
+      max_length, exposed.data(), codes.data())
+#define OSH_OV_ALL(X)        \
   if (dim == 3 && md == 3)   \
-    OSH_OV(3, 3, F32);       \
+    OSH_OV(3, 3, X);         \
   else if (dim == 3)         \
-    OSH_OV(3, 1, F32);       \
+    OSH_OV(3, 1, X);         \
   else if (md == 2)          \
-    OSH_OV(2, 2, F32);       \
+    OSH_OV(2, 2, X);         \
   else                       \
-    OSH_OV(2, 1, F32)
+    OSH_OV(2, 1, X)
   if (mixed) {
     OSH_OV_ALL(true);
+  } else {
+    OSH_OV_ALL(false);
   }
-  OSH_OV_ALL(false);
 #undef OSH_OV_ALL
 #undef OSH_OV
-  OSH_LAUNCH(apply_vetoes, ncands, c, cands.data(), veto.data(), codes.data());
   overshoot_range.end();
   if (o.should_prevent_coarsen_flip) prevent_coarsen_flip(c, m, cands, codes);
-  // sides without a candidate left are skipped by every sweep below, and the
-  // check after the quality filter returns
+  // sides without a candidate left are skipped by every sweep below
   Range quality_range(c, "coarsen_qualities");
-  Reals quals(c, ne * 2);
+  Reals quals(c, ne * 2);  // read where a side is kept
   LOs const& cv2v = verts_of(c, m, dim);
-  Adj v2c = marked_up(c, m, 0, dim, vmarks, nullptr, false);
-  Reals partial(c, nlanes);
-  Bytes unsure;
-  if (mixed) unsure = fill_i8(c, ncands * 2, 0);
-#define OSH_CQ(D, M, F32)                                                                \
-  OSH_LAUNCH((coarsen_quality_lanes<D, M, F32>), nlanes, c, lshift, cands.data(), ev2v,     \
-      cv2v.data(), v2c.a2ab.data(), v2c.ab2b.data(), v2c.codes.data(), m.coords.data(),     \
-      m.metric.data(), codes.data(), mixed ? need.data() : (I8 const*)nullptr,              \
-      mixed ? unsure.data() : (I8*)nullptr, partial.data())
-#define OSH_CQ_ALL(F32)      \
-  if (dim == 3 && md == 3)   \
-    OSH_CQ(3, 3, F32);       \
-  else if (dim == 3)         \
-    OSH_CQ(3, 1, F32);       \
-  else if (md == 2)          \
-    OSH_CQ(2, 2, F32);       \
-  else                       \
-    OSH_CQ(2, 1, F32)
-  if (mixed) {
-    OSH_CQ_ALL(true);
-    OSH_LAUNCH(screen_quality_sides, ncands * 2, c, lanes, cands.data(), codes.data(),
-        unsure.data(), partial.data(), o.min_quality_allowed, need.data());
-  }
-  OSH_CQ_ALL(false);
-#undef OSH_CQ_ALL
-#undef OSH_CQ
-  OSH_LAUNCH(combine_quality_lanes, ncands, c, lanes, cands.data(), codes.data(),
-      mixed ? need.data() : (I8 const*)nullptr, partial.data(), quals.data());
-  Reals vold;
-  if (improve) {
-    // read only at collapsing vertices, whose rows are built
-    vold = Reals(c, nv);
-    OSH_LAUNCH(vert_min_quality, nv, c, v2c.a2ab.data(), v2c.ab2b.data(),
-        ask_qualities(c, m).data(), vold.data());
-  }
-  OSH_LAUNCH(filter_quals_kernel, ncands, c, cands.data(), ev2v, quals.data(),
-      o.min_quality_allowed, improve ? vold.data() : (Real const*)nullptr, codes.data());
+  Reals dets = metric_dets(c, m);
+  SideQualities sq{cands.data(), ev2v, cv2v.data(), v2c.a2ab.data(), v2c.ab2b.data(),
+      v2c.codes.data(), m.coords.data(), m.metric.data(), dets.data(), o.min_quality_allowed,
+      improve ? ask_qualities(c, m).data() : (Real const*)nullptr, codes.data(), quals.data()};
+  launch_side_qualities<true>(c, m, ncands, o.precision, sq);
   quality_range.end();
-  if (max_i8(c, codes) <= kDont) return false;
-  Reals const& lengths = ask_lengths(c, m);
   Bytes vcand(c, nv);
   Reals vqual(c, nv);
   LOs vrail(c, nv);
-  OSH_LAUNCH(choose_rails_kernel, nv, c, v2e.a2ab.data(), v2e.ab2b.data(), v2e.codes.data(),
-      codes.data(), lengths.data(), quals.data(), vcand.data(), vqual.data(), vrail.data());
   // the independent set reads the star rows of candidate vertices only
   Adj star;
   star.a2ab = v2e.a2ab;
   star.ab2b = LOs(c, v2e.ab2b.size());
-  OSH_LAUNCH(star_from_v2e, nv, c, v2e.a2ab.data(), v2e.ab2b.data(), v2e.codes.data(), ev2v,
-      star.ab2b.data());
-  Bytes keys = find_indset(c, m, 0, vqual, vcand, nullptr, nullptr, &star);
-  LOs keys2verts = collect_marked(c, keys);
-  LO nkeys = keys2verts.size();
-  note_changed_parts(c, m, 0, keys2verts);
-  if (o.verbosity >= 2) std::printf("coarsening %d vertices\n", int(nkeys));
+  Rails rails{v2e.a2ab.data(), v2e.ab2b.data(), v2e.codes.data(), codes.data(), ev2v,
+      ask_lengths(c, m).data(), quals.data()};
+  OSH_LAUNCH64(choose_rails_kernel, std::int64_t(nv) * kLanes, c, rails, vcand.data(), vqual.data(),
+      vrail.data(), star.ab2b.data());
+  bool any;
+  Bytes keys = find_indset(c, m, 0, vqual, vcand, &any, nullptr, &star);
+  if (!any) return false;
   Range modify_range(c, "modify_ents");
-  LOs rails2edges(c, nkeys), col_dirs(c, nkeys), keys2onto(c, nkeys);
-  OSH_LAUNCH(find_rails_kernel, nkeys, c, keys2verts.data(), vrail.data(), v2e.a2ab.data(),
-      v2e.ab2b.data(), v2e.codes.data(), ev2v, rails2edges.data(), col_dirs.data(),
-      keys2onto.data());
   Bytes dead[4];
-  dead[1] = fill_i8(c, ne, 0);
-  Bytes rail_col = fill_i8(c, ne, -1);
-  OSH_LAUNCH(mark_rails, nkeys, c, rails2edges.data(), col_dirs.data(), dead[1].data(),
-      rail_col.data());
-  for (int d = 2; d <= dim; ++d) dead[d] = fill_i8(c, m.nents[d], 0);
-  for (int cell_dim = dim; cell_dim > 1; --cell_dim) {
-    LO const* c2e = ask_down(c, m, cell_dim, 1, nullptr).data();
-    LO const* cv2v = verts_of(c, m, cell_dim).data();
-    if (cell_dim == 3)
-      OSH_LAUNCH(mark_dead_cells<3>, m.nents[3], c, c2e, cv2v, m.down[3].data(), ev2v,
-          rail_col.data(), dead[3].data(), dead[2].data());
-    else
-      OSH_LAUNCH(mark_dead_cells<2>, m.nents[2], c, c2e, cv2v, m.down[2].data(), ev2v,
-          rail_col.data(), dead[2].data(), dead[1].data());
+  dead[1] = fills.bytes(ne, 0);
+  for (int d = 2; d <= dim; ++d) dead[d] = fills.bytes(m.nents[d], 0);
+  Bytes rail_col = fills.bytes(ne, -1);
+  fills.run();
+  LOs onto(c, nv);
+  OSH_LAUNCH(mark_rails, nv, c, keys.data(), vrail.data(), ev2v, dead[1].data(),
+      rail_col.data(), onto.data());
+  for (int w = 0; w < cells.n; ++w) {
+    cells.dead_cells[w] = dead[cells.dim[w]].data();
+    cells.dead_sides[w] = dead[cells.dim[w] - 1].data();
   }
+  hipLaunchKernelGGL(mark_dead_cells, dim3(cell_blocks), dim3(kBlock), 0, c.stream, cells, ev2v,
+      static_cast<I8 const*>(rail_col.data()));
+  OSH_HIP(hipGetLastError());
   // the keys' rows of every dimension, in order: products follow them
   Adj v2d[4];
   v2d[1] = v2e;
-  for (int d = 2; d <= dim; ++d) v2d[d] = marked_up(c, m, 0, d, keys);
+  {
+    int const hs[2] = {2, 3};
+    bool const in_order[2] = {true, true};
+    marked_ups(c, m, 0, keys, dim - 1, hs, in_order, v2d + 2);
+  }
+  KeyedMods km;  // no key vertex has a product vertex
+  LiveRows live{};
+  live.n = dim;
+  for (int d = 1; d <= dim; ++d) {
+    km.prod_counts[d] = LOs(c, nv);
+    live.a2ab[d - 1] = v2d[d].a2ab.data();
+    live.ab2b[d - 1] = v2d[d].ab2b.data();
+    live.dead[d - 1] = dead[d].data();
+    live.counts[d - 1] = km.prod_counts[d].data();
+  }
+  OSH_LAUNCH64(live_counts, std::int64_t(nv) * kLanes, c, keys.data(), live);
+  plan_keys(c, m, 0, 0, dim, keys, km);
+  LO nkeys = km.nkeys;
+  LOs const& keys2verts = km.keys2kds;
+  ModPlan const* plans = km.plans;
+  note_changed_parts(c, m, 0, keys2verts);
+  if (o.verbosity >= 2) std::printf("coarsening %d vertices\n", int(nkeys));
   DMesh nw;
   nw.dim = dim;
   nw.metric_ncomps = nc;
-  // products per key of every dimension, numbered by one scan launch
-  LOs k2p[4];
-  LO nprods[4] = {0, 0, 0, 0};
-  k2p[0] = fill_lo(c, nkeys + 1, 0);  // no key vertex has a product vertex
-  {
-    LOs counts = fill_lo(c, dim * nkeys, 0);
-    LiveRows rows{};
-    ScanJob jobs[3];
-    for (int d = 1; d <= dim; ++d) {
-      rows.a2ab[d - 1] = v2d[d].a2ab.data();
-      rows.ab2b[d - 1] = v2d[d].ab2b.data();
-      rows.dead[d - 1] = dead[d].data();
-      rows.counts[d - 1] = counts.data() + (d - 1) * nkeys;
-      k2p[d] = LOs(c, nkeys + 1);
-      jobs[d - 1] = {rows.counts[d - 1], kScanLO, nkeys, k2p[d].data(), slot_ptr<LO>(c, d)};
-    }
-    OSH_LAUNCH(live_counts, dim * nkeys * kLanes, c, nkeys, keys2verts.data(), rows);
-    offset_scans(c, jobs, dim);
-    c.wait();
-    for (int d = 1; d <= dim; ++d) nprods[d] = read_slot<LO>(c, d);
-  }
-  // every dimension's new numbering by one more scan launch
-  ModPlan plans[4];
-  modify_plans(c, m, 0, 0, dim, keys2verts, k2p, plans);
-  modify_scan(c, plans, dim + 1);
   ModOut mo[4];
   rebuild_same(c, m, nw, 0, plans, mo);
   Products prods[4];
   CoarsenRows rows{};
   for (int d = 1; d <= dim; ++d) {
     Products& p = prods[d];
-    p.n = nprods[d];
-    p.keys2prods = k2p[d];
+    p.n = km.nprods[d];
+    p.keys2prods = km.k2p[d];
     p.verts = LOs(c, p.n * (d + 1));
     p.src = LOs(c, p.n);
     p.src_dim = d;
@@ -932,12 +1013,12 @@ bool coarsen(Ctx& c, DMesh& m, AdaptOptions const& o, Bytes& codes, bool oversho
     rows.codes[d - 1] = v2d[d].codes.data();
     rows.dead[d - 1] = dead[d].data();
     rows.verts[d - 1] = verts_of(c, m, d).data();
-    rows.keys2prods[d - 1] = k2p[d].data();
+    rows.keys2prods[d - 1] = km.k2p[d].data();
     rows.pv[d - 1] = p.verts.data();
     rows.psrc[d - 1] = p.src.data();
   }
-  OSH_LAUNCH(coarsen_products, dim * nkeys * kLanes, c, nkeys, keys2verts.data(),
-      keys2onto.data(), plans[0].offsets.data(), rows);
+  OSH_LAUNCH64(coarsen_products, std::int64_t(nkeys) * dim * kLanes, c, nkeys, keys2verts.data(), onto.data(),
+      plans[0].offsets.data(), rows);
   place_products(c, m, nw, 1, dim, 0, plans, keys2verts, prods, mo);
   match_sides(c, nw, prods, mo);
   measure_products(c, nw, mo);
@@ -946,30 +1027,20 @@ bool coarsen(Ctx& c, DMesh& m, AdaptOptions const& o, Bytes& codes, bool oversho
   for (std::size_t t = 0; t < m.itags.size(); ++t)
     nw.itags[t].data[0] =
         transfer<Real>(c, mo[0], m.itags[t].ncomps, m.itags[t].data[0], nullptr);
-  transfer_pointwise(c, m, nw, mo[dim], 0, keys2verts, k2p[dim], prods[dim].verts);
-  conserve_pass(c, m, nw, 1, 0, keys2verts, k2p[dim], mo[dim]);
+  transfer_pointwise(c, m, nw, mo[dim], 0, keys2verts, km.k2p[dim], prods[dim].verts);
+  conserve_pass(c, m, nw, 1, 0, keys2verts, km.k2p[dim], mo[dim]);
   m = nw;
   return true;
-}
-
-bool coarsen_verts(Ctx& c, DMesh& m, AdaptOptions const& o, Bytes const& vmarks,
-    bool overshoot_allowed, bool improve) {
-  LO ne = m.nents[1];
-  Bytes codes(c, ne);
-  OSH_LAUNCH(edge_codes_from_verts, ne, c, m.down[1].data(), vmarks.data(), codes.data());
-  return coarsen(c, m, o, codes, overshoot_allowed, improve);
 }
 
 }  // namespace
 
 bool coarsen_by_size(Ctx& c, DMesh& m, AdaptOptions const& o) {
-  LO ne = m.nents[1];
   Reals const& lengths = ask_lengths(c, m);
   ask_qualities(c, m);
-  Bytes cand(c, ne);
-  OSH_LAUNCH(lt_kernel, ne, c, lengths.data(), o.min_length_desired, cand.data());
-  if (max_i8(c, cand) != 1) return false;
-  Bytes vm = mark_down(c, m, 1, 0, cand);
+  Bytes vm = fill_i8(c, m.nents[0], 0);
+  OSH_LAUNCH(mark_short_edges, m.nents[1], c, lengths.data(), o.min_length_desired,
+      m.down[1].data(), vm.data());
   return coarsen_verts(c, m, o, vm, false, false);
 }
 
@@ -982,48 +1053,16 @@ bool coarsen_slivers(Ctx& c, DMesh& m, AdaptOptions const& o) {
 
 void coarsen_qualities(Ctx& c, DMesh& m, LO ncands, LO const* cands, I8 const* cand_codes,
     Real* out, int precision, Real qmin) {
-  int dim = m.dim;
-  int md = (m.metric_ncomps == 1) ? 1 : dim;
   if (ncands == 0) return;
-  LO const* ev2v = m.down[1].data();
-  LOs const& cv2v = verts_of(c, m, dim);
-  Adj const& v2c = ask_up(c, m, 0, dim);
+  LOs const& cv2v = verts_of(c, m, m.dim);
+  Adj const& v2c = ask_up(c, m, 0, m.dim);
   Bytes codes = fill_i8(c, m.nents[1], kDont);
   OSH_LAUNCH(scatter_codes, ncands, c, cands, cand_codes, codes.data());
-  int lanes = fit_lanes(ncands * 2, c.tuning.coarsen_lanes);
-  int lshift = lanes_shift(lanes);
-  LO nlanes = ncands * 2 * lanes;
-  Reals partial(c, nlanes);
-  bool mixed = precision == 1;
-  Bytes need, unsure;
-  if (mixed) {
-    need = Bytes(c, ncands * 2);
-    unsure = fill_i8(c, ncands * 2, 0);
-  }
-#define OSH_CQ(D, M, F32)                                                                \
-  OSH_LAUNCH((coarsen_quality_lanes<D, M, F32>), nlanes, c, lshift, cands, ev2v,            \
-      cv2v.data(), v2c.a2ab.data(), v2c.ab2b.data(), v2c.codes.data(), m.coords.data(),     \
-      m.metric.data(), codes.data(), mixed ? need.data() : (I8 const*)nullptr,              \
-      mixed ? unsure.data() : (I8*)nullptr, partial.data())
-#define OSH_CQ_ALL(F32)      \
-  if (dim == 3 && md == 3)   \
-    OSH_CQ(3, 3, F32);       \
-  else if (dim == 3)         \
-    OSH_CQ(3, 1, F32);       \
-  else if (md == 2)          \
-    OSH_CQ(2, 2, F32);       \
-  else                       \
-    OSH_CQ(2, 1, F32)
-  if (mixed) {
-    OSH_CQ_ALL(true);
-    OSH_LAUNCH(screen_quality_sides, ncands * 2, c, lanes, cands, codes.data(), unsure.data(),
-        partial.data(), qmin, need.data());
-  }
-  OSH_CQ_ALL(false);
-#undef OSH_CQ_ALL
-#undef OSH_CQ
-  OSH_LAUNCH(combine_to_cands, ncands, c, lanes, cands, codes.data(),
-      mixed ? need.data() : (I8 const*)nullptr, partial.data(), out);
+  Reals dets = metric_dets(c, m);
+  SideQualities sq{cands, m.down[1].data(), cv2v.data(), v2c.a2ab.data(), v2c.ab2b.data(),
+      v2c.codes.data(), m.coords.data(), m.metric.data(), dets.data(), qmin, nullptr,
+      codes.data(), out};
+  launch_side_qualities<false>(c, m, ncands, precision, sq);
 }
 
 }  // namespace osh

@@ -738,20 +738,10 @@ OSH_HD void barycentric(double const* x, double const (*p)[3], double* xi) {
   }
 }
 
-// maxdet_metric + metric_element_quality, src/Omega_h_metric.hpp:170-181,
-// src/Omega_h_quality.hpp:8-37
+// metric_element_quality with the chosen metric (the one of the largest
+// determinant, maxdet), src/Omega_h_quality.hpp:8-37
 template <int D, int M>
-OSH_HD double element_quality(double const* const* p, double const* const* ms) {
-  Mat m = get_symm<M>(ms[0]);
-  double maxdet = det<M>(m);
-  for (int i = 1; i < D + 1; ++i) {
-    Mat mi = get_symm<M>(ms[i]);
-    double d = det<M>(mi);
-    if (d > maxdet) {
-      m = mi;
-      maxdet = d;
-    }
-  }
+OSH_HD double quality_with(double const* const* p, Mat const& m, double maxdet) {
   double b[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
   for (int i = 0; i < D; ++i)
     for (int j = 0; j < D; ++j) b[i][j] = p[i + 1][j] - p[0][j];
@@ -801,6 +791,37 @@ OSH_HD double element_quality(double const* const* p, double const* const* ms) {
   double x = s / eq;
   double num = (D == 3) ? math::cbrt_(x * x) : x;
   return num / msl;
+}
+
+// maxdet_metric + metric_element_quality, src/Omega_h_metric.hpp:170-181
+template <int D, int M>
+OSH_HD double element_quality(double const* const* p, double const* const* ms) {
+  Mat m = get_symm<M>(ms[0]);
+  double maxdet = det<M>(m);
+  for (int i = 1; i < D + 1; ++i) {
+    Mat mi = get_symm<M>(ms[i]);
+    double d = det<M>(mi);
+    if (d > maxdet) {
+      m = mi;
+      maxdet = d;
+    }
+  }
+  return quality_with<D, M>(p, m, maxdet);
+}
+
+// the same with the vertices' determinants in hand: only the chosen metric is
+// read
+template <int D, int M>
+OSH_HD double element_quality(double const* const* p, double const* const* ms,
+    double const* dets) {
+  double const* best = ms[0];
+  double maxdet = dets[0];
+  for (int i = 1; i < D + 1; ++i)
+    if (dets[i] > maxdet) {
+      best = ms[i];
+      maxdet = dets[i];
+    }
+  return quality_with<D, M>(p, get_symm<M>(best), maxdet);
 }
 
 // ------------------------------------------------------------ FP32 screens

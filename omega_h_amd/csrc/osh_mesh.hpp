@@ -120,15 +120,13 @@ int simplex_degree(int from_dim, int to_dim);
 LOs const& verts_of(Ctx& c, DMesh& m, int d);
 LOs const& ask_down(Ctx& c, DMesh& m, int high, int low, Bytes const** codes);
 Adj const& ask_up(Ctx& c, DMesh& m, int low, int high);
-// the upward adjacency with only the rows of marked lows filled (the others
-// are empty; entries past a2ab[nlow] are unused); not cached.  With
-// `marked`, also the list of marked lows (collect_marked), from the same scan
-// launch.  Without `sorted`, a row's order is arbitrary, which suits uses
-// that do not depend on it (counts, any/all tests, min/max)
-// `marked_index` (with `marked`) receives, for each marked low, its position
-// in the list (the scan of the marks)
-Adj marked_up(Ctx& c, DMesh& m, int low, int high, Bytes const& marks, LOs* marked = nullptr,
-    bool sorted = true, LOs* marked_index = nullptr);
+// the upward adjacencies low -> highs[w] with only the rows of marked lows
+// filled (the others are empty; entries past a2ab[nlow] are unused), up to
+// three by the same launches; not cached.  Without sorted[w], a row's order is
+// arbitrary, which suits uses that do not depend on it (counts, any/all
+// tests, min/max)
+void marked_ups(Ctx& c, DMesh& m, int low, Bytes const& marks, int n, int const* highs,
+    bool const* sorted, Adj* out);
 Adj const& ask_star(Ctx& c, DMesh& m, int d);
 DArray<unsigned long long> const& ask_side_elems(Ctx& c, DMesh& m);
 // Mesh::ask_dual (src/Omega_h_mesh.cpp:260): elements_across_sides

@@ -9,6 +9,7 @@
 //   indset::find / QualityCompare         src/Omega_h_indset_inline.hpp:12-72,
 //                                         src/Omega_h_indset.cpp:5-35
 //   mark_down / mark_dual_layers / mark_sliver_layers src/Omega_h_mark.cpp:12-47,190-212
+#include "osh_indset.hpp"
 #include "osh_math.hpp"
 #include "osh_passes.hpp"
 
@@ -16,35 +17,43 @@ namespace osh {
 
 namespace {
 
-// the same entities of dimension > key dimension: those with no key among
-// their lower entities, each counting one new entity; each key also receives
-// the lowest index among the entities above it, which is the first entry of
-// its row of the upward adjacency (rows are sorted by index), without
-// building that adjacency
-// the dimensions above the keys in one launch: job w owns the threads
-// [start[w], start[w + 1])
-struct SameUpJobs {
-  LO start[4];
-  int deg[3];
-  LO const* hl2l[3];
-  I8* same[3];
-  LO* counts[3];
-  LO* first_up[3];
+// The plans of a pass's dimensions from its keys, given as a mask over the key
+// dimension, in one sweep.  A key is no longer the same and counts its
+// products; in the dimensions above, an entity is the same when no key is
+// among its lower entities, and each key receives the lowest index among the
+// entities above it (the first entry of its row of the upward adjacency,
+// whose rows are sorted by index), without building that adjacency.  Job w
+// owns the workgroups [first[w], first[w + 1]).
+struct SameMarks {
   int n;
+  unsigned first[5];
+  LO nents[4];
+  int deg[4];             // lower entities per entity; 0: the key dimension itself
+  LO const* lows[4];
+  I8* same[4];
+  LO* counts[4];
+  LO* first_up[4];
+  LO const* key_prods;    // products of the key dimension per entity (null: fixed)
+  LO fixed_key_prods;
 };
 
-__global__ void mark_same_up_kernel(LO nt, I8 const* low_marks, SameUpJobs j) {
-  LO t = thread_index();
-  if (t >= nt) return;
+__global__ void __launch_bounds__(kBlock) mark_same_kernel(I8 const* keys, SameMarks j) {
   int w = 0;
-  while (w + 1 < j.n && t >= j.start[w + 1]) ++w;
-  LO h = t - j.start[w];
+  while (w + 1 < j.n && blockIdx.x >= j.first[w + 1]) ++w;
+  LO h = LO(blockIdx.x - j.first[w]) * kBlock + LO(threadIdx.x);
+  if (h >= j.nents[w]) return;
   int deg = j.deg[w];
-  LO const* hl2l = j.hl2l[w];
+  if (deg == 0) {
+    bool key = keys[h] != 0;
+    j.same[w][h] = key ? 0 : 1;
+    j.counts[w][h] = key ? (j.key_prods ? j.key_prods[h] : j.fixed_key_prods) : 1;
+    return;
+  }
+  LO const* lows = j.lows[w] + std::size_t(h) * deg;
   I8 r = 1;
   for (int k = 0; k < deg; ++k) {
-    LO l = hl2l[h * deg + k];
-    if (low_marks[l]) {
+    LO l = lows[k];
+    if (keys[l]) {
       r = 0;
       atomicMin(&j.first_up[w][l], h);
     }
@@ -53,106 +62,80 @@ __global__ void mark_same_up_kernel(LO nt, I8 const* low_marks, SameUpJobs j) {
   j.counts[w][h] = r;
 }
 
-// One sweep over the key-dimension entities starts the plans of every
-// dimension of a pass: no key marked, no entity above found yet, and (when
-// the key dimension itself is rebuilt) every entity the same, counting one.
-struct KeyDimInit {
-  I8* key_marks;
-  LO* first_up[4];  // per dimension above the keys (null elsewhere)
-  I8* same;         // when the key dimension is rebuilt
-  LO* counts;
-  // with a key mask, the keys are marked in the same sweep: no longer the
-  // same, each counting its products
-  I8 const* key_mask;
-  LO const* key_prod_counts;
+// the keys' representatives (get_mods2reps, src/Omega_h_modify.cpp:20-45)
+// count their products (get_rep_counts, :47-70): the lowest entity above the
+// key, or in the dimension below the key's first lower entity, where the keys
+// of one representative are also chained for their order (get_rep2md_order)
+struct RepCounts {
+  int n;
+  LO const* first_up[4];   // dimensions above
+  LO const* down[4];       // the dimension below
+  int deg[4];
+  LO const* prods[4];      // per key-dimension entity (null: fixed)
+  LO fixed[4];
+  LO* counts[4];
+  LO* head;                // per representative below: a key, or -1
+  LO* next;                // per key-dimension entity: the chain's next key
 };
 
-__global__ void init_key_dim(LO n, KeyDimInit a) {
-  LO i = thread_index();
-  if (i >= n) return;
-  if (a.key_marks) a.key_marks[i] = 0;
-  for (int d = 0; d < 4; ++d)
-    if (a.first_up[d]) a.first_up[d][i] = 0x7fffffff;
-  if (a.same) {
-    bool key = a.key_mask && a.key_mask[i];
-    a.same[i] = key ? 0 : 1;
-    a.counts[i] = key ? a.key_prod_counts[i] : 1;
-  }
-}
-
-// the keys: marked; when the key dimension is rebuilt, a key is its own
-// representative (get_mods2reps, src/Omega_h_modify.cpp:20-45), is no longer
-// the same and counts its products (get_rep_counts, :47-70)
-__global__ void mark_keys(LO nkeys, LO const* keys2kds, LO const* keys2prods, I8* key_marks,
-    I8* same, LO* counts, LO* reps) {
-  LO k = thread_index();
-  if (k >= nkeys) return;
-  LO kd = keys2kds[k];
-  if (key_marks) key_marks[kd] = 1;
-  if (same) {
-    same[kd] = 0;
-    counts[kd] = keys2prods[k + 1] - keys2prods[k];
-    reps[k] = kd;
-  }
-}
-
-// representatives of the keys for up to three dimensions in one launch: the
-// lowest entity above the key (first_up) or the key's first lower entity
-// (down); the representative counts the key's products
-struct RepsJob {
-  LO const* first_up[3];
-  LO const* down[3];
-  int deg[3];
-  LO const* keys2prods[3];
-  LO* reps[3];
-  LO* counts[3];
-};
-
-__global__ void reps_kernel(LO nt, LO nkeys, LO const* keys2kds, RepsJob j, int* error) {
-  LO t = thread_index();
-  if (t >= nt) return;
-  int w = t / nkeys;
-  LO k = t % nkeys;
-  LO kd = keys2kds[k];
-  LO r;
-  if (j.first_up[w]) {
-    r = j.first_up[w][kd];
-    if (r == 0x7fffffff) {  // keeps every index in range until the host sees it
-      r = 0;
-      *error = kKeyWithoutUp;
+__global__ void rep_counts_kernel(LO nkd, I8 const* keys, RepCounts j, int* error) {
+  LO kd = thread_index();
+  if (kd >= nkd || !keys[kd]) return;
+  for (int w = 0; w < j.n; ++w) {
+    LO r;
+    if (j.first_up[w]) {
+      r = j.first_up[w][kd];
+      if (r == 0x7fffffff) {  // keeps every index in range until the host sees it
+        r = 0;
+        *error = kKeyWithoutUp;
+      }
+    } else {
+      r = j.down[w][std::size_t(kd) * j.deg[w]];
+      j.next[kd] = atomicExch(&j.head[r], kd);
     }
-  } else {
-    r = j.down[w][kd * j.deg[w]];
+    atomicAdd(&j.counts[w][r], j.prods[w] ? j.prods[w][kd] : j.fixed[w]);
   }
-  j.reps[w][k] = r;
-  atomicAdd(&j.counts[w][r], j.keys2prods[w][k + 1] - j.keys2prods[w][k]);
 }
 
-// the same starts with the keys given as a mask over the key dimension and
-// their product counts per key-dimension entity: a key of the rebuilt key
-// dimension is no longer the same and counts its products; for the
-// dimensions above, each key's representative (kept per key-dimension
-// entity) counts the key's products
-struct MaskedReps {
-  LO const* first_up[3];
-  LO const* prod_counts[3];
-  LO* rep_of[3];
-  LO* counts[3];
+// per key (and one past the last): its product offsets and representatives in
+// every dimension and, below the key dimension, how many products of earlier
+// keys share its representative
+struct KeyList {
+  int n;
+  int kind[4];  // 0: the key dimension, 1: above, -1: below
+  LO const* first_up[4];
+  LO const* down[4];
+  int deg[4];
+  LO const* prod_off[4];  // scan of the products per entity (null: fixed)
+  LO fixed[4];
+  LO* k2p[4];
+  LO* reps[4];
+  LO nkd;
+  LO const* head;
+  LO const* next;
+  LO* order;  // per key-dimension entity
 };
 
-__global__ void reps_masked(LO nt, LO nkd, I8 const* key_mask, MaskedReps j, int* error) {
-  LO t = thread_index();
-  if (t >= nt) return;
-  int w = t / nkd;
-  LO kd = t % nkd;
-  if (!key_mask[kd]) return;
-  LO r = j.first_up[w][kd];
-  if (r == 0x7fffffff) {  // keeps every index in range until the host sees it
-    r = 0;
-    *error = kKeyWithoutUp;
+__global__ void list_keys_kernel(LO n, LO nkeys, LO const* keys2kds, KeyList j) {
+  LO k = thread_index();
+  if (k >= n) return;
+  LO kd = k < nkeys ? keys2kds[k] : j.nkd;
+  for (int w = 0; w < j.n; ++w) {
+    j.k2p[w][k] = j.prod_off[w] ? j.prod_off[w][kd] : k * j.fixed[w];
+    if (k == nkeys) continue;
+    LO r = kd;
+    if (j.kind[w] > 0) {
+      r = j.first_up[w][kd];
+      r = r == 0x7fffffff ? 0 : r;
+    } else if (j.kind[w] < 0) {
+      r = j.down[w][std::size_t(kd) * j.deg[w]];
+      // one product a key: the order counts the representative's smaller keys
+      LO before = 0;
+      for (LO o = j.head[r]; o >= 0; o = j.next[o]) before += o < kd;
+      j.order[kd] = before * j.fixed[w];
+    }
+    j.reps[w][k] = r;
   }
-  j.rep_of[w][kd] = r;
-  atomicAdd(&j.counts[w][r], j.prod_counts[w][kd]);
 }
 
 // a same entity's new number is its offset (assign_new_numbering,
@@ -275,26 +258,6 @@ __global__ void __launch_bounds__(kBlock) rebuild_same_kernel(SameJobs j) {
   }
 }
 
-__global__ void scatter_index(LO n, LO const* a2b, LO* b2a) {
-  LO i = thread_index();
-  if (i < n) b2a[a2b[i]] = i;
-}
-
-__global__ void rep2md_order_kernel(LO nreps, LO const* a2ab, LO const* ab2b, I8 const* codes,
-    LO const* md2mod, LO const* keys2prods, LO* order) {
-  LO rep = thread_index();
-  if (rep >= nreps) return;
-  LO offset = 0;
-  for (LO j = a2ab[rep]; j < a2ab[rep + 1]; ++j) {
-    LO md = ab2b[j];
-    LO mod = md2mod[md];
-    if (mod >= 0 && code_which_down(codes[j]) == 0) {
-      order[md] = offset;
-      offset += keys2prods[mod + 1] - keys2prods[mod];
-    }
-  }
-}
-
 // the products' new numbers, following their representative
 // (src/Omega_h_modify.cpp:141-161), with their vertex lists and their
 // classification, inherited from the entity each came from
@@ -330,13 +293,14 @@ struct PlaceJobs {
   PlaceDim d[4];
 };
 
-__global__ void __launch_bounds__(kBlock) place_products_kernel(LO nt, LO nkeys, PlaceJobs j) {
-  LO t = thread_index();
+__global__ void __launch_bounds__(kBlock) place_products_kernel(std::int64_t nt, LO nkeys,
+    PlaceJobs j) {
+  std::int64_t t = thread_index64();
   if (t >= nt) return;
-  LO per = nkeys * kProdLanes;
-  PlaceDim const& a = j.d[t / per];
-  LO k = (t % per) / kProdLanes;
-  int lane = t % kProdLanes;
+  std::int64_t row = t / kProdLanes;
+  PlaceDim const& a = j.d[row / nkeys];
+  LO k = LO(row % nkeys);
+  int lane = int(t % kProdLanes);
   LO first = a.keys2prods[k];
   LO end = a.keys2prods[k + 1];
   LO key = j.keys2kds[k];
@@ -469,50 +433,6 @@ __global__ void inherit_kernel(LO n, LO nold, int nc, LO const* old2new, Real co
   LO s = src[p];
   LO w = prods2new[p];
   for (int k = 0; k < nc; ++k) out[std::size_t(w) * nc + k] = from[std::size_t(s) * nc + k];
-}
-
-// one round of indset::find (src/Omega_h_indset.cpp:5-35).  In the first
-// round the states come straight from the candidate marks (2 for a
-// candidate, 0 otherwise), so no node is in the set yet.
-template <bool FIRST>
-__device__ __forceinline__ I8 indset_state(I8 const* old_state, LO x) {
-  I8 s = old_state[x];
-  return FIRST ? I8(s ? 2 : 0) : s;
-}
-
-// A node joins the set once every neighbor that beats it (higher quality,
-// or the same quality and a higher index) is out, and leaves once one of
-// them is in: a neighbor it beats can be in only after the node is out, so
-// this is the round above restated over the beating neighbors alone.  The
-// first round records, per candidate, which row positions hold candidates
-// that beat it (bits of `dom`); later rounds read the states at those
-// positions only, not the qualities.  A row longer than 64 positions is
-// read whole every round.
-constexpr int kDomBits = 64;
-
-// Each batch of rounds ends with a wait for two words: kUndecidedWord, set by
-// the last round's nodes that stay undecided, and kCandWord, set by the first
-// round's candidates, so that no reduction over the states is needed.
-constexpr int kUndecidedWord = 0;
-constexpr int kCandWord = 1;
-
-// one lane a wave stores, and only where the word does not hold the tag yet
-__device__ __forceinline__ void tell(bool is, unsigned* word, unsigned tag) {
-  unsigned long long b = __ballot(is);
-  if (b == 0ull || int(threadIdx.x & 63) != __ffsll(static_cast<long long>(b)) - 1) return;
-  if (__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != tag)
-    __hip_atomic_store(word, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-struct IndsetWords {
-  unsigned* words;
-  unsigned cand_tag;  // 0: not the first round
-  unsigned last_tag;  // 0: not the last round of its batch
-};
-
-__device__ __forceinline__ void tell_round(I8 before, I8 after, IndsetWords w) {
-  if (w.cand_tag) tell(before == 2, w.words + kCandWord, w.cand_tag);
-  if (w.last_tag) tell(after == 2, w.words + kUndecidedWord, w.last_tag);
 }
 
 // an undecided node's next state
@@ -678,10 +598,10 @@ __global__ void below_kernel(LO n, Real const* q, Real ceil, I8* out) {
 // elements_across_sides, src/Omega_h_adj.cpp:591-657): the max over the
 // elements across each side that has two, -128 for an element with none; a
 // side with more than two elements (not a manifold mesh) is an error.  The
-// input is `in`, or, when `q` is given, the sliver test q < ceil.
+// first layer: the input is the sliver test q < ceil.
 template <int NSPE>
 __device__ __forceinline__ I8 dual_max_at(LO e, LO const* es2s,
-    unsigned long long const* side_elems, I8 const* in, Real const* q, Real ceil, int* error) {
+    unsigned long long const* side_elems, Real const* q, Real ceil, int* error) {
   I8 r = -128;
 #pragma unroll
   for (int j = 0; j < NSPE; ++j) {
@@ -689,7 +609,7 @@ __device__ __forceinline__ I8 dual_max_at(LO e, LO const* es2s,
     unsigned count = unsigned(w >> 32);
     if (count == 2) {
       LO o = LO(unsigned(w)) - e;
-      I8 x = q ? I8(q[o] < ceil) : in[o];
+      I8 x = I8(q[o] < ceil);
       r = (r < x) ? x : r;
     } else if (count > 2) {
       *error = kNonManifoldSide;
@@ -699,12 +619,33 @@ __device__ __forceinline__ I8 dual_max_at(LO e, LO const* es2s,
 }
 
 __global__ void dual_max_kernel(LO n, int nspe, LO const* es2s,
-    unsigned long long const* side_elems, I8 const* in, Real const* q, Real ceil, I8* out,
-    int* error) {
+    unsigned long long const* side_elems, Real const* q, Real ceil, I8* out, int* error) {
   LO e = thread_index();
   if (e >= n) return;
-  out[e] = nspe == 4 ? dual_max_at<4>(e, es2s, side_elems, in, q, ceil, error)
-                     : dual_max_at<3>(e, es2s, side_elems, in, q, ceil, error);
+  out[e] = nspe == 4 ? dual_max_at<4>(e, es2s, side_elems, q, ceil, error)
+                     : dual_max_at<3>(e, es2s, side_elems, q, ceil, error);
+}
+
+// a later layer, pushed from the marked elements (the first one's output has
+// looked at every side): few elements are marked, and the rest read one byte
+// instead of four side words (2.5 us against 4.5 us at 167,000 tets).  `out`
+// starts at 0; an element without neighbors keeps its -128.
+template <int NSPE>
+__global__ void push_layer_kernel(LO n, LO const* es2s, unsigned long long const* side_elems,
+    I8 const* in, I8* out) {
+  LO e = thread_index();
+  if (e >= n) return;
+  I8 s = in[e];
+  if (s == 0) return;
+  if (s < 0) {
+    out[e] = s;
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < NSPE; ++j) {
+    unsigned long long w = side_elems[es2s[std::size_t(e) * NSPE + j]];
+    if (unsigned(w >> 32) == 2) out[LO(unsigned(w)) - e] = 1;
+  }
 }
 
 __global__ void degrees_kernel(LO n, LO const* a2ab, LO const* rows, LO* out) {
@@ -724,124 +665,106 @@ LOs degrees_of(Ctx& c, LOs const& a2ab, LOs const& rows) {
   return out;
 }
 
-void modify_plans(Ctx& c, DMesh& old, int key_dim, int d0, int d1, LOs const& keys2kds,
-    LOs const* keys2prods, ModPlan* plans) {
-  LO nkeys = keys2kds.size();
+void plan_keys(Ctx& c, DMesh& old, int key_dim, int d0, int d1, Bytes const& keys,
+    KeyedMods& out) {
   LO nkd = old.nents[key_dim];
-  KeyDimInit init{};
-  Bytes key_marks;
-  LOs first_up[4];
-  bool above = false;
+  int nd = d1 - d0 + 1;
+  OSH_CHECK(nd >= 1 && nd <= 4 && key_dim - d0 <= 1 && key_dim >= d0, "plan_keys: dimensions");
+  Fills fills(c);
+  LOs first_up[4], head, next;
+  SameMarks sm{};
+  RepCounts rc{};
+  KeyList kl{};
+  unsigned blocks = 0;
   for (int d = d0; d <= d1; ++d) {
-    ModPlan& plan = plans[d - d0];
+    ModPlan& plan = out.plans[d - d0];
     plan.ent_dim = d;
     plan.key_dim = key_dim;
     plan.nold = old.nents[d];
-    plan.reps = LOs(c, nkeys);
-    // same entities: those not adjacent to a key (collect_same); without a
-    // `same` array every old entity is the same
-    if (d >= key_dim) {
+    LO const* prods = out.prod_counts[d].exists() ? out.prod_counts[d].data() : nullptr;
+    int w = kl.n++;
+    kl.kind[w] = d == key_dim ? 0 : (d > key_dim ? 1 : -1);
+    kl.fixed[w] = out.fixed_prods[d];
+    if (d < key_dim) {
+      // every entity stays; without a `same` array all are the same
+      OSH_CHECK(!prods, "plan_keys: a fixed count below the keys");
+      plan.counts = fills.ints(plan.nold, 1);
+      head = fills.ints(plan.nold, -1);
+      next = LOs(c, nkd);
+      out.order = LOs(c, nkd);
+      kl.deg[w] = simplex_degree(key_dim, d);
+      kl.down[w] = ask_down(c, old, key_dim, d, nullptr).data();
+      kl.head = rc.head = head.data();
+      rc.next = next.data();
+      kl.next = next.data();
+      kl.order = out.order.data();
+    } else {
       plan.same = Bytes(c, plan.nold);
       plan.counts = LOs(c, plan.nold);
+      int v = sm.n;
+      sm.first[v] = blocks;
+      blocks += nblocks(plan.nold);
+      sm.first[v + 1] = blocks;
+      sm.nents[v] = plan.nold;
+      sm.same[v] = plan.same.data();
+      sm.counts[v] = plan.counts.data();
+      if (d == key_dim) {
+        sm.key_prods = prods;
+        sm.fixed_key_prods = out.fixed_prods[d];
+      } else {
+        first_up[d] = fills.ints(nkd, 0x7fffffff);
+        sm.deg[v] = simplex_degree(d, key_dim);
+        sm.lows[v] = ask_down(c, old, d, key_dim, nullptr).data();
+        sm.first_up[v] = first_up[d].data();
+        kl.first_up[w] = first_up[d].data();
+      }
+      ++sm.n;
     }
-    if (d > key_dim) {
-      first_up[d] = LOs(c, nkd);
-      init.first_up[d] = first_up[d].data();
-      above = true;
-    }
-    if (d == key_dim) {
-      init.same = plan.same.data();
-      init.counts = plan.counts.data();
-    }
-  }
-  if (above) {
-    key_marks = Bytes(c, nkd);
-    init.key_marks = key_marks.data();
-  }
-  if (above || init.same) {
-    OSH_LAUNCH(init_key_dim, nkd, c, init);
-    ModPlan* kp = (key_dim >= d0 && key_dim <= d1) ? &plans[key_dim - d0] : nullptr;
-    OSH_LAUNCH(mark_keys, nkeys, c, keys2kds.data(),
-        kp ? keys2prods[key_dim].data() : (LO const*)nullptr, init.key_marks,
-        kp ? kp->same.data() : (I8*)nullptr, kp ? kp->counts.data() : (LO*)nullptr,
-        kp ? kp->reps.data() : (LO*)nullptr);
-  }
-  RepsJob jobs{};
-  int njobs = 0;
-  SameUpJobs up{};
-  for (int d = d0; d <= d1; ++d) {
-    ModPlan& plan = plans[d - d0];
-    if (d > key_dim) {
-      up.deg[up.n] = simplex_degree(d, key_dim);
-      up.hl2l[up.n] = ask_down(c, old, d, key_dim, nullptr).data();
-      up.same[up.n] = plan.same.data();
-      up.counts[up.n] = plan.counts.data();
-      up.first_up[up.n] = first_up[d].data();
-      up.start[up.n + 1] = up.start[up.n] + plan.nold;
-      ++up.n;
-      jobs.first_up[njobs] = first_up[d].data();
-    } else if (d < key_dim) {
-      plan.counts = fill_lo(c, plan.nold, 1);
-      jobs.deg[njobs] = simplex_degree(key_dim, d);
-      jobs.down[njobs] = ask_down(c, old, key_dim, d, nullptr).data();
-    } else {
-      continue;
-    }
-    jobs.keys2prods[njobs] = keys2prods[d].data();
-    jobs.reps[njobs] = plan.reps.data();
-    jobs.counts[njobs] = plan.counts.data();
-    ++njobs;
-  }
-  OSH_CHECK(njobs <= 3, "modify_plans: too many dimensions");
-  if (up.n) OSH_LAUNCH(mark_same_up_kernel, up.start[up.n], c, key_marks.data(), up);
-  if (njobs) OSH_LAUNCH(reps_kernel, njobs * nkeys, c, nkeys, keys2kds.data(), jobs,
-      c.error_word());
-}
-
-void modify_plans_masked(Ctx& c, DMesh& old, int key_dim, int d1, Bytes const& key_mask,
-    LO const* const* prod_counts, ModPlan* plans, LOs* rep_of) {
-  LO nkd = old.nents[key_dim];
-  KeyDimInit init{};
-  LOs first_up[4];
-  for (int d = key_dim; d <= d1; ++d) {
-    ModPlan& plan = plans[d - key_dim];
-    plan.ent_dim = d;
-    plan.key_dim = key_dim;
-    plan.nold = old.nents[d];
-    plan.same = Bytes(c, plan.nold);
-    plan.counts = LOs(c, plan.nold);
-    if (d > key_dim) {
-      first_up[d] = LOs(c, nkd);
-      init.first_up[d] = first_up[d].data();
-      rep_of[d] = LOs(c, nkd);
+    if (d != key_dim) {
+      int r = rc.n++;
+      rc.first_up[r] = kl.first_up[w];
+      rc.down[r] = kl.down[w];
+      rc.deg[r] = kl.deg[w];
+      rc.prods[r] = prods;
+      rc.fixed[r] = kl.fixed[w];
+      rc.counts[r] = plan.counts.data();
     }
   }
-  init.same = plans[0].same.data();
-  init.counts = plans[0].counts.data();
-  init.key_mask = key_mask.data();
-  init.key_prod_counts = prod_counts[key_dim];
-  OSH_LAUNCH(init_key_dim, nkd, c, init);
-  MaskedReps j{};
+  fills.run();
+  hipLaunchKernelGGL(mark_same_kernel, dim3(blocks), dim3(kBlock), 0, c.stream, keys.data(), sm);
+  OSH_HIP(hipGetLastError());
+  if (rc.n) OSH_LAUNCH(rep_counts_kernel, nkd, c, keys.data(), rc, c.error_word());
+  // the keys, their products and every dimension's new numbering by one scan
+  // and one wait
+  ScanJob jobs[kMaxScanJobs];
+  LOs off[4];
+  out.keys2kds = LOs(c, nkd);
   int nj = 0;
-  SameUpJobs up{};
-  for (int d = key_dim + 1; d <= d1; ++d) {
-    ModPlan& plan = plans[d - key_dim];
-    up.deg[up.n] = simplex_degree(d, key_dim);
-    up.hl2l[up.n] = ask_down(c, old, d, key_dim, nullptr).data();
-    up.same[up.n] = plan.same.data();
-    up.counts[up.n] = plan.counts.data();
-    up.first_up[up.n] = first_up[d].data();
-    up.start[up.n + 1] = up.start[up.n] + plan.nold;
-    ++up.n;
-    j.first_up[nj] = first_up[d].data();
-    j.prod_counts[nj] = prod_counts[d];
-    j.rep_of[nj] = rep_of[d].data();
-    j.counts[nj] = plan.counts.data();
-    ++nj;
+  jobs[nj++] = {keys.data(), kScanNonzero, nkd, nullptr, slot_ptr<LO>(c, 0),
+      out.keys2kds.data()};
+  for (int d = d0; d <= d1; ++d) {
+    if (!out.prod_counts[d].exists()) continue;
+    off[d] = LOs(c, nkd + 1);
+    kl.prod_off[d - d0] = off[d].data();
+    jobs[nj++] = {out.prod_counts[d].data(), kScanLO, nkd, off[d].data(),
+        slot_ptr<LO>(c, 1 + d)};
   }
-  OSH_CHECK(nj <= 3, "modify_plans_masked: too many dimensions");
-  if (up.n) OSH_LAUNCH(mark_same_up_kernel, up.start[up.n], c, key_mask.data(), up);
-  if (nj) OSH_LAUNCH(reps_masked, nj * nkd, c, nkd, key_mask.data(), j, c.error_word());
+  nj += modify_scan_jobs(c, out.plans, nd, jobs + nj, 5);
+  offset_scans(c, jobs, nj);
+  c.wait();
+  modify_scan_totals(c, out.plans, nd, 5);
+  out.nkeys = read_slot<LO>(c, 0);
+  out.keys2kds.shrink(out.nkeys);
+  for (int d = d0; d <= d1; ++d) {
+    out.nprods[d] = out.prod_counts[d].exists() ? read_slot<LO>(c, 1 + d)
+                                                 : out.nkeys * out.fixed_prods[d];
+    out.k2p[d] = LOs(c, out.nkeys + 1);
+    out.plans[d - d0].reps = LOs(c, out.nkeys);
+    kl.k2p[d - d0] = out.k2p[d].data();
+    kl.reps[d - d0] = out.plans[d - d0].reps.data();
+  }
+  kl.nkd = nkd;
+  OSH_LAUNCH(list_keys_kernel, out.nkeys + 1, c, out.nkeys, out.keys2kds.data(), kl);
 }
 
 int modify_scan_jobs(Ctx& c, ModPlan* plans, int nplans, ScanJob* jobs, int first_slot) {
@@ -856,15 +779,6 @@ int modify_scan_jobs(Ctx& c, ModPlan* plans, int nplans, ScanJob* jobs, int firs
 
 void modify_scan_totals(Ctx& c, ModPlan* plans, int nplans, int first_slot) {
   for (int i = 0; i < nplans; ++i) plans[i].nnew = read_slot<LO>(c, first_slot + i);
-}
-
-void modify_scan(Ctx& c, ModPlan* plans, int nplans) {
-  OSH_CHECK(nplans >= 1 && nplans <= 4, "modify_scan: too many dimensions");
-  ScanJob jobs[kMaxScanJobs];
-  int njobs = modify_scan_jobs(c, plans, nplans, jobs, 1);
-  offset_scans(c, jobs, njobs);
-  c.wait();
-  modify_scan_totals(c, plans, nplans, 1);
 }
 
 bool has_tags(DMesh const& m) {
@@ -956,29 +870,18 @@ void rebuild_same(Ctx& c, DMesh& old, DMesh& nw, int d0, ModPlan const* plans, M
 
 void place_products(Ctx& c, DMesh& old, DMesh& nw, int d0, int d1, int plan0,
     ModPlan const* plans, LOs const& keys2kds, Products const* prods, ModOut* mo,
-    I8* new_edges_valid) {
+    LOs const* order, I8* new_edges_valid) {
   LO nkeys = keys2kds.size();
   PlaceJobs j{};
   j.keys2kds = keys2kds.data();
   LOs src[4];
-  LOs order;
   for (int d = d0; d <= d1; ++d) {
     ModPlan const& plan = plans[d - plan0];
     Products const& p = prods[d];
     PlaceDim& a = j.d[d - d0];
     mo[d].nprods = p.n;
     mo[d].prods2new = LOs(c, p.n);
-    if (plan.key_dim > d) {
-      OSH_CHECK(!order.exists(), "one dimension below the keys");
-      LO nkd = old.nents[plan.key_dim];
-      order = fill_lo(c, nkd, -1);
-      LOs md2mod = fill_lo(c, nkd, -1);
-      OSH_LAUNCH(scatter_index, nkeys, c, keys2kds.data(), md2mod.data());
-      Adj const& up = ask_up(c, old, d, plan.key_dim);
-      OSH_LAUNCH(rep2md_order_kernel, plan.nold, c, up.a2ab.data(), up.ab2b.data(),
-          up.codes.data(), md2mod.data(), p.keys2prods.data(), order.data());
-      a.order = order.data();
-    }
+    a.order = plan.key_dim > d ? order->data() : nullptr;
     a.reps = plan.reps.data();
     a.offsets = plan.offsets.data();
     a.keys2prods = p.keys2prods.data();
@@ -1006,9 +909,7 @@ void place_products(Ctx& c, DMesh& old, DMesh& nw, int d0, int d1, int plan0,
     if (d == 1) a.zeroed = new_edges_valid;
   }
   int nd = d1 - d0 + 1;
-  OSH_CHECK(std::int64_t(nkeys) * kProdLanes * nd <= std::int64_t(0x7fffffff),
-      "place_products: too many keys");
-  OSH_LAUNCH(place_products_kernel, nkeys * kProdLanes * nd, c, nkeys, j);
+  OSH_LAUNCH64(place_products_kernel, std::int64_t(nkeys) * nd * kProdLanes, c, nkeys, j);
   if (nw.itags.size() != old.itags.size()) nw.itags = old.itags;
   for (int d = d0; d <= d1; ++d) {
     Products const& p = prods[d];
@@ -1099,45 +1000,28 @@ Bytes find_indset(Ctx& c, DMesh& m, int d, Reals const& quality, Bytes const& ca
   }
   Bytes a(c, n), b(c, n);
   DArray<unsigned long long> dom(c, n);
-  // rounds leave decided nodes as they are and take no node from the set, so
-  // extra rounds after convergence change nothing: run two rounds before each
-  // of the first four checks, then 4, 8 and 16 (long chains of decreasing
-  // quality, as on the first coarsening passes of a large smooth mesh, take
-  // some 200 rounds and would otherwise spend a wait every two)
   int first_lanes = fit_lanes(n, c.tuning.first_lanes);
-  for (LO round = 0;;) {
-    OSH_CHECK(round <= n + 1, "independent set does not converge");
-    int batch = round < 8 ? 2 : (round < 16 ? 4 : (round < 32 ? 8 : 16));
-    unsigned tag = c.wait_tag();
-    for (int k = 0; k < batch; ++k, ++round) {
-      bool first = round == 0;
-      IndsetWords w{c.words, first ? tag : 0u, k == batch - 1 ? tag : 0u};
-      I8 const* in = first ? cands.data() : a.data();
-      if (g && first)
-        OSH_LAUNCH(indset_iteration<true>, n, c, g->a2ab.data(), g->ab2b.data(),
-            quality.data(), in, b.data(), dom.data(), w);
-      else if (g)
-        OSH_LAUNCH(indset_iteration<false>, n, c, g->a2ab.data(), g->ab2b.data(),
-            quality.data(), in, b.data(), dom.data(), w);
-      else if (first && m.dim == 3)
-        OSH_LAUNCH((indset_first_edges<6>), n * first_lanes, c, first_lanes, e2c->a2ab.data(),
-            e2c->ab2b.data(), c2e, quality.data(), in, b.data(), dom.data(), w);
-      else if (first)
-        OSH_LAUNCH((indset_first_edges<3>), n * first_lanes, c, first_lanes, e2c->a2ab.data(),
-            e2c->ab2b.data(), c2e, quality.data(), in, b.data(), dom.data(), w);
-      else if (m.dim == 3)
-        OSH_LAUNCH(indset_iteration_edges<6>, n, c, e2c->a2ab.data(), e2c->ab2b.data(), c2e,
-            quality.data(), in, b.data(), dom.data(), w);
-      else
-        OSH_LAUNCH(indset_iteration_edges<3>, n, c, e2c->a2ab.data(), e2c->ab2b.data(), c2e,
-            quality.data(), in, b.data(), dom.data(), w);
-      std::swap(a, b);
-    }
-    c.wait();
-    if (any_cands && round == 2) *any_cands = c.word_set(kCandWord, tag);
-    if (!c.word_set(kUndecidedWord, tag)) break;
-  }
-  return a;
+  return indset_rounds(c, n, cands, a, b, any_cands,
+      [&](bool first, I8 const* in, I8* out, IndsetWords w) {
+        if (g && first)
+          OSH_LAUNCH(indset_iteration<true>, n, c, g->a2ab.data(), g->ab2b.data(),
+              quality.data(), in, out, dom.data(), w);
+        else if (g)
+          OSH_LAUNCH(indset_iteration<false>, n, c, g->a2ab.data(), g->ab2b.data(),
+              quality.data(), in, out, dom.data(), w);
+        else if (first && m.dim == 3)
+          OSH_LAUNCH((indset_first_edges<6>), n * first_lanes, c, first_lanes,
+              e2c->a2ab.data(), e2c->ab2b.data(), c2e, quality.data(), in, out, dom.data(), w);
+        else if (first)
+          OSH_LAUNCH((indset_first_edges<3>), n * first_lanes, c, first_lanes,
+              e2c->a2ab.data(), e2c->ab2b.data(), c2e, quality.data(), in, out, dom.data(), w);
+        else if (m.dim == 3)
+          OSH_LAUNCH(indset_iteration_edges<6>, n, c, e2c->a2ab.data(), e2c->ab2b.data(), c2e,
+              quality.data(), in, out, dom.data(), w);
+        else
+          OSH_LAUNCH(indset_iteration_edges<3>, n, c, e2c->a2ab.data(), e2c->ab2b.data(), c2e,
+              quality.data(), in, out, dom.data(), w);
+      });
 }
 
 Bytes mark_down(Ctx& c, DMesh& m, int high, int low, Bytes const& marks) {
@@ -1166,12 +1050,26 @@ Bytes mark_sliver_layers(Ctx& c, DMesh& m, Real qual_ceil, int nlayers) {
     return marks;
   }
   auto const& se = ask_side_elems(c, m);
-  // the first layer reads the sliver test itself
-  for (int i = 0; i < nlayers; ++i) {
-    Bytes next(c, ne);
-    OSH_LAUNCH(dual_max_kernel, ne, c, m.dim + 1, m.down[m.dim].data(), se.data(), marks.data(),
-        i == 0 ? q.data() : (Real const*)nullptr, qual_ceil, next.data(), c.error_word());
-    marks = next;
+  // the first layer reads the sliver test itself; later ones push, into
+  // buffers cleared eight at a time
+  marks = Bytes(c, ne);
+  OSH_LAUNCH(dual_max_kernel, ne, c, m.dim + 1, m.down[m.dim].data(), se.data(), q.data(),
+      qual_ceil, marks.data(), c.error_word());
+  Bytes next[8];
+  for (int i = 1; i < nlayers; ++i) {
+    int b = (i - 1) % 8;
+    if (b == 0) {
+      Fills fills(c);
+      for (int k = 0; k < 8 && i + k < nlayers; ++k) next[k] = fills.bytes(ne, 0);
+      fills.run();
+    }
+    if (m.dim == 3)
+      OSH_LAUNCH(push_layer_kernel<4>, ne, c, m.down[3].data(), se.data(), marks.data(),
+          next[b].data());
+    else
+      OSH_LAUNCH(push_layer_kernel<3>, ne, c, m.down[2].data(), se.data(), marks.data(),
+          next[b].data());
+    marks = next[b];
   }
   return marks;
 }

@@ -44,10 +44,9 @@ struct ModOut {
 };
 
 // modify_ents_adapt (src/Omega_h_modify.cpp:468-517) in steps that each cover
-// every dimension of a pass in one launch: modify_plans marks the same
-// entities, counts the new entities each old one stands for and finds the
-// representatives (no sync); modify_scan scans the counts of up to four
-// dimensions together; rebuild_same moves the same entities with all they
+// every dimension of a pass in one launch: plan_keys marks the same entities,
+// counts the new entities each old one stands for, finds the representatives
+// and scans the counts; rebuild_same moves the same entities with all they
 // carry; place_products numbers the products; match_sides connects them
 struct ModPlan {
   int ent_dim = 0, key_dim = 0;
@@ -55,20 +54,25 @@ struct ModPlan {
   Bytes same;
   LOs counts, reps, offsets;
 };
-// the plans of dimensions d0..d1 (keys2prods indexed by dimension)
-void modify_plans(Ctx& c, DMesh& old, int key_dim, int d0, int d1, LOs const& keys2kds,
-    LOs const* keys2prods, ModPlan* plans);
-void modify_scan(Ctx& c, ModPlan* plans, int nplans);
-// the same plans for dimensions key_dim..d1 with the keys given as a mask
-// over the key dimension and their product counts per key-dimension entity
-// (prod_counts[d]); plans' reps stay empty and rep_of[d] (d > key_dim)
-// receives each key's representative by key-dimension entity, so that the
-// keys need not be listed before the scan
-void modify_plans_masked(Ctx& c, DMesh& old, int key_dim, int d1, Bytes const& key_mask,
-    LO const* const* prod_counts, ModPlan* plans, LOs* rep_of);
-// modify_scan in two halves, for callers that add the plans' scans to a
-// launch of their own: the jobs (totals in pinned slots first_slot...), then,
-// after the caller's wait, the totals
+// what a pass's keys come to.  The caller sets, per rebuilt dimension, the
+// products of every key-dimension entity (0 where it is no key), or the fixed
+// count of each key.
+struct KeyedMods {
+  LOs prod_counts[4];
+  LO fixed_prods[4] = {0, 0, 0, 0};
+  LO nkeys = 0;
+  LOs keys2kds;
+  LOs k2p[4];
+  LO nprods[4] = {0, 0, 0, 0};
+  ModPlan plans[4];  // plans[d - d0]
+  LOs order;         // of the dimension below the keys, by key-dimension entity
+};
+// the plans of dimensions d0..d1 from the keys, a mask over the key dimension,
+// with one wait for everything that depends on the keys
+void plan_keys(Ctx& c, DMesh& old, int key_dim, int d0, int d1, Bytes const& keys,
+    KeyedMods& out);
+// the scans of plans' counts, for a launch of the caller's: the jobs (totals in
+// pinned slots first_slot...), then, after the caller's wait, the totals
 int modify_scan_jobs(Ctx& c, ModPlan* plans, int nplans, ScanJob* jobs, int first_slot);
 void modify_scan_totals(Ctx& c, ModPlan* plans, int nplans, int first_slot);
 
@@ -100,11 +104,12 @@ struct Products {
 };
 // numbers the products of dimensions d0..d1 (prods[d], mo[d], plans[d -
 // plan0]) and writes their vertex lists and classification, in one launch;
-// inheritance tags of those dimensions follow.  new_edges_valid, when given,
-// is zeroed at new edges.
+// inheritance tags of those dimensions follow.  order: KeyedMods::order, for
+// the dimension below the keys; new_edges_valid, when given, is zeroed at new
+// edges.
 void place_products(Ctx& c, DMesh& old, DMesh& nw, int d0, int d1, int plan0,
     ModPlan const* plans, LOs const& keys2kds, Products const* prods, ModOut* mo,
-    I8* new_edges_valid = nullptr);
+    LOs const* order = nullptr, I8* new_edges_valid = nullptr);
 // the sides and codes of the placed products of dimensions 2..dim, by their
 // vertices among the new mesh's entities (reflect_down)
 void match_sides(Ctx& c, DMesh& nw, Products const* prods, ModOut const* mo);

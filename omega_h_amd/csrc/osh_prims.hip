@@ -864,10 +864,10 @@ namespace {
 
 struct FillJobs {
   int n;
-  unsigned first[9];
-  void* p[8];
-  std::size_t bytes[8];
-  unsigned pattern[8];
+  unsigned first[17];
+  void* p[16];
+  std::size_t bytes[16];
+  unsigned pattern[16];
 };
 
 // 16 bytes a thread; blocks come from the pool, so every start is aligned and

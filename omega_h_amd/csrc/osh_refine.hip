@@ -120,15 +120,19 @@ struct RefineRows {
   I8* psrc_dim[3];
 };
 
-__global__ void prod_counts(LO nt, LO nkeys, LO const* keys2edges, RefineRows r) {
-  LO t = thread_index();
-  if (t >= nt) return;
-  int d = t / nkeys;
-  LO k = t % nkeys;
-  LO e = keys2edges[k];
-  LO n = r.pairs_a2ab[d] ? 2 * (r.pairs_a2ab[d][e + 1] - r.pairs_a2ab[d][e]) : 2;
-  if (r.cuts_a2ab[d]) n += r.cuts_a2ab[d][e + 1] - r.cuts_a2ab[d][e];
-  r.counts[d][k] = n;
+// the products of every edge in dimensions 1..n (0 for edges that are no keys)
+__global__ void prod_counts(LO nedges, int n, I8 const* keys, RefineRows r) {
+  LO e = thread_index();
+  if (e >= nedges) return;
+  bool key = keys[e] != 0;
+  for (int d = 0; d < n; ++d) {
+    LO k = 0;
+    if (key) {
+      k = r.pairs_a2ab[d] ? 2 * (r.pairs_a2ab[d][e + 1] - r.pairs_a2ab[d][e]) : 2;
+      if (r.cuts_a2ab[d]) k += r.cuts_a2ab[d][e + 1] - r.cuts_a2ab[d][e];
+    }
+    r.counts[d][e] = k;
+  }
 }
 
 // every product's position follows from its row entry, so kRowLanes threads
@@ -201,14 +205,14 @@ __device__ __forceinline__ void refine_products_of(int lane, LO e, LO mid, LO pr
   }
 }
 
-__global__ void refine_products(LO nt, LO nkeys, LO const* keys2edges, LO const* keys2mid,
-    LO const* ev2v, LO const* vert_offsets, RefineRows r) {
-  LO t = thread_index();
+__global__ void refine_products(std::int64_t nt, LO nkeys, LO const* keys2edges,
+    LO const* keys2mid, LO const* ev2v, LO const* vert_offsets, RefineRows r) {
+  std::int64_t t = thread_index64();
   if (t >= nt) return;
-  LO per = nkeys * kRowLanes;
-  int d = t / per;
-  LO k = (t % per) / kRowLanes;
-  int lane = t % kRowLanes;
+  std::int64_t row = t / kRowLanes;
+  int d = int(row / nkeys);
+  LO k = LO(row % nkeys);
+  int lane = int(t % kRowLanes);
   LO e = keys2edges[k];
   LO mid = keys2mid[k];
   LO prod0 = r.keys2prods[d][k];
@@ -302,65 +306,55 @@ bool refine_by_size(Ctx& c, DMesh& m, AdaptOptions const& o) {
   Reals cand_metrics;
   Reals quals = refine_qualities(c, m, cands, &cand_metrics);
   Bytes initial = fill_i8(c, ne, 0);
-  Reals edge_quals = fill_real(c, ne, 0.0);
+  Reals edge_quals(c, ne);  // read where an edge is a candidate
   OSH_LAUNCH(seed_keys, cands.size(), c, cands.data(), quals.data(), o.min_quality_allowed,
       initial.data(), edge_quals.data());
   bool any;
   Bytes keys = find_indset(c, m, 1, edge_quals, initial, &any);
   if (!any) return false;
   Range modify_range(c, "modify_ents");
-  LOs keys2edges = collect_marked(c, keys);
-  LO nkeys = keys2edges.size();
-  note_changed_parts(c, m, 1, keys2edges);
-  if (o.verbosity >= 2) std::printf("refining %d edges\n", int(nkeys));
   int nc = m.metric_ncomps;
   DMesh nw;
   nw.dim = dim;
   nw.metric_ncomps = nc;
-  // products per key of every dimension, numbered by one scan launch
-  LOs k2p[4];
-  LO nprods[4] = {nkeys, 0, 0, 0};
   RefineRows rows{};
-  k2p[0] = iota(c, nkeys + 1);
-  {
-    LOs counts(c, dim * nkeys);
-    ScanJob jobs[3];
-    for (int d = 1; d <= dim; ++d) {
-      if (d > 1) {
-        Adj const& pr = ask_up(c, m, 1, d);
-        rows.pairs_a2ab[d - 1] = pr.a2ab.data();
-        rows.pairs_ab2b[d - 1] = pr.ab2b.data();
-        rows.pairs_codes[d - 1] = pr.codes.data();
-        rows.pair_verts[d - 1] = verts_of(c, m, d).data();
-      }
-      if (d < dim) {
-        Adj const& ct = ask_up(c, m, 1, d + 1);
-        rows.cuts_a2ab[d - 1] = ct.a2ab.data();
-        rows.cuts_ab2b[d - 1] = ct.ab2b.data();
-        rows.cuts_codes[d - 1] = ct.codes.data();
-        rows.cut_verts[d - 1] = verts_of(c, m, d + 1).data();
-      }
-      rows.counts[d - 1] = counts.data() + std::size_t(d - 1) * nkeys;
-      k2p[d] = LOs(c, nkeys + 1);
-      rows.keys2prods[d - 1] = k2p[d].data();
-      jobs[d - 1] = {rows.counts[d - 1], kScanLO, nkeys, k2p[d].data(), slot_ptr<LO>(c, d)};
+  KeyedMods km;
+  km.fixed_prods[0] = 1;
+  for (int d = 1; d <= dim; ++d) {
+    if (d > 1) {
+      Adj const& pr = ask_up(c, m, 1, d);
+      rows.pairs_a2ab[d - 1] = pr.a2ab.data();
+      rows.pairs_ab2b[d - 1] = pr.ab2b.data();
+      rows.pairs_codes[d - 1] = pr.codes.data();
+      rows.pair_verts[d - 1] = verts_of(c, m, d).data();
     }
-    OSH_LAUNCH(prod_counts, dim * nkeys, c, nkeys, keys2edges.data(), rows);
-    offset_scans(c, jobs, dim);
-    c.wait();
-    for (int d = 1; d <= dim; ++d) nprods[d] = read_slot<LO>(c, d);
+    if (d < dim) {
+      Adj const& ct = ask_up(c, m, 1, d + 1);
+      rows.cuts_a2ab[d - 1] = ct.a2ab.data();
+      rows.cuts_ab2b[d - 1] = ct.ab2b.data();
+      rows.cuts_codes[d - 1] = ct.codes.data();
+      rows.cut_verts[d - 1] = verts_of(c, m, d + 1).data();
+    }
+    km.prod_counts[d] = LOs(c, ne);
+    rows.counts[d - 1] = km.prod_counts[d].data();
   }
-  // every dimension's new numbering by one more scan launch
-  ModPlan plans[4];
-  modify_plans(c, m, 1, 0, dim, keys2edges, k2p, plans);
-  modify_scan(c, plans, dim + 1);
+  OSH_LAUNCH(prod_counts, ne, c, dim, keys.data(), rows);
+  plan_keys(c, m, 1, 0, dim, keys, km);
+  LO nkeys = km.nkeys;
+  LOs const& keys2edges = km.keys2kds;
+  LOs const* k2p = km.k2p;
+  LO const* nprods = km.nprods;
+  ModPlan const* plans = km.plans;
+  for (int d = 1; d <= dim; ++d) rows.keys2prods[d - 1] = k2p[d].data();
+  note_changed_parts(c, m, 1, keys2edges);
+  if (o.verbosity >= 2) std::printf("refining %d edges\n", int(nkeys));
   ModOut mo[4];
   rebuild_same(c, m, nw, 0, plans, mo);
   Products prods[4];
   prods[0].n = nkeys;
   prods[0].keys2prods = k2p[0];
   prods[0].src_dim = 1;
-  place_products(c, m, nw, 0, 0, 0, plans, keys2edges, prods, mo);
+  place_products(c, m, nw, 0, 0, 0, plans, keys2edges, prods, mo, &km.order);
   LO const* keys2mid = mo[0].prods2new.data();
   OSH_LAUNCH(place_midpoints, nkeys, c, dim, nc, keys2edges.data(), keys2mid,
       m.down[1].data(), m.coords.data(), cand_of_edge.data(), cand_metrics.data(),
@@ -377,7 +371,7 @@ bool refine_by_size(Ctx& c, DMesh& m, AdaptOptions const& o) {
     rows.psrc[d - 1] = p.src.data();
     rows.psrc_dim[d - 1] = p.src_dims.data();
   }
-  OSH_LAUNCH(refine_products, dim * nkeys * kRowLanes, c, nkeys, keys2edges.data(), keys2mid,
+  OSH_LAUNCH64(refine_products, std::int64_t(nkeys) * dim * kRowLanes, c, nkeys, keys2edges.data(), keys2mid,
       m.down[1].data(), plans[0].offsets.data(), rows);
   place_products(c, m, nw, 1, dim, 0, plans, keys2edges, prods, mo);
   match_sides(c, nw, prods, mo);

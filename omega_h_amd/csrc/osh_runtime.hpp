@@ -311,6 +311,23 @@ inline unsigned nblocks(LO n, int block = kBlock) {
     }                                                                          \
   } while (0)
 
+// the same for thread counts past 32 bits (several lanes per row in several
+// dimensions)
+#define OSH_LAUNCH64(kernel, n, c, ...)                                        \
+  do {                                                                         \
+    std::int64_t osh_n_ = (n);                                                 \
+    if (osh_n_ > 0) {                                                          \
+      hipLaunchKernelGGL(kernel,                                               \
+          dim3(unsigned((osh_n_ + ::osh::kBlock - 1) / ::osh::kBlock)),        \
+          dim3(::osh::kBlock), 0, (c).stream, osh_n_, __VA_ARGS__);            \
+      OSH_HIP(hipGetLastError());                                              \
+    }                                                                          \
+  } while (0)
+
+__device__ __forceinline__ std::int64_t thread_index64() {
+  return std::int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+}
+
 __device__ __forceinline__ LO thread_index() {
   return LO(blockIdx.x) * LO(blockDim.x) + LO(threadIdx.x);
 }
@@ -396,7 +413,7 @@ class Fills {
   void run();
 
  private:
-  static constexpr int kMax = 8;
+  static constexpr int kMax = 16;
   void add(void* p, std::size_t bytes, unsigned pattern);
   Ctx& c_;
   int n_ = 0;

@@ -12,6 +12,7 @@
 //   transfer_swap / transfer_copy                src/Omega_h_transfer.cpp:631-730
 #include <cstdio>
 
+#include "osh_indset.hpp"
 #include "osh_math.hpp"
 #include "osh_passes.hpp"
 #include "osh_swap_tables.hpp"
@@ -22,7 +23,21 @@ namespace {
 
 using swap::Tables;
 
-constexpr int kLoopLanes = 8;  // at least swap::kMaxLoop
+// The tets around the candidate edges of a swap pass: kRow slots per
+// candidate, in the order of the atomics, each the use index tet * 6 +
+// local edge.  Only edges with at most swap::kMaxLoop tets can be swapped, so
+// a candidate with more just counts them; fixed rows need no scan of counts.
+constexpr int kRow = 8;
+static_assert(swap::kMaxLoop <= kRow, "a loop fits a row");
+
+struct EdgeRings {
+  LO const* cands;     // the candidate edges
+  LO const* cand_of;   // candidate index of an edge
+  LO const* counts;    // tets around an edge, by edge
+  LO const* rows;      // kRow use indices per candidate
+  LO const* t2e;       // the elements' edges and their codes
+  I8 const* t2e_codes;
+};
 
 struct Loop {
   int size;
@@ -131,329 +146,386 @@ __device__ double length_between(LO a, LO b, Real const* coords, Real const* met
   return edge_length<S, M>(p0, p1, m0, m1);
 }
 
-// swap3d_qualities (src/Omega_h_swap3d_qualities.cpp:11-75) in four flat
-// sweeps instead of one thread per candidate edge:
-//   swap3d_loops:     the loop of each candidate and its counts of unique
-//                     triangles and unique interior edges
-//   swap3d_loop_measures: one thread per (candidate, unique triangle): the
-//                     min quality of the two tets on that triangle, and one
-//                     per (candidate, unique edge): its length
-//   swap3d_mesh_quals: one thread per (candidate, triangulation): its value
-//                     for choose() of src/Omega_h_swap3d_choice.hpp
-//   swap3d_choose:    per candidate, the choice over those values in the
-//                     reference's order
-// Every value is the one the reference computes (each unique triangle and
-// edge evaluated once), so the choice is the same.
-__global__ void swap3d_loops(LO nt, LO const* cands, LO const* e2t_a2ab, LO const* e2t_ab2b,
-    I8 const* e2t_codes, LO const* ev2v, LO const* tv2v, Tables const* tb, I8 const* cached,
-    LO* lsize, LO* leev, LO* lverts, LO* ntris, LO* nedges, int* error) {
-  // kLoopLanes threads per candidate: lane le reads the le-th tet around
-  // the edge; the group then orders the loop as find_loop does
-  LO t = thread_index();
-  if (t >= nt) return;
-  LO cand = t / kLoopLanes;
-  int lane = t % kLoopLanes;
-  LO edge = cands[cand];
-  LO begin = e2t_a2ab[edge];
-  int size = e2t_a2ab[edge + 1] - begin;
-  LO x0 = -1, x1 = -1;
-  if (size <= swap::kMaxLoop && lane < size) {
-    LO tet = e2t_ab2b[begin + lane];
-    I8 code = e2t_codes[begin + lane];
-    int rre_opp = opposite_template(3, 1, code_which_down(code));
-    int rot = code_rotation(code);
-    x0 = tv2v[tet * 4 + down_template(3, 1, rre_opp, rot)];
-    x1 = tv2v[tet * 4 + down_template(3, 1, rre_opp, rot ^ 1)];
-  }
-  int base = int(threadIdx.x % 64) & ~(kLoopLanes - 1);
-  LO tmp[swap::kMaxLoop][2];
-#pragma unroll
-  for (int k = 0; k < swap::kMaxLoop; ++k) {
-    tmp[k][0] = __shfl(x0, base + k, 64);
-    tmp[k][1] = __shfl(x1, base + k, 64);
-  }
-  if (lane != 0) return;
-  lsize[cand] = size;
-  if (size > swap::kMaxLoop) {
-    ntris[cand] = 0;
-    nedges[cand] = 0;
-    return;
-  }
-  for (int i = 0; i < size - 1; ++i) {
-    int j;
-    for (j = i + 1; j < size; ++j)
-      if (tmp[j][0] == tmp[i][1]) break;
-    if (j >= size) {
-      // the tets around the edge do not close a ring (the reference aborts,
-      // src/Omega_h_swap3d_loop.hpp:71): no configuration, and an error
-      *error = kBrokenSwapLoop;
-      ntris[cand] = 0;
-      nedges[cand] = 0;
-      lsize[cand] = swap::kMaxLoop + 1;
-      return;
-    }
-    LO t0 = tmp[i + 1][0], t1 = tmp[i + 1][1];
-    tmp[i + 1][0] = tmp[j][0];
-    tmp[i + 1][1] = tmp[j][1];
-    tmp[j][0] = t0;
-    tmp[j][1] = t1;
-  }
-  leev[cand * 2 + 0] = ev2v[edge * 2];
-  leev[cand * 2 + 1] = ev2v[edge * 2 + 1];
-  for (int k = 0; k < swap::kMaxLoop; ++k)
-    lverts[cand * swap::kMaxLoop + k] = (k < size) ? tmp[k][0] : -1;
-  // a carried-over choice needs the loop (for products) but no qualities
-  bool carried = cached && cached[edge];
-  ntris[cand] = carried ? 0 : tb->ntris[size];
-  nedges[cand] = carried ? 0 : tb->nuedges[size];
+__global__ void swap3d_rows(LO nuses, LO const* t2e, I8 const* marks, LO const* cand_of,
+    LO* counts, LO* rows) {
+  LO i = thread_index();
+  if (i >= nuses) return;
+  LO e = t2e[i];
+  if (!marks[e]) return;
+  LO slot = atomicAdd(&counts[e], 1);
+  if (slot < kRow) rows[std::size_t(cand_of[e]) * kRow + slot] = i;
 }
 
-// F32 (mixed precision): FP32 estimates, and a candidate with an element
-// whose max-determinant metric is not clear is marked in `unsure`; with
-// `need` given, the FP64 sweep evaluates only the marked candidates
-// the loop measures of the candidates in one launch: threads [0, ntp) take
-// the (candidate, unique triangle) slots, the rest the (candidate, unique
-// edge) slots
-struct LoopMeasures {
-  LO ntp;
-  LO const* ntris;
-  LO const* nedges;
-  LO const* lsize;
-  LO const* leev;
-  LO const* lverts;
+// The loop of vertices around a candidate edge (find_loop,
+// src/Omega_h_swap3d_loop.hpp:24-78) by a group of at least kRow lanes, the
+// lanes from `base` on in the wave: lane k < size brings use index `use` and
+// returns with the loop's k-th vertex.  The ring starts at the tet with the
+// smallest index, and each tet is followed by the one that begins at its last
+// vertex.  *ok is false (in every lane) where no such tet is left: the tets
+// do not close a ring (the reference aborts,
+// src/Omega_h_swap3d_loop.hpp:71).
+__device__ __forceinline__ LO ring_vertex(int size, int lane, int base, LO use,
+    I8 const* t2e_codes, LO const* tv2v, bool* ok) {
+  LO x0 = -1, x1 = -1;
+  bool in = lane < size;
+  if (in) {
+    LO tet = use / 6;
+    int rot = code_rotation(t2e_codes[use]);
+    int opp = opposite_template(3, 1, int(use % 6));
+    x0 = tv2v[tet * 4 + down_template(3, 1, opp, rot)];
+    x1 = tv2v[tet * 4 + down_template(3, 1, opp, rot ^ 1)];
+  }
+  // the lane with the smallest use
+  LO least = in ? use : 0x7fffffff;
+  for (int d = kRow / 2; d > 0; d >>= 1) {
+    LO o = __shfl_xor(least, d, 64);
+    least = o < least ? o : least;
+  }
+  least = __shfl(least, base, 64);  // lanes of the row's first eight hold it
+  unsigned long long group = ((1ull << kRow) - 1ull) << base;
+  unsigned long long at = __ballot(in && use == least) & group;
+  int cur = __ffsll(static_cast<long long>(at)) - 1;
+  unsigned long long done = at;
+  LO mine = __shfl(x0, cur, 64);
+  if (lane != 0) mine = -1;
+  *ok = true;
+  for (int i = 1; i < size; ++i) {
+    LO v = __shfl(x1, cur, 64);
+    unsigned long long next = __ballot(in && x0 == v) & group & ~done;
+    if (next == 0ull) {
+      *ok = false;
+      break;
+    }
+    cur = __ffsll(static_cast<long long>(next)) - 1;
+    done |= 1ull << cur;
+    if (lane == i) mine = v;
+  }
+  return mine;
+}
+
+// swap3d_qualities (src/Omega_h_swap3d_qualities.cpp:11-75) and choose
+// (src/Omega_h_swap3d_choice.hpp:16-100) in one launch: a group of lanes per
+// candidate finds the edge's loop, measures each (unique triangle, side) and
+// each unique interior edge once, in LDS, values every triangulation and
+// takes the best.  A triangulation's value is its minimum triangle quality, or
+// -1 when one of its interior edges is longer than max_length; choose() keeps
+// the first triangulation whose quality exceeds every earlier kept one
+// (starting from 0) and whose edges pass, so it equals the first one attaining
+// the largest of these values, when that is positive.
+//
+// Most candidates of a late pass carry their choice over and return at once,
+// so the launch is bound by the latency of one evaluation, not by the FP64
+// rate: loops, measures, triangulations and choice in launches of their own,
+// with their intermediate arrays, took 32 us where this takes 16 us.
+//
+// MIXED: an FP32 estimate first.  Its best value, where an interior edge
+// counts as too long only when its FP32 length exceeds max_length by more
+// than the band, is an upper estimate of the FP64 choice's quality; the
+// candidate needs no FP64 when that is below the edge's current minimum
+// quality by more than the band, with every element's metric clear and that
+// minimum positive.
+struct EvalArgs {
+  EdgeRings r;
+  LO ncands;
+  LO const* ev2v;
+  LO const* tv2v;
   Real const* coords;
   Real const* metric;
+  Real const* elem_quals;
+  Real max_length;
   Tables const* tb;
-  I8 const* need;
-  I8* unsure;
-  Real* tq;
-  Real* el;
+  I8* configs;
+  Real* quals;
+  I8* keep;
+  I8* c_valid;  // null: no cache
+  I8* c_cfg;
+  I8* c_keep;
+  Real* c_q;
+  int* error;
 };
 
-template <int M, bool F32>
-__device__ __forceinline__ void swap3d_tri_qual(LO p, LO const* ntris, LO const* lsize,
-    LO const* leev, LO const* lverts, Real const* coords, Real const* metric, Tables const* tb,
-    I8 const* need, I8* unsure, Real* tq) {
-  // a fixed stride of kMaxUniqueTris slots per candidate
-  LO cand = p / swap::kMaxUniqueTris;
-  int ut = p % swap::kMaxUniqueTris;
-  if (ut >= ntris[cand]) return;
-  if (!F32 && need && !need[cand]) return;
-  int n = lsize[cand];
-  LO tv[4];
-  for (int k = 0; k < 3; ++k) tv[k] = lverts[cand * swap::kMaxLoop + tb->tris[n][ut][k]];
-  double tri_minqual = 1.0;
-  float minq32 = 1.0f;
-  bool unclear = false;
-  for (int tri_tet = 0; tri_tet < 2; ++tri_tet) {
-    tv[3] = leev[cand * 2 + 1 - tri_tet];
-    if constexpr (F32) {
-      float q = tet_quality32<M>(tv, coords, metric, &unclear);
-      minq32 = (q < minq32) ? q : minq32;
-    } else {
-      tri_minqual = math::min2(tri_minqual, tet_quality<M>(tv, coords, metric));
+constexpr int kMinEvalLanes = kRow;
+
+// LDS written by some lanes of a wave and read by others of the same wave
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <int M, bool MIXED>
+__global__ void __launch_bounds__(kBlock) swap3d_evaluate_kernel(LO nt, int lshift, EvalArgs a) {
+  constexpr int kGroups = kBlock / kMinEvalLanes;
+  __shared__ double s_tq[kGroups][swap::kMaxUniqueTris];
+  __shared__ double s_el[kGroups][swap::kMaxUniqueEdges];
+  __shared__ LO s_lv[kGroups][kRow];
+  LO t = thread_index();
+  if (t >= nt) return;
+  int lanes = 1 << lshift;
+  LO cand = t >> lshift;
+  int lane = int(t) & (lanes - 1);
+  int base = int(threadIdx.x % 64) & ~(lanes - 1);
+  int g = int(threadIdx.x) >> lshift;
+  LO edge = a.r.cands[cand];
+  if (a.c_valid && a.c_valid[edge]) {
+    if (lane == 0) {
+      a.configs[edge] = a.c_cfg[edge];
+      if (a.c_keep[edge]) {
+        a.keep[edge] = 1;
+        a.quals[edge] = a.c_q[edge];
+      }
     }
-    LO t = tv[1];
-    tv[1] = tv[2];
-    tv[2] = t;
+    return;
   }
-  if constexpr (F32) {
-    if (unclear) unsure[cand] = 1;
-    tq[p] = double(minq32);
-  } else {
-    tq[p] = tri_minqual;
-  }
-}
-
-template <int M, bool F32>
-__device__ __forceinline__ void swap3d_edge_len(LO q, LO const* nedges, LO const* lsize,
-    LO const* lverts, Real const* coords, Real const* metric, Tables const* tb, I8 const* need,
-    Real* el) {
-  // a fixed stride of kMaxUniqueEdges slots per candidate
-  LO cand = q / swap::kMaxUniqueEdges;
-  int ue = q % swap::kMaxUniqueEdges;
-  if (ue >= nedges[cand]) return;
-  if (!F32 && need && !need[cand]) return;
-  int n = lsize[cand];
-  LO const* lv = lverts + cand * swap::kMaxLoop;
-  LO a = lv[tb->uedges[n][ue][0]], b = lv[tb->uedges[n][ue][1]];
-  if constexpr (F32)
-    el[q] = double(length_between32<3, M>(a, b, coords, metric));
-  else
-    el[q] = length_between<3, M>(a, b, coords, metric);
-}
-
-template <int M, bool F32>
-__global__ void swap3d_loop_measures(LO nt, LoopMeasures a) {
-  LO t = thread_index();
-  if (t >= nt) return;
-  if (t < a.ntp)
-    swap3d_tri_qual<M, F32>(t, a.ntris, a.lsize, a.leev, a.lverts, a.coords, a.metric, a.tb,
-        a.need, a.unsure, a.tq);
-  else
-    swap3d_edge_len<M, F32>(t - a.ntp, a.nedges, a.lsize, a.lverts, a.coords, a.metric, a.tb,
-        a.need, a.el);
-}
-
-// one thread per (candidate, triangulation) on a fixed stride of
-// kMaxMeshes: the triangulation's minimum triangle quality, or -1 when one of
-// its interior edges is longer than max_length.  choose() keeps the first
-// triangulation whose quality exceeds every earlier kept one (starting from
-// 0) and whose edges pass, so it equals the first triangulation attaining
-// the largest of these values, when that is positive; a minimum that went
-// negative (where choose() stops early) is never kept either way.
-constexpr int kMaxMeshes = 42;
-
-__global__ void swap3d_mesh_quals(LO nt, LO const* lsize, LO const* ntris, Real const* tq,
-    Real const* el, Real max_length, Tables const* tb, I8 const* need, Real* mq) {
-  LO t = thread_index();
-  if (t >= nt) return;
-  LO cand = t / kMaxMeshes;
-  int mesh = t % kMaxMeshes;
-  int n = lsize[cand];
-  if (n > swap::kMaxLoop || mesh >= tb->mesh_counts[n]) return;
-  if (ntris[cand] == 0) return;  // a carried-over choice
-  if (need && !need[cand]) return;  // rejected by the mixed-precision screen
-  int nmesh_tris = tb->mesh_sizes[n];
-  int nmesh_edges = tb->nedges[n];
-  Real const* ctq = tq + LO(cand) * swap::kMaxUniqueTris;
-  Real const* cel = el + LO(cand) * swap::kMaxUniqueEdges;
-  double q = 1.0;
-  for (int mt = 0; mt < nmesh_tris; ++mt)
-    q = math::min2(q, ctq[tb->meshes[n][mesh * nmesh_tris + mt]]);
-  for (int me = 0; me < nmesh_edges; ++me)
-    if (cel[tb->medges[n][mesh * nmesh_edges + me]] > max_length) q = -1.0;
-  mq[t] = q;
-}
-
-// the mixed-precision screen of one candidate (Tuning::choose_lanes threads): the
-// best FP32 triangulation value, where an interior edge counts as too long
-// only when its FP32 length exceeds max_length by more than the band, is an
-// upper estimate of the FP64 choice's quality; the candidate needs FP64
-// unless that estimate is below the edge's current minimum quality by more
-// than the band (with every element's metric clear and that minimum
-// positive)
-__global__ void swap3d_screen(LO nt, int lanes, LO const* cands, LO const* lsize,
-    LO const* ntris, Real const* tq, Real const* el, Real max_length, Tables const* tb,
-    LO const* e2t_a2ab, LO const* e2t_ab2b, Real const* elem_quals, I8 const* unsure,
-    I8* need) {
-  LO t = thread_index();
-  if (t >= nt) return;
-  LO cand = t / lanes;
-  int lane = t % lanes;
-  LO edge = cands[cand];
-  int n = lsize[cand];
-  bool open = ntris[cand] != 0 && n <= swap::kMaxLoop;  // not carried over, a loop
-  double best = -1.0;
+  int n = a.r.counts[edge];
+  Tables const* tb = a.tb;
+  // old: the smallest quality around the edge; each lane keeps the first of
+  // its triangulations with the largest value above 0
+  double old = 1.79769313486231570815e+308;
+  int choice = -1;
+  double choice_quality = n <= swap::kMaxLoop ? 0.0 : -1.0;
+  bool open = n >= 1 && n <= swap::kMaxLoop;
+  LO use = 0;
+  LO eev[2] = {0, 0};
   if (open) {
-    int nmesh_tris = tb->mesh_sizes[n];
-    int nmesh_edges = tb->nedges[n];
-    Real const* ctq = tq + LO(cand) * swap::kMaxUniqueTris;
-    Real const* cel = el + LO(cand) * swap::kMaxUniqueEdges;
-    double lmax = max_length * (1.0 + double(f32::kScreenBand));
-    for (int mesh = lane; mesh < tb->mesh_counts[n]; mesh += lanes) {
-      double q = 1.0;
-      for (int mt = 0; mt < nmesh_tris; ++mt)
-        q = math::min2(q, ctq[tb->meshes[n][mesh * nmesh_tris + mt]]);
-      for (int me = 0; me < nmesh_edges; ++me)
-        if (cel[tb->medges[n][mesh * nmesh_edges + me]] > lmax) q = -1.0;
-      best = math::max2(best, q);
+    use = lane < n ? a.r.rows[std::size_t(cand) * kRow + lane] : 0;
+    bool ok;
+    LO v = ring_vertex(n, lane, base, use, a.r.t2e_codes, a.tv2v, &ok);
+    if (!ok) {
+      if (lane == 0) *a.error = kBrokenSwapLoop;
+      open = false;
+      choice_quality = -1.0;
     }
+    if (lane < kRow) s_lv[g][lane] = v;
+    eev[0] = a.ev2v[edge * 2];
+    eev[1] = a.ev2v[edge * 2 + 1];
+    if (lane < n) old = math::min2(old, a.elem_quals[use / 6]);
+    for (int d = kRow / 2; d > 0; d >>= 1) old = math::min2(old, __shfl_xor(old, d, 64));
+    old = __shfl(old, base, 64);
+    wave_lds_fence();
   }
-  double old = 1.79769313486231570815e+308;
-  for (LO j = e2t_a2ab[edge] + lane; j < e2t_a2ab[edge + 1]; j += lanes)
-    old = math::min2(old, elem_quals[e2t_ab2b[j]]);
-  for (int d = lanes / 2; d > 0; d >>= 1) {
-    best = math::max2(best, __shfl_xor(best, d, 64));
-    old = math::min2(old, __shfl_xor(old, d, 64));
-  }
-  if (lane != 0) return;
-  bool reject = open && !unsure[cand] && old > 0.0 &&
-                best < old * (1.0 - double(f32::kScreenBand));
-  need[cand] = reject ? 0 : 1;
-}
-
-__global__ void swap3d_choose(LO nt, int lanes, LO const* cands, LO const* lsize,
-    Real const* mq, LO const* e2t_a2ab, LO const* e2t_ab2b, Real const* elem_quals,
-    Tables const* tb, I8 const* need, I8* configs, Real* quals, I8* keep, I8* c_valid,
-    I8* c_cfg, I8* c_keep, Real* c_q) {
-  // `lanes` threads (a power of two, Tuning::choose_lanes) per candidate
-  // share its triangulations and tets
-  LO t = thread_index();
-  if (t >= nt) return;
-  LO cand = t / lanes;
-  int lane = t % lanes;
-  LO edge = cands[cand];
-  if (c_valid && c_valid[edge]) {
-    if (lane == 0) {
-      configs[edge] = c_cfg[edge];
-      if (c_keep[edge]) {
-        keep[edge] = 1;
-        quals[edge] = c_q[edge];
-      }
-    }
-    return;
-  }
-  if (need && !need[cand]) {
-    // the mixed-precision screen showed that no triangulation improves on
-    // the edge's elements: not kept, as the FP64 choice would decide
-    if (lane == 0) {
-      configs[edge] = -1;
-      if (c_valid) {
-        c_cfg[edge] = -1;
-        c_keep[edge] = 0;
-        c_q[edge] = -1.0;
-        c_valid[edge] = 1;
-      }
-    }
-    return;
-  }
-  int n = lsize[cand];
-  // each lane keeps the first of its triangulations with the largest value
-  // above 0; the group then takes the largest value, the lowest index on
-  // ties: the first triangulation attaining the maximum, as the sequential
-  // choice finds it
-  int choice_mesh = -1;
-  double choice_quality = -1.0;
-  if (n <= swap::kMaxLoop) {
-    choice_quality = 0.0;
+  bool rejected = false;
+  if (open) {
+    int ntris = tb->ntris[n], nedges = tb->nuedges[n];
     int nmeshes = tb->mesh_counts[n];
-    Real const* cmq = mq + LO(cand) * kMaxMeshes;
-    for (int mesh = lane; mesh < nmeshes; mesh += lanes) {
-      double q = cmq[mesh];
-      if (q > choice_quality) {
-        choice_mesh = mesh;
-        choice_quality = q;
+    int mesh_tris = tb->mesh_sizes[n], mesh_edges = tb->nedges[n];
+    LO const* lv = s_lv[g];
+    double* tq = s_tq[g];
+    double* el = s_el[g];
+    // the vertices of (triangle i / 2, side i % 2)
+    auto tet = [&](int i, LO* tv) {
+      int ut = i >> 1;
+      bool second = i & 1;
+      LO p = lv[tb->tris[n][ut][0]], q = lv[tb->tris[n][ut][1]], r = lv[tb->tris[n][ut][2]];
+      tv[0] = p;
+      tv[1] = second ? r : q;
+      tv[2] = second ? q : r;
+      tv[3] = second ? eev[0] : eev[1];
+    };
+    auto value = [&](int mesh, double lmax) {
+      double q = 1.0;
+      for (int mt = 0; mt < mesh_tris; ++mt)
+        q = math::min2(q, tq[tb->meshes[n][mesh * mesh_tris + mt]]);
+      for (int me = 0; me < mesh_edges; ++me)
+        if (el[tb->medges[n][mesh * mesh_edges + me]] > lmax) q = -1.0;
+      return q;
+    };
+    if constexpr (MIXED) {
+      bool unclear = false;
+      for (int i = lane; i < 2 * ntris; i += lanes) {
+        LO tv[4];
+        tet(i, tv);
+        float q = tet_quality32<M>(tv, a.coords, a.metric, &unclear);
+        q = q < 1.0f ? q : 1.0f;
+        float o = __shfl_xor(q, 1, 64);
+        if (!(i & 1)) tq[i >> 1] = double(o < q ? o : q);
       }
+      for (int i = lane; i < nedges; i += lanes)
+        el[i] = double(length_between32<3, M>(lv[tb->uedges[n][i][0]], lv[tb->uedges[n][i][1]],
+            a.coords, a.metric));
+      wave_lds_fence();
+      double best = -1.0;
+      double lmax = a.max_length * (1.0 + double(f32::kScreenBand));
+      for (int mesh = lane; mesh < nmeshes; mesh += lanes)
+        best = math::max2(best, value(mesh, lmax));
+      int unsure = unclear ? 1 : 0;
+      for (int d = lanes / 2; d > 0; d >>= 1) {
+        best = math::max2(best, __shfl_xor(best, d, 64));
+        unsure |= __shfl_xor(unsure, d, 64);
+      }
+      rejected = ntris != 0 && !unsure && old > 0.0 &&
+                 best < old * (1.0 - double(f32::kScreenBand));
+      wave_lds_fence();
     }
-  }
-  double old = 1.79769313486231570815e+308;
-  for (LO j = e2t_a2ab[edge] + lane; j < e2t_a2ab[edge + 1]; j += lanes)
-    old = math::min2(old, elem_quals[e2t_ab2b[j]]);
-  for (int d = lanes / 2; d > 0; d >>= 1) {
-    double oq = __shfl_xor(choice_quality, d, 64);
-    int om = __shfl_xor(choice_mesh, d, 64);
-    if (oq > choice_quality || (oq == choice_quality && om >= 0 &&
-                                   (choice_mesh < 0 || om < choice_mesh))) {
-      choice_quality = oq;
-      choice_mesh = om;
+    if (!rejected) {
+      for (int i = lane; i < 2 * ntris; i += lanes) {
+        LO tv[4];
+        tet(i, tv);
+        double q = math::min2(1.0, tet_quality<M>(tv, a.coords, a.metric));
+        double o = __shfl_xor(q, 1, 64);
+        if (!(i & 1)) tq[i >> 1] = math::min2(q, o);
+      }
+      for (int i = lane; i < nedges; i += lanes)
+        el[i] = length_between<3, M>(lv[tb->uedges[n][i][0]], lv[tb->uedges[n][i][1]], a.coords,
+            a.metric);
+      wave_lds_fence();
+      for (int mesh = lane; mesh < nmeshes; mesh += lanes) {
+        double q = value(mesh, a.max_length);
+        if (q > choice_quality) {
+          choice = mesh;
+          choice_quality = q;
+        }
+      }
+      // the largest value, the lowest index on ties
+      for (int d = lanes / 2; d > 0; d >>= 1) {
+        double oq = __shfl_xor(choice_quality, d, 64);
+        int om = __shfl_xor(choice, d, 64);
+        if (oq > choice_quality || (oq == choice_quality && om >= 0 &&
+                                       (choice < 0 || om < choice))) {
+          choice_quality = oq;
+          choice = om;
+        }
+      }
+    } else {
+      choice_quality = -1.0;
     }
-    old = math::min2(old, __shfl_xor(old, d, 64));
   }
   if (lane != 0) return;
-  configs[edge] = I8(choice_mesh);
+  a.configs[edge] = I8(choice);
   // a key needs a triangulation; with inverted elements the reference can
   // keep an edge without one and then index its tables out of bounds
-  bool kept = choice_mesh >= 0 && choice_quality > old;
+  bool kept = choice >= 0 && choice_quality > old;
   if (kept) {
-    keep[edge] = 1;
-    quals[edge] = choice_quality;
+    a.keep[edge] = 1;
+    a.quals[edge] = choice_quality;
   }
-  if (c_valid) {
-    c_cfg[edge] = I8(choice_mesh);
-    c_keep[edge] = I8(kept);
-    c_q[edge] = choice_quality;
-    c_valid[edge] = 1;
+  if (a.c_valid) {
+    a.c_cfg[edge] = I8(choice);
+    a.c_keep[edge] = I8(kept);
+    a.c_q[edge] = choice_quality;
+    a.c_valid[edge] = 1;
+  }
+}
+
+// indset::find over the candidates kept by the choice, through their rows
+// (see indset_first_edges and indset_edge for the rounds' rules): a thread or
+// a group of lanes per candidate instead of one per edge of the mesh
+template <bool FIRST>
+__global__ void swap3d_indset(LO nt, int lanes, EdgeRings r, Real const* q, I8 const* old_state,
+    I8* new_state, unsigned long long* dom, IndsetWords w) {
+  LO t = thread_index();
+  if (t >= nt) return;
+  LO cand = t / lanes;
+  int lane = t % lanes;
+  LO v = r.cands[cand];
+  I8 s = indset_state<FIRST>(old_state, v);
+  I8 res = s;
+  if (s == 2) {
+    LO const* row = r.rows + std::size_t(cand) * kRow;
+    unsigned long long mask = 0;
+    int undecided = 0;
+    bool out = false;
+    if (FIRST) {
+      Real qv = q[v];
+      int np = r.counts[v] * 6;
+      for (int p = lane; p < np; p += lanes) {
+        LO u = r.t2e[row[p / 6] / 6 * 6 + p % 6];
+        if (u == v || !old_state[u]) continue;
+        Real qu = q[u];
+        bool beaten = (qu != qv) ? (qu < qv) : (u < v);
+        if (beaten) continue;
+        undecided = 1;
+        mask |= 1ull << p;
+      }
+      for (int d = lanes / 2; d > 0; d >>= 1) {
+        mask |= __shfl_xor(mask, d, 64);
+        undecided |= __shfl_xor(undecided, d, 64);
+      }
+      if (lane == 0) dom[cand] = mask;
+    } else {
+      mask = dom[cand];
+      while (mask && !out) {
+        int p = __ffsll(static_cast<long long>(mask)) - 1;
+        mask &= mask - 1;
+        I8 su = old_state[r.t2e[row[p / 6] / 6 * 6 + p % 6]];
+        out = su == 1;
+        if (su == 2) undecided = 1;
+      }
+    }
+    res = out ? I8(0) : (undecided ? I8(2) : I8(1));
+  }
+  if (lane != 0) return;
+  new_state[v] = res;
+  tell_round(s, res, w);
+}
+
+// The rebuild plans of a swap from its keys' rows alone: a key edge and the
+// faces and tets around it are no longer the same, the lowest of each stands
+// for the key's products, and all else stays (one launch of fills).  Keys share
+// no element, so every entity is written for one key only.  Sweeps over every
+// edge, face and tet of the mesh (counts, key marks, same entities,
+// representatives) took 17 us where this takes 5 us.
+struct KeyPlan {
+  I8* same[3];    // edges, faces, tets
+  LO* counts[3];
+  I8* is_key;     // per candidate
+  LO* nprods[3];  // per candidate: product edges, faces, tets
+  LO* reps[2];    // per candidate: face, tet
+  I8* dirty;      // edges whose tets change (null: not wanted)
+};
+
+__global__ void swap3d_plan_keys(LO nt, EdgeRings r, I8 const* keys, LO const* t2f,
+    Tables const* tb, KeyPlan a) {
+  LO t = thread_index();
+  if (t >= nt) return;
+  LO cand = t / kRow;
+  int lane = t % kRow;
+  LO e = r.cands[cand];
+  if (!keys[e]) {
+    if (lane == 0) {
+      a.is_key[cand] = 0;
+      for (int d = 0; d < 3; ++d) a.nprods[d][cand] = 0;
+    }
+    return;
+  }
+  int n = r.counts[e];
+  int npt = tb->mesh_sizes[n], npe = tb->nedges[n];
+  LO tet = 0x7fffffff, f[2] = {0x7fffffff, 0x7fffffff};
+  if (lane < n) {
+    LO use = r.rows[std::size_t(cand) * kRow + lane];
+    tet = use / 6;
+    int opp = opposite_template(3, 1, int(use % 6));
+    // the two faces of the tet that hold the edge lie across from the ends of
+    // the opposite edge
+    for (int k = 0; k < 2; ++k)
+      f[k] = t2f[tet * 4 + opposite_template(3, 0, down_template(3, 1, opp, k))];
+    if (a.dirty)
+      for (int i = 0; i < 6; ++i) a.dirty[r.t2e[tet * 6 + i]] = 1;
+  }
+  LO trep = tet, frep = f[0] < f[1] ? f[0] : f[1];
+  for (int d = kRow / 2; d > 0; d >>= 1) {
+    LO o = __shfl_xor(trep, d, 64);
+    trep = o < trep ? o : trep;
+    o = __shfl_xor(frep, d, 64);
+    frep = o < frep ? o : frep;
+  }
+  LO nf = npt + 2 * npe;
+  if (lane < n) {
+    a.same[2][tet] = 0;
+    a.counts[2][tet] = tet == trep ? 2 * npt : 0;
+    for (int k = 0; k < 2; ++k) {
+      a.same[1][f[k]] = 0;
+      a.counts[1][f[k]] = f[k] == frep ? nf : 0;
+    }
+  }
+  if (lane == 0) {
+    a.same[0][e] = 0;
+    a.counts[0][e] = npe;
+    a.is_key[cand] = 1;
+    a.nprods[0][cand] = npe;
+    a.nprods[1][cand] = nf;
+    a.nprods[2][cand] = 2 * npt;
+    a.reps[0][cand] = frep;
+    a.reps[1][cand] = trep;
   }
 }
 
@@ -483,7 +555,7 @@ struct LocalSides {
 
 template <int HIGH>
 __device__ __forceinline__ void local_side(LO t, int lanes, LO const* keys2edges,
-    LO const* e2t_a2ab, LO const* e2t_ab2b, LocalSides const& a, int* error) {
+    EdgeRings const& r, LocalSides const& a, int* error) {
   LO u = t / lanes;
   int lane = t % lanes;
   constexpr int LOW = HIGH - 1;
@@ -503,8 +575,8 @@ __device__ __forceinline__ void local_side(LO t, int lanes, LO const* keys2edges
     LO q0 = a.k2p_low[key];
     LO nq = a.k2p_low[key + 1] - q0;
     LO e = keys2edges[key];
-    LO r0 = e2t_a2ab[e];
-    LO ncand = nq + (e2t_a2ab[e + 1] - r0) * nlpt;
+    LO const* row = r.rows + std::size_t(r.cand_of[e]) * kRow;
+    LO ncand = nq + r.counts[e] * nlpt;
     for (LO cnd = lane; cnd < ncand; cnd += lanes) {
       LO id;
       LO bv[3];
@@ -513,8 +585,8 @@ __device__ __forceinline__ void local_side(LO t, int lanes, LO const* keys2edges
 #pragma unroll
         for (int k = 0; k < nvl; ++k) bv[k] = a.pv_low[(q0 + cnd) * nvl + k];
       } else {
-        LO r = cnd - nq;
-        LO o = a.t2low[e2t_ab2b[r0 + r / nlpt] * nlpt + r % nlpt];
+        LO s = cnd - nq;
+        LO o = a.t2low[row[s / nlpt] / 6 * nlpt + s % nlpt];
         if (!a.low_same[o]) continue;
         id = a.low_offsets[o];
 #pragma unroll
@@ -551,120 +623,108 @@ __device__ __forceinline__ void local_side(LO t, int lanes, LO const* keys2edges
 }
 
 __global__ void __launch_bounds__(kBlock) swap3d_local_down(int lanes, unsigned face_blocks,
-    LO const* keys2edges, LO const* e2t_a2ab, LO const* e2t_ab2b, LocalSides faces,
-    LocalSides tets, int* error) {
+    LO const* keys2edges, EdgeRings r, LocalSides faces, LocalSides tets, int* error) {
   if (blockIdx.x < face_blocks)
-    local_side<2>(LO(blockIdx.x) * kBlock + LO(threadIdx.x), lanes, keys2edges, e2t_a2ab,
-        e2t_ab2b, faces, error);
+    local_side<2>(LO(blockIdx.x) * kBlock + LO(threadIdx.x), lanes, keys2edges, r, faces, error);
   else
-    local_side<3>(LO(blockIdx.x - face_blocks) * kBlock + LO(threadIdx.x), lanes, keys2edges,
-        e2t_a2ab, e2t_ab2b, tets, error);
+    local_side<3>(LO(blockIdx.x - face_blocks) * kBlock + LO(threadIdx.x), lanes, keys2edges, r,
+        tets, error);
 }
 
-// the edges of the tets the pass replaces: their tet rings change
-__global__ void swap3d_mark_dirty(LO ntets, I8 const* tet_same, LO const* t2e, I8* dirty) {
+// the interior edges (mark_by_class_dim) of the marked elements
+__global__ void mark_interior_edges(LO nelems, int nepe, LO const* elem2edges,
+    I8 const* elem_marks, int dim, I8 const* edim, I8* marks) {
   LO t = thread_index();
-  if (t >= ntets || tet_same[t]) return;
-  for (int i = 0; i < 6; ++i) dirty[t2e[t * 6 + i]] = 1;
-}
-
-// the interior edges among the marked ones (mark_by_class_dim), and the
-// swap choice arrays set to "none"
-__global__ void and_interior(LO ne, int dim, I8 const* edim, I8* marks, I8* configs, I8* keep,
-    Real* quals) {
-  LO e = thread_index();
-  if (e >= ne) return;
-  marks[e] = I8(marks[e] && (edim[e] == dim));
-  if (configs) configs[e] = -1;
-  keep[e] = 0;
-  quals[e] = -1.0;
-}
-
-// per edge, the edges, faces and tets a key edge's swap produces (0 for
-// other edges), so that one scan launch numbers the keys and their products
-__global__ void swap3d_counts(LO nedges, I8 const* keys, LO const* e2t_a2ab, Tables const* tb,
-    LO* ne, LO* nf, LO* nt) {
-  LO e = thread_index();
-  if (e >= nedges) return;
-  int npt = 0, npe = 0;
-  if (keys[e]) {
-    int ls = e2t_a2ab[e + 1] - e2t_a2ab[e];
-    npt = tb->mesh_sizes[ls];
-    npe = tb->nedges[ls];
+  if (t >= nelems || !elem_marks[t]) return;
+  for (int i = 0; i < nepe; ++i) {
+    LO e = elem2edges[t * nepe + i];
+    if (edim[e] == dim) marks[e] = 1;
   }
-  ne[e] = npe;
-  nf[e] = npt + 2 * npe;
-  nt[e] = 2 * npt;
 }
 
-// the key list, each key's product offsets and its representatives in the
-// rebuild of faces and tets, from the per-edge scans and sweeps
-__global__ void swap3d_key_offsets(LO nedges, I8 const* keys, LO const* key_off,
-    LO const* eoff, LO const* foff, LO const* toff, LO const* frep_of, LO const* trep_of,
-    LO* keys2edges, LO* k2e, LO* k2f, LO* k2t, LO* ereps, LO* freps, LO* treps) {
-  LO e = thread_index();
-  if (e >= nedges) return;
-  if (e == 0) {
-    LO nk = key_off[nedges];
-    k2e[nk] = eoff[nedges];
-    k2f[nk] = foff[nedges];
-    k2t[nk] = toff[nedges];
-  }
-  if (!keys[e]) return;
-  LO k = key_off[e];
-  keys2edges[k] = e;
-  k2e[k] = eoff[e];
-  k2f[k] = foff[e];
-  k2t[k] = toff[e];
-  ereps[k] = e;
-  freps[k] = frep_of[e];
-  treps[k] = trep_of[e];
-}
+// swap3d_topology (src/Omega_h_swap3d_topology.cpp:12-119): the key list, each
+// key's product offsets and representatives from the per-candidate scans, and
+// its new edges, faces and tets in template order; kRow threads per candidate
+// find a key's loop again and share its products
+struct KeyProducts {
+  I8 const* is_key;
+  LO const* key_off;
+  LO const* off[3];   // product offsets by candidate
+  LO const* reps[2];  // face and tet representatives by candidate
+  LO* keys2edges;
+  LO* k2p[3];
+  LO* key_reps[3];
+  LO* pv[3];
+  LO* fkey;
+  LO* tkey;
+};
 
-// swap3d_topology (src/Omega_h_swap3d_topology.cpp:12-119): each key's new
-// edges, faces and tets in template order, from the loop its candidate sweep
-// already found; kLanes threads per key share the products
-constexpr int kLanes = 8;
-
-__global__ void swap3d_products(LO nt, LO const* keys2edges, I8 const* configs,
-    LO const* cand_of_edge, LO const* lsize, LO const* leev, LO const* lverts, Tables const* tb,
-    LO const* k2e, LO const* k2f, LO const* k2t, LO* pe, LO* pf, LO* pt, LO* fkey, LO* tkey) {
+__global__ void swap3d_products(LO nt, LO ncands, EdgeRings r, LO const* ev2v, LO const* tv2v,
+    I8 const* configs, Tables const* tb, KeyProducts a) {
   LO t = thread_index();
   if (t >= nt) return;
-  LO k = t / kLanes;
-  int lane = t % kLanes;
-  LO edge = keys2edges[k];
+  LO cand = t / kRow;
+  int lane = t % kRow;
+  if (t == 0)
+    for (int d = 0; d < 3; ++d) a.k2p[d][a.key_off[ncands]] = a.off[d][ncands];
+  if (!a.is_key[cand]) return;
+  LO k = a.key_off[cand];
+  LO edge = r.cands[cand];
+  int n = r.counts[edge];
+  int base = int(threadIdx.x % 64) & ~(kRow - 1);
+  LO use = lane < n ? r.rows[std::size_t(cand) * kRow + lane] : 0;
+  bool ok;  // the choice has found the same ring
+  LO mine = ring_vertex(n, lane, base, use, r.t2e_codes, tv2v, &ok);
+  LO lv[kRow];
+#pragma unroll
+  for (int i = 0; i < kRow; ++i) lv[i] = __shfl(mine, base + i, 64);
+  auto vertex = [&](int i) {
+    LO v = lv[0];
+#pragma unroll
+    for (int j = 1; j < kRow; ++j) v = i == j ? lv[j] : v;
+    return v;
+  };
+  LO k2e = a.off[0][cand], k2f = a.off[1][cand], k2t = a.off[2][cand];
+  if (lane == 0) {
+    a.keys2edges[k] = edge;
+    a.k2p[0][k] = k2e;
+    a.k2p[1][k] = k2f;
+    a.k2p[2][k] = k2t;
+    a.key_reps[0][k] = edge;
+    a.key_reps[1][k] = a.reps[0][cand];
+    a.key_reps[2][k] = a.reps[1][cand];
+  }
   int config = configs[edge];
-  LO cand = cand_of_edge[edge];
-  int n = lsize[cand];
-  LO const* lv = lverts + cand * swap::kMaxLoop;
-  LO eev2v[2] = {leev[cand * 2], leev[cand * 2 + 1]};
+  LO eev2v[2] = {ev2v[edge * 2], ev2v[edge * 2 + 1]};
   int npt = tb->mesh_sizes[n], npe = tb->nedges[n];
-  for (int pe_i = lane; pe_i < npe; pe_i += kLanes) {
-    int ue = tb->medges[n][config * npe + pe_i];
-    LO a = lv[tb->uedges[n][ue][0]];
-    LO b = lv[tb->uedges[n][ue][1]];
-    LO pedge = k2e[k] + pe_i;
-    pe[pedge * 2] = a;
-    pe[pedge * 2 + 1] = b;
+  LO* pe = a.pv[0];
+  LO* pf = a.pv[1];
+  LO* pt = a.pv[2];
+  for (int i = lane; i < npe; i += kRow) {
+    int ue = tb->medges[n][config * npe + i];
+    LO va = vertex(tb->uedges[n][ue][0]);
+    LO vb = vertex(tb->uedges[n][ue][1]);
+    LO pedge = k2e + i;
+    pe[pedge * 2] = va;
+    pe[pedge * 2 + 1] = vb;
     for (int eev = 0; eev < 2; ++eev) {
-      LO ptri = k2f[k] + 2 * pe_i + eev;
-      pf[ptri * 3 + 0] = a;
-      pf[ptri * 3 + 1] = b;
+      LO ptri = k2f + 2 * i + eev;
+      pf[ptri * 3 + 0] = va;
+      pf[ptri * 3 + 1] = vb;
       pf[ptri * 3 + 2] = eev2v[eev];
-      fkey[ptri] = k;
+      a.fkey[ptri] = k;
     }
   }
-  for (int pt_i = lane; pt_i < npt; pt_i += kLanes) {
-    int ut = tb->meshes[n][config * npt + pt_i];
+  for (int i = lane; i < npt; i += kRow) {
+    int ut = tb->meshes[n][config * npt + i];
     LO tv[3];
-    for (int j = 0; j < 3; ++j) tv[j] = lv[tb->tris[n][ut][j]];
-    LO ptri = k2f[k] + 2 * npe + pt_i;
+    for (int j = 0; j < 3; ++j) tv[j] = vertex(tb->tris[n][ut][j]);
+    LO ptri = k2f + 2 * npe + i;
     for (int j = 0; j < 3; ++j) pf[ptri * 3 + j] = tv[j];
-    fkey[ptri] = k;
+    a.fkey[ptri] = k;
     for (int eev = 0; eev < 2; ++eev) {
-      LO ptet = k2t[k] + 2 * pt_i + eev;
-      tkey[ptet] = k;
+      LO ptet = k2t + 2 * i + eev;
+      a.tkey[ptet] = k;
       LO nt4[4] = {tv[0], tv[1], tv[2], eev2v[eev]};
       if (eev == 0) {
         LO tmp = nt4[1];
@@ -777,10 +837,10 @@ Tables const* device_tables(Ctx& c) {
       static_cast<DArray<unsigned char>*>(c.swap_tables.get())->data());
 }
 
-// `plans` (when given) are the rebuild plans of dimensions 1..dim, scanned
+// `plans` are the rebuild plans of dimensions 1..dim, scanned
 void swap_rebuild(Ctx& c, DMesh& m, LOs const& keys2edges, LOs const* k2p, LO const* nprods,
-    LOs const* pv, ModPlan* plans = nullptr, SwapCache* cache = nullptr,
-    Bytes const* dirty = nullptr, Adj const* key_tets = nullptr,
+    LOs const* pv, ModPlan const* plans, SwapCache* cache = nullptr,
+    Bytes const* dirty = nullptr, EdgeRings const* rings = nullptr,
     LOs const* prod_keys = nullptr) {
   int dim = m.dim;
   DMesh nw;
@@ -793,12 +853,6 @@ void swap_rebuild(Ctx& c, DMesh& m, LOs const& keys2edges, LOs const* k2p, LO co
   nw.itags = m.itags;
   nw.class_id[0] = m.class_id[0];
   nw.class_dim[0] = m.class_dim[0];
-  ModPlan own[3];
-  if (!plans) {
-    plans = own;
-    modify_plans(c, m, 1, 1, dim, keys2edges, k2p, plans);
-    modify_scan(c, plans, dim);
-  }
   ModOut mo[4];
   SwapCache next;
   CacheMove move{cache, &next, dirty};
@@ -810,10 +864,10 @@ void swap_rebuild(Ctx& c, DMesh& m, LOs const& keys2edges, LOs const* k2p, LO co
     prods[d].verts = pv[d];
     prods[d].src_dim = 1;  // products come from their key edge
   }
-  place_products(c, m, nw, 1, dim, 1, plans, keys2edges, prods, mo,
+  place_products(c, m, nw, 1, dim, 1, plans, keys2edges, prods, mo, nullptr,
       cache ? next.valid.data() : nullptr);
   if (cache) *cache = next;
-  if (key_tets && prod_keys) {
+  if (rings) {
     // in 3D the products' sides come from a search around each key
     LO most = nprods[2] * 3 > nprods[3] * 4 ? nprods[2] * 3 : nprods[3] * 4;
     int lanes = fit_lanes(most, c.tuning.side_lanes);
@@ -838,8 +892,7 @@ void swap_rebuild(Ctx& c, DMesh& m, LOs const& keys2edges, LOs const* k2p, LO co
     }
     if (blocks[0] + blocks[1]) {
       hipLaunchKernelGGL(swap3d_local_down, dim3(blocks[0] + blocks[1]), dim3(kBlock), 0,
-          c.stream, lanes, blocks[0], keys2edges.data(), key_tets->a2ab.data(),
-          key_tets->ab2b.data(), s[0], s[1], c.error_word());
+          c.stream, lanes, blocks[0], keys2edges.data(), *rings, s[0], s[1], c.error_word());
       OSH_HIP(hipGetLastError());
     }
   } else {
@@ -851,142 +904,139 @@ void swap_rebuild(Ctx& c, DMesh& m, LOs const& keys2edges, LOs const* k2p, LO co
   m = nw;
 }
 
-// sliver-layer elements' interior edges (src/Omega_h_swap.cpp:21-30); the
-// same launch sets the choice arrays
-Bytes swap_candidates(Ctx& c, DMesh& m, AdaptOptions const& o, Bytes* configs, Bytes& keep,
-    Reals& quals) {
-  int dim = m.dim;
-  LO ne = m.nents[1];
-  Bytes elems = mark_sliver_layers(c, m, o.min_quality_desired, o.nsliver_layers);
-  Bytes edges = mark_down(c, m, dim, 1, elems);
-  if (configs) *configs = Bytes(c, ne);
-  keep = Bytes(c, ne);
-  quals = Reals(c, ne);
-  OSH_LAUNCH(and_interior, ne, c, dim, m.class_dim[1].data(), edges.data(),
-      configs ? configs->data() : (I8*)nullptr, keep.data(), quals.data());
-  return edges;
+// what a 3D pass knows about its candidates' rings, with the storage behind it
+struct Rings {
+  LOs cands, cand_of, rows;
+  EdgeRings r{};
+};
+
+// the rings of the marked edges; counts: zeros per edge
+void build_rings(Ctx& c, DMesh& m, Bytes const& marks, LOs const& counts, Rings& out) {
+  out.cands = collect_marked(c, marks, &out.cand_of);
+  LO ncands = out.cands.size();
+  if (ncands == 0) return;
+  Bytes const* codes;
+  LOs const& t2e = ask_down(c, m, 3, 1, &codes);
+  out.rows = LOs(c, ncands * kRow);
+  OSH_LAUNCH(swap3d_rows, m.nents[3] * 6, c, t2e.data(), marks.data(), out.cand_of.data(),
+      counts.data(), out.rows.data());
+  out.r = EdgeRings{out.cands.data(), out.cand_of.data(), counts.data(), out.rows.data(),
+      t2e.data(), codes->data()};
 }
 
 // swap3d_qualities (src/Omega_h_swap3d_qualities.cpp:11-75) with the choice
-// of each candidate's triangulation (src/Omega_h_swap3d_choice.hpp): for the
-// candidate edges `cands`, whose edge -> tet rows e2t holds, configs[e]
-// receives the chosen triangulation (-1 for none) and, when it improves on
-// the elements around the edge, keep[e] = 1 and quals[e] its quality
-// (entries of other edges are left as they are).  The candidates' loops stay
-// in `loops` for the products.
-struct SwapLoops {
-  LOs lsize, leev, lverts;
-};
-
-void swap3d_evaluate(Ctx& c, DMesh& m, AdaptOptions const& o, LOs const& cands, Adj const& e2t,
-    SwapCache* cache, Bytes& configs, Reals& quals, Bytes& keep, SwapLoops& loops) {
-  LO ne = m.nents[1];
-  int md = (m.metric_ncomps == 1) ? 1 : 3;
-  Tables const* tb = device_tables(c);
-  LOs const& tv2v = verts_of(c, m, 3);
-  Reals const& eq = ask_qualities(c, m);
-  LO ncands = cands.size();
-  int choose_lanes = fit_lanes(ncands, c.tuning.choose_lanes);
-  if (cache && !cache->valid.exists()) {
-    cache->valid = fill_i8(c, ne, 0);
-    cache->cfg = Bytes(c, ne);
-    cache->keep = Bytes(c, ne);
-    cache->q = Reals(c, ne);
-  }
+// of each candidate's triangulation (src/Omega_h_swap3d_choice.hpp):
+// configs[e] receives the chosen triangulation (-1 for none) and, when it
+// improves on the elements around the edge, keep[e] = 1 and quals[e] its
+// quality (entries of other edges are left as they are)
+void swap3d_evaluate(Ctx& c, DMesh& m, AdaptOptions const& o, Rings const& rings,
+    SwapCache* cache, Bytes& configs, Reals& quals, Bytes& keep) {
   Range quality_range(c, "swap3d_qualities");
-  loops.lsize = LOs(c, ncands);
-  loops.leev = LOs(c, ncands * 2);
-  loops.lverts = LOs(c, ncands * swap::kMaxLoop);
-  LOs const& lsize = loops.lsize;
-  LOs const& leev = loops.leev;
-  LOs const& lverts = loops.lverts;
-  LOs ntris(c, ncands), nedges(c, ncands);
-  OSH_LAUNCH(swap3d_loops, ncands * kLoopLanes, c, cands.data(), e2t.a2ab.data(), e2t.ab2b.data(),
-      e2t.codes.data(), m.down[1].data(), tv2v.data(), tb,
-      cache ? cache->valid.data() : (I8 const*)nullptr, lsize.data(), leev.data(),
-      lverts.data(), ntris.data(), nedges.data(), c.error_word());
-  // the unique triangles and edges of all loops at fixed strides per
-  // candidate, so that neither a scan nor a sync sizes them
-  LO ntp = ncands * swap::kMaxUniqueTris, nep = ncands * swap::kMaxUniqueEdges;
-  Reals tq(c, ntp), el(c, nep);
-  // mixed precision: an FP32 screen of every candidate first, then the FP64
-  // sweeps, choice included, only for the candidates it left open
+  LO ncands = rings.cands.size();
+  int md = (m.metric_ncomps == 1) ? 1 : 3;
+  // one evaluation keeps up to 70 lanes busy (a loop of seven); four lanes
+  // to each one that the choice alone is given, 32 by default
+  int lanes = 4 * c.tuning.choose_lanes;
+  lanes = lanes < kMinEvalLanes ? kMinEvalLanes : (lanes > 64 ? 64 : lanes);
+  lanes = fit_lanes(ncands, lanes);
+  OSH_CHECK(lanes >= kMinEvalLanes, "swap: too many candidates");
+  EvalArgs a{rings.r, ncands, m.down[1].data(), verts_of(c, m, 3).data(), m.coords.data(),
+      m.metric.data(), ask_qualities(c, m).data(), o.max_length_allowed, device_tables(c),
+      configs.data(), quals.data(), keep.data(), cache ? cache->valid.data() : nullptr,
+      cache ? cache->cfg.data() : nullptr, cache ? cache->keep.data() : nullptr,
+      cache ? cache->q.data() : nullptr, c.error_word()};
+  int lshift = lanes_shift(lanes);
+#define OSH_SWE(M, X) OSH_LAUNCH((swap3d_evaluate_kernel<M, X>), ncands * lanes, c, lshift, a)
   bool mixed = o.precision == 1;
-  Bytes need, unsure;
-  if (mixed) {
-    need = Bytes(c, ncands);
-    unsure = fill_i8(c, ncands, 0);
-  }
-  I8 const* needp = mixed ? need.data() : nullptr;
-  LoopMeasures lm{ntp, ntris.data(), nedges.data(), lsize.data(), leev.data(), lverts.data(),
-      m.coords.data(), m.metric.data(), tb, needp, mixed ? unsure.data() : (I8*)nullptr,
-      tq.data(), el.data()};
-#define OSH_SWQ(M, F32) OSH_LAUNCH((swap3d_loop_measures<M, F32>), ntp + nep, c, lm)
-  if (mixed) {
-    if (md == 3) {
-      OSH_SWQ(3, true);
-    } else {
-      OSH_SWQ(1, true);
-    }
-    OSH_LAUNCH(swap3d_screen, ncands * choose_lanes, c, choose_lanes, cands.data(),
-        lsize.data(),
-        ntris.data(), tq.data(), el.data(), o.max_length_allowed, tb, e2t.a2ab.data(),
-        e2t.ab2b.data(), eq.data(), unsure.data(), need.data());
-  }
-  if (md == 3) {
-    OSH_SWQ(3, false);
-  } else {
-    OSH_SWQ(1, false);
-  }
-#undef OSH_SWQ
-  Reals mq(c, ncands * kMaxMeshes);
-  OSH_LAUNCH(swap3d_mesh_quals, ncands * kMaxMeshes, c, lsize.data(), ntris.data(),
-      tq.data(), el.data(), o.max_length_allowed, tb, needp, mq.data());
-  OSH_LAUNCH(swap3d_choose, ncands * choose_lanes, c, choose_lanes, cands.data(),
-      lsize.data(), mq.data(),
-      e2t.a2ab.data(),
-      e2t.ab2b.data(), eq.data(), tb, needp, configs.data(), quals.data(), keep.data(),
-      cache ? cache->valid.data() : (I8*)nullptr, cache ? cache->cfg.data() : (I8*)nullptr,
-      cache ? cache->keep.data() : (I8*)nullptr, cache ? cache->q.data() : (Real*)nullptr);
+  if (md == 3 && mixed)
+    OSH_SWE(3, true);
+  else if (md == 3)
+    OSH_SWE(3, false);
+  else if (mixed)
+    OSH_SWE(1, true);
+  else
+    OSH_SWE(1, false);
+#undef OSH_SWE
 }
 
 bool swap_edges_3d(Ctx& c, DMesh& m, AdaptOptions const& o, SwapCache* cache) {
   ask_lengths(c, m);
-  Bytes configs, keep;
-  Reals quals;
-  Bytes cand = swap_candidates(c, m, o, &configs, keep, quals);
-  // every edge -> tet row this pass reads is a candidate's
-  LOs cands, cand_of_edge;
-  Adj e2t = marked_up(c, m, 1, 3, cand, &cands, true, &cand_of_edge);
-  if (cands.size() == 0) return false;
-  LO ne = m.nents[1];
-  Tables const* tb = device_tables(c);
-  SwapLoops loops;
-  swap3d_evaluate(c, m, o, cands, e2t, cache, configs, quals, keep, loops);
-  LOs const& lsize = loops.lsize;
-  LOs const& leev = loops.leev;
-  LOs const& lverts = loops.lverts;
-  bool any;
-  Bytes keys = find_indset(c, m, 1, quals, keep, &any, &e2t);
+  LO ne = m.nents[1], nf = m.nents[2], nt = m.nents[3];
+  Bytes elems = mark_sliver_layers(c, m, o.min_quality_desired, o.nsliver_layers);
+  // every array of the pass that starts out constant, in one launch
+  Fills fills(c);
+  Bytes marks = fills.bytes(ne, 0);
+  LOs ring_counts = fills.ints(ne, 0);
+  Bytes keep = fills.bytes(ne, 0);
+  Bytes state[2] = {fills.bytes(ne, 0), fills.bytes(ne, 0)};
+  Bytes dirty;
+  if (cache) dirty = fills.bytes(ne, 0);
+  ModPlan plans[3];
+  LO nents[3] = {ne, nf, nt};
+  for (int d = 0; d < 3; ++d) {
+    plans[d].ent_dim = d + 1;
+    plans[d].key_dim = 1;
+    plans[d].nold = nents[d];
+    plans[d].same = fills.bytes(nents[d], 1);
+    plans[d].counts = fills.ints(nents[d], 1);
+  }
+  if (cache && !cache->valid.exists()) {
+    cache->valid = fills.bytes(ne, 0);
+    cache->cfg = Bytes(c, ne);
+    cache->keep = Bytes(c, ne);
+    cache->q = Reals(c, ne);
+  }
+  fills.run();
+  LOs const& t2e = ask_down(c, m, 3, 1, nullptr);
+  OSH_LAUNCH(mark_interior_edges, nt, c, 6, t2e.data(), elems.data(), 3,
+      m.class_dim[1].data(), marks.data());
+  Rings rings;
+  build_rings(c, m, marks, ring_counts, rings);
+  LO ncands = rings.cands.size();
+  if (ncands == 0) return false;
+  Bytes configs(c, ne);
+  Reals quals(c, ne);
+  swap3d_evaluate(c, m, o, rings, cache, configs, quals, keep);
+  bool any = false;
+  Bytes keys;
+  {
+    Range indset_range(c, "find_indset");
+    DArray<unsigned long long> dom(c, ncands);
+    int first_lanes = fit_lanes(ncands, c.tuning.first_lanes);
+    keys = indset_rounds(c, ne, keep, state[0], state[1], &any,
+        [&](bool first, I8 const* in, I8* out, IndsetWords w) {
+          if (first)
+            OSH_LAUNCH(swap3d_indset<true>, ncands * first_lanes, c, first_lanes, rings.r,
+                quals.data(), in, out, dom.data(), w);
+          else
+            OSH_LAUNCH(swap3d_indset<false>, ncands, c, 1, rings.r, quals.data(), in, out,
+                dom.data(), w);
+        });
+  }
   if (!any) return false;
   Range modify_range(c, "modify_ents");
-  // per-edge product counts and the rebuild plans from the key mask, then
-  // one scan launch and one sync for the keys, their products and the new
-  // numbering of edges, faces and tets
-  LOs counts[4], offs[4], rep_of[4];
+  // the plans from the keys, then one scan launch and one wait for the keys,
+  // their products and the new numbering of edges, faces and tets
+  Tables const* tb = device_tables(c);
+  Bytes is_key(c, ncands);
+  LOs np[3], off[3], reps[2] = {LOs(c, ncands), LOs(c, ncands)};
+  LOs key_off(c, ncands + 1);
   ScanJob jobs[kMaxScanJobs];
-  offs[0] = LOs(c, ne + 1);
-  jobs[0] = {keys.data(), kScanNonzero, ne, offs[0].data(), slot_ptr<LO>(c, 0)};
-  for (int d = 1; d <= 3; ++d) {
-    counts[d] = LOs(c, ne);
-    offs[d] = LOs(c, ne + 1);
-    jobs[d] = {counts[d].data(), kScanLO, ne, offs[d].data(), slot_ptr<LO>(c, d)};
+  jobs[0] = {is_key.data(), kScanNonzero, ncands, key_off.data(), slot_ptr<LO>(c, 0)};
+  KeyPlan kp{};
+  for (int d = 0; d < 3; ++d) {
+    np[d] = LOs(c, ncands);
+    off[d] = LOs(c, ncands + 1);
+    jobs[d + 1] = {np[d].data(), kScanLO, ncands, off[d].data(), slot_ptr<LO>(c, d + 1)};
+    kp.same[d] = plans[d].same.data();
+    kp.counts[d] = plans[d].counts.data();
+    kp.nprods[d] = np[d].data();
   }
-  OSH_LAUNCH(swap3d_counts, ne, c, keys.data(), e2t.a2ab.data(), tb, counts[1].data(),
-      counts[2].data(), counts[3].data());
-  ModPlan plans[3];
-  LO const* pc[4] = {nullptr, counts[1].data(), counts[2].data(), counts[3].data()};
-  modify_plans_masked(c, m, 1, 3, keys, pc, plans, rep_of);
+  kp.is_key = is_key.data();
+  kp.reps[0] = reps[0].data();
+  kp.reps[1] = reps[1].data();
+  kp.dirty = cache ? dirty.data() : nullptr;
+  OSH_LAUNCH(swap3d_plan_keys, ncands * kRow, c, rings.r, keys.data(), m.down[3].data(), tb, kp);
   int njobs = 4 + modify_scan_jobs(c, plans, 3, jobs + 4, 4);
   offset_scans(c, jobs, njobs);
   c.wait();
@@ -996,40 +1046,46 @@ bool swap_edges_3d(Ctx& c, DMesh& m, AdaptOptions const& o, SwapCache* cache) {
   LOs keys2edges(c, nkeys);
   LOs k2p[4], pv[4];
   LO nprods[4] = {0, 0, 0, 0};
+  KeyProducts pr{};
+  pr.is_key = is_key.data();
+  pr.key_off = key_off.data();
+  pr.reps[0] = reps[0].data();
+  pr.reps[1] = reps[1].data();
+  pr.keys2edges = keys2edges.data();
   for (int d = 1; d <= 3; ++d) {
     nprods[d] = read_slot<LO>(c, d);
     pv[d] = LOs(c, nprods[d] * (d + 1));
     k2p[d] = LOs(c, nkeys + 1);
     plans[d - 1].reps = LOs(c, nkeys);
+    pr.off[d - 1] = off[d - 1].data();
+    pr.k2p[d - 1] = k2p[d].data();
+    pr.key_reps[d - 1] = plans[d - 1].reps.data();
+    pr.pv[d - 1] = pv[d].data();
   }
-  OSH_LAUNCH(swap3d_key_offsets, ne, c, keys.data(), offs[0].data(), offs[1].data(),
-      offs[2].data(), offs[3].data(), rep_of[2].data(), rep_of[3].data(), keys2edges.data(),
-      k2p[1].data(), k2p[2].data(), k2p[3].data(), plans[0].reps.data(), plans[1].reps.data(),
-      plans[2].reps.data());
-  note_changed_parts(c, m, 1, keys2edges);
   LOs prod_keys[4];  // the key of each product face and tet
   prod_keys[2] = LOs(c, nprods[2]);
   prod_keys[3] = LOs(c, nprods[3]);
-  OSH_LAUNCH(swap3d_products, nkeys * kLanes, c, keys2edges.data(), configs.data(),
-      cand_of_edge.data(), lsize.data(), leev.data(), lverts.data(), tb, k2p[1].data(),
-      k2p[2].data(), k2p[3].data(), pv[1].data(), pv[2].data(), pv[3].data(),
-      prod_keys[2].data(), prod_keys[3].data());
-  Bytes dirty;
-  if (cache) {
-    dirty = fill_i8(c, ne, 0);
-    OSH_LAUNCH(swap3d_mark_dirty, m.nents[3], c, plans[2].same.data(),
-        ask_down(c, m, 3, 1, nullptr).data(), dirty.data());
-  }
-  swap_rebuild(c, m, keys2edges, k2p, nprods, pv, plans, cache, cache ? &dirty : nullptr, &e2t,
-      prod_keys);
+  pr.fkey = prod_keys[2].data();
+  pr.tkey = prod_keys[3].data();
+  OSH_LAUNCH(swap3d_products, ncands * kRow, c, ncands, rings.r, m.down[1].data(),
+      verts_of(c, m, 3).data(), configs.data(), tb, pr);
+  note_changed_parts(c, m, 1, keys2edges);
+  swap_rebuild(c, m, keys2edges, k2p, nprods, pv, plans, cache, cache ? &dirty : nullptr,
+      &rings.r, prod_keys);
   return true;
 }
 
 bool swap_edges_2d(Ctx& c, DMesh& m, AdaptOptions const& o) {
   ask_lengths(c, m);
-  Bytes keep;
-  Reals quals;
-  Bytes cand = swap_candidates(c, m, o, nullptr, keep, quals);
+  LO ne = m.nents[1];
+  Bytes elems = mark_sliver_layers(c, m, o.min_quality_desired, o.nsliver_layers);
+  Fills fills(c);
+  Bytes cand = fills.bytes(ne, 0);
+  Bytes keep = fills.bytes(ne, 0);
+  fills.run();
+  Reals quals(c, ne);  // read where an edge is kept
+  OSH_LAUNCH(mark_interior_edges, m.nents[2], c, 3, m.down[2].data(), elems.data(), 2,
+      m.class_dim[1].data(), cand.data());
   LOs cands = collect_marked(c, cand);
   if (cands.size() == 0) return false;
   int md = (m.metric_ncomps == 1) ? 1 : 2;
@@ -1050,19 +1106,19 @@ bool swap_edges_2d(Ctx& c, DMesh& m, AdaptOptions const& o) {
   Bytes keys = find_indset(c, m, 1, quals, keep, &any);
   if (!any) return false;
   Range modify_range(c, "modify_ents");
-  LOs keys2edges = collect_marked(c, keys);
-  LO nkeys = keys2edges.size();
-  note_changed_parts(c, m, 1, keys2edges);
-  if (o.verbosity >= 2) std::printf("swapping %d 2D edges\n", int(nkeys));
-  LOs k2p[4], pv[4];
-  k2p[1] = iota(c, nkeys + 1);
-  k2p[2] = iota(c, nkeys + 1, 0, 2);
-  LO nprods[3] = {0, nkeys, 2 * nkeys};
-  pv[1] = LOs(c, nkeys * 2);
-  pv[2] = LOs(c, nkeys * 6);
-  OSH_LAUNCH(swap2d_products, nkeys, c, keys2edges.data(), e2t.a2ab.data(), e2t.ab2b.data(),
-      e2t.codes.data(), m.down[1].data(), tv2v.data(), pv[1].data(), pv[2].data());
-  swap_rebuild(c, m, keys2edges, k2p, nprods, pv);
+  KeyedMods km;
+  km.fixed_prods[1] = 1;
+  km.fixed_prods[2] = 2;
+  plan_keys(c, m, 1, 1, 2, keys, km);
+  note_changed_parts(c, m, 1, km.keys2kds);
+  if (o.verbosity >= 2) std::printf("swapping %d 2D edges\n", int(km.nkeys));
+  LOs pv[4];
+  pv[1] = LOs(c, km.nkeys * 2);
+  pv[2] = LOs(c, km.nkeys * 6);
+  OSH_LAUNCH(swap2d_products, km.nkeys, c, km.keys2kds.data(), e2t.a2ab.data(),
+      e2t.ab2b.data(), e2t.codes.data(), m.down[1].data(), tv2v.data(), pv[1].data(),
+      pv[2].data());
+  swap_rebuild(c, m, km.keys2kds, km.k2p, km.nprods, pv, km.plans);
   return true;
 }
 
@@ -1096,17 +1152,18 @@ void swap3d_choices(Ctx& c, DMesh& m, AdaptOptions const& o, LOs const& edges,
   OSH_CHECK(m.dim == 3, "swap3d choices need a 3D mesh");
   LO ne = m.nents[1];
   LO n = edges.size();
-  Bytes marks = fill_i8(c, ne, 0);
+  Fills fills(c);
+  Bytes marks = fills.bytes(ne, 0);
+  LOs counts = fills.ints(ne, 0);
+  Bytes configs = fills.bytes(ne, -1);
+  Bytes keep = fills.bytes(ne, 0);
+  fills.run();
   OSH_LAUNCH(mark_listed, n, c, edges.data(), marks.data());
-  LOs cands, cand_of_edge;
-  Adj e2t = marked_up(c, m, 1, 3, marks, &cands, true, &cand_of_edge);
-  Bytes configs = fill_i8(c, ne, -1);
-  Bytes keep = fill_i8(c, ne, 0);
-  Reals quals = fill_real(c, ne, -1.0);
-  if (cands.size() > 0) {
-    SwapLoops loops;
-    swap3d_evaluate(c, m, o, cands, e2t, nullptr, configs, quals, keep, loops);
-  }
+  Rings rings;
+  build_rings(c, m, marks, counts, rings);
+  Reals quals(c, ne);  // read where an edge is kept
+  if (rings.cands.size() > 0)
+    swap3d_evaluate(c, m, o, rings, nullptr, configs, quals, keep);
   configs_out = LOs(c, n);
   quals_out = Reals(c, n);
   OSH_LAUNCH(gather_choices, n, c, edges.data(), configs.data(), quals.data(), keep.data(),
