@@ -94,6 +94,14 @@ __device__ __forceinline__ void check_exposure(LO c, CellSweep const& a, int w,
     LO const* ev2v, I8 const* codes, I8* veto) {
   if (c >= a.ncells[w]) return;
   constexpr int nepc = (CD == 3) ? 6 : 3;
+  // a cell whose sides are all classified like itself vetoes nothing: most
+  // cells stop here, before they look at their edges
+  I8 own = a.cdim[w][c];
+  unsigned differ = 0u;
+#pragma unroll
+  for (int k = 0; k <= CD; ++k)
+    if (a.sdim[w][a.cs2s[w][std::size_t(c) * (CD + 1) + k]] != own) differ |= 1u << k;
+  if (differ == 0u) return;
   LO const* cv = a.cv2v[w] + std::size_t(c) * (CD + 1);
   for (int j = 0; j < nepc; ++j) {
     LO e = a.c2e[w][std::size_t(c) * nepc + j];
@@ -102,9 +110,7 @@ __device__ __forceinline__ void check_exposure(LO c, CellSweep const& a, int w,
     for (int col = 0; col < 2; ++col) {
       if (!collapses(code, col)) continue;
       int ccv_onto = local_vertex<CD>(cv, ev2v[e * 2 + (1 - col)]);
-      int ccs_opp = opposite_template(CD, 0, ccv_onto);
-      if (a.sdim[w][a.cs2s[w][std::size_t(c) * (CD + 1) + ccs_opp]] != a.cdim[w][c])
-        veto[e * 2 + col] = 1;
+      if ((differ >> opposite_template(CD, 0, ccv_onto)) & 1u) veto[e * 2 + col] = 1;
     }
   }
 }
@@ -239,7 +245,7 @@ __global__ void vert_dets(LO nv, Real const* metric, Real* dets) {
 // Bound by FP64 issue (166 operations a quality and its correctly rounded
 // divisions), so work is left out where it decides nothing: the determinants
 // come from vert_dets, a lane reads only the metric it uses, and a side stops
-// at the first cell below qmin unless it has to know the old minimum too.
+// at the first cell below qmin.
 //
 // MIXED: FP32 estimates first; a side is rejected (quality -1) when their
 // minimum is below qmin by more than the band and every element's
@@ -333,7 +339,7 @@ __global__ void __launch_bounds__(kBlock) coarsen_quality_lanes(LO nt, int lshif
         minq = math::min2(minq, element_quality<D, M>(pp, ms, dets));
       }
     }
-    if (FILTER && !a.old_quals && s.any(minq < a.qmin)) break;
+    if (FILTER && s.any(minq < a.qmin)) break;
   }
   for (int d = lanes / 2; d > 0; d >>= 1) {
     minq = math::min2(minq, __shfl_xor(minq, d, 64));

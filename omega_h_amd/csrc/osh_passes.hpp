@@ -185,8 +185,11 @@ void swap3d_choices(Ctx& c, DMesh& m, AdaptOptions const& o, LOs const& edges,
     LOs& configs_out, Reals& quals_out);
 
 // known-answer hooks used by the tests
-Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands,
-    Reals* midpoint_metrics = nullptr);
+Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands);
+// the same over an edge -> element adjacency with at least the candidates'
+// rows, also handing over the midpoints' metrics
+Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands, Adj const& e2c,
+    Reals* midpoint_metrics);
 // coarsen_qualities (src/Omega_h_coarsen_qualities.cpp:65-88) on device
 // arrays, stream-ordered: out[2 i + col] is the quality after collapsing
 // candidate i's edge in direction col (-1 where cand_codes[i] does not

@@ -262,7 +262,12 @@ __global__ void midpoint_coords(LO nkeys, int dim, LO const* keys2edges, LO cons
 
 }  // namespace
 
-Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands, Reals* midpoint_metrics) {
+Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands) {
+  return refine_qualities(c, m, cands, ask_up(c, m, 1, m.dim), nullptr);
+}
+
+Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands, Adj const& e2c,
+    Reals* midpoint_metrics) {
   Range range(c, "refine_qualities");
   LO n = cands.size();
   int dim = m.dim;
@@ -273,7 +278,6 @@ Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands, Reals* midpoint_metri
   mident_metrics(c, m, n, cands.data(), mm.data());
   Reals out(c, n);
   LOs const& cv2v = verts_of(c, m, dim);
-  Adj const& e2c = ask_up(c, m, 1, dim);
   // lanes share a candidate's children, as the coarsen sweeps share a side's
   int lanes = fit_lanes(n, c.tuning.coarsen_lanes);
   int lshift = lanes_shift(lanes);
@@ -303,14 +307,21 @@ bool refine_by_size(Ctx& c, DMesh& m, AdaptOptions const& o) {
   LOs cand_of_edge;
   LOs cands = collect_marked(c, cand, &cand_of_edge);
   if (cands.size() == 0) return false;
+  // the candidates' faces and elements; an attempt with a few long edges left
+  // (most of the 64^3 workload's) would otherwise invert the whole mesh
+  Adj up[2];
+  int const highs[2] = {2, 3};
+  bool const sorted[2] = {true, true};
+  marked_ups(c, m, 1, cand, dim - 1, highs, sorted, up);
+  Adj const& e2c = up[dim - 2];
   Reals cand_metrics;
-  Reals quals = refine_qualities(c, m, cands, &cand_metrics);
+  Reals quals = refine_qualities(c, m, cands, e2c, &cand_metrics);
   Bytes initial = fill_i8(c, ne, 0);
   Reals edge_quals(c, ne);  // read where an edge is a candidate
   OSH_LAUNCH(seed_keys, cands.size(), c, cands.data(), quals.data(), o.min_quality_allowed,
       initial.data(), edge_quals.data());
   bool any;
-  Bytes keys = find_indset(c, m, 1, edge_quals, initial, &any);
+  Bytes keys = find_indset(c, m, 1, edge_quals, initial, &any, &e2c);
   if (!any) return false;
   Range modify_range(c, "modify_ents");
   int nc = m.metric_ncomps;
@@ -322,14 +333,14 @@ bool refine_by_size(Ctx& c, DMesh& m, AdaptOptions const& o) {
   km.fixed_prods[0] = 1;
   for (int d = 1; d <= dim; ++d) {
     if (d > 1) {
-      Adj const& pr = ask_up(c, m, 1, d);
+      Adj const& pr = up[d - 2];
       rows.pairs_a2ab[d - 1] = pr.a2ab.data();
       rows.pairs_ab2b[d - 1] = pr.ab2b.data();
       rows.pairs_codes[d - 1] = pr.codes.data();
       rows.pair_verts[d - 1] = verts_of(c, m, d).data();
     }
     if (d < dim) {
-      Adj const& ct = ask_up(c, m, 1, d + 1);
+      Adj const& ct = up[d - 1];
       rows.cuts_a2ab[d - 1] = ct.a2ab.data();
       rows.cuts_ab2b[d - 1] = ct.ab2b.data();
       rows.cuts_codes[d - 1] = ct.codes.data();
