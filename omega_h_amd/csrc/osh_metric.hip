@@ -14,6 +14,7 @@
 #include <cmath>
 #include <cstdio>
 
+#include "osh_indset.hpp"
 #include "osh_metric.hpp"
 #include "osh_passes.hpp"
 
@@ -21,9 +22,34 @@ namespace osh {
 
 namespace {
 
+// are_close (src/Omega_h_scalar.hpp:266-277) of two values, negated
+__device__ __forceinline__ bool not_close(double a, double b, double tol) {
+  double am = math::fabs_(a), bm = math::fabs_(b);
+  double rd = (am <= kMetricEpsilon && bm <= kMetricEpsilon)
+                  ? 0.0
+                  : math::fabs_(b - a) / math::max2(am, bm);
+  return !(rd <= tol);
+}
+
+// vertex u's metric as its neighbour sees it at distance vec
+template <int S, int M>
+__device__ __forceinline__ Mat graded_metric(Real const* in, LO u, double const* vec,
+    double max_rate) {
+  constexpr int nc = (M * (M + 1)) / 2;
+  Mat am = get_symm<M>(in + std::size_t(u) * nc);
+  double dist = math::sqrt_(metric_product<S, M>(am, vec));
+  double h = 1.0 + dist * max_rate;
+  double factor = 1.0 / (h * h);
+  for (int c = 0; c < M; ++c)
+    for (int r = 0; r < M; ++r) am.m[c][r] = am.m[c][r] * factor;
+  return am;
+}
+
+// one sweep; `word` receives the tag when some value moved by more than tol
 template <int S, int M>
 __global__ void limit_gradation_kernel(LO nv, LO const* a2ab, LO const* ab2b,
-    Real const* coords, Real const* in, Real max_rate, Real* out, int* error) {
+    Real const* coords, Real const* in, Real max_rate, Real tol, Real* out, unsigned* word,
+    unsigned tag, int* error) {
   LO v = xcd_thread_index();
   if (v >= nv) return;
   int bad = 0;
@@ -33,28 +59,19 @@ __global__ void limit_gradation_kernel(LO nv, LO const* a2ab, LO const* ab2b,
   for (int i = 0; i < S; ++i) x[i] = coords[std::size_t(v) * S + i];
   for (LO j = a2ab[v]; j < a2ab[v + 1]; ++j) {
     LO av = ab2b[j];
-    Mat am = get_symm<M>(in + std::size_t(av) * nc);
     double vec[3] = {0.0, 0.0, 0.0};
     for (int i = 0; i < S; ++i) vec[i] = coords[std::size_t(av) * S + i] - x[i];
-    double dist = math::sqrt_(metric_product<S, M>(am, vec));
-    double h = 1.0 + dist * max_rate;
-    double factor = 1.0 / (h * h);
-    for (int c = 0; c < M; ++c)
-      for (int r = 0; r < M; ++r) am.m[c][r] = am.m[c][r] * factor;
-    m = intersect_metrics<M>(m, am, &bad);
+    m = intersect_metrics<M>(m, graded_metric<S, M>(in, av, vec, max_rate), &bad);
   }
-  set_symm<M>(m, out + std::size_t(v) * nc);
+  double r[nc];
+  set_symm<M>(m, r);
+  bool moved = false;
+  for (int k = 0; k < nc; ++k) {
+    out[std::size_t(v) * nc + k] = r[k];
+    moved = moved || not_close(in[std::size_t(v) * nc + k], r[k], tol);
+  }
+  tell(moved, word, tag);
   if (bad) *error = kDegenerateEigen;
-}
-
-__global__ void not_close_kernel(LO n, Real const* a, Real const* b, Real tol, Real floor,
-    I8* out) {
-  LO i = thread_index();
-  if (i >= n) return;
-  double am = math::fabs_(a[i]), bm = math::fabs_(b[i]);
-  double rd = (am <= floor && bm <= floor) ? 0.0
-                                           : math::fabs_(b[i] - a[i]) / math::max2(am, bm);
-  out[i] = !(rd <= tol);
 }
 
 template <int M>
@@ -106,46 +123,88 @@ __global__ void element_implied_kernel(LO ne, LO const* ev2v, Real const* coords
 
 // project_metrics, src/Omega_h_metric.cpp:221-245: log-Euclidean average of
 // the metrics of a vertex's elements (average_metric_contrib/_finish with
-// degenerate metrics skipped, src/Omega_h_metric.hpp:125-139)
-template <int D>
-__global__ void project_metrics_kernel(LO nv, LO const* a2ab, LO const* ab2b, Real const* e2m,
-    Real* out, int* error) {
-  LO v = thread_index();
-  if (v >= nv) return;
+// degenerate metrics skipped, src/Omega_h_metric.hpp:125-139).  Each element's
+// logarithm is taken once, not once by each of its vertices; the full matrix
+// is kept, since its halves can differ in the last bit.
+template <int M>
+__global__ void metric_logs_kernel(LO ne, Real const* e2m, Real* logs, I8* counts, int* error) {
+  LO e = thread_index();
+  if (e >= ne) return;
+  constexpr int nc = (M * (M + 1)) / 2;
   int bad = 0;
-  constexpr int nc = (D * (D + 1)) / 2;
-  Mat am;
-  mat_zero(am);
-  int n = 0;
-  for (LO j = a2ab[v]; j < a2ab[v + 1]; ++j) {
-    Mat em = get_symm<D>(e2m + std::size_t(ab2b[j]) * nc);
-    double mx = 0.0;
-    for (int c = 0; c < D; ++c)
-      for (int r = 0; r < D; ++r) mx = math::max2(mx, math::fabs_(em.m[c][r]));
-    if (mx < kMetricEpsilon) continue;
-    Mat lm = log_spd<D>(em, &bad);
-    for (int c = 0; c < D; ++c)
-      for (int r = 0; r < D; ++r) am.m[c][r] = am.m[c][r] + lm.m[c][r];
-    ++n;
-  }
-  Mat r = am;
-  if (n > 0) {
-    for (int c = 0; c < D; ++c)
-      for (int rr = 0; rr < D; ++rr) am.m[c][rr] = am.m[c][rr] / n;
-    r = exp_spd<D>(am, &bad);
-  }
-  set_symm<D>(r, out + std::size_t(v) * nc);
+  Mat em = get_symm<M>(e2m + std::size_t(e) * nc);
+  double mx = 0.0;
+  for (int c = 0; c < M; ++c)
+    for (int r = 0; r < M; ++r) mx = math::max2(mx, math::fabs_(em.m[c][r]));
+  bool skip = mx < kMetricEpsilon;
+  counts[e] = skip ? 0 : 1;
+  if (skip) return;
+  Mat lm = log_spd<M>(em, &bad);
+  for (int c = 0; c < M; ++c)
+    for (int r = 0; r < M; ++r) logs[std::size_t(e) * M * M + c * M + r] = lm.m[c][r];
   if (bad) *error = kDegenerateEigen;
 }
 
-Reals limit_gradation_once(Ctx& c, DMesh& m, Reals const& values, Real max_rate) {
+// kLogLanes lanes per vertex: lane k sums component k of the logarithms in row
+// order (a row of 24 elements one after another, 72 bytes each, in one
+// coalesced load); the exponentials are a sweep of their own, at full waves.
+// With the logarithms taken here by one thread per vertex, 33,000 vertices took
+// 123 us; the three sweeps take 18, 22 and 9 us.
+template <int M>
+__global__ void sum_logs_kernel(std::int64_t nt, LO const* a2ab, LO const* ab2b,
+    Real const* logs, I8 const* counts, Real* sums, LO* ns) {
+  constexpr int kLogLanes = M == 3 ? 16 : (M == 2 ? 4 : 1);
+  std::int64_t t = thread_index64();
+  if (t >= nt) return;
+  LO v = LO(t / kLogLanes);
+  int lane = int(t % kLogLanes);
+  if (lane >= M * M) return;
+  double sum = 0.0;
+  int n = 0;
+  LO end = a2ab[v + 1];
+#pragma unroll 4
+  for (LO j = a2ab[v]; j < end; ++j) {
+    LO e = ab2b[j];
+    if (counts[e]) {
+      sum = sum + logs[std::size_t(e) * M * M + lane];
+      ++n;
+    }
+  }
+  sums[std::size_t(v) * M * M + lane] = sum;
+  if (lane == 0) ns[v] = n;
+}
+
+template <int M>
+__global__ void mean_exps_kernel(LO nv, Real const* sums, LO const* ns, Real* out, int* error) {
+  LO v = thread_index();
+  if (v >= nv) return;
+  constexpr int nc = (M * (M + 1)) / 2;
+  int n = ns[v];
+  int bad = 0;
+  Mat r;
+  mat_zero(r);
+  for (int c = 0; c < M; ++c)
+    for (int rr = 0; rr < M; ++rr) r.m[c][rr] = sums[std::size_t(v) * M * M + c * M + rr];
+  if (n > 0) {
+    for (int c = 0; c < M; ++c)
+      for (int rr = 0; rr < M; ++rr) r.m[c][rr] = r.m[c][rr] / n;
+    r = exp_spd<M>(r, &bad);
+  }
+  set_symm<M>(r, out + std::size_t(v) * nc);
+  if (bad) *error = kDegenerateEigen;
+}
+
+Reals limit_gradation_once(Ctx& c, DMesh& m, Reals const& values, Real max_rate, Real tol,
+    int word) {
   LO nv = m.nents[0];
   Adj const& star = ask_star(c, m, 0);
   Reals out(c, values.size());
   int md = (m.metric_ncomps == 1) ? 1 : m.dim;
+  unsigned* w = c.words + word;
+  unsigned tag = c.wait_tag();
 #define OSH_LG(S, M)                                                                       \
   OSH_LAUNCH((limit_gradation_kernel<S, M>), nv, c, star.a2ab.data(), star.ab2b.data(),    \
-      m.coords.data(), values.data(), max_rate, out.data(), c.error_word())
+      m.coords.data(), values.data(), max_rate, tol, out.data(), w, tag, c.error_word())
   if (m.dim == 3 && md == 3)
     OSH_LG(3, 3);
   else if (m.dim == 3)
@@ -163,21 +222,29 @@ Reals limit_gradation_once(Ctx& c, DMesh& m, Reals const& values, Real max_rate)
 int limit_metric_gradation(Ctx& c, DMesh& m, Real max_rate, Real tol) {
   OSH_CHECK(max_rate > 0.0, "max_rate must be positive");
   OSH_CHECK(m.metric.exists(), "mesh has no metric");
+  // Sweeps run until one moves nothing.  An isotropic one costs little more
+  // than the wait that tells, so after the first they run two to a wait, each
+  // with a word of its own, and the first quiet one's values are the result,
+  // whatever the next made of them.
+  int batch = 1;
   Reals values2 = m.metric;
-  Reals values;
-  LO n = values2.size();
-  Bytes flags(c, n);
   int steps = 0;
-  bool close;
-  do {
-    values = values2;
-    values2 = limit_gradation_once(c, m, values, max_rate);
-    ++steps;
-    OSH_LAUNCH(not_close_kernel, n, c, values.data(), values2.data(), tol, kMetricEpsilon,
-        flags.data());
-    close = max_i8(c, flags) <= 0;
-    OSH_CHECK(close || steps < 10000, "gradation limiting does not converge in 10000 sweeps");
-  } while (!close);
+  for (;; batch = m.metric_ncomps == 1 ? 2 : 1) {
+    static_assert(Ctx::kWords >= 2, "a word for each sweep of a batch");
+    Reals made[2];
+    unsigned tag = c.wait_tag();
+    for (int k = 0; k < batch; ++k)
+      made[k] = limit_gradation_once(c, m, k ? made[k - 1] : values2, max_rate, tol, k);
+    c.wait();
+    bool close = false;
+    for (int k = 0; k < batch && !close; ++k) {
+      ++steps;
+      values2 = made[k];
+      close = !c.word_set(k, tag);
+      OSH_CHECK(close || steps < 10000, "gradation limiting does not converge in 10000 sweeps");
+    }
+    if (close) break;
+  }
   // a new metric invalidates cached lengths and qualities
   // (src/Omega_h_mesh.cpp:167-177)
   m.metric = values2;
@@ -202,16 +269,28 @@ Reals element_implied_array(Ctx& c, DMesh& m, Real scalar) {
 Reals project_metric_array(Ctx& c, DMesh& m, int mdim, Reals const& e2m) {
   Adj const& v2e = ask_up(c, m, 0, m.dim);
   int nc = (mdim * (mdim + 1)) / 2;
-  Reals out(c, m.nents[0] * nc);
+  LO nv = m.nents[0], ne = m.nents[m.dim];
+  Reals out(c, nv * nc);
+  DArray<Real> logs(c, ne * mdim * mdim);
+  Bytes counts(c, ne);
+  Reals sums(c, nv * mdim * mdim);
+  LOs ns(c, nv);
+#define OSH_PM(M, LANES)                                                                     \
+  do {                                                                                       \
+    OSH_LAUNCH(metric_logs_kernel<M>, ne, c, e2m.data(), logs.data(), counts.data(),           \
+        c.error_word());                                                                     \
+    OSH_LAUNCH64(sum_logs_kernel<M>, std::int64_t(nv) * LANES, c, v2e.a2ab.data(),             \
+        v2e.ab2b.data(), logs.data(), counts.data(), sums.data(), ns.data());                 \
+    OSH_LAUNCH(mean_exps_kernel<M>, nv, c, sums.data(), ns.data(), out.data(),                 \
+        c.error_word());                                                                     \
+  } while (0)
   if (mdim == 3)
-    OSH_LAUNCH(project_metrics_kernel<3>, m.nents[0], c, v2e.a2ab.data(), v2e.ab2b.data(),
-        e2m.data(), out.data(), c.error_word());
+    OSH_PM(3, 16);
   else if (mdim == 2)
-    OSH_LAUNCH(project_metrics_kernel<2>, m.nents[0], c, v2e.a2ab.data(), v2e.ab2b.data(),
-        e2m.data(), out.data(), c.error_word());
+    OSH_PM(2, 4);
   else
-    OSH_LAUNCH(project_metrics_kernel<1>, m.nents[0], c, v2e.a2ab.data(), v2e.ab2b.data(),
-        e2m.data(), out.data(), c.error_word());
+    OSH_PM(1, 1);
+#undef OSH_PM
   return out;
 }
 
