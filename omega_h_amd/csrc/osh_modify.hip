@@ -740,18 +740,21 @@ void plan_keys(Ctx& c, DMesh& old, int key_dim, int d0, int d1, Bytes const& key
   LOs off[4];
   out.keys2kds = LOs(c, nkd);
   int nj = 0;
-  jobs[nj++] = {keys.data(), kScanNonzero, nkd, nullptr, slot_ptr<LO>(c, 0),
+  jobs[nj++] = {keys.data(), kScanNonzero, nkd, nullptr, total_slot(c, 0),
       out.keys2kds.data()};
   for (int d = d0; d <= d1; ++d) {
     if (!out.prod_counts[d].exists()) continue;
     off[d] = LOs(c, nkd + 1);
     kl.prod_off[d - d0] = off[d].data();
     jobs[nj++] = {out.prod_counts[d].data(), kScanLO, nkd, off[d].data(),
-        slot_ptr<LO>(c, 1 + d)};
+        total_slot(c, 1 + d)};
   }
   nj += modify_scan_jobs(c, out.plans, nd, jobs + nj, 5);
   offset_scans(c, jobs, nj);
-  c.wait();
+  unsigned slots = 1u;
+  for (int d = d0; d <= d1; ++d)
+    slots |= (out.prod_counts[d].exists() ? 1u << (1 + d) : 0u) | 1u << (5 + d - d0);
+  c.wait_totals(slots);
   modify_scan_totals(c, out.plans, nd, 5);
   out.nkeys = read_slot<LO>(c, 0);
   out.keys2kds.shrink(out.nkeys);
@@ -772,7 +775,7 @@ int modify_scan_jobs(Ctx& c, ModPlan* plans, int nplans, ScanJob* jobs, int firs
     ModPlan& p = plans[i];
     p.offsets = LOs(c, p.nold + 1);
     jobs[i] = {p.counts.data(), kScanLO, p.nold, p.offsets.data(),
-        slot_ptr<LO>(c, first_slot + i)};
+        total_slot(c, first_slot + i)};
   }
   return nplans;
 }

@@ -145,14 +145,17 @@ struct Ctx {
   // (not for copies into host memory, which only sync() completes)
   void wait();
   // Device words that kernels set to the tag of the coming wait and that the
-  // wait brings to the host: word_set(i, tag) after it.  A tag is never used
-  // twice, so nothing has to be cleared.
+  // wait brings to the host: word_set(i, tag) after it.  A tag (never 0) does
+  // not come again for 2^32 waits, so nothing has to be cleared.
   static constexpr int kWords = 4;
   unsigned* words = nullptr;
-  unsigned wait_tag() const { return signal_value + 1; }
+  unsigned wait_tag() const { return signal_value + 1u ? signal_value + 1u : 1u; }
   bool word_set(int i, unsigned tag) const {
     return __atomic_load_n(host_words() + i, __ATOMIC_RELAXED) == tag;
   }
+  // waits for the scan totals of the given slots (bits) that the last
+  // offset_scans call since the last wait writes
+  void wait_totals(unsigned slots);
   // for a kernel that signals by itself, as its last store (a release at
   // system scope of wait_tag() into signal_word()): waits for that
   void wait_signalled();
@@ -164,6 +167,8 @@ struct Ctx {
   unsigned signal_value = 0;
   unsigned* host_words() const { return signal_word() + 16; }
   void raise_device_error();
+  template <class Arrived>
+  void poll(Arrived const& arrived);
 };
 
 void range_begin(Ctx& c, char const* name);
@@ -278,6 +283,16 @@ enum DeviceError {
   kPolytopeOverflow = 11
 };
 
+// the pinned slot for a scan's total, and the total there once waited for
+// (Ctx::wait_totals, or any later wait): the low half of the slot's word
+inline unsigned long long* total_slot(Ctx& c, int slot) {
+  return slot_ptr<unsigned long long>(c, slot);
+}
+inline LO scan_total(Ctx& c, int slot) {
+  c.wait_totals(1u << slot);
+  return read_slot<LO>(c, slot);
+}
+
 // what a raised kReflectDownNoMatch says
 constexpr char const* kNoMatchMessage = "reflect_down: entity without a unique match";
 
@@ -368,7 +383,8 @@ struct ScanJob {
   int kind;
   LO n;
   LO* out;    // n + 1 entries
-  LO* total;  // device-visible grand total (a pinned slot), or nullptr
+  // where the grand total goes (total_slot), or nullptr
+  unsigned long long* total;
   LO* list = nullptr;  // for nonzero flags: the indices of the nonzero ones
 };
 void offset_scans(Ctx& c, ScanJob const* jobs, int njobs);

@@ -1022,12 +1022,12 @@ bool swap_edges_3d(Ctx& c, DMesh& m, AdaptOptions const& o, SwapCache* cache) {
   LOs np[3], off[3], reps[2] = {LOs(c, ncands), LOs(c, ncands)};
   LOs key_off(c, ncands + 1);
   ScanJob jobs[kMaxScanJobs];
-  jobs[0] = {is_key.data(), kScanNonzero, ncands, key_off.data(), slot_ptr<LO>(c, 0)};
+  jobs[0] = {is_key.data(), kScanNonzero, ncands, key_off.data(), total_slot(c, 0)};
   KeyPlan kp{};
   for (int d = 0; d < 3; ++d) {
     np[d] = LOs(c, ncands);
     off[d] = LOs(c, ncands + 1);
-    jobs[d + 1] = {np[d].data(), kScanLO, ncands, off[d].data(), slot_ptr<LO>(c, d + 1)};
+    jobs[d + 1] = {np[d].data(), kScanLO, ncands, off[d].data(), total_slot(c, d + 1)};
     kp.same[d] = plans[d].same.data();
     kp.counts[d] = plans[d].counts.data();
     kp.nprods[d] = np[d].data();
@@ -1039,7 +1039,7 @@ bool swap_edges_3d(Ctx& c, DMesh& m, AdaptOptions const& o, SwapCache* cache) {
   OSH_LAUNCH(swap3d_plan_keys, ncands * kRow, c, rings.r, keys.data(), m.down[3].data(), tb, kp);
   int njobs = 4 + modify_scan_jobs(c, plans, 3, jobs + 4, 4);
   offset_scans(c, jobs, njobs);
-  c.wait();
+  c.wait_totals(0x7fu);
   modify_scan_totals(c, plans, 3, 4);
   LO nkeys = read_slot<LO>(c, 0);
   if (o.verbosity >= 2) std::printf("swapping %d 3D edges\n", int(nkeys));
