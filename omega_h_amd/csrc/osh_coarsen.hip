@@ -38,9 +38,10 @@ __global__ void mark_short_edges(LO ne, Real const* lengths, Real shortest, LO c
 
 // the collapse directions of each edge: away from its marked ends
 // (src/Omega_h_coarsen.cpp:29-47), as far as classification allows
-// (check_collapse_class, src/Omega_h_check_collapse.cpp:10-40)
+// (check_collapse_class, src/Omega_h_check_collapse.cpp:10-40); `verts` marks
+// the vertices that collapse along some edge
 __global__ void collapse_codes(LO ne, LO const* ev2v, I8 const* vmarks, I8 const* vdim,
-    I8 const* edim, I8* codes) {
+    I8 const* edim, I8* codes, I8* verts) {
   LO e = thread_index();
   if (e >= ne) return;
   LO v[2] = {ev2v[e * 2], ev2v[e * 2 + 1]};
@@ -58,12 +59,10 @@ __global__ void collapse_codes(LO ne, LO const* ev2v, I8 const* vmarks, I8 const
     }
   }
   codes[e] = code;
+  for (int eev = 0; eev < 2; ++eev)
+    if (collapses(code, eev)) verts[v[eev]] = 1;
 }
 
-// check_collapse_exposure from the cells' side: every cell of dimension CD
-// looks at its own edges, and a collapse side whose cell's side opposite the
-// target vertex is classified differently from the cell is vetoed (the
-// order of the cells does not matter, so no edge -> cell rows are built)
 template <int CD>
 __device__ __forceinline__ int local_vertex(LO const* cv, LO v) {
   int k = 0;
@@ -83,37 +82,9 @@ struct CellSweep {
   LO const* c2e[2];
   LO const* cv2v[2];
   LO const* cs2s[2];
-  I8 const* cdim[2];
-  I8 const* sdim[2];
   I8* dead_cells[2];
   I8* dead_sides[2];
 };
-
-template <int CD>
-__device__ __forceinline__ void check_exposure(LO c, CellSweep const& a, int w,
-    LO const* ev2v, I8 const* codes, I8* veto) {
-  if (c >= a.ncells[w]) return;
-  constexpr int nepc = (CD == 3) ? 6 : 3;
-  // a cell whose sides are all classified like itself vetoes nothing: most
-  // cells stop here, before they look at their edges
-  I8 own = a.cdim[w][c];
-  unsigned differ = 0u;
-#pragma unroll
-  for (int k = 0; k <= CD; ++k)
-    if (a.sdim[w][a.cs2s[w][std::size_t(c) * (CD + 1) + k]] != own) differ |= 1u << k;
-  if (differ == 0u) return;
-  LO const* cv = a.cv2v[w] + std::size_t(c) * (CD + 1);
-  for (int j = 0; j < nepc; ++j) {
-    LO e = a.c2e[w][std::size_t(c) * nepc + j];
-    I8 code = codes[e];
-    if (code == kDont) continue;
-    for (int col = 0; col < 2; ++col) {
-      if (!collapses(code, col)) continue;
-      int ccv_onto = local_vertex<CD>(cv, ev2v[e * 2 + (1 - col)]);
-      if ((differ >> opposite_template(CD, 0, ccv_onto)) & 1u) veto[e * 2 + col] = 1;
-    }
-  }
-}
 
 __device__ __forceinline__ int cell_job(CellSweep const& a, LO* c) {
   int w = (a.n > 1 && blockIdx.x >= a.first[1]) ? 1 : 0;
@@ -121,108 +92,9 @@ __device__ __forceinline__ int cell_job(CellSweep const& a, LO* c) {
   return w;
 }
 
-__global__ void __launch_bounds__(kBlock) check_exposure_cells(CellSweep a, LO const* ev2v,
-    I8 const* codes, I8* veto) {
-  LO c;
-  int w = cell_job(a, &c);
-  if (a.dim[w] == 3)
-    check_exposure<3>(c, a, w, ev2v, codes, veto);
-  else
-    check_exposure<2>(c, a, w, ev2v, codes, veto);
-}
-
-// Each collapse side (candidate edge, direction) gets 2^lshift threads
-// (Tuning::coarsen_lanes, at most 32 so that an edge's two sides share a
-// wave), which split the collapsing vertex's row between them, so that passes
-// with few candidates still spread their work over the device.  Minima do not
-// depend on how a row is split, so the lane count changes no result.  The two
-// sides' verdicts meet through ballots and one lane writes the edge's code.
 // The product builders below use kLanes threads per key.
 constexpr int kLanes = 8;
 constexpr int kMaxSideLanes = 32;
-
-// the lanes of a side and of its edge in the wave
-struct SideLanes {
-  int lane;
-  int base;  // the side's first lane
-  unsigned long long side;  // its lanes
-  __device__ __forceinline__ SideLanes(LO t, int lshift) {
-    int lanes = 1 << lshift;
-    lane = int(t) & (lanes - 1);
-    base = int(threadIdx.x % 64) & ~(lanes - 1);
-    side = ((1ull << lanes) - 1ull) << base;
-  }
-  __device__ __forceinline__ bool any(bool x) const { return (__ballot(x) & side) != 0ull; }
-};
-
-// writes the code of the edge whose sides' verdicts are `keep`
-__device__ __forceinline__ void write_code(SideLanes const& s, int lshift, int col, bool keep,
-    I8 code, LO e, I8* codes) {
-  unsigned long long b = __ballot(keep);
-  if (col != 0 || s.lane != 0) return;
-  I8 out = code;
-  if (!((b >> s.base) & 1ull)) out = dont_collapse(out, 0);
-  if (!((b >> (s.base + (1 << lshift))) & 1ull)) out = dont_collapse(out, 1);
-  if (out != code) codes[e] = out;
-}
-
-// prevent_coarsen_overshoot: a side is vetoed when any new edge would reach
-// max_length (the order of the row does not matter); sides vetoed by exposure
-// leave their codes here too.  MIXED: FP32 estimates first; a side is vetoed
-// when one is over max_length by more than the screening band, and measured
-// in FP64 only when none is but one lies inside the band.
-template <int D, int M, bool MIXED>
-__global__ void overshoot_lanes(LO nt, int lshift, LO const* cands, LO const* ev2v,
-    LO const* v2e_a2ab, LO const* v2e_ab2b, I8 const* v2e_codes, Real const* coords,
-    Real const* metric, Real max_length, I8 const* exposed, I8* codes) {
-  LO t = thread_index();
-  if (t >= nt) return;
-  LO side = t >> lshift;
-  SideLanes s(t, lshift);
-  LO e = cands[side / 2];
-  int col = side % 2;
-  I8 code = codes[e];
-  constexpr int nc = (M == 1) ? 1 : (M == 2 ? 3 : 6);
-  LO v_col = ev2v[e * 2 + col];
-  LO v_onto = ev2v[e * 2 + (1 - col)];
-  bool open = collapses(code, col) && !exposed[e * 2 + col];
-  LO row = open ? v2e_a2ab[v_col] : 0;
-  LO end = open ? v2e_a2ab[v_col + 1] : 0;
-  // the ends of the new edge at row entry ve; false for the candidate itself
-  auto ends = [&](LO ve, double (&p0)[D], double (&p1)[D], double (&m0)[nc], double (&m1)[nc]) {
-    LO e2 = v2e_ab2b[ve];
-    if (e2 == e) return false;
-    int eev_in = code_which_down(v2e_codes[ve]);
-    LO out = ev2v[e2 * 2 + 1 - eev_in];
-    LO a = eev_in == 0 ? v_onto : out, b = eev_in == 0 ? out : v_onto;
-    for (int k = 0; k < D; ++k) {
-      p0[k] = coords[a * D + k];
-      p1[k] = coords[b * D + k];
-    }
-    for (int k = 0; k < nc; ++k) {
-      m0[k] = metric[a * nc + k];
-      m1[k] = metric[b * nc + k];
-    }
-    return true;
-  };
-  double p0[D], p1[D], m0[nc], m1[nc];
-  bool veto = false;
-  if constexpr (MIXED) {
-    bool unsure = false;
-    float lmax = float(max_length);
-    for (LO ve = row + s.lane; ve < end; ve += (1 << lshift)) {
-      if (!ends(ve, p0, p1, m0, m1)) continue;
-      float l = f32::edge_length<D, M>(p0, p1, m0, m1);
-      veto = veto || l >= lmax * (1.0f + f32::kScreenBand);
-      unsure = unsure || !(l < lmax * (1.0f - f32::kScreenBand));
-    }
-    veto = s.any(veto);
-    if (veto || !s.any(unsure)) end = row;
-  }
-  for (LO ve = row + s.lane; ve < end && !veto; ve += (1 << lshift))
-    if (ends(ve, p0, p1, m0, m1)) veto = edge_length<D, M>(p0, p1, m0, m1) >= max_length;
-  write_code(s, lshift, col, open && !s.any(veto), code, e, codes);
-}
 
 // the vertices' metric determinants, which every quality around a vertex
 // needs (24 times in a tet mesh)
@@ -236,20 +108,9 @@ __global__ void vert_dets(LO nv, Real const* metric, Real* dets) {
   dets[v] = det<M>(get_symm<M>(m));
 }
 
-// coarsen_qualities with its filters (src/Omega_h_coarsen_qualities.cpp:16-122):
-// the minimum quality of the cells that survive a collapse, with v_col moved
-// onto v_onto; a side is kept when it reaches qmin and, with `improve`, exceeds
-// the old minimum around v_col.  FILTER off: every side's minimum goes to
-// quals and nothing is kept or dropped.
-//
-// Bound by FP64 issue (166 operations a quality and its correctly rounded
-// divisions), so work is left out where it decides nothing: the determinants
-// come from vert_dets, a lane reads only the metric it uses, and a side stops
-// at the first cell below qmin.
-//
-// MIXED: FP32 estimates first; a side is rejected (quality -1) when their
-// minimum is below qmin by more than the band and every element's
-// max-determinant metric was clear, else evaluated in FP64.
+// coarsen_qualities without its filters: every collapse side's minimum quality
+// of the cells that survive, with v_col moved onto v_onto, or -1 for a side
+// that is not asked for.  MIXED as in collapse_stars.
 struct SideQualities {
   LO const* cands;
   LO const* ev2v;
@@ -261,56 +122,62 @@ struct SideQualities {
   Real const* metric;
   Real const* dets;
   Real qmin;
-  Real const* old_quals;  // improve: the elements' qualities (else null)
-  I8* codes;
-  Real* quals;  // by (edge, direction); by (candidate, direction) with FILTER off
+  I8 const* codes;
+  Real* quals;  // by (candidate, direction)
 };
 
-template <int D, int M, bool MIXED, bool FILTER>
+// the vertices of a row's cell once its vertex has moved onto v_onto; false if
+// it dies
+template <int D>
+__device__ __forceinline__ bool moved_cell(LO const* cv2v, LO c, int ccv_col, LO v_onto,
+    LO (&cv)[D + 1]) {
+  bool lives = true;
+#pragma unroll
+  for (int k = 0; k < D + 1; ++k) {
+    cv[k] = cv2v[std::size_t(c) * (D + 1) + k];
+    if (k != ccv_col && cv[k] == v_onto) lives = false;
+  }
+#pragma unroll
+  for (int k = 0; k < D + 1; ++k)
+    if (k == ccv_col) cv[k] = v_onto;
+  return lives;
+}
+
+template <int D, int M, bool MIXED>
 __global__ void __launch_bounds__(kBlock) coarsen_quality_lanes(LO nt, int lshift,
     SideQualities a) {
   LO t = thread_index();
   if (t >= nt) return;
   LO side = t >> lshift;
-  SideLanes s(t, lshift);
   int lanes = 1 << lshift;
+  int lane = int(t) & (lanes - 1);
+  unsigned long long group = ((1ull << lanes) - 1ull) << (int(threadIdx.x % 64) & ~(lanes - 1));
   LO e = a.cands[side / 2];
   int col = side % 2;
-  I8 code = a.codes[e];
   constexpr int nc = (M == 1) ? 1 : (M == 2 ? 3 : 6);
-  bool open = collapses(code, col);
+  bool open = collapses(a.codes[e], col);
   LO v_col = a.ev2v[e * 2 + col];
   LO v_onto = a.ev2v[e * 2 + (1 - col)];
   LO row = open ? a.v2c_a2ab[v_col] : 0;
   LO end = open ? a.v2c_a2ab[v_col + 1] : 0;
-  // the vertices of row entry vc's cell after the collapse; false if it dies
-  auto moved = [&](LO vc, LO (&cv)[D + 1]) {
-    LO c = a.v2c_ab2b[vc];
-    int ccv_col = code_which_down(a.v2c_codes[vc]);
-    bool lives = true;
-#pragma unroll
-    for (int k = 0; k < D + 1; ++k) {
-      cv[k] = a.cv2v[std::size_t(c) * (D + 1) + k];
-      if (k != ccv_col && cv[k] == v_onto) lives = false;
-    }
-#pragma unroll
-    for (int k = 0; k < D + 1; ++k)
-      if (k == ccv_col) cv[k] = v_onto;
-    return lives;
-  };
   bool rejected = false;
   double const* pp[D + 1];
   double const* ms[D + 1];
+  auto points = [&](LO vc) {
+    LO cv[D + 1];
+    if (!moved_cell<D>(a.cv2v, a.v2c_ab2b[vc], code_which_down(a.v2c_codes[vc]), v_onto, cv))
+      return false;
+    for (int k = 0; k < D + 1; ++k) {
+      pp[k] = a.coords + std::size_t(cv[k]) * D;
+      ms[k] = a.metric + std::size_t(cv[k]) * nc;
+    }
+    return true;
+  };
   if constexpr (MIXED) {
     float minq = 1.0f;
     bool unclear = false;
-    for (LO vc = row + s.lane; vc < end; vc += lanes) {
-      LO cv[D + 1];
-      if (!moved(vc, cv)) continue;
-      for (int k = 0; k < D + 1; ++k) {
-        pp[k] = a.coords + std::size_t(cv[k]) * D;
-        ms[k] = a.metric + std::size_t(cv[k]) * nc;
-      }
+    for (LO vc = row + lane; vc < end; vc += lanes) {
+      if (!points(vc)) continue;
       float q = f32::element_quality<D, M>(pp, ms, &unclear);
       minq = (q < minq) ? q : minq;
     }
@@ -318,41 +185,542 @@ __global__ void __launch_bounds__(kBlock) coarsen_quality_lanes(LO nt, int lshif
       float o = __shfl_xor(minq, d, 64);
       minq = (o < minq) ? o : minq;
     }
-    rejected = open && !s.any(unclear) &&
+    rejected = open && (__ballot(unclear) & group) == 0ull &&
                double(minq) < a.qmin * (1.0 - double(f32::kScreenBand));
     if (rejected) end = row;
   }
   double minq = 1.0;
-  double vold = 1.79769313486231570815e+308;
-  for (LO b = row; b < end; b += lanes) {
-    LO vc = b + s.lane;
-    LO cv[D + 1];
-    if (vc < end) {
-      if (FILTER && a.old_quals) vold = math::min2(vold, a.old_quals[a.v2c_ab2b[vc]]);
-      if (moved(vc, cv)) {
-        double dets[D + 1];
-        for (int k = 0; k < D + 1; ++k) {
-          pp[k] = a.coords + std::size_t(cv[k]) * D;
-          ms[k] = a.metric + std::size_t(cv[k]) * nc;
-          dets[k] = a.dets[cv[k]];
-        }
-        minq = math::min2(minq, element_quality<D, M>(pp, ms, dets));
+  for (LO vc = row + lane; vc < end; vc += lanes) {
+    if (!points(vc)) continue;
+    double dets[D + 1];
+    for (int k = 0; k < D + 1; ++k) dets[k] = a.dets[(ms[k] - a.metric) / nc];
+    minq = math::min2(minq, element_quality<D, M>(pp, ms, dets));
+  }
+  for (int d = lanes / 2; d > 0; d >>= 1) minq = math::min2(minq, __shfl_xor(minq, d, 64));
+  if (lane == 0) a.quals[side] = (rejected || !open) ? -1.0 : minq;
+}
+
+// What a collapsing vertex decides from its star, a wave each:
+//  - check_collapse_exposure (src/Omega_h_check_collapse.cpp:64-117): a side is
+//    vetoed where a cell around its edge (triangle or tet) has its side opposite
+//    the target classified differently from itself;
+//  - prevent_coarsen_overshoot: where a new edge would reach max_length;
+//  - coarsen_qualities with its filters
+//    (src/Omega_h_coarsen_qualities.cpp:16-122): a side is kept when the cells
+//    that survive reach qmin and, with `improve`, exceed the old minimum;
+//  - choose_rails (src/Omega_h_collapse_rail.cpp:15-60): the shortest edge left,
+//    the one of higher quality among equally long ones, the first of those;
+//  - the vertex star (verts_across_edges, src/Omega_h_adj.cpp:512-530).
+//
+// Bound by FP64 issue (81 % of the cycles issue vector instructions): some 100
+// operations a new edge, 166 a quality, with their correctly rounded divisions.
+// A star's vertices are neighbors of all its sides, so they are brought to LDS
+// once, and the (target, edge) and (target, cell) pairs of the sides still open
+// are dealt out to the lanes together, a few edges or cells of each side at a
+// time.  As sweeps of their own with 16 lanes a side, each side gathering the
+// star again, exposure, overshoot, qualities and rails took 1.85 ms for 1.9 M
+// sides of 275,000 vertices and 165 us for 239,000 sides of which none was
+// kept; this takes 1.47 ms and 71 us.
+//
+// MIXED: FP32 estimates first.  A side is vetoed when an estimated length is
+// over max_length by more than the screening band, and measured in FP64 only
+// when none is but one lies inside the band; it is rejected when the estimated
+// minimum quality is below qmin by more than the band and every cell's
+// max-determinant metric was clear, else evaluated in FP64.
+struct StarSweep {
+  LO nverts;
+  LO const* verts;
+  LO const* ev2v;
+  LO const* e_a2ab;
+  LO const* e_ab2b;
+  I8 const* e_codes;
+  LO const* c_a2ab;
+  LO const* c_ab2b;
+  I8 const* c_codes;
+  LO const* cv2v;
+  LO const* c2s;  // the cells' sides
+  LO const* f2e;  // 3D: the faces' edges and vertices
+  LO const* fv2v;
+  I8 const* edim;
+  I8 const* sdim;
+  I8 const* cdim;
+  Real const* coords;
+  Real const* metric;
+  Real const* lengths;
+  Real const* old_quals;  // improve: the elements' qualities (else null)
+  Real max_length;
+  Real qmin;
+  I8 const* codes;
+  bool sides_only;  // stop after the overshoot check, with the verdicts in `sides`
+  bool checked;     // the codes are those of such a sweep
+  unsigned* word;   // receives the tag where a star is large
+  unsigned tag;
+  I8* sides;        // by (edge, direction)
+  I8* vcand;        // zero on entry
+  Real* vqual;
+  LO* vrail;
+  LO* star;
+};
+
+// a star in LDS, shared by the WAVES waves that work on it
+template <int D, int M, int WAVES>
+struct StarData {
+  static constexpr int nc = (M == 1) ? 1 : (M == 2 ? 3 : 6);
+  static constexpr int kThreads = WAVES * 64;
+  static constexpr int kEdges = kThreads - 1;  // at most a thread each; a byte holds a position
+  static constexpr int kCells = WAVES * 128;
+  double coords[kThreads * D];
+  double metric[kThreads * nc];
+  double dets[kThreads];
+  double lens[kThreads];
+  unsigned long long minq[kThreads];
+  double least[WAVES];
+  int counts[WAVES];
+  LO verts[kThreads];
+  unsigned cells[kCells];  // positions of a cell's vertices, a byte each; kSelf: the vertex
+  unsigned char list[kThreads];
+  I8 edim[kThreads];
+  I8 second[kThreads];  // the vertex is its edge's second
+  I8 veto[kThreads];
+  I8 unsure[kThreads];
+
+  __device__ __forceinline__ static void sync() {
+    if constexpr (WAVES > 1) {
+      __syncthreads();
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+  // lists the sides whose thread says so, in order; how many
+  __device__ __forceinline__ int list_sides(bool in, int t) {
+    unsigned long long b = __ballot(in);
+    sync();
+    if (WAVES > 1 && t % 64 == 0) counts[t / 64] = __popcll(b);
+    if (WAVES > 1) sync();
+    int before = 0, total = __popcll(b);
+    if constexpr (WAVES > 1) {
+      total = 0;
+      for (int w = 0; w < WAVES; ++w) {
+        before += w < t / 64 ? counts[w] : 0;
+        total += counts[w];
       }
     }
-    if (FILTER && s.any(minq < a.qmin)) break;
+    if (in) list[before + __popcll(b & ((1ull << (t % 64)) - 1ull))] = static_cast<unsigned char>(t);
+    sync();
+    return total;
   }
-  for (int d = lanes / 2; d > 0; d >>= 1) {
-    minq = math::min2(minq, __shfl_xor(minq, d, 64));
-    vold = math::min2(vold, __shfl_xor(vold, d, 64));
+  // op(target, k) for the listed targets and k < n, over the threads
+  template <class Op>
+  __device__ __forceinline__ void for_pairs(int nlist, int n, int t, Op const& op) const {
+    int at = t / n, k = t % n, step = kThreads / n, rest = kThreads % n;
+#pragma unroll 1
+    while (at < nlist) {
+      op(int(list[at]), k);
+      at += step;
+      k += rest;
+      if (k >= n) {
+        k -= n;
+        ++at;
+      }
+    }
   }
-  if (rejected || !open) minq = -1.0;
-  if constexpr (FILTER) {
-    bool keep = open && minq >= a.qmin && (!a.old_quals || minq > vold);
-    if (keep && s.lane == 0) a.quals[std::size_t(e) * 2 + col] = minq;
-    write_code(s, lshift, col, keep, code, e, a.codes);
+  // the same while the sides still stand: few rows of the pairs at a time, the
+  // sides vetoed by then left out of the next (a list is some 30 instructions,
+  // a quality 500)
+  template <class Op>
+  __device__ __forceinline__ void for_standing_pairs(int nlist, int n, int t, bool open,
+      Op const& op) {
+    for (int first = 0; first < n && nlist > 0;) {
+      int rows = (nlist > kThreads / 4 ? 2 * kThreads : kThreads) / nlist;
+      rows = rows < n - first ? rows : n - first;
+#pragma unroll 1
+      for (int p = t; p < nlist * rows; p += kThreads) op(int(list[p / rows]), first + p % rows);
+      first += rows;
+      sync();
+      if (first < n) nlist = list_sides(open && !veto[t], t);
+    }
+  }
+  __device__ __forceinline__ double min_of(double x, int t) {
+    for (int d = 32; d > 0; d >>= 1) x = math::min2(x, __shfl_xor(x, d, 64));
+    if constexpr (WAVES > 1) {
+      sync();
+      if (t % 64 == 0) least[t / 64] = x;
+      sync();
+      x = least[0];
+      for (int w = 1; w < WAVES; ++w) x = math::min2(x, least[w]);
+    }
+    return x;
+  }
+};
+constexpr unsigned kSelf = 0xffu;
+constexpr int kLargeStarWord = 2;  // the sets use the words before
+
+// doubles as whole numbers in the same order (atomicMin)
+__device__ __forceinline__ unsigned long long ordered(double x) {
+  unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(x));
+  return (b >> 63) ? ~b : b | (1ull << 63);
+}
+__device__ __forceinline__ double unordered(unsigned long long b) {
+  return __longlong_as_double(
+      static_cast<long long>((b >> 63) ? b & ~(1ull << 63) : ~b));
+}
+
+// the choice among a vertex's rails so far
+struct Rail {
+  LO edge = -1;
+  double len = 0.0;
+  double qual = 0.0;
+  __device__ __forceinline__ void visit(LO e, double l, double q) {
+    if (edge != -1 && !(l < len || (l == len && q > qual))) return;
+    edge = e;
+    len = l;
+    qual = q;
+  }
+};
+
+template <int D, int M, bool MIXED, int WAVES>
+__device__ __forceinline__ void small_star(StarSweep const& a, LO row, int nedges, LO crow,
+    int ncells, int t, StarData<D, M, WAVES>& s, Rail& rail) {
+  using S = StarData<D, M, WAVES>;
+  constexpr int nc = S::nc;
+  LO e = -1;
+  int eev = 0;
+  bool open = false;
+  if (t < nedges) {
+    e = a.e_ab2b[row + t];
+    eev = code_which_down(a.e_codes[row + t]);
+    LO u = a.ev2v[e * 2 + 1 - eev];
+    open = collapses(a.codes[e], eev);
+    if (!a.sides_only) a.star[row + t] = u;
+    s.verts[t] = u;
+    s.edim[t] = a.edim[e];
+    s.second[t] = eev == 1;
+    double m[nc];
+    for (int k = 0; k < D; ++k) s.coords[t * D + k] = a.coords[std::size_t(u) * D + k];
+    for (int k = 0; k < nc; ++k) s.metric[t * nc + k] = m[k] = a.metric[std::size_t(u) * nc + k];
+    s.dets[t] = M == 1 ? m[0] : det<M>(get_symm<M>(m));
+  }
+  s.veto[t] = s.unsure[t] = 0;
+  int nopen = s.list_sides(open, t);
+  if (!a.checked && nopen) {
+    // the ends of the new edge from target w at neighbor u
+    auto length_of = [&](auto const& length, int w, int u) {
+      int p = s.second[u] ? u : w, q = s.second[u] ? w : u;
+      return length(s.coords + p * D, s.coords + q * D, s.metric + p * nc, s.metric + q * nc);
+    };
+    if constexpr (MIXED) {
+      float lmax = float(a.max_length);
+      s.for_standing_pairs(nopen, nedges, t, open, [&](int w, int u) {
+        if (u == w) return;
+        float l = length_of(
+            [](auto... x) { return f32::edge_length<D, M>(x...); }, w, u);
+        if (l >= lmax * (1.0f + f32::kScreenBand))
+          s.veto[w] = 1;
+        else if (!(l < lmax * (1.0f - f32::kScreenBand)))
+          s.unsure[w] = 1;
+      });
+      nopen = s.list_sides(open && s.unsure[t] && !s.veto[t], t);
+    }
+    s.for_standing_pairs(nopen, nedges, t, MIXED ? open && s.unsure[t] : open, [&](int w, int u) {
+      if (u == w) return;
+      double l = length_of([](auto... x) { return edge_length<D, M>(x...); }, w, u);
+      if (l >= a.max_length) s.veto[w] = 1;
+    });
+    open = open && !s.veto[t];
+    nopen = s.list_sides(open, t);
+  }
+  double vold = 1.79769313486231570815e+308;
+  for (int i = t; nopen && i < ncells; i += S::kThreads) {
+    LO c = a.c_ab2b[crow + i];
+    int at = code_which_down(a.c_codes[crow + i]);
+    unsigned pos[D + 1];
+    LO cv[D + 1];
+#pragma unroll
+    for (int k = 0; k < D + 1; ++k) {
+      cv[k] = a.cv2v[std::size_t(c) * (D + 1) + k];
+      pos[k] = kSelf;
+    }
+    I8 own = 0, sd[D + 1];
+    if (!a.checked) {
+      // the side opposite a vertex other than the star's has that one in it
+      own = a.cdim[c];
+#pragma unroll
+      for (int k = 0; k < D + 1; ++k)
+        sd[k] = a.sdim[a.c2s[std::size_t(c) * (D + 1) + opposite_template(D, 0, k)]];
+    }
+    if (a.old_quals && !a.sides_only) vold = math::min2(vold, a.old_quals[c]);
+#pragma unroll 2
+    for (int j = 0; j < nedges; ++j) {
+      LO u = s.verts[j];
+#pragma unroll
+      for (int k = 0; k < D + 1; ++k)
+        if (cv[k] == u) pos[k] = unsigned(j);
+    }
+    unsigned packed = 0u;
+#pragma unroll
+    for (int k = 0; k < D + 1; ++k) packed |= pos[k] << (8 * k);
+    s.cells[i] = packed;
+    if (a.checked) continue;
+#pragma unroll
+    for (int k = 0; k < D + 1; ++k) {
+      if (k == at) continue;
+      if (sd[k] != own) s.veto[pos[k] % S::kThreads] = 1;
+      if (D == 3) {
+        // the triangle's edges from the vertex, each opposite the other's end
+        unsigned x = kSelf, y = kSelf;
+#pragma unroll
+        for (int j = 0; j < D + 1; ++j) {
+          if (j == at || j == k) continue;
+          y = x;
+          x = pos[j];
+        }
+        x %= S::kThreads;
+        y %= S::kThreads;
+        if (s.edim[y] != sd[k]) s.veto[x] = 1;
+        if (s.edim[x] != sd[k]) s.veto[y] = 1;
+      }
+    }
+  }
+  S::sync();
+  open = open && !s.veto[t];
+  if (a.sides_only) {
+    if (t < nedges) a.sides[std::size_t(e) * 2 + eev] = open ? 1 : 0;
+    return;
+  }
+  nopen = s.list_sides(open, t);
+  if (nopen == 0) return;
+  if (a.old_quals) vold = s.min_of(vold, t);
+  // the positions of cell i's vertices with its vertex moved onto target w;
+  // false if it dies
+  auto moved = [&](int w, int i, int (&at)[D + 1]) {
+    unsigned packed = s.cells[i];
+    bool lives = true;
+#pragma unroll
+    for (int k = 0; k < D + 1; ++k) {
+      int j = int((packed >> (8 * k)) & 0xffu);
+      lives = lives && j != w;
+      at[k] = j == int(kSelf) ? w : j;
+    }
+    return lives;
+  };
+  if constexpr (MIXED) {
+    // estimated minima, as ordered whole numbers; `unsure`: an unclear metric
+    s.unsure[t] = 0;
+    s.minq[t] = ordered(1.0);
+    S::sync();
+    s.for_pairs(nopen, ncells, t, [&](int w, int i) {
+      int at[D + 1];
+      if (!moved(w, i, at)) return;
+      double const* pp[D + 1];
+      double const* ms[D + 1];
+#pragma unroll
+      for (int k = 0; k < D + 1; ++k) {
+        pp[k] = s.coords + at[k] * D;
+        ms[k] = s.metric + at[k] * nc;
+      }
+      bool unclear = false;
+      float q = f32::element_quality<D, M>(pp, ms, &unclear);
+      if (unclear) s.unsure[w] = 1;
+      if (q < 1.0f) atomicMin(&s.minq[w], ordered(double(q)));
+    });
+    S::sync();
+    bool rejected =
+        !s.unsure[t] && unordered(s.minq[t]) < a.qmin * (1.0 - double(f32::kScreenBand));
+    open = open && !rejected;
+    nopen = s.list_sides(open, t);
+  }
+  s.minq[t] = ordered(1.0);
+  if (open) s.lens[t] = a.lengths[e];
+  s.veto[t] = 0;
+  S::sync();
+  s.for_standing_pairs(nopen, ncells, t, open, [&](int w, int i) {
+    int at[D + 1];
+    if (!moved(w, i, at)) return;
+    // element_quality, from the positions
+    double p[D + 1][D];
+    double const* pp[D + 1];
+    int best = at[0];
+    double maxdet = s.dets[at[0]];
+#pragma unroll
+    for (int k = 0; k < D + 1; ++k) {
+      pp[k] = p[k];
+#pragma unroll
+      for (int j = 0; j < D; ++j) p[k][j] = s.coords[at[k] * D + j];
+      if (s.dets[at[k]] > maxdet) {
+        best = at[k];
+        maxdet = s.dets[at[k]];
+      }
+    }
+    double q = quality_with<D, M>(pp, get_symm<M>(s.metric + best * nc), maxdet);
+    if (q < a.qmin || (a.old_quals && q <= vold))
+      s.veto[w] = 1;
+    else if (q < 1.0)
+      atomicMin(&s.minq[w], ordered(q));
+  });
+  double minq = unordered(s.minq[t]);
+  int nkept = s.list_sides(open && !s.veto[t] && minq >= a.qmin &&
+                               (!a.old_quals || minq > vold), t);
+  if (t != 0) return;
+  for (int i = 0; i < nkept; ++i) {
+    int w = s.list[i];
+    rail.visit(w, s.lens[w], unordered(s.minq[w]));
+  }
+  if (nkept) rail.edge = a.e_ab2b[row + rail.edge];
+}
+
+// a star of any size: one side after another, from memory
+template <int D, int M, bool MIXED>
+__device__ __forceinline__ void large_star(StarSweep const& a, LO row, LO end, LO crow, LO cend,
+    int lane, Rail& rail) {
+  constexpr int nc = StarData<D, M, 1>::nc;
+  if (!a.sides_only)
+    for (LO ve = row + lane; ve < end; ve += 64)
+      a.star[ve] = a.ev2v[a.e_ab2b[ve] * 2 + 1 - code_which_down(a.e_codes[ve])];
+  double vold = 1.79769313486231570815e+308;
+  if (a.old_quals && !a.sides_only) {
+    for (LO vc = crow + lane; vc < cend; vc += 64)
+      vold = math::min2(vold, a.old_quals[a.c_ab2b[vc]]);
+    for (int d = 32; d > 0; d >>= 1) vold = math::min2(vold, __shfl_xor(vold, d, 64));
+  }
+  for (LO vw = row; vw < end; ++vw) {
+    LO e = a.e_ab2b[vw];
+    int eev = code_which_down(a.e_codes[vw]);
+    LO onto = a.ev2v[e * 2 + 1 - eev];
+    bool open = collapses(a.codes[e], eev);
+    if (open && !a.checked) {
+      bool veto = false;
+      for (LO vc = crow + lane; vc < cend; vc += 64) {
+        LO c = a.c_ab2b[vc];
+        int at = code_which_down(a.c_codes[vc]);
+        int k_onto = -1;
+        for (int k = 0; k < D + 1; ++k)
+          if (a.cv2v[std::size_t(c) * (D + 1) + k] == onto) k_onto = k;
+        if (k_onto < 0) continue;
+        for (int k = 0; k < D + 1; ++k) {
+          if (k == at) continue;
+          LO f = a.c2s[std::size_t(c) * (D + 1) + opposite_template(D, 0, k)];
+          if (k == k_onto) {
+            veto = veto || a.sdim[f] != a.cdim[c];
+          } else if (D == 3) {
+            int j = local_vertex<2>(a.fv2v + std::size_t(f) * 3, onto);
+            veto = veto || a.edim[a.f2e[std::size_t(f) * 3 + opposite_template(2, 0, j)]] != a.sdim[f];
+          }
+        }
+      }
+      bool unsure = !MIXED;
+      bool over = false;
+      auto length_of = [&](auto const& length, LO ve) {
+        LO e2 = a.e_ab2b[ve];
+        int in = code_which_down(a.e_codes[ve]);
+        LO out = a.ev2v[e2 * 2 + 1 - in];
+        LO p = in == 0 ? onto : out, q = in == 0 ? out : onto;
+        return length(a.coords + std::size_t(p) * D, a.coords + std::size_t(q) * D,
+            a.metric + std::size_t(p) * nc, a.metric + std::size_t(q) * nc);
+      };
+      if constexpr (MIXED) {
+        float lmax = float(a.max_length);
+        for (LO ve = row + lane; ve < end; ve += 64) {
+          if (ve == vw) continue;
+          float l = length_of([](auto... x) { return f32::edge_length<D, M>(x...); }, ve);
+          over = over || l >= lmax * (1.0f + f32::kScreenBand);
+          unsure = unsure || !(l < lmax * (1.0f - f32::kScreenBand));
+        }
+      }
+      veto = __any(veto || over);
+      if (!veto && __any(unsure)) {
+        for (LO ve = row + lane; ve < end && !over; ve += 64)
+          if (ve != vw)
+            over = length_of([](auto... x) { return edge_length<D, M>(x...); }, ve) >=
+                   a.max_length;
+        veto = __any(over);
+      }
+      open = !veto;
+    }
+    if (a.sides_only) {
+      if (lane == 0) a.sides[std::size_t(e) * 2 + eev] = open ? 1 : 0;
+      continue;
+    }
+    if (!open) continue;
+    double const* pp[D + 1];
+    double const* ms[D + 1];
+    auto moved = [&](LO vc) {
+      LO cv[D + 1];
+      if (!moved_cell<D>(a.cv2v, a.c_ab2b[vc], code_which_down(a.c_codes[vc]), onto, cv))
+        return false;
+      for (int k = 0; k < D + 1; ++k) {
+        pp[k] = a.coords + std::size_t(cv[k]) * D;
+        ms[k] = a.metric + std::size_t(cv[k]) * nc;
+      }
+      return true;
+    };
+    if constexpr (MIXED) {
+      double least = 1.0;
+      bool unclear = false;
+      for (LO vc = crow + lane; vc < cend; vc += 64)
+        if (moved(vc)) least = math::min2(least, f32::element_quality<D, M>(pp, ms, &unclear));
+      for (int d = 32; d > 0; d >>= 1) least = math::min2(least, __shfl_xor(least, d, 64));
+      if (!__any(unclear) && least < a.qmin * (1.0 - double(f32::kScreenBand))) continue;
+    }
+    double minq = 1.0;
+    for (LO vc = crow + lane; vc < cend; vc += 64)
+      if (moved(vc)) {
+        double dets[D + 1];
+#pragma unroll
+        for (int k = 0; k < D + 1; ++k) dets[k] = M == 1 ? ms[k][0] : det<M>(get_symm<M>(ms[k]));
+        minq = math::min2(minq, element_quality<D, M>(pp, ms, dets));
+      }
+    for (int d = 32; d > 0; d >>= 1) minq = math::min2(minq, __shfl_xor(minq, d, 64));
+    if (minq >= a.qmin && (!a.old_quals || minq > vold)) rail.visit(e, a.lengths[e], minq);
+  }
+}
+
+// WAVES 1: a wave a star, four stars a workgroup; 4: a workgroup a star, for the
+// stars too large for that; 0: a wave a star of any size, for those that are too
+// large for a workgroup.  `rest`: only the stars that the forms before do not
+// take; stars that do not fit are told by `word`.  One wave a star is the
+// faster form also for few stars (2400: 28 us against 33 with four), since it
+// drops vetoed sides sooner.
+template <int D, int M, bool MIXED, int WAVES>
+__global__ void __launch_bounds__(kBlock, WAVES ? 5 : 1) collapse_stars(StarSweep a, bool rest) {
+  using S = StarData<D, M, (WAVES ? WAVES : 1)>;
+  using Less = StarData<D, M, (WAVES ? 1 : 4)>;
+  constexpr int kStars = kBlock / S::kThreads;
+  int star = int(threadIdx.x) / S::kThreads, t = int(threadIdx.x) % S::kThreads;
+  std::int64_t i = std::int64_t(blockIdx.x) * kStars + star;
+  if (i >= a.nverts) return;
+  LO v = a.verts[i];
+  LO row = a.e_a2ab[v], end = a.e_a2ab[v + 1];
+  LO crow = a.c_a2ab[v], cend = a.c_a2ab[v + 1];
+  if (rest && end - row <= Less::kEdges && cend - crow <= Less::kCells) return;
+  Rail rail;
+  if constexpr (WAVES == 0) {
+    large_star<D, M, MIXED>(a, row, end, crow, cend, t, rail);
   } else {
-    if (s.lane == 0) a.quals[side] = minq;
+    __shared__ S data[kStars];
+    if (end - row > S::kEdges || cend - crow > S::kCells) {
+      if (t == 0)
+        __hip_atomic_store(a.word, a.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return;
+    }
+    small_star<D, M, MIXED, WAVES>(a, row, int(end - row), crow, int(cend - crow), t, data[star],
+        rail);
   }
+  if (a.sides_only || t != 0 || rail.edge < 0) return;
+  a.vcand[v] = 1;
+  a.vqual[v] = rail.qual;
+  a.vrail[v] = rail.edge;
+}
+
+// drops the candidates' directions that a sweep has vetoed
+__global__ void drop_sides(LO n, LO const* cands, I8 const* sides, I8* codes) {
+  LO i = thread_index();
+  if (i >= n) return;
+  LO e = cands[i];
+  I8 code = codes[e];
+  for (int col = 0; col < 2; ++col)
+    if (collapses(code, col) && !sides[std::size_t(e) * 2 + col]) code = dont_collapse(code, col);
+  codes[e] = code;
 }
 
 __global__ void scatter_codes(LO n, LO const* cands, I8 const* cand_codes, I8* codes) {
@@ -369,86 +737,6 @@ __global__ void mark_collapsing_verts(LO ncands, LO const* cands, LO const* ev2v
   I8 code = codes[e];
   for (int col = 0; col < 2; ++col)
     if (collapses(code, col)) vmarks[ev2v[e * 2 + col]] = 1;
-}
-
-// choose_rails (src/Omega_h_collapse_rail.cpp:15-60): each vertex that can
-// collapse takes the shortest of its edges that allow it, the one of higher
-// quality among equally long ones, the first one of those; and the vertex star
-// (verts_across_edges, src/Omega_h_adj.cpp:512-530) of the vertices whose rows
-// are built.  kLanes threads per vertex share its row: a chain of some 14
-// dependent gathers a vertex otherwise (41 us for the two sweeps on the 64^3
-// workload).  A length or quality that is not a number leaves the row to one
-// lane, since the choice then depends on the order of the comparisons.
-struct Rails {
-  LO const* a2ab;
-  LO const* ab2b;
-  I8 const* v2e_codes;
-  I8 const* codes;
-  LO const* ev2v;
-  Real const* lengths;
-  Real const* quals;
-};
-
-__device__ __forceinline__ bool better_rail(double len, double q, double best_len,
-    double best_q) {
-  return len < best_len || (len == best_len && q > best_q);
-}
-
-__global__ void choose_rails_kernel(std::int64_t nt, Rails r, I8* vcand, Real* vqual,
-    LO* vrail, LO* star) {
-  std::int64_t t = thread_index64();
-  if (t >= nt) return;
-  LO v = LO(t / kLanes);
-  int lane = int(t % kLanes);
-  LO b = r.a2ab[v], end = r.a2ab[v + 1];
-  if (b == end) {
-    if (lane == 0) vcand[v] = 0;
-    return;
-  }
-  LO best = -1, at = 0x7fffffff;
-  double best_len = 0.0, best_q = 0.0;
-  bool nan = false;
-  auto visit = [&](LO ve) {
-    LO e = r.ab2b[ve];
-    int eev = code_which_down(r.v2e_codes[ve]);
-    if (!collapses(r.codes[e], eev)) return;
-    double len = r.lengths[e];
-    double q = r.quals[std::size_t(e) * 2 + eev];
-    nan = nan || len != len || q != q;
-    if (best == -1 || better_rail(len, q, best_len, best_q)) {
-      best = e;
-      at = ve;
-      best_len = len;
-      best_q = q;
-    }
-  };
-  for (LO ve = b + lane; ve < end; ve += kLanes) {
-    star[ve] = r.ev2v[r.ab2b[ve] * 2 + (1 - code_which_down(r.v2e_codes[ve]))];
-    visit(ve);
-  }
-  int base = int(threadIdx.x % 64) & ~(kLanes - 1);
-  bool any_nan = ((__ballot(nan) >> base) & ((1ull << kLanes) - 1ull)) != 0ull;
-  if (any_nan) {
-    if (lane != 0) return;
-    best = -1;
-    for (LO ve = b; ve < end; ++ve) visit(ve);
-  } else {
-    for (int d = kLanes / 2; d > 0; d >>= 1) {
-      LO ob = __shfl_xor(best, d, 64), oa = __shfl_xor(at, d, 64);
-      double ol = __shfl_xor(best_len, d, 64), oq = __shfl_xor(best_q, d, 64);
-      bool tie = ol == best_len && oq == best_q;
-      if (ob >= 0 && (best < 0 || better_rail(ol, oq, best_len, best_q) || (tie && oa < at))) {
-        best = ob;
-        at = oa;
-        best_len = ol;
-        best_q = oq;
-      }
-    }
-    if (lane != 0) return;
-  }
-  vcand[v] = best >= 0 ? 1 : 0;
-  vqual[v] = best_q;
-  vrail[v] = best;
 }
 
 // mark_dead_ents (src/Omega_h_coarsen_topology.cpp:15-60): the rails die,
@@ -831,38 +1119,56 @@ Reals metric_dets(Ctx& c, DMesh& m) {
   return d;
 }
 
-// the lanes of each collapse side
-int side_lanes(Ctx& c, LO ncands) {
-  int lanes = c.tuning.coarsen_lanes < kMaxSideLanes ? c.tuning.coarsen_lanes : kMaxSideLanes;
-  return fit_lanes(ncands * 2, lanes);
-}
-
-template <bool FILTER>
-void launch_side_qualities(Ctx& c, DMesh& m, LO ncands, int precision, SideQualities const& a) {
-  int dim = m.dim;
-  int md = (m.metric_ncomps == 1) ? 1 : dim;
-  int lanes = side_lanes(c, ncands);
-  int lshift = lanes_shift(lanes);
-  bool mixed = precision == 1;
-#define OSH_CQ(D, M)                                                                       \
-  do {                                                                                     \
-    if (mixed)                                                                             \
-      OSH_LAUNCH((coarsen_quality_lanes<D, M, true, FILTER>), ncands * 2 * lanes, c, lshift, a); \
-    else                                                                                   \
-      OSH_LAUNCH((coarsen_quality_lanes<D, M, false, FILTER>), ncands * 2 * lanes, c, lshift, a); \
+// a kernel template over dimension, metric dimension and precision
+#define OSH_BY_FORM(LAUNCH, dim, md, mixed) \
+  do {                                      \
+    if (dim == 3 && md == 3 && mixed)       \
+      LAUNCH(3, 3, true);                   \
+    else if (dim == 3 && md == 3)           \
+      LAUNCH(3, 3, false);                  \
+    else if (dim == 3 && mixed)             \
+      LAUNCH(3, 1, true);                   \
+    else if (dim == 3)                      \
+      LAUNCH(3, 1, false);                  \
+    else if (md == 2 && mixed)              \
+      LAUNCH(2, 2, true);                   \
+    else if (md == 2)                       \
+      LAUNCH(2, 2, false);                  \
+    else if (mixed)                         \
+      LAUNCH(2, 1, true);                   \
+    else                                    \
+      LAUNCH(2, 1, false);                  \
   } while (0)
-  if (dim == 3 && md == 3)
-    OSH_CQ(3, 3);
-  else if (dim == 3)
-    OSH_CQ(3, 1);
-  else if (md == 2)
-    OSH_CQ(2, 2);
-  else
-    OSH_CQ(2, 1);
-#undef OSH_CQ
+
+template <int WAVES>
+void launch_stars(Ctx& c, int dim, int md, bool mixed, StarSweep const& a, bool rest) {
+  int waves = WAVES ? WAVES : 1;
+  unsigned blocks = unsigned((std::int64_t(a.nverts) * 64 * waves + kBlock - 1) / kBlock);
+#define OSH_STARS(D, M, X)                                                                     \
+  hipLaunchKernelGGL((collapse_stars<D, M, X, WAVES>), dim3(blocks), dim3(kBlock), 0, c.stream, \
+      a, rest)
+  OSH_BY_FORM(OSH_STARS, dim, md, mixed);
+#undef OSH_STARS
+  OSH_HIP(hipGetLastError());
 }
 
-bool coarsen_verts(Ctx& c, DMesh& m, AdaptOptions const& o, Bytes const& vm,
+// the stars that fit a wave, the others being told by the sweep's word
+void sweep_stars(Ctx& c, int dim, int md, bool mixed, StarSweep const& a) {
+  launch_stars<1>(c, dim, md, mixed, a, false);
+}
+void sweep_large_stars(Ctx& c, int dim, int md, bool mixed, StarSweep const& a) {
+  launch_stars<4>(c, dim, md, mixed, a, true);
+  launch_stars<0>(c, dim, md, mixed, a, true);
+}
+
+// the pass's byte arrays by vertex that start out zero
+struct VertMarks {
+  Bytes wanted;      // collapses of these are tried
+  Bytes collapsing;  // those that have a candidate edge
+  Bytes cand;        // those that have a rail
+};
+
+bool coarsen_verts(Ctx& c, DMesh& m, AdaptOptions const& o, VertMarks& vm,
     bool overshoot_allowed, bool improve) {
   int dim = m.dim;
   LO ne = m.nents[1];
@@ -871,17 +1177,83 @@ bool coarsen_verts(Ctx& c, DMesh& m, AdaptOptions const& o, Bytes const& vm,
   int md = (nc == 1) ? 1 : dim;
   LO const* ev2v = m.down[1].data();
   Bytes codes(c, ne);
-  OSH_LAUNCH(collapse_codes, ne, c, ev2v, vm.data(), m.class_dim[0].data(),
-      m.class_dim[1].data(), codes.data());
-  // the candidate edges: every later sweep runs over this list
-  LOs cands = collect_marked(c, codes);
-  LO ncands = cands.size();
-  if (ncands == 0) return false;
-  Fills fills(c);
-  Bytes vmarks = fills.bytes(nv, 0);
-  Bytes exposed = fills.bytes(2 * ne, 0);
-  fills.run();
-  OSH_LAUNCH(mark_collapsing_verts, ncands, c, cands.data(), ev2v, codes.data(), vmarks.data());
+  OSH_LAUNCH(collapse_codes, ne, c, ev2v, vm.wanted.data(), m.class_dim[0].data(),
+      m.class_dim[1].data(), codes.data(), vm.collapsing.data());
+  LOs verts = collect_marked(c, vm.collapsing);
+  if (verts.size() == 0) return false;
+  // upward rows only where the candidates look: the collapsing vertices' edges
+  // (ordered: the first best rail is kept) and cells (order-free minima)
+  Adj up[2];
+  int const highs[2] = {1, dim};
+  bool const sorted[2] = {true, false};
+  marked_ups(c, m, 0, vm.collapsing, 2, highs, sorted, up);
+  Adj const& v2e = up[0];
+  Adj const& v2c = up[1];
+  Range quality_range(c, "coarsen_qualities");
+  Reals vqual(c, nv);
+  LOs vrail(c, nv);
+  // the independent set reads the star rows of candidate vertices only
+  Adj star;
+  star.a2ab = v2e.a2ab;
+  star.ab2b = LOs(c, v2e.ab2b.size());
+  StarSweep sw{};
+  sw.nverts = verts.size();
+  sw.verts = verts.data();
+  sw.ev2v = ev2v;
+  sw.e_a2ab = v2e.a2ab.data();
+  sw.e_ab2b = v2e.ab2b.data();
+  sw.e_codes = v2e.codes.data();
+  sw.c_a2ab = v2c.a2ab.data();
+  sw.c_ab2b = v2c.ab2b.data();
+  sw.c_codes = v2c.codes.data();
+  sw.cv2v = verts_of(c, m, dim).data();
+  sw.c2s = m.down[dim].data();
+  if (dim == 3) {
+    sw.f2e = m.down[2].data();
+    sw.fv2v = verts_of(c, m, 2).data();
+  }
+  sw.edim = m.class_dim[1].data();
+  sw.sdim = m.class_dim[dim - 1].data();
+  sw.cdim = m.class_dim[dim].data();
+  sw.coords = m.coords.data();
+  sw.metric = m.metric.data();
+  sw.lengths = ask_lengths(c, m).data();
+  sw.old_quals = improve ? ask_qualities(c, m).data() : nullptr;
+  sw.max_length = overshoot_allowed ? o.max_length_allowed : o.max_length_desired;
+  sw.qmin = o.min_quality_allowed;
+  sw.codes = codes.data();
+  sw.vcand = vm.cand.data();
+  sw.vqual = vqual.data();
+  sw.vrail = vrail.data();
+  sw.star = star.ab2b.data();
+  bool mixed = o.precision == 1;
+  sw.word = c.words + kLargeStarWord;
+  sw.tag = c.wait_tag();
+  if (o.should_prevent_coarsen_flip) {
+    // the flip check looks at the edges that the overshoot check leaves
+    LOs cands = collect_marked(c, codes);
+    Bytes sides(c, ne * 2);
+    sw.sides_only = true;
+    sw.sides = sides.data();
+    sweep_stars(c, dim, md, mixed, sw);
+    sweep_large_stars(c, dim, md, mixed, sw);
+    OSH_LAUNCH(drop_sides, cands.size(), c, cands.data(), sides.data(), codes.data());
+    prevent_coarsen_flip(c, m, cands, codes);
+    sw.sides_only = false;
+    sw.checked = true;
+  }
+  sweep_stars(c, dim, md, mixed, sw);
+  quality_range.end();
+  bool any;
+  // waits below bring the word along; a tag lasts until a sweep stores the next
+  unsigned tag = sw.tag;
+  Bytes keys = find_indset(c, m, 0, vqual, vm.cand, &any, nullptr, &star);
+  if (c.word_set(kLargeStarWord, tag)) {
+    sweep_large_stars(c, dim, md, mixed, sw);
+    keys = find_indset(c, m, 0, vqual, vm.cand, &any, nullptr, &star);
+  }
+  if (!any) return false;
+  Range modify_range(c, "modify_ents");
   CellSweep cells{};
   unsigned cell_blocks = 0;
   for (int d = dim; d > 1; --d) {
@@ -891,75 +1263,11 @@ bool coarsen_verts(Ctx& c, DMesh& m, AdaptOptions const& o, Bytes const& vm,
     cells.c2e[w] = ask_down(c, m, d, 1, nullptr).data();
     cells.cv2v[w] = verts_of(c, m, d).data();
     cells.cs2s[w] = m.down[d].data();
-    cells.cdim[w] = m.class_dim[d].data();
-    cells.sdim[w] = m.class_dim[d - 1].data();
     cells.first[w] = cell_blocks;
     cell_blocks += nblocks(m.nents[d]);
     cells.first[w + 1] = cell_blocks;
   }
-  hipLaunchKernelGGL(check_exposure_cells, dim3(cell_blocks), dim3(kBlock), 0, c.stream, cells,
-      ev2v, static_cast<I8 const*>(codes.data()), exposed.data());
-  OSH_HIP(hipGetLastError());
-  // upward rows only where the candidates look: the collapsing vertices' edges
-  // (ordered: the first best rail is kept) and cells (order-free minima)
-  Adj up[2];
-  int const highs[2] = {1, dim};
-  bool const sorted[2] = {true, false};
-  marked_ups(c, m, 0, vmarks, 2, highs, sorted, up);
-  Adj const& v2e = up[0];
-  Adj const& v2c = up[1];
-  Real max_length = overshoot_allowed ? o.max_length_allowed : o.max_length_desired;
-  bool mixed = o.precision == 1;
-  int lanes = side_lanes(c, ncands);
-  int lshift = lanes_shift(lanes);
-  Range overshoot_range(c, "prevent_overshoot");
-#define OSH_OV(D, M, X)                                                                    \
-  OSH_LAUNCH((overshoot_lanes<D, M, X>), ncands * 2 * lanes, c, lshift, cands.data(), ev2v,  \
-      v2e.a2ab.data(), v2e.ab2b.data(), v2e.codes.data(), m.coords.data(), m.metric.data(), \
-      max_length, exposed.data(), codes.data())
-#define OSH_OV_ALL(X)        \
-  if (dim == 3 && md == 3)   \
-    OSH_OV(3, 3, X);         \
-  else if (dim == 3)         \
-    OSH_OV(3, 1, X);         \
-  else if (md == 2)          \
-    OSH_OV(2, 2, X);         \
-  else                       \
-    OSH_OV(2, 1, X)
-  if (mixed) {
-    OSH_OV_ALL(true);
-  } else {
-    OSH_OV_ALL(false);
-  }
-#undef OSH_OV_ALL
-#undef OSH_OV
-  overshoot_range.end();
-  if (o.should_prevent_coarsen_flip) prevent_coarsen_flip(c, m, cands, codes);
-  // sides without a candidate left are skipped by every sweep below
-  Range quality_range(c, "coarsen_qualities");
-  Reals quals(c, ne * 2);  // read where a side is kept
-  LOs const& cv2v = verts_of(c, m, dim);
-  Reals dets = metric_dets(c, m);
-  SideQualities sq{cands.data(), ev2v, cv2v.data(), v2c.a2ab.data(), v2c.ab2b.data(),
-      v2c.codes.data(), m.coords.data(), m.metric.data(), dets.data(), o.min_quality_allowed,
-      improve ? ask_qualities(c, m).data() : (Real const*)nullptr, codes.data(), quals.data()};
-  launch_side_qualities<true>(c, m, ncands, o.precision, sq);
-  quality_range.end();
-  Bytes vcand(c, nv);
-  Reals vqual(c, nv);
-  LOs vrail(c, nv);
-  // the independent set reads the star rows of candidate vertices only
-  Adj star;
-  star.a2ab = v2e.a2ab;
-  star.ab2b = LOs(c, v2e.ab2b.size());
-  Rails rails{v2e.a2ab.data(), v2e.ab2b.data(), v2e.codes.data(), codes.data(), ev2v,
-      ask_lengths(c, m).data(), quals.data()};
-  OSH_LAUNCH64(choose_rails_kernel, std::int64_t(nv) * kLanes, c, rails, vcand.data(), vqual.data(),
-      vrail.data(), star.ab2b.data());
-  bool any;
-  Bytes keys = find_indset(c, m, 0, vqual, vcand, &any, nullptr, &star);
-  if (!any) return false;
-  Range modify_range(c, "modify_ents");
+  Fills fills(c);
   Bytes dead[4];
   dead[1] = fills.bytes(ne, 0);
   for (int d = 2; d <= dim; ++d) dead[d] = fills.bytes(m.nents[d], 0);
@@ -1044,16 +1352,22 @@ bool coarsen_verts(Ctx& c, DMesh& m, AdaptOptions const& o, Bytes const& vm,
 bool coarsen_by_size(Ctx& c, DMesh& m, AdaptOptions const& o) {
   Reals const& lengths = ask_lengths(c, m);
   ask_qualities(c, m);
-  Bytes vm = fill_i8(c, m.nents[0], 0);
+  LO nv = m.nents[0];
+  Fills fills(c);
+  VertMarks vm{fills.bytes(nv, 0), fills.bytes(nv, 0), fills.bytes(nv, 0)};
+  fills.run();
   OSH_LAUNCH(mark_short_edges, m.nents[1], c, lengths.data(), o.min_length_desired,
-      m.down[1].data(), vm.data());
+      m.down[1].data(), vm.wanted.data());
   return coarsen_verts(c, m, o, vm, false, false);
 }
 
 bool coarsen_slivers(Ctx& c, DMesh& m, AdaptOptions const& o) {
   ask_lengths(c, m);
   Bytes marks = mark_sliver_layers(c, m, o.min_quality_desired, o.nsliver_layers);
-  Bytes vm = mark_down(c, m, m.dim, 0, marks);
+  LO nv = m.nents[0];
+  Fills fills(c);
+  VertMarks vm{mark_down(c, m, m.dim, 0, marks), fills.bytes(nv, 0), fills.bytes(nv, 0)};
+  fills.run();
   return coarsen_verts(c, m, o, vm, true, true);
 }
 
@@ -1066,9 +1380,16 @@ void coarsen_qualities(Ctx& c, DMesh& m, LO ncands, LO const* cands, I8 const* c
   OSH_LAUNCH(scatter_codes, ncands, c, cands, cand_codes, codes.data());
   Reals dets = metric_dets(c, m);
   SideQualities sq{cands, m.down[1].data(), cv2v.data(), v2c.a2ab.data(), v2c.ab2b.data(),
-      v2c.codes.data(), m.coords.data(), m.metric.data(), dets.data(), qmin, nullptr,
-      codes.data(), out};
-  launch_side_qualities<false>(c, m, ncands, precision, sq);
+      v2c.codes.data(), m.coords.data(), m.metric.data(), dets.data(), qmin, codes.data(), out};
+  // an edge's two sides share a wave
+  int lanes = c.tuning.coarsen_lanes < kMaxSideLanes ? c.tuning.coarsen_lanes : kMaxSideLanes;
+  lanes = fit_lanes(ncands * 2, lanes);
+  int lshift = lanes_shift(lanes);
+#define OSH_CQ(D, M, X) \
+  OSH_LAUNCH((coarsen_quality_lanes<D, M, X>), ncands * 2 * lanes, c, lshift, sq)
+  int md = (m.metric_ncomps == 1) ? 1 : m.dim;
+  OSH_BY_FORM(OSH_CQ, m.dim, md, precision == 1);
+#undef OSH_CQ
 }
 
 }  // namespace osh
