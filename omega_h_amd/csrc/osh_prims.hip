@@ -219,20 +219,20 @@ constexpr int kScanItems = 16;
 constexpr int kScanTile = kBlock * kScanItems;  // 4096 values per block
 constexpr int kWave = 64;
 
+// both with every lane active: the lane before takes part in the addition itself
+// (row_shr 1, 2, 4, 8, then the last lanes of rows 0 and 2 and of rows 0-1)
 __device__ __forceinline__ LO wave_inclusive_scan(LO v) {
-  int lane = threadIdx.x & (kWave - 1);
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    LO u = __shfl_up(v, d, kWave);
-    if (lane >= d) v += u;
-  }
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
   return v;
 }
 
 __device__ __forceinline__ LO wave_sum(LO v) {
-#pragma unroll
-  for (int d = kWave / 2; d > 0; d >>= 1) v += __shfl_xor(v, d, kWave);
-  return v;
+  return __builtin_amdgcn_readlane(wave_inclusive_scan(v), kWave - 1);
 }
 
 // Block-wide exclusive scan of one value per thread; returns the block total.
@@ -324,24 +324,28 @@ __device__ __forceinline__ LO look_back(unsigned long long* status, unsigned til
 // tiles [first[j], first[j + 1]) of the launch and the same range of status
 // words, so its look-back never leaves its own tiles
 struct ScanBatch {
-  void const* in[kMaxScanJobs];
-  LO* out[kMaxScanJobs];
-  LO* list[kMaxScanJobs];
-  unsigned long long* total[kMaxScanJobs];
-  unsigned tag;
-  LO n[kMaxScanJobs];
-  int kind[kMaxScanJobs];
+  struct Job {
+    void const* in;
+    LO* out;
+    LO* list;
+    unsigned long long* total;
+    LO n;
+    int kind;
+  };
+  // a job's arguments are one load
+  Job job[kMaxScanJobs];
   unsigned first[kMaxScanJobs + 1];
   int count;
+  unsigned tag;
 };
 
 // a grand total goes to its pinned slot as one word with the tag that the host
 // polls for, so that a scan ends its own wait: no order among the totals, and
 // no kernel after the scan, is needed
-__device__ __forceinline__ void put_total(ScanBatch const& b, int job, LO total) {
-  if (b.total[job])
-    __hip_atomic_store(b.total[job],
-        (static_cast<unsigned long long>(b.tag) << 32) | static_cast<unsigned>(total),
+__device__ __forceinline__ void put_total(unsigned long long* slot, unsigned tag, LO total) {
+  if (slot)
+    __hip_atomic_store(slot,
+        (static_cast<unsigned long long>(tag) << 32) | static_cast<unsigned>(total),
         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
@@ -371,11 +375,11 @@ __global__ void __launch_bounds__(kBlock) scan_lookback(ScanBatch b,
   while (job + 1 < b.count && t >= b.first[job + 1]) ++job;
   unsigned tile = t - b.first[job];
   unsigned ntiles = b.first[job + 1] - b.first[job];
-  LO n = b.n[job];
-  int kind = b.kind[job];
-  void const* in = b.in[job];
-  LO* out = b.out[job];
-  LO* list = b.list[job];
+  LO n = b.job[job].n;
+  int kind = b.job[job].kind;
+  void const* in = b.job[job].in;
+  LO* out = b.job[job].out;
+  LO* list = b.job[job].list;
   unsigned long long* st = status + b.first[job];
   LO tile_base = LO(tile) * kScanTile;
 #pragma unroll
@@ -409,7 +413,7 @@ __global__ void __launch_bounds__(kBlock) scan_lookback(ScanBatch b,
             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       s_prefix = prefix;
       if (tile == 0 && out) out[0] = 0;
-      if (tile == ntiles - 1) put_total(b, job, prefix + total);
+      if (tile == ntiles - 1) put_total(b.job[job].total, b.tag, prefix + total);
     }
   }
   __syncthreads();
@@ -433,11 +437,18 @@ __global__ void __launch_bounds__(kBlock) scan_lookback(ScanBatch b,
 // next scans each tile behind the sum of its job's earlier tile sums, which
 // every workgroup adds up for itself.  A look-back has to carry the prefix
 // from workgroup to workgroup across the XCDs, a device-scope round trip at
-// a time: 10 us from two tiles on, 21 us at 542, against 11 us for the two
-// launches.  Jobs of one tile of 4096 or 16384 values need only the second
-// launch (workgroups of 256 and of 1024 threads: the smaller one starts sooner),
-// and in moderate jobs (kOwnTiles) each workgroup adds up the values in front
-// of its tile itself, from L2, which costs less than the first launch.
+// a time: 10 us from two tiles on, 21 us at 542, against 7.4 us for the two
+// launches.  Jobs of one tile of 1024, 4096 or 16384 values need only the second
+// launch, with 256 threads or, for the largest, 1024; in moderate jobs
+// (kOwnTiles) each workgroup adds up the values in front of its tile itself,
+// from L2, which costs less than the first launch.
+//
+// Small scans are bound by the chain of latencies from the arguments to the
+// stores.  A job's arguments are one load, a workgroup of a one-tile job knows
+// its job from its index, the lanes add with DPP moves instead of LDS
+// permutes, and every wave scans the partial sums itself behind one barrier:
+// 2.65 us for up to 1024 values, 3.3 for 4096 and 4.0 for 16384, against 5.7,
+// 5.7 and 6.5 before.
 //
 // A thread takes four consecutive values per round (one 16-byte load, or one
 // 4-byte load of byte values, where the array is so aligned) and writes the
@@ -487,8 +498,7 @@ __device__ __forceinline__ int job_of(ScanBatch const& b, unsigned t) {
 constexpr int kSumBlock = 256;
 constexpr int kSumRounds = 2;
 constexpr int kSumTile = TileScan<kSumBlock, kSumRounds>::kTile;
-constexpr int kSmallRounds = 4;
-constexpr int kSmallTile = TileScan<kSumBlock, kSmallRounds>::kTile;
+constexpr int kLeastTile = TileScan<kSumBlock, 1>::kTile;
 constexpr int kOneBlock = 1024;
 constexpr int kOneRounds = 4;
 constexpr int kOneTile = TileScan<kOneBlock, kOneRounds>::kTile;
@@ -497,23 +507,24 @@ constexpr int kOneTile = TileScan<kOneBlock, kOneRounds>::kTile;
 constexpr unsigned kMaxSumTiles = Ctx::kScanTiles;
 // a workgroup of the one-launch form reads at most this many tiles of 4096
 // values, and all of a launch at most kOwnBytes: at up to 16 tiles it takes 6
-// us against 8.5 us for the two launches and 10 us for the look-back, at 32
+// us against 7.4 us for the two launches and 10 us for the look-back, at 32
 // tiles 10 us
 constexpr int kOwnTile = TileScan<kOneBlock, 1>::kTile;
+static_assert(kOwnTile == TileScan<kSumBlock, 4>::kTile && kOneTile == 4 * kOwnTile, "one tile");
 constexpr unsigned kOwnTiles = 16;
 constexpr double kOwnBytes = 8e6;
 
 __global__ void __launch_bounds__(kSumBlock) sum_tiles(ScanBatch b, LO* sums) {
   unsigned t = blockIdx.x;
   int job = job_of(b, t);
+  ScanBatch::Job a = b.job[job];
   LO base = LO(t - b.first[job]) * kSumTile;
-  bool wide = wide_input(b.in[job], b.kind[job]);
+  bool wide = wide_input(a.in, a.kind);
   LO acc = 0;
 #pragma unroll
   for (int r = 0; r < kSumRounds; ++r) {
     LO v[4];
-    load_four(b.in[job], b.kind[job], base + (r * kSumBlock + LO(threadIdx.x)) * 4, b.n[job],
-        wide, v);
+    load_four(a.in, a.kind, base + (r * kSumBlock + LO(threadIdx.x)) * 4, a.n, wide, v);
     acc += (v[0] + v[1]) + (v[2] + v[3]);
   }
   __shared__ LO part[kSumBlock / kWave];
@@ -527,40 +538,46 @@ __global__ void __launch_bounds__(kSumBlock) sum_tiles(ScanBatch b, LO* sums) {
   }
 }
 
-// with OWN each workgroup sums its job's earlier values instead of reading
-// their tile sums
-template <int BLOCK, int ROUNDS, bool OWN>
+// How a workgroup knows what lies in front of its tile: kOnly, nothing does,
+// every job being one tile; kSums, from the tile sums; kOwn, by adding up its
+// job's earlier values itself.
+enum ScanBefore { kOnly, kSums, kOwn };
+
+template <int BLOCK, int ROUNDS, ScanBefore BEFORE>
 __global__ void __launch_bounds__(BLOCK) scan_tiles(ScanBatch b, LO const* sums) {
   using T = TileScan<BLOCK, ROUNDS>;
   __shared__ LO part[T::kParts];
   __shared__ LO before[T::kWaves];
   unsigned t = blockIdx.x;
-  int job = job_of(b, t);
-  unsigned tile = t - b.first[job];
-  unsigned ntiles = b.first[job + 1] - b.first[job];
-  LO n = b.n[job];
+  int job = BEFORE == kOnly ? int(t) : job_of(b, t);
+  ScanBatch::Job a = b.job[job];
+  unsigned tile = BEFORE == kOnly ? 0u : t - b.first[job];
+  bool last = BEFORE == kOnly || t + 1 == b.first[job + 1];
+  LO n = a.n;
   int lane = int(threadIdx.x) & (kWave - 1);
   int wave = int(threadIdx.x) / kWave;
   LO base = LO(tile) * T::kTile;
-  bool wide = wide_input(b.in[job], b.kind[job]);
+  bool wide = wide_input(a.in, a.kind);
   LO v[ROUNDS][4];
 #pragma unroll
   for (int r = 0; r < ROUNDS; ++r)
-    load_four(b.in[job], b.kind[job], base + (r * BLOCK + LO(threadIdx.x)) * 4, n, wide, v[r]);
-  LO earlier = 0;
-  if constexpr (OWN) {
-    // whole tiles, all in range
+    load_four(a.in, a.kind, base + (r * BLOCK + LO(threadIdx.x)) * 4, n, wide, v[r]);
+  if constexpr (BEFORE != kOnly) {
+    LO earlier = 0;
+    if constexpr (BEFORE == kOwn) {
+      // whole tiles, all in range
 #pragma unroll 4
-    for (LO i = LO(threadIdx.x) * 4; i < base; i += BLOCK * 4) {
-      LO u[4];
-      load_four(b.in[job], b.kind[job], i, n, wide, u);
-      earlier += (u[0] + u[1]) + (u[2] + u[3]);
+      for (LO i = LO(threadIdx.x) * 4; i < base; i += BLOCK * 4) {
+        LO u[4];
+        load_four(a.in, a.kind, i, n, wide, u);
+        earlier += (u[0] + u[1]) + (u[2] + u[3]);
+      }
+    } else {
+      for (unsigned j = threadIdx.x; j < tile; j += BLOCK) earlier += sums[b.first[job] + j];
     }
-  } else {
-    for (unsigned j = threadIdx.x; j < tile; j += BLOCK) earlier += sums[b.first[job] + j];
+    if (tile) earlier = wave_sum(earlier);
+    if (lane == 0) before[wave] = earlier;
   }
-  if (tile) earlier = wave_sum(earlier);
-  if (lane == 0) before[wave] = earlier;
   LO inc[ROUNDS];
 #pragma unroll
   for (int r = 0; r < ROUNDS; ++r) {
@@ -568,40 +585,41 @@ __global__ void __launch_bounds__(BLOCK) scan_tiles(ScanBatch b, LO const* sums)
     if (lane == kWave - 1) part[r * T::kWaves + wave] = inc[r];
   }
   __syncthreads();
-  if (wave == 0) {
-    LO p = lane < T::kParts ? part[lane] : 0;
-    LO s = lane < T::kWaves ? before[lane] : 0;
-    LO prefix = wave_sum(s);
-    LO i = wave_inclusive_scan(p);
-    if (lane < T::kParts) part[lane] = prefix + i - p;
-    if (lane == kWave - 1 && tile == ntiles - 1) {
-      if (b.out[job]) b.out[job][n] = prefix + i;
-      put_total(b, job, prefix + i);
-    }
+  // every wave scans the partial sums for itself
+  LO p = lane < T::kParts ? part[lane] : 0;
+  LO i = wave_inclusive_scan(p);
+  LO prefix = 0;
+  if constexpr (BEFORE != kOnly) prefix = wave_sum(lane < T::kWaves ? before[lane] : 0);
+  LO total = prefix + __builtin_amdgcn_readlane(i, kWave - 1);
+  if (last && threadIdx.x == 0) {
+    if (a.out) a.out[n] = total;
+    put_total(a.total, b.tag, total);
   }
-  __syncthreads();
-  LO* out = b.out[job];
+  i += prefix - p;
+  LO* out = a.out;
+  LO* list = a.list;
   bool wide_out = (reinterpret_cast<std::uintptr_t>(out) & 15u) == 0;
 #pragma unroll
   for (int r = 0; r < ROUNDS; ++r) {
-    LO i = base + (r * BLOCK + LO(threadIdx.x)) * 4;
-    LO o0 = part[r * T::kWaves + wave] + inc[r] - ((v[r][0] + v[r][1]) + (v[r][2] + v[r][3]));
+    LO at = base + (r * BLOCK + LO(threadIdx.x)) * 4;
+    LO o0 = __builtin_amdgcn_readlane(i, __builtin_amdgcn_readfirstlane(r * T::kWaves + wave)) +
+            inc[r] - ((v[r][0] + v[r][1]) + (v[r][2] + v[r][3]));
     LO o1 = o0 + v[r][0], o2 = o1 + v[r][1], o3 = o2 + v[r][2];
-    if (LO* list = b.list[job]) {
+    if (list) {
       // values past the end are 0
-      if (v[r][0]) list[o0] = i;
-      if (v[r][1]) list[o1] = i + 1;
-      if (v[r][2]) list[o2] = i + 2;
-      if (v[r][3]) list[o3] = i + 3;
+      if (v[r][0]) list[o0] = at;
+      if (v[r][1]) list[o1] = at + 1;
+      if (v[r][2]) list[o2] = at + 2;
+      if (v[r][3]) list[o3] = at + 3;
     }
     if (!out) continue;
-    if (wide_out && i + 4 <= n) {
-      *reinterpret_cast<int4*>(out + i) = make_int4(o0, o1, o2, o3);
+    if (wide_out && at + 4 <= n) {
+      *reinterpret_cast<int4*>(out + at) = make_int4(o0, o1, o2, o3);
     } else {
-      if (i < n) out[i] = o0;
-      if (i + 1 < n) out[i + 1] = o1;
-      if (i + 2 < n) out[i + 2] = o2;
-      if (i + 3 < n) out[i + 3] = o3;
+      if (at < n) out[at] = o0;
+      if (at + 1 < n) out[at + 1] = o1;
+      if (at + 2 < n) out[at + 2] = o2;
+      if (at + 3 < n) out[at + 3] = o3;
     }
   }
 }
@@ -645,14 +663,9 @@ unsigned batch_jobs(ScanJob const* jobs, int njobs, int tile, ScanBatch& b, unsi
   *most = 0;
   for (int j = 0; j < njobs; ++j) {
     OSH_CHECK(jobs[j].n >= 0 && (jobs[j].out || jobs[j].list), "offset_scans: bad job");
-    b.in[j] = jobs[j].in;
-    b.out[j] = jobs[j].out;
-    b.list[j] = jobs[j].list;
-    b.total[j] = jobs[j].total;
+    b.job[j] = {jobs[j].in, jobs[j].out, jobs[j].list, jobs[j].total, jobs[j].n, jobs[j].kind};
     // a value of another kind left in the slot could look like the coming tag
     if (jobs[j].total) __atomic_store_n(jobs[j].total, 0ull, __ATOMIC_RELAXED);
-    b.n[j] = jobs[j].n;
-    b.kind[j] = jobs[j].kind;
     b.first[j] = tiles;
     // an empty job still takes one tile, which writes its 0 and its total
     unsigned nt = jobs[j].n == 0 ? 1u : unsigned((std::int64_t(jobs[j].n) + tile - 1) / tile);
@@ -671,21 +684,26 @@ void offset_scans(Ctx& c, ScanJob const* jobs, int njobs) {
   ScanBatch b{};
   b.tag = c.wait_tag();
   unsigned most = 0;
-  unsigned tiles = batch_jobs(jobs, njobs, kSmallTile, b, &most);
+  unsigned tiles = batch_jobs(jobs, njobs, kOwnTile, b, &most);
   if (most <= 1) {
-    hipLaunchKernelGGL((scan_tiles<kSumBlock, kSmallRounds, false>), dim3(tiles),
-        dim3(kSumBlock), 0, c.stream, b, (LO const*)nullptr);
+    LO n = 0;
+    for (int j = 0; j < njobs; ++j) n = jobs[j].n > n ? jobs[j].n : n;
+    if (n <= kLeastTile)
+      hipLaunchKernelGGL((scan_tiles<kSumBlock, 1, kOnly>), dim3(tiles), dim3(kSumBlock), 0,
+          c.stream, b, (LO const*)nullptr);
+    else
+      hipLaunchKernelGGL((scan_tiles<kSumBlock, 4, kOnly>), dim3(tiles), dim3(kSumBlock), 0,
+          c.stream, b, (LO const*)nullptr);
     OSH_HIP(hipGetLastError());
     return;
   }
-  tiles = batch_jobs(jobs, njobs, kOneTile, b, &most);
-  if (most <= 1) {
-    hipLaunchKernelGGL((scan_tiles<kOneBlock, kOneRounds, false>), dim3(tiles), dim3(kOneBlock),
+  if (most <= 4) {
+    tiles = batch_jobs(jobs, njobs, kOneTile, b, &most);
+    hipLaunchKernelGGL((scan_tiles<kOneBlock, kOneRounds, kOnly>), dim3(tiles), dim3(kOneBlock),
         0, c.stream, b, (LO const*)nullptr);
     OSH_HIP(hipGetLastError());
     return;
   }
-  tiles = batch_jobs(jobs, njobs, kOwnTile, b, &most);
   if (most <= kOwnTiles) {
     double read = 0.0;
     for (int j = 0; j < njobs; ++j) {
@@ -693,7 +711,7 @@ void offset_scans(Ctx& c, ScanJob const* jobs, int njobs) {
       read += 0.5 * nt * nt * kOwnTile * (jobs[j].kind == kScanLO ? 4.0 : 1.0);
     }
     if (read <= kOwnBytes) {
-      hipLaunchKernelGGL((scan_tiles<kOneBlock, 1, true>), dim3(tiles), dim3(kOneBlock), 0,
+      hipLaunchKernelGGL((scan_tiles<kOneBlock, 1, kOwn>), dim3(tiles), dim3(kOneBlock), 0,
           c.stream, b, (LO const*)nullptr);
       OSH_HIP(hipGetLastError());
       return;
@@ -704,7 +722,7 @@ void offset_scans(Ctx& c, ScanJob const* jobs, int njobs) {
     LO* sums = c.tile_sums;
     hipLaunchKernelGGL(sum_tiles, dim3(tiles), dim3(kSumBlock), 0, c.stream, b, sums);
     OSH_HIP(hipGetLastError());
-    hipLaunchKernelGGL((scan_tiles<kSumBlock, kSumRounds, false>), dim3(tiles), dim3(kSumBlock), 0,
+    hipLaunchKernelGGL((scan_tiles<kSumBlock, kSumRounds, kSums>), dim3(tiles), dim3(kSumBlock), 0,
         c.stream, b, static_cast<LO const*>(sums));
     OSH_HIP(hipGetLastError());
     return;
@@ -753,11 +771,7 @@ void offset_scans_noalloc(Ctx& c, ScanJob const* jobs, int njobs) {
   bool multi = false;
   for (int j = 0; j < njobs; ++j) {
     OSH_CHECK(jobs[j].n >= 0 && jobs[j].out, "offset_scans: bad job");
-    b.in[j] = jobs[j].in;
-    b.out[j] = jobs[j].out;
-    b.total[j] = jobs[j].total;
-    b.n[j] = jobs[j].n;
-    b.kind[j] = jobs[j].kind;
+    b.job[j] = {jobs[j].in, jobs[j].out, nullptr, jobs[j].total, jobs[j].n, jobs[j].kind};
     b.first[j] = unsigned(tiles);
     std::int64_t nt = jobs[j].n == 0 ? 1 : (std::int64_t(jobs[j].n) + kScanTile - 1) / kScanTile;
     multi = multi || nt > 1;

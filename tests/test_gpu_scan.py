@@ -41,10 +41,10 @@ def test_single_scan(ctx, n):
     assert np.array_equal(got, expected(a)), n
 
 
-@pytest.mark.parametrize("n", [16383, 16384, 16385, 20479, 20480, 16 * 4096,
+@pytest.mark.parametrize("n", [1023, 1024, 1025, 16383, 16384, 16385, 20479, 20480, 16 * 4096,
                                16 * 4096 + 1, 8192 * 2048, 8192 * 2048 + 1])
 def test_sizes_at_the_edges_of_tiles_and_launch_forms(ctx, n):
-    """One 16384-value tile, the 4096-value tiles of the one-launch form and
+    """One tile of 1024, 4096 or 16384 values, the 4096-value tiles of the one-launch form and
     its largest job, and the largest job of the two-launch form."""
     a = np.random.default_rng(n).integers(0, 8, size=n, dtype=np.int32)
     (got,) = run_scans(ctx, [a])
