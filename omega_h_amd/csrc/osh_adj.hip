@@ -21,6 +21,7 @@ int simplex_degree(int from_dim, int to_dim) {
 }
 
 void DMesh::clear_caches() {
+  linked = false;
   for (int d = 0; d < 4; ++d) {
     verts[d] = LOs();
     for (int e = 0; e < 4; ++e) up[d][e] = Adj();

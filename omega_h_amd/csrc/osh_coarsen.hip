@@ -1169,7 +1169,7 @@ struct VertMarks {
 };
 
 bool coarsen_verts(Ctx& c, DMesh& m, AdaptOptions const& o, VertMarks& vm,
-    bool overshoot_allowed, bool improve) {
+    bool overshoot_allowed, bool improve, SliverLayers* layers = nullptr) {
   int dim = m.dim;
   LO ne = m.nents[1];
   LO nv = m.nents[0];
@@ -1252,6 +1252,7 @@ bool coarsen_verts(Ctx& c, DMesh& m, AdaptOptions const& o, VertMarks& vm,
     sweep_large_stars(c, dim, md, mixed, sw);
     keys = find_indset(c, m, 0, vqual, vm.cand, &any, nullptr, &star);
   }
+  if (layers) layers->settle();
   if (!any) return false;
   Range modify_range(c, "modify_ents");
   CellSweep cells{};
@@ -1363,12 +1364,13 @@ bool coarsen_by_size(Ctx& c, DMesh& m, AdaptOptions const& o) {
 
 bool coarsen_slivers(Ctx& c, DMesh& m, AdaptOptions const& o) {
   ask_lengths(c, m);
-  Bytes marks = mark_sliver_layers(c, m, o.min_quality_desired, o.nsliver_layers);
   LO nv = m.nents[0];
   Fills fills(c);
-  VertMarks vm{mark_down(c, m, m.dim, 0, marks), fills.bytes(nv, 0), fills.bytes(nv, 0)};
+  SliverLayers layers(c, m, o.nsliver_layers, fills);
+  VertMarks vm{Bytes(), fills.bytes(nv, 0), fills.bytes(nv, 0)};
   fills.run();
-  return coarsen_verts(c, m, o, vm, true, true);
+  vm.wanted = mark_down(c, m, m.dim, 0, layers.mark(o.min_quality_desired));
+  return coarsen_verts(c, m, o, vm, true, true, &layers);
 }
 
 void coarsen_qualities(Ctx& c, DMesh& m, LO ncands, LO const* cands, I8 const* cand_codes,

@@ -110,6 +110,9 @@ struct DMesh {
   // side_elems[s]: the number of elements on side s (high 32 bits) and the
   // sum of their indices (low 32 bits)
   DArray<unsigned long long> side_elems;
+  // known to hold: no side has more than two elements, and every element has
+  // another across one of its sides
+  bool linked = false;
   Adj dual;    // element -> elements across sides (on demand, for callers)
   Reals size;  // element sizes (on demand)
   void clear_caches();

@@ -619,11 +619,45 @@ __device__ __forceinline__ I8 dual_max_at(LO e, LO const* es2s,
 }
 
 __global__ void dual_max_kernel(LO n, int nspe, LO const* es2s,
-    unsigned long long const* side_elems, Real const* q, Real ceil, I8* out, int* error) {
+    unsigned long long const* side_elems, Real const* q, Real ceil, I8* out, unsigned* word,
+    unsigned tag, int* error) {
   LO e = thread_index();
   if (e >= n) return;
-  out[e] = nspe == 4 ? dual_max_at<4>(e, es2s, side_elems, q, ceil, error)
-                     : dual_max_at<3>(e, es2s, side_elems, q, ceil, error);
+  I8 r = nspe == 4 ? dual_max_at<4>(e, es2s, side_elems, q, ceil, error)
+                   : dual_max_at<3>(e, es2s, side_elems, q, ceil, error);
+  out[e] = r;
+  tell(r < 0, word, tag);
+}
+
+// The same in a mesh known to be linked (DMesh::linked), without the per-side
+// words, whose 660,000 atomics took 18 of a pass's 34 us for four layers at
+// 165,000 tets: the few elements of a layer count themselves at their sides,
+// and an element is in the next layer when one of its sides has a count that
+// is not its own.  A side's counts are two bits a layer of one word.
+constexpr int kCountedLayers = 16;
+constexpr int kUnlinkedWord = 3;  // the sets and the star sweeps use the others
+
+template <int NSPE>
+__global__ void sliver_layer(LO n, int layer, int nlayers, LO const* es2s, Real const* q,
+    Real ceil, unsigned* counts, I8* marks) {
+  LO e = thread_index();
+  if (e >= n) return;
+  LO sides[NSPE];
+#pragma unroll
+  for (int j = 0; j < NSPE; ++j) sides[j] = es2s[std::size_t(e) * NSPE + j];
+  bool in = false;
+  if (layer == 0) {
+    in = q[e] < ceil;
+  } else {
+    unsigned own = marks[e] != 0;
+#pragma unroll
+    for (int j = 0; j < NSPE; ++j)
+      in = in || ((counts[sides[j]] >> (2 * (layer - 1))) & 3u) > own;
+  }
+  marks[e] = in;
+  if (!in || layer == nlayers) return;
+#pragma unroll
+  for (int j = 0; j < NSPE; ++j) atomicAdd(&counts[sides[j]], 1u << (2 * layer));
 }
 
 // a later layer, pushed from the marked elements (the first one's output has
@@ -1043,38 +1077,60 @@ Bytes mark_down(Ctx& c, DMesh& m, int high, int low, Bytes const& marks) {
   return out;
 }
 
-Bytes mark_sliver_layers(Ctx& c, DMesh& m, Real qual_ceil, int nlayers) {
+SliverLayers::SliverLayers(Ctx& c, DMesh& m, int nlayers, Fills& fills)
+    : c_(c), m_(m), nlayers_(nlayers) {
+  if (m.linked && nlayers > 0 && nlayers <= kCountedLayers)
+    counts_ = fills.ints(m.nents[m.dim - 1], 0);
+}
+
+Bytes SliverLayers::mark(Real qual_ceil) {
+  Ctx& c = c_;
+  DMesh& m = m_;
   LO ne = m.nents[m.dim];
   Reals const& q = ask_qualities(c, m);
-  Bytes marks;
-  if (nlayers == 0) {
-    marks = Bytes(c, ne);
+  Bytes marks(c, ne);
+  if (nlayers_ == 0) {
     OSH_LAUNCH(below_kernel, ne, c, q.data(), qual_ceil, marks.data());
+    return marks;
+  }
+  LO const* es2s = m.down[m.dim].data();
+  if (counts_.exists()) {
+    unsigned* counts = reinterpret_cast<unsigned*>(counts_.data());
+    for (int k = 0; k <= nlayers_; ++k) {
+      if (m.dim == 3)
+        OSH_LAUNCH(sliver_layer<4>, ne, c, k, nlayers_, es2s, q.data(), qual_ceil, counts,
+            marks.data());
+      else
+        OSH_LAUNCH(sliver_layer<3>, ne, c, k, nlayers_, es2s, q.data(), qual_ceil, counts,
+            marks.data());
+    }
     return marks;
   }
   auto const& se = ask_side_elems(c, m);
   // the first layer reads the sliver test itself; later ones push, into
   // buffers cleared eight at a time
-  marks = Bytes(c, ne);
-  OSH_LAUNCH(dual_max_kernel, ne, c, m.dim + 1, m.down[m.dim].data(), se.data(), q.data(),
-      qual_ceil, marks.data(), c.error_word());
+  tag_ = c.wait_tag();
+  OSH_LAUNCH(dual_max_kernel, ne, c, m.dim + 1, es2s, se.data(), q.data(), qual_ceil,
+      marks.data(), c.words + kUnlinkedWord, tag_, c.error_word());
   Bytes next[8];
-  for (int i = 1; i < nlayers; ++i) {
+  for (int i = 1; i < nlayers_; ++i) {
     int b = (i - 1) % 8;
     if (b == 0) {
       Fills fills(c);
-      for (int k = 0; k < 8 && i + k < nlayers; ++k) next[k] = fills.bytes(ne, 0);
+      for (int k = 0; k < 8 && i + k < nlayers_; ++k) next[k] = fills.bytes(ne, 0);
       fills.run();
     }
     if (m.dim == 3)
-      OSH_LAUNCH(push_layer_kernel<4>, ne, c, m.down[3].data(), se.data(), marks.data(),
-          next[b].data());
+      OSH_LAUNCH(push_layer_kernel<4>, ne, c, es2s, se.data(), marks.data(), next[b].data());
     else
-      OSH_LAUNCH(push_layer_kernel<3>, ne, c, m.down[2].data(), se.data(), marks.data(),
-          next[b].data());
+      OSH_LAUNCH(push_layer_kernel<3>, ne, c, es2s, se.data(), marks.data(), next[b].data());
     marks = next[b];
   }
   return marks;
+}
+
+void SliverLayers::settle() {
+  if (tag_) m_.linked = !c_.word_set(kUnlinkedWord, tag_);
 }
 
 void default_options(int dim, AdaptOptions& o) {

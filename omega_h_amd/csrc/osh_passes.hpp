@@ -153,7 +153,23 @@ void conserve_correct(Ctx& c, DMesh& m, int max_sweeps);
 Bytes find_indset(Ctx& c, DMesh& m, int d, Reals const& quality, Bytes const& cands,
     bool* any_cands = nullptr, Adj const* edge_elems = nullptr, Adj const* star = nullptr);
 Bytes mark_down(Ctx& c, DMesh& m, int high, int low, Bytes const& marks);
-Bytes mark_sliver_layers(Ctx& c, DMesh& m, Real qual_ceil, int nlayers);
+// mark_sliver_layers: the arrays that start out constant go into `fills`, which
+// has to run before mark()
+class SliverLayers {
+ public:
+  SliverLayers(Ctx& c, DMesh& m, int nlayers, Fills& fills);
+  Bytes mark(Real qual_ceil);
+  // after a find_indset that follows mark(): records what it has found out
+  // about the mesh (DMesh::linked)
+  void settle();
+
+ private:
+  Ctx& c_;
+  DMesh& m_;
+  int nlayers_;
+  LOs counts_;
+  unsigned tag_ = 0;
+};
 LOs degrees_of(Ctx& c, LOs const& a2ab, LOs const& rows);
 
 bool refine_by_size(Ctx& c, DMesh& m, AdaptOptions const& o);

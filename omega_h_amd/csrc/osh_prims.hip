@@ -922,10 +922,10 @@ namespace {
 
 struct FillJobs {
   int n;
-  unsigned first[17];
-  void* p[16];
-  std::size_t bytes[16];
-  unsigned pattern[16];
+  unsigned first[25];
+  void* p[24];
+  std::size_t bytes[24];
+  unsigned pattern[24];
 };
 
 // 16 bytes a thread; blocks come from the pool, so every start is aligned and

@@ -327,6 +327,7 @@ bool refine_by_size(Ctx& c, DMesh& m, AdaptOptions const& o) {
   int nc = m.metric_ncomps;
   DMesh nw;
   nw.dim = dim;
+  nw.linked = m.linked;
   nw.metric_ncomps = nc;
   RefineRows rows{};
   KeyedMods km;

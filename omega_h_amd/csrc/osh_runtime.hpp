@@ -429,7 +429,7 @@ class Fills {
   void run();
 
  private:
-  static constexpr int kMax = 16;
+  static constexpr int kMax = 24;
   void add(void* p, std::size_t bytes, unsigned pattern);
   Ctx& c_;
   int n_ = 0;

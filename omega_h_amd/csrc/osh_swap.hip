@@ -845,6 +845,7 @@ void swap_rebuild(Ctx& c, DMesh& m, LOs const& keys2edges, LOs const* k2p, LO co
   int dim = m.dim;
   DMesh nw;
   nw.dim = dim;
+  nw.linked = m.linked;
   nw.metric_ncomps = m.metric_ncomps;
   nw.nents[0] = m.nents[0];
   nw.coords = m.coords;
@@ -962,9 +963,9 @@ void swap3d_evaluate(Ctx& c, DMesh& m, AdaptOptions const& o, Rings const& rings
 bool swap_edges_3d(Ctx& c, DMesh& m, AdaptOptions const& o, SwapCache* cache) {
   ask_lengths(c, m);
   LO ne = m.nents[1], nf = m.nents[2], nt = m.nents[3];
-  Bytes elems = mark_sliver_layers(c, m, o.min_quality_desired, o.nsliver_layers);
   // every array of the pass that starts out constant, in one launch
   Fills fills(c);
+  SliverLayers layers(c, m, o.nsliver_layers, fills);
   Bytes marks = fills.bytes(ne, 0);
   LOs ring_counts = fills.ints(ne, 0);
   Bytes keep = fills.bytes(ne, 0);
@@ -987,6 +988,7 @@ bool swap_edges_3d(Ctx& c, DMesh& m, AdaptOptions const& o, SwapCache* cache) {
     cache->q = Reals(c, ne);
   }
   fills.run();
+  Bytes elems = layers.mark(o.min_quality_desired);
   LOs const& t2e = ask_down(c, m, 3, 1, nullptr);
   OSH_LAUNCH(mark_interior_edges, nt, c, 6, t2e.data(), elems.data(), 3,
       m.class_dim[1].data(), marks.data());
@@ -1013,6 +1015,7 @@ bool swap_edges_3d(Ctx& c, DMesh& m, AdaptOptions const& o, SwapCache* cache) {
                 dom.data(), w);
         });
   }
+  layers.settle();
   if (!any) return false;
   Range modify_range(c, "modify_ents");
   // the plans from the keys, then one scan launch and one wait for the keys,
@@ -1078,11 +1081,12 @@ bool swap_edges_3d(Ctx& c, DMesh& m, AdaptOptions const& o, SwapCache* cache) {
 bool swap_edges_2d(Ctx& c, DMesh& m, AdaptOptions const& o) {
   ask_lengths(c, m);
   LO ne = m.nents[1];
-  Bytes elems = mark_sliver_layers(c, m, o.min_quality_desired, o.nsliver_layers);
   Fills fills(c);
+  SliverLayers layers(c, m, o.nsliver_layers, fills);
   Bytes cand = fills.bytes(ne, 0);
   Bytes keep = fills.bytes(ne, 0);
   fills.run();
+  Bytes elems = layers.mark(o.min_quality_desired);
   Reals quals(c, ne);  // read where an edge is kept
   OSH_LAUNCH(mark_interior_edges, m.nents[2], c, 3, m.down[2].data(), elems.data(), 2,
       m.class_dim[1].data(), cand.data());
@@ -1104,6 +1108,7 @@ bool swap_edges_2d(Ctx& c, DMesh& m, AdaptOptions const& o) {
   quality_range.end();
   bool any;
   Bytes keys = find_indset(c, m, 1, quals, keep, &any);
+  layers.settle();
   if (!any) return false;
   Range modify_range(c, "modify_ents");
   KeyedMods km;
