@@ -196,16 +196,21 @@ struct Invert {
   bool sorted;
 };
 
-void invert_adjs(Ctx& c, int n, Invert const* in, Adj* out) {
+void invert_adjs(Ctx& c, int n, Invert const* in, Adj* out, LOs const* zeros = nullptr) {
   OSH_CHECK(n >= 1 && n <= kMaxUseJobs, "invert_adjs: too many maps");
   UseJobs j{};
-  LOs counts[kMaxUseJobs], slot[kMaxUseJobs], ab2hl[kMaxUseJobs];
+  LOs slot[kMaxUseJobs], ab2hl[kMaxUseJobs];
   ScanJob scans[kMaxUseJobs];
-  Fills fills(c);
+  LOs counts = zeros ? *zeros : LOs();
+  if (!zeros) {
+    LO total = 0;
+    for (int w = 0; w < n; ++w) total += in[w].nlow;
+    counts = fill_lo(c, total, 0);
+  }
+  LO* count = counts.data();
   unsigned blocks = 0;
   for (int w = 0; w < n; ++w) {
     LO nhl = in[w].nhigh * in[w].deg;
-    counts[w] = fills.ints(in[w].nlow, 0);
     slot[w] = LOs(c, nhl);
     out[w].a2ab = LOs(c, in[w].nlow + 1);
     // with marks the rows hold at most nhl uses; the size stays an upper bound
@@ -213,16 +218,16 @@ void invert_adjs(Ctx& c, int n, Invert const* in, Adj* out) {
     out[w].codes = Bytes(c, nhl);
     if (in[w].sorted) ab2hl[w] = LOs(c, nhl);
     j.d[w] = UseJob{nhl, in[w].hl2l.data(), in[w].marks ? in[w].marks->data() : nullptr,
-        counts[w].data(), slot[w].data(), out[w].a2ab.data(), in[w].deg,
+        count, slot[w].data(), out[w].a2ab.data(), in[w].deg,
         in[w].down_codes ? in[w].down_codes->data() : nullptr, in[w].sorted ? 1 : 0,
         in[w].sorted ? ab2hl[w].data() : nullptr, out[w].ab2b.data(), out[w].codes.data()};
-    scans[w] = {counts[w].data(), kScanLO, in[w].nlow, out[w].a2ab.data(), nullptr};
+    scans[w] = {count, kScanLO, in[w].nlow, out[w].a2ab.data(), nullptr};
+    count += in[w].nlow;
     j.first[w] = blocks;
     blocks += nblocks(nhl);
     j.first[w + 1] = blocks;
   }
   j.n = n;
-  fills.run();
   auto launch = [&](auto kernel, UseJobs const& jobs, unsigned nb) {
     if (nb == 0) return;
     hipLaunchKernelGGL(kernel, dim3(nb), dim3(kBlock), 0, c.stream, jobs);
@@ -543,7 +548,7 @@ LOs const& ask_down(Ctx& c, DMesh& m, int high, int low, Bytes const** codes) {
 }
 
 void marked_ups(Ctx& c, DMesh& m, int low, Bytes const& marks, int n, int const* highs,
-    bool const* sorted, Adj* out) {
+    bool const* sorted, Adj* out, LOs const* zeros) {
   Invert in[kMaxUseJobs];
   OSH_CHECK(n <= kMaxUseJobs, "marked_ups: too many dimensions");
   for (int w = 0; w < n; ++w) {
@@ -556,7 +561,8 @@ void marked_ups(Ctx& c, DMesh& m, int low, Bytes const& marks, int n, int const*
     in[w].marks = &marks;
     in[w].sorted = sorted[w];
   }
-  invert_adjs(c, n, in, out);
+  OSH_CHECK(!zeros || zeros->size() >= n * m.nents[low], "marked_ups: too few zeros");
+  invert_adjs(c, n, in, out, zeros);
 }
 
 Adj const& ask_up(Ctx& c, DMesh& m, int low, int high) {
@@ -584,9 +590,10 @@ unsigned side_blocks(SideJobs& j, std::int64_t const* n) {
   return b;
 }
 
-void run_sides(Ctx& c, DMesh& m, SideJobs& j) {
+void run_sides(Ctx& c, DMesh& m, SideJobs& j, LOs const* zeros = nullptr) {
   LO nv = m.nents[0];
-  LOs counts = fill_lo(c, nv * j.n, 0);
+  bool enough = zeros && zeros->size() >= nv * j.n;
+  LOs counts = enough ? *zeros : fill_lo(c, nv * j.n, 0);
   LOs slot[2], a2ab[2];
   DArray<int4> rows[2];
   ScanJob scans[2];
@@ -641,7 +648,8 @@ void reflect_down(Ctx& c, DMesh& m, int high_dim, LO nprods, LOs const& prod_ver
   run_sides(c, m, j);
 }
 
-void match_sides(Ctx& c, DMesh& nw, Products const* prods, ModOut const* mo) {
+void match_sides(Ctx& c, DMesh& nw, Products const* prods, ModOut const* mo,
+    LOs const* zeros) {
   SideJobs j{};
   for (int d = 2; d <= nw.dim; ++d) {
     if (prods[d].n == 0) continue;
@@ -655,7 +663,7 @@ void match_sides(Ctx& c, DMesh& nw, Products const* prods, ModOut const* mo) {
     a.out = nw.down[d].data();
     a.codes = nw.down_codes[d].data();
   }
-  if (j.n) run_sides(c, nw, j);
+  if (j.n) run_sides(c, nw, j, zeros);
 }
 
 Adj const& ask_star(Ctx& c, DMesh& m, int d) {

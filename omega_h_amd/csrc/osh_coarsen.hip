@@ -1161,14 +1161,45 @@ void sweep_large_stars(Ctx& c, int dim, int md, bool mixed, StarSweep const& a) 
   launch_stars<0>(c, dim, md, mixed, a, true);
 }
 
-// the pass's byte arrays by vertex that start out zero
-struct VertMarks {
+// Up to this many cells the collapsing vertices' rows of all dimensions are
+// built at once, in order; beyond, the faces' (and ordered cells') rows are
+// built for the chosen keys alone.  The five launches of the second inversion
+// take some 25 us; for all candidates it adds about 10 us at 30,000 cells.
+constexpr LO kJointCells = 32768;
+
+// the pass's arrays that start out constant, in one launch for the attempt and
+// another for the rebuild, or all in the first in small meshes
+struct CoarsenArrays {
+  bool joint;
+  // by vertex
   Bytes wanted;      // collapses of these are tried
   Bytes collapsing;  // those that have a candidate edge
   Bytes cand;        // those that have a rail
+  LOs up_zeros, key_up_zeros, side_zeros;
+  // by entity
+  Bytes dead[4];
+  Bytes rail_col;
+  KeyedMods km;
+
+  CoarsenArrays(DMesh const& m, Fills& fills, bool with_wanted) {
+    joint = m.nents[m.dim] <= kJointCells;
+    LO nv = m.nents[0];
+    if (with_wanted) wanted = fills.bytes(nv, 0);
+    collapsing = fills.bytes(nv, 0);
+    cand = fills.bytes(nv, 0);
+    up_zeros = fills.ints(nv * (joint ? m.dim : 2), 0);
+    if (joint) add_rebuild(m, fills);
+  }
+  void add_rebuild(DMesh const& m, Fills& fills) {
+    for (int d = 1; d <= m.dim; ++d) dead[d] = fills.bytes(m.nents[d], 0);
+    rail_col = fills.bytes(m.nents[1], -1);
+    prepare_keys(m, 0, 0, m.dim, fills, km);
+    if (!joint) key_up_zeros = fills.ints(m.nents[0] * (m.dim - 1), 0);
+    side_zeros = fills.ints(m.nents[0] * (m.dim - 1), 0);
+  }
 };
 
-bool coarsen_verts(Ctx& c, DMesh& m, AdaptOptions const& o, VertMarks& vm,
+bool coarsen_verts(Ctx& c, DMesh& m, AdaptOptions const& o, CoarsenArrays& vm,
     bool overshoot_allowed, bool improve, SliverLayers* layers = nullptr) {
   int dim = m.dim;
   LO ne = m.nents[1];
@@ -1183,12 +1214,21 @@ bool coarsen_verts(Ctx& c, DMesh& m, AdaptOptions const& o, VertMarks& vm,
   if (verts.size() == 0) return false;
   // upward rows only where the candidates look: the collapsing vertices' edges
   // (ordered: the first best rail is kept) and cells (order-free minima)
-  Adj up[2];
-  int const highs[2] = {1, dim};
-  bool const sorted[2] = {true, false};
-  marked_ups(c, m, 0, vm.collapsing, 2, highs, sorted, up);
-  Adj const& v2e = up[0];
-  Adj const& v2c = up[1];
+  Adj v2d[4];
+  if (vm.joint) {
+    int const highs[3] = {1, 2, 3};
+    bool const sorted[3] = {true, true, true};
+    marked_ups(c, m, 0, vm.collapsing, dim, highs, sorted, v2d + 1, &vm.up_zeros);
+  } else {
+    Adj up[2];
+    int const highs[2] = {1, dim};
+    bool const sorted[2] = {true, false};
+    marked_ups(c, m, 0, vm.collapsing, 2, highs, sorted, up, &vm.up_zeros);
+    v2d[1] = up[0];
+    v2d[dim] = up[1];
+  }
+  Adj const v2e = v2d[1];
+  Adj const v2c = v2d[dim];
   Range quality_range(c, "coarsen_qualities");
   Reals vqual(c, nv);
   LOs vrail(c, nv);
@@ -1268,31 +1308,29 @@ bool coarsen_verts(Ctx& c, DMesh& m, AdaptOptions const& o, VertMarks& vm,
     cell_blocks += nblocks(m.nents[d]);
     cells.first[w + 1] = cell_blocks;
   }
-  Fills fills(c);
-  Bytes dead[4];
-  dead[1] = fills.bytes(ne, 0);
-  for (int d = 2; d <= dim; ++d) dead[d] = fills.bytes(m.nents[d], 0);
-  Bytes rail_col = fills.bytes(ne, -1);
-  fills.run();
+  if (!vm.joint) {
+    Fills fills(c);
+    vm.add_rebuild(m, fills);
+    fills.run();
+  }
+  Bytes const* dead = vm.dead;
   LOs onto(c, nv);
-  OSH_LAUNCH(mark_rails, nv, c, keys.data(), vrail.data(), ev2v, dead[1].data(),
-      rail_col.data(), onto.data());
+  OSH_LAUNCH(mark_rails, nv, c, keys.data(), vrail.data(), ev2v, vm.dead[1].data(),
+      vm.rail_col.data(), onto.data());
   for (int w = 0; w < cells.n; ++w) {
-    cells.dead_cells[w] = dead[cells.dim[w]].data();
-    cells.dead_sides[w] = dead[cells.dim[w] - 1].data();
+    cells.dead_cells[w] = vm.dead[cells.dim[w]].data();
+    cells.dead_sides[w] = vm.dead[cells.dim[w] - 1].data();
   }
   hipLaunchKernelGGL(mark_dead_cells, dim3(cell_blocks), dim3(kBlock), 0, c.stream, cells, ev2v,
-      static_cast<I8 const*>(rail_col.data()));
+      static_cast<I8 const*>(vm.rail_col.data()));
   OSH_HIP(hipGetLastError());
   // the keys' rows of every dimension, in order: products follow them
-  Adj v2d[4];
-  v2d[1] = v2e;
-  {
+  if (!vm.joint) {
     int const hs[2] = {2, 3};
     bool const in_order[2] = {true, true};
-    marked_ups(c, m, 0, keys, dim - 1, hs, in_order, v2d + 2);
+    marked_ups(c, m, 0, keys, dim - 1, hs, in_order, v2d + 2, &vm.key_up_zeros);
   }
-  KeyedMods km;  // no key vertex has a product vertex
+  KeyedMods& km = vm.km;  // no key vertex has a product vertex
   LiveRows live{};
   live.n = dim;
   for (int d = 1; d <= dim; ++d) {
@@ -1335,7 +1373,7 @@ bool coarsen_verts(Ctx& c, DMesh& m, AdaptOptions const& o, VertMarks& vm,
   OSH_LAUNCH64(coarsen_products, std::int64_t(nkeys) * dim * kLanes, c, nkeys, keys2verts.data(), onto.data(),
       plans[0].offsets.data(), rows);
   place_products(c, m, nw, 1, dim, 0, plans, keys2verts, prods, mo);
-  match_sides(c, nw, prods, mo);
+  match_sides(c, nw, prods, mo, &vm.side_zeros);
   measure_products(c, nw, mo);
   for (auto const& t : m.vtags)
     nw.vtags.push_back(t.with_data(transfer<Real>(c, mo[0], t.ncomps, t.data, nullptr)));
@@ -1353,9 +1391,8 @@ bool coarsen_verts(Ctx& c, DMesh& m, AdaptOptions const& o, VertMarks& vm,
 bool coarsen_by_size(Ctx& c, DMesh& m, AdaptOptions const& o) {
   Reals const& lengths = ask_lengths(c, m);
   ask_qualities(c, m);
-  LO nv = m.nents[0];
   Fills fills(c);
-  VertMarks vm{fills.bytes(nv, 0), fills.bytes(nv, 0), fills.bytes(nv, 0)};
+  CoarsenArrays vm(m, fills, true);
   fills.run();
   OSH_LAUNCH(mark_short_edges, m.nents[1], c, lengths.data(), o.min_length_desired,
       m.down[1].data(), vm.wanted.data());
@@ -1364,10 +1401,9 @@ bool coarsen_by_size(Ctx& c, DMesh& m, AdaptOptions const& o) {
 
 bool coarsen_slivers(Ctx& c, DMesh& m, AdaptOptions const& o) {
   ask_lengths(c, m);
-  LO nv = m.nents[0];
   Fills fills(c);
   SliverLayers layers(c, m, o.nsliver_layers, fills);
-  VertMarks vm{Bytes(), fills.bytes(nv, 0), fills.bytes(nv, 0)};
+  CoarsenArrays vm(m, fills, false);
   fills.run();
   vm.wanted = mark_down(c, m, m.dim, 0, layers.mark(o.min_quality_desired));
   return coarsen_verts(c, m, o, vm, true, true, &layers);

@@ -128,8 +128,9 @@ Adj const& ask_up(Ctx& c, DMesh& m, int low, int high);
 // three by the same launches; not cached.  Without sorted[w], a row's order is
 // arbitrary, which suits uses that do not depend on it (counts, any/all
 // tests, min/max)
+// `zeros` (when given): n * nents[low] zeros, to be used up
 void marked_ups(Ctx& c, DMesh& m, int low, Bytes const& marks, int n, int const* highs,
-    bool const* sorted, Adj* out);
+    bool const* sorted, Adj* out, LOs const* zeros = nullptr);
 Adj const& ask_star(Ctx& c, DMesh& m, int d);
 DArray<unsigned long long> const& ask_side_elems(Ctx& c, DMesh& m);
 // Mesh::ask_dual (src/Omega_h_mesh.cpp:260): elements_across_sides

@@ -699,13 +699,23 @@ LOs degrees_of(Ctx& c, LOs const& a2ab, LOs const& rows) {
   return out;
 }
 
+void prepare_keys(DMesh const& old, int key_dim, int d0, int d1, Fills& fills, KeyedMods& out) {
+  for (int d = d0; d <= d1; ++d) {
+    if (d < key_dim) {
+      out.plans[d - d0].counts = fills.ints(old.nents[d], 1);
+      out.head = fills.ints(old.nents[d], -1);
+    } else if (d > key_dim) {
+      out.first_up[d] = fills.ints(old.nents[key_dim], 0x7fffffff);
+    }
+  }
+}
+
 void plan_keys(Ctx& c, DMesh& old, int key_dim, int d0, int d1, Bytes const& keys,
     KeyedMods& out) {
   LO nkd = old.nents[key_dim];
   int nd = d1 - d0 + 1;
   OSH_CHECK(nd >= 1 && nd <= 4 && key_dim - d0 <= 1 && key_dim >= d0, "plan_keys: dimensions");
-  Fills fills(c);
-  LOs first_up[4], head, next;
+  LOs next;
   SameMarks sm{};
   RepCounts rc{};
   KeyList kl{};
@@ -722,13 +732,11 @@ void plan_keys(Ctx& c, DMesh& old, int key_dim, int d0, int d1, Bytes const& key
     if (d < key_dim) {
       // every entity stays; without a `same` array all are the same
       OSH_CHECK(!prods, "plan_keys: a fixed count below the keys");
-      plan.counts = fills.ints(plan.nold, 1);
-      head = fills.ints(plan.nold, -1);
       next = LOs(c, nkd);
       out.order = LOs(c, nkd);
       kl.deg[w] = simplex_degree(key_dim, d);
       kl.down[w] = ask_down(c, old, key_dim, d, nullptr).data();
-      kl.head = rc.head = head.data();
+      kl.head = rc.head = out.head.data();
       rc.next = next.data();
       kl.next = next.data();
       kl.order = out.order.data();
@@ -746,11 +754,10 @@ void plan_keys(Ctx& c, DMesh& old, int key_dim, int d0, int d1, Bytes const& key
         sm.key_prods = prods;
         sm.fixed_key_prods = out.fixed_prods[d];
       } else {
-        first_up[d] = fills.ints(nkd, 0x7fffffff);
         sm.deg[v] = simplex_degree(d, key_dim);
         sm.lows[v] = ask_down(c, old, d, key_dim, nullptr).data();
-        sm.first_up[v] = first_up[d].data();
-        kl.first_up[w] = first_up[d].data();
+        sm.first_up[v] = out.first_up[d].data();
+        kl.first_up[w] = out.first_up[d].data();
       }
       ++sm.n;
     }
@@ -764,7 +771,6 @@ void plan_keys(Ctx& c, DMesh& old, int key_dim, int d0, int d1, Bytes const& key
       rc.counts[r] = plan.counts.data();
     }
   }
-  fills.run();
   hipLaunchKernelGGL(mark_same_kernel, dim3(blocks), dim3(kBlock), 0, c.stream, keys.data(), sm);
   OSH_HIP(hipGetLastError());
   if (rc.n) OSH_LAUNCH(rep_counts_kernel, nkd, c, keys.data(), rc, c.error_word());

@@ -66,7 +66,12 @@ struct KeyedMods {
   LO nprods[4] = {0, 0, 0, 0};
   ModPlan plans[4];  // plans[d - d0]
   LOs order;         // of the dimension below the keys, by key-dimension entity
+  LOs head;          // by entity of the dimension below the keys
+  LOs first_up[4];   // by key-dimension entity
 };
+// allocates what plan_keys needs to start out constant; `fills` has to run
+// before it
+void prepare_keys(DMesh const& old, int key_dim, int d0, int d1, Fills& fills, KeyedMods& out);
 // the plans of dimensions d0..d1 from the keys, a mask over the key dimension,
 // with one wait for everything that depends on the keys
 void plan_keys(Ctx& c, DMesh& old, int key_dim, int d0, int d1, Bytes const& keys,
@@ -111,8 +116,11 @@ void place_products(Ctx& c, DMesh& old, DMesh& nw, int d0, int d1, int plan0,
     ModPlan const* plans, LOs const& keys2kds, Products const* prods, ModOut* mo,
     LOs const* order = nullptr, I8* new_edges_valid = nullptr);
 // the sides and codes of the placed products of dimensions 2..dim, by their
-// vertices among the new mesh's entities (reflect_down)
-void match_sides(Ctx& c, DMesh& nw, Products const* prods, ModOut const* mo);
+// vertices among the new mesh's entities (reflect_down); `zeros` (when given
+// and long enough): a zero per vertex of the new mesh and such dimension, to be
+// used up
+void match_sides(Ctx& c, DMesh& nw, Products const* prods, ModOut const* mo,
+    LOs const* zeros = nullptr);
 // lengths of new edges and qualities of new elements, in one launch
 void measure_products(Ctx& c, DMesh& nw, ModOut const* mo);
 // every tag of a rebuilt mesh but the vertex tags' and refinement's own
@@ -202,10 +210,6 @@ void swap3d_choices(Ctx& c, DMesh& m, AdaptOptions const& o, LOs const& edges,
 
 // known-answer hooks used by the tests
 Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands);
-// the same over an edge -> element adjacency with at least the candidates'
-// rows, also handing over the midpoints' metrics
-Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands, Adj const& e2c,
-    Reals* midpoint_metrics);
 // coarsen_qualities (src/Omega_h_coarsen_qualities.cpp:65-88) on device
 // arrays, stream-ordered: out[2 i + col] is the quality after collapsing
 // candidate i's edge in direction col (-1 where cand_codes[i] does not

@@ -20,6 +20,13 @@ __global__ void gt_kernel(LO n, Real const* a, Real v, I8* out) {
   if (i < n) out[i] = a[i] > v;
 }
 
+// by edge: whether a candidate's quality reaches qmin, and the quality
+struct RefineSeeds {
+  Real qmin = 0.0;
+  I8* keep = nullptr;
+  Real* quals = nullptr;
+};
+
 // 2^lshift lanes per candidate edge (consecutive threads of one wave): the
 // lanes share the 2 x (elements around the edge) children, each measured
 // with the max-determinant metric of its cell-side vertices and the edge
@@ -30,7 +37,7 @@ template <int D, int M>
 __global__ void __launch_bounds__(kBlock) refine_qualities_kernel(LO nt, int lshift,
     LO ncands, LO const* cands, LO const* ev2v, LO const* cv2v, LO const* e2c_a2ab,
     LO const* e2c_ab2b, I8 const* e2c_codes, Real const* coords, Real const* metric,
-    Real const* midpt_metrics, Real* out) {
+    Real const* midpt_metrics, Real* out, RefineSeeds seeds) {
   LO t = thread_index();
   int lanes = 1 << lshift;
   LO cand = t >> lshift;
@@ -89,15 +96,12 @@ __global__ void __launch_bounds__(kBlock) refine_qualities_kernel(LO nt, int lsh
     }
   }
   for (int d = lanes / 2; d > 0; d /= 2) minqual = math::min2(minqual, __shfl_xor(minqual, d, 64));
-  if (valid && lane == 0) out[cand] = minqual;
-}
-
-__global__ void seed_keys(LO ncands, LO const* cands, Real const* quals, Real qmin,
-    I8* initial, Real* edge_quals) {
-  LO c = thread_index();
-  if (c >= ncands) return;
-  initial[cands[c]] = quals[c] >= qmin;
-  edge_quals[cands[c]] = quals[c];
+  if (!valid || lane != 0) return;
+  if (out) out[cand] = minqual;
+  if (seeds.keep) {
+    seeds.keep[e] = minqual >= seeds.qmin;
+    seeds.quals[e] = minqual;
+  }
 }
 
 // the rows that refinement products of dimensions 1..3 come from: pairs (the
@@ -260,23 +264,18 @@ __global__ void midpoint_coords(LO nkeys, int dim, LO const* keys2edges, LO cons
   }
 }
 
-}  // namespace
-
-Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands) {
-  return refine_qualities(c, m, cands, ask_up(c, m, 1, m.dim), nullptr);
-}
-
+// the qualities of splitting the candidates over an edge -> element adjacency
+// with at least their rows: to `out` (when given), and to `seeds` (when set);
+// returns the midpoints' metrics
 Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands, Adj const& e2c,
-    Reals* midpoint_metrics) {
+    RefineSeeds const& seeds, Real* out) {
   Range range(c, "refine_qualities");
   LO n = cands.size();
   int dim = m.dim;
   int nc = m.metric_ncomps;
   int md = (nc == 1) ? 1 : dim;
   Reals mm(c, n * nc);
-  if (midpoint_metrics) *midpoint_metrics = mm;
   mident_metrics(c, m, n, cands.data(), mm.data());
-  Reals out(c, n);
   LOs const& cv2v = verts_of(c, m, dim);
   // lanes share a candidate's children, as the coarsen sweeps share a side's
   int lanes = fit_lanes(n, c.tuning.coarsen_lanes);
@@ -284,7 +283,7 @@ Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands, Adj const& e2c,
 #define OSH_RQ(D, M)                                                                    \
   OSH_LAUNCH((refine_qualities_kernel<D, M>), n * lanes, c, lshift, n, cands.data(),       \
       m.down[1].data(), cv2v.data(), e2c.a2ab.data(), e2c.ab2b.data(), e2c.codes.data(),    \
-      m.coords.data(), m.metric.data(), mm.data(), out.data())
+      m.coords.data(), m.metric.data(), mm.data(), out, seeds)
   if (dim == 3 && md == 3)
     OSH_RQ(3, 3);
   else if (dim == 3)
@@ -294,6 +293,14 @@ Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands, Adj const& e2c,
   else
     OSH_RQ(2, 1);
 #undef OSH_RQ
+  return mm;
+}
+
+}  // namespace
+
+Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands) {
+  Reals out(c, cands.size());
+  refine_qualities(c, m, cands, ask_up(c, m, 1, m.dim), RefineSeeds{}, out.data());
   return out;
 }
 
@@ -312,14 +319,20 @@ bool refine_by_size(Ctx& c, DMesh& m, AdaptOptions const& o) {
   Adj up[2];
   int const highs[2] = {2, 3};
   bool const sorted[2] = {true, true};
-  marked_ups(c, m, 1, cand, dim - 1, highs, sorted, up);
+  // every array of the pass that starts out constant, in one launch
+  Fills fills(c);
+  KeyedMods km;
+  km.fixed_prods[0] = 1;
+  prepare_keys(m, 1, 0, dim, fills, km);
+  LOs up_zeros = fills.ints((dim - 1) * ne, 0);
+  LOs side_zeros = fills.ints((dim - 1) * (m.nents[0] + cands.size()), 0);
+  Bytes initial = fills.bytes(ne, 0);
+  fills.run();
+  marked_ups(c, m, 1, cand, dim - 1, highs, sorted, up, &up_zeros);
   Adj const& e2c = up[dim - 2];
-  Reals cand_metrics;
-  Reals quals = refine_qualities(c, m, cands, e2c, &cand_metrics);
-  Bytes initial = fill_i8(c, ne, 0);
   Reals edge_quals(c, ne);  // read where an edge is a candidate
-  OSH_LAUNCH(seed_keys, cands.size(), c, cands.data(), quals.data(), o.min_quality_allowed,
-      initial.data(), edge_quals.data());
+  RefineSeeds seeds{o.min_quality_allowed, initial.data(), edge_quals.data()};
+  Reals cand_metrics = refine_qualities(c, m, cands, e2c, seeds, nullptr);
   bool any;
   Bytes keys = find_indset(c, m, 1, edge_quals, initial, &any, &e2c);
   if (!any) return false;
@@ -330,8 +343,6 @@ bool refine_by_size(Ctx& c, DMesh& m, AdaptOptions const& o) {
   nw.linked = m.linked;
   nw.metric_ncomps = nc;
   RefineRows rows{};
-  KeyedMods km;
-  km.fixed_prods[0] = 1;
   for (int d = 1; d <= dim; ++d) {
     if (d > 1) {
       Adj const& pr = up[d - 2];
@@ -386,7 +397,7 @@ bool refine_by_size(Ctx& c, DMesh& m, AdaptOptions const& o) {
   OSH_LAUNCH64(refine_products, std::int64_t(nkeys) * dim * kRowLanes, c, nkeys, keys2edges.data(), keys2mid,
       m.down[1].data(), plans[0].offsets.data(), rows);
   place_products(c, m, nw, 1, dim, 0, plans, keys2edges, prods, mo);
-  match_sides(c, nw, prods, mo);
+  match_sides(c, nw, prods, mo, &side_zeros);
   measure_products(c, nw, mo);
   for (auto const& t : m.vtags) {
     Reals pt(c, nkeys * t.ncomps);

@@ -841,7 +841,7 @@ Tables const* device_tables(Ctx& c) {
 void swap_rebuild(Ctx& c, DMesh& m, LOs const& keys2edges, LOs const* k2p, LO const* nprods,
     LOs const* pv, ModPlan const* plans, SwapCache* cache = nullptr,
     Bytes const* dirty = nullptr, EdgeRings const* rings = nullptr,
-    LOs const* prod_keys = nullptr) {
+    LOs const* prod_keys = nullptr, LOs const* side_zeros = nullptr) {
   int dim = m.dim;
   DMesh nw;
   nw.dim = dim;
@@ -897,7 +897,7 @@ void swap_rebuild(Ctx& c, DMesh& m, LOs const& keys2edges, LOs const* k2p, LO co
       OSH_HIP(hipGetLastError());
     }
   } else {
-    match_sides(c, nw, prods, mo);
+    match_sides(c, nw, prods, mo, side_zeros);
   }
   measure_products(c, nw, mo);
   transfer_pointwise(c, m, nw, mo[dim], 1, keys2edges, k2p[dim], pv[dim]);
@@ -1085,6 +1085,11 @@ bool swap_edges_2d(Ctx& c, DMesh& m, AdaptOptions const& o) {
   SliverLayers layers(c, m, o.nsliver_layers, fills);
   Bytes cand = fills.bytes(ne, 0);
   Bytes keep = fills.bytes(ne, 0);
+  KeyedMods km;
+  km.fixed_prods[1] = 1;
+  km.fixed_prods[2] = 2;
+  prepare_keys(m, 1, 1, 2, fills, km);
+  LOs side_zeros = fills.ints(m.nents[0], 0);
   fills.run();
   Bytes elems = layers.mark(o.min_quality_desired);
   Reals quals(c, ne);  // read where an edge is kept
@@ -1111,9 +1116,6 @@ bool swap_edges_2d(Ctx& c, DMesh& m, AdaptOptions const& o) {
   layers.settle();
   if (!any) return false;
   Range modify_range(c, "modify_ents");
-  KeyedMods km;
-  km.fixed_prods[1] = 1;
-  km.fixed_prods[2] = 2;
   plan_keys(c, m, 1, 1, 2, keys, km);
   note_changed_parts(c, m, 1, km.keys2kds);
   if (o.verbosity >= 2) std::printf("swapping %d 2D edges\n", int(km.nkeys));
@@ -1123,7 +1125,8 @@ bool swap_edges_2d(Ctx& c, DMesh& m, AdaptOptions const& o) {
   OSH_LAUNCH(swap2d_products, km.nkeys, c, km.keys2kds.data(), e2t.a2ab.data(),
       e2t.ab2b.data(), e2t.codes.data(), m.down[1].data(), tv2v.data(), pv[1].data(),
       pv[2].data());
-  swap_rebuild(c, m, km.keys2kds, km.k2p, km.nprods, pv, km.plans);
+  swap_rebuild(c, m, km.keys2kds, km.k2p, km.nprods, pv, km.plans, nullptr, nullptr, nullptr,
+      nullptr, &side_zeros);
   return true;
 }
 
