@@ -84,8 +84,39 @@ double now() {
       .count();
 }
 
-// *qmin receives the minimum element quality after the pass, whose reduction is
-// also the pass's closing wait
+// the reductions for pre_adapt: least and largest length, least quality
+void goal_jobs(Ctx& c, DMesh& m, ReduceJob* jobs) {
+  Reals const& l = ask_lengths(c, m);
+  Reals const& q = ask_qualities(c, m);
+  jobs[0] = {l.data(), l.size(), 1, false};
+  jobs[1] = {l.data(), l.size(), 1, true};
+  jobs[2] = {q.data(), q.size(), 1, false};
+}
+void goal_extremes(Ctx& c, DMesh& m, Real* goals) {
+  ReduceJob jobs[3];
+  goal_jobs(c, m, jobs);
+  reduce_reals(c, jobs, 3, goals);
+}
+
+// those of the meshes whose least quality is below `desired`
+std::vector<int> below_quality(Ctx& c, std::vector<DMesh>& meshes, std::vector<int> const& ids,
+    Real desired) {
+  std::vector<ReduceJob> jobs;
+  for (int i : ids) {
+    Reals const& q = ask_qualities(c, meshes[std::size_t(i)]);
+    jobs.push_back({q.data(), q.size(), 1, false});
+  }
+  std::vector<Real> least(jobs.size());
+  reduce_reals(c, jobs.data(), int(jobs.size()), least.data());
+  std::vector<int> low;
+  for (std::size_t k = 0; k < ids.size(); ++k)
+    if (least[k] < desired) low.push_back(ids[k]);
+  return low;
+}
+
+// *qmin (when given) receives the minimum element quality after a pass that
+// changed the mesh, whose reduction is also the pass's closing wait; one that
+// did not has waited for what it looked at
 // the most passes one adapt() records: a guard on the log, far above real
 // runs (the reference's loops have no limit; one 1.3M-tet box of the serving
 // workload under a constant anisotropic metric takes 4,639 swap and 283
@@ -99,7 +130,6 @@ bool run_pass(Ctx& c, DMesh& m, AdaptOptions const& o, int kind,
   static char const* const kPassNames[4] = {"refine_by_size", "coarsen_by_size", "swap_edges",
       "coarsen_slivers"};
   LO nin = m.nents[m.dim];
-  c.sync();
   Range range(c, kPassNames[kind]);
   double t0 = now();
   bool r;
@@ -111,7 +141,10 @@ bool run_pass(Ctx& c, DMesh& m, AdaptOptions const& o, int kind,
     r = swap_edges(c, m, o, cache);
   else
     r = coarsen_slivers(c, m, o);
-  *qmin = min_real_wait(c, ask_qualities(c, m));
+  if (r && qmin)
+    *qmin = min_real_wait(c, ask_qualities(c, m));
+  else if (r)
+    c.wait();
   double t1 = now();
   range.end();
   if (r && log) log->push_back({kind, nin, m.nents[m.dim], t1 - t0});
@@ -140,9 +173,9 @@ bool adapt(Ctx& c, DMesh& m, AdaptOptions const& o, std::vector<PassRecord>* log
   Range pre_range(c, "pre_adapt");
   if (o.verbosity >= 1) std::printf("before adapting:\n");
   print_status(c, m, o);
-  Reals const& l = ask_lengths(c, m);
-  Real lmin = min_real(c, l), lmax = max_real(c, l);
-  Real qmin = min_real(c, ask_qualities(c, m));
+  Real goals[3];
+  goal_extremes(c, m, goals);
+  Real lmin = goals[0], lmax = goals[1], qmin = goals[2];
   if (qmin >= o.min_quality_desired && lmin >= o.min_length_desired &&
       lmax <= o.max_length_desired)
     return false;
@@ -153,12 +186,15 @@ bool adapt(Ctx& c, DMesh& m, AdaptOptions const& o, std::vector<PassRecord>* log
   double t1 = now();
   bool did;
   Real q = qmin;  // the minimum quality of the current mesh
+  bool changed = false;
   Range lengths_range(c, "satisfy_lengths");
   do {
     did = false;
-    if (o.should_refine && run_pass(c, m, o, 0, log, &q, hook)) did = true;
-    if (o.should_coarsen && run_pass(c, m, o, 1, log, &q, hook)) did = true;
+    if (o.should_refine && run_pass(c, m, o, 0, log, nullptr, hook)) did = true;
+    if (o.should_coarsen && run_pass(c, m, o, 1, log, nullptr, hook)) did = true;
+    changed = changed || did;
   } while (did);
+  if (changed) q = min_real(c, ask_qualities(c, m));
   lengths_range.end();
   double t2 = now();
   Range quality_range(c, "satisfy_quality");
@@ -256,15 +292,14 @@ void batch_lengths(Ctx& c, std::vector<DMesh>& meshes, std::vector<int> active,
     int np = int(active.size());
     DMesh joined = joined_of(c, meshes, active);
     PartFlags pf(c, np);
-    Real q = 0.0;
     std::vector<char> frozen;
     bool finished = false;
     for (;;) {
       bool did = false;
       if (o.should_refine)
-        did = run_pass(c, joined, o, 0, log, &q, nullptr) || did;
+        did = run_pass(c, joined, o, 0, log, nullptr, nullptr) || did;
       if (o.should_coarsen)
-        did = run_pass(c, joined, o, 1, log, &q, nullptr) || did;
+        did = run_pass(c, joined, o, 1, log, nullptr, nullptr) || did;
       if (!did) {
         finished = true;
         break;
@@ -334,16 +369,12 @@ void batch_quality(Ctx& c, std::vector<DMesh>& meshes, std::vector<int> group,
       if (out.empty()) finished = true;
       put_back(c, joined, meshes, active);
       if (finished) break;
-      std::vector<int> next;
-      for (int k = 0; k < np; ++k) {
-        int id = active[std::size_t(k)];
-        if (!out[std::size_t(k)]) {
-          next.push_back(id);
-        } else if (min_real(c, ask_qualities(c, meshes[std::size_t(id)])) <
-                   o.min_quality_desired) {
-          stalled.push_back(id);  // its next pass is a sliver pass
-        }
-      }
+      std::vector<int> next, set_aside;
+      for (int k = 0; k < np; ++k)
+        (out[std::size_t(k)] ? set_aside : next).push_back(active[std::size_t(k)]);
+      // the next pass of those below the goal is a sliver pass
+      for (int id : below_quality(c, meshes, set_aside, o.min_quality_desired))
+        stalled.push_back(id);
       active = next;
     }
     if (!stalled.empty()) groups.push_back(stalled);
@@ -363,14 +394,21 @@ std::vector<int> adapt_batch(Ctx& c, std::vector<DMesh>& meshes, AdaptOptions co
   Range pre_range(c, "pre_adapt");
   std::vector<int> did(std::size_t(n), 0);
   std::vector<int> todo;
+  std::vector<ReduceJob> jobs;
   for (int i = 0; i < n; ++i) {
     DMesh& m = meshes[std::size_t(i)];
     OSH_CHECK(m.etags.empty() && m.itags.empty(),
         "batched adapt: meshes with element or inheritance tags");
+    ReduceJob j[3];
+    goal_jobs(c, m, j);
+    jobs.insert(jobs.end(), j, j + 3);
+  }
+  std::vector<Real> goals(jobs.size());
+  reduce_reals(c, jobs.data(), int(jobs.size()), goals.data());
+  for (int i = 0; i < n; ++i) {
     // pre_adapt (src/Omega_h_adapt.cpp:153-167) per mesh
-    Reals const& l = ask_lengths(c, m);
-    Real lmin = min_real(c, l), lmax = max_real(c, l);
-    Real qmin = min_real(c, ask_qualities(c, m));
+    Real const* g = goals.data() + 3 * std::size_t(i);
+    Real lmin = g[0], lmax = g[1], qmin = g[2];
     if (qmin >= o.min_quality_desired && lmin >= o.min_length_desired &&
         lmax <= o.max_length_desired)
       continue;
@@ -381,10 +419,7 @@ std::vector<int> adapt_batch(Ctx& c, std::vector<DMesh>& meshes, AdaptOptions co
   AdaptOptions quiet = o;
   quiet.verbosity = 0;
   batch_lengths(c, meshes, todo, quiet, log);
-  std::vector<int> low;
-  for (int i : todo)
-    if (min_real(c, ask_qualities(c, meshes[std::size_t(i)])) < o.min_quality_desired)
-      low.push_back(i);
+  std::vector<int> low = below_quality(c, meshes, todo, o.min_quality_desired);
   batch_quality(c, meshes, low, quiet, log);
   return did;
 }

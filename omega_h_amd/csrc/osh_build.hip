@@ -200,11 +200,6 @@ __global__ void hilbert_keys(LO nv, Real const* coords, Real const* s, Real cons
   for (int j = 0; j < D; ++j) keys[I64(v) * D + j] = I64(Y[j]);
 }
 
-__global__ void coord_column(LO nv, int dim, int j, Real const* coords, Real* out) {
-  LO v = thread_index();
-  if (v < nv) out[v] = coords[v * dim + j];
-}
-
 __global__ void first_vertex_rank(LO n, int deg, LO const* ev2v, LO const* old2new_v, I64* keys) {
   LO e = thread_index();
   if (e < n) keys[e] = old2new_v[ev2v[e * deg]];
@@ -282,11 +277,13 @@ void reorder_by_hilbert(Ctx& c, DMesh& m) {
   int dim = m.dim;
   LO nv = m.nents[0];
   std::vector<Real> bmin(dim), bmax(dim);
-  Reals col(c, nv);
+  ReduceJob jobs[6];
+  Real ends[6];
+  for (int j = 0; j < 2 * dim; ++j) jobs[j] = {m.coords.data() + j % dim, nv, dim, j >= dim};
+  reduce_reals(c, jobs, 2 * dim, ends);
   for (int j = 0; j < dim; ++j) {
-    OSH_LAUNCH(coord_column, nv, c, dim, j, m.coords.data(), col.data());
-    bmin[j] = min_real(c, col);
-    bmax[j] = max_real(c, col);
+    bmin[j] = ends[j];
+    bmax[j] = ends[dim + j];
   }
   Real maxl = bmax[0] - bmin[0];
   for (int j = 1; j < dim; ++j) {

@@ -76,7 +76,8 @@ Ctx::Ctx() : pool(std::make_shared<Pool>()) {
   OSH_HIP(hipMalloc((void**)&words, sizeof(unsigned) * kWords));
   unsigned none[kWords] = {0};
   OSH_HIP(hipMemcpy(words, none, sizeof(none), hipMemcpyHostToDevice));
-  OSH_HIP(hipMalloc(&partials, 1024 * sizeof(double)));
+  OSH_HIP(hipHostMalloc((void**)&partials, sizeof(Partial) * kPartials, hipHostMallocDefault));
+  std::memset(partials, 0, sizeof(Partial) * kPartials);
   OSH_HIP(hipMalloc((void**)&tile_counter, sizeof(unsigned)));
   OSH_HIP(hipMalloc((void**)&tile_sums, sizeof(LO) * kScanTiles * kMaxScanJobs));
   unsigned zero = 0;
@@ -100,7 +101,7 @@ Ctx::~Ctx() {
   if (tile_sums) (void)hipFree(tile_sums);
   if (words) (void)hipFree(words);
   if (pool) pool->close();
-  if (partials) (void)hipFree(partials);
+  if (partials) (void)hipHostFree(partials);
   if (pinned) (void)hipHostFree(pinned);
 }
 
@@ -185,6 +186,18 @@ void Ctx::wait_totals(unsigned slots) {
   };
   poll(arrived);
   OSH_CHECK(arrived(), "a scan's total is missing");
+}
+
+void Ctx::wait_partials(int n) {
+  unsigned long long tag = signal_value = wait_tag();
+  Partial const* a = partials;
+  auto arrived = [=] {
+    for (int i = 0; i < n; ++i)
+      if (__atomic_load_n(&a[i].tag, __ATOMIC_ACQUIRE) != tag) return false;
+    return true;
+  };
+  poll(arrived);
+  OSH_CHECK(arrived(), "a reduction's result is missing");
 }
 
 void Ctx::raise_device_error() {
@@ -830,63 +843,115 @@ __global__ void iota_kernel(LO n, LO* out, LO start, LO stride) {
 
 enum ReduceOp { kMin, kMax, kSum };
 
-template <class T, int Op>
-__device__ __forceinline__ T combine(T a, T b) {
-  if (Op == kMin) return (b < a) ? b : a;
-  if (Op == kMax) return (a < b) ? b : a;
+template <class T>
+__host__ __device__ __forceinline__ T combine(int op, T a, T b) {
+  if (op == kMin) return (b < a) ? b : a;
+  if (op == kMax) return (a < b) ? b : a;
   return a + b;
 }
 
-// grid-stride partial reductions into out[blockIdx.x]; a one-block launch
-// over the partials then writes the result into host-visible memory (the
-// kernel boundary orders the two, so no device-wide fences are needed)
-template <class T, int Op>
-__global__ void __launch_bounds__(kBlock) reduce_blocks(LO n, T const* in, T* out, T init,
-    unsigned* signal, unsigned value) {
-  __shared__ T buf[kBlock];
-  T acc = init;
-  for (LO i = LO(blockIdx.x) * kBlock + LO(threadIdx.x); i < n; i += LO(gridDim.x) * kBlock)
-    acc = combine<T, Op>(acc, in[i]);
-  buf[threadIdx.x] = acc;
+// Reductions: each job's workgroups write their partial results to pinned
+// memory, tagged for the host, which polls for the tags and combines the few
+// there are.  A second launch for that, and a wait a job, cost a pass 7 us and
+// the start of an adapt two more waits.
+template <class T>
+struct ReduceBatch {
+  struct Job {
+    T const* in;
+    LO n;
+    LO stride;
+    int op;
+    unsigned first;
+  };
+  Job job[kMaxReduceJobs + 1];  // one past the last: where its workgroups end
+  int count;
+  unsigned tag;
+  Ctx::Partial* out;
+};
+constexpr int kReduceBlock = 1024;
+constexpr unsigned kReduceBlocks = Ctx::kPartials / kMaxReduceJobs;
+
+template <class T, class A>
+__global__ void __launch_bounds__(kReduceBlock) reduce_partials(ReduceBatch<T> b, A init_min,
+    A init_max, A init_sum) {
+  __shared__ A part[kReduceBlock / kWave];
+  int w = 0;
+  while (w + 1 < b.count && blockIdx.x >= b.job[w + 1].first) ++w;
+  typename ReduceBatch<T>::Job a = b.job[w];
+  unsigned block = blockIdx.x - a.first, blocks = b.job[w + 1].first - a.first;
+  A acc = a.op == kMin ? init_min : (a.op == kMax ? init_max : init_sum);
+  std::int64_t step = std::int64_t(blocks) * blockDim.x;
+#pragma unroll 4
+  for (std::int64_t i = std::int64_t(block) * blockDim.x + threadIdx.x; i < a.n; i += step)
+    acc = combine<A>(a.op, acc, A(a.in[i * a.stride]));
+  for (int d = kWave / 2; d > 0; d >>= 1) acc = combine<A>(a.op, acc, __shfl_xor(acc, d, kWave));
+  if (threadIdx.x % kWave == 0) part[threadIdx.x / kWave] = acc;
   __syncthreads();
-  for (int s = kBlock / 2; s > 0; s >>= 1) {
-    if (int(threadIdx.x) < s) buf[threadIdx.x] = combine<T, Op>(buf[threadIdx.x], buf[threadIdx.x + s]);
-    __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (unsigned k = 1; k < blockDim.x / kWave; ++k) acc = combine<A>(a.op, acc, part[k]);
+  unsigned long long bits = 0;
+  __builtin_memcpy(&bits, &acc, sizeof(A));
+  b.out[blockIdx.x].value = bits;
+  __hip_atomic_store(&b.out[blockIdx.x].tag, static_cast<unsigned long long>(b.tag),
+      __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// the reductions of up to kMaxReduceJobs jobs, waited for; an empty one gives
+// its init
+template <class T, class A>
+void reduce(Ctx& c, ReduceBatch<T>& b, A const (&init)[3], A* out) {
+  unsigned blocks = 0;
+  LO most = 0;
+  for (int j = 0; j < b.count; ++j) {
+    b.job[j].first = blocks;
+    unsigned nb = nblocks(b.job[j].n, kReduceBlock * 4);
+    blocks += nb > kReduceBlocks ? kReduceBlocks : nb;
+    most = b.job[j].n > most ? b.job[j].n : most;
   }
-  if (threadIdx.x == 0) {
-    out[blockIdx.x] = buf[0];
-    // the one-block launch that ends a reduction can end the wait for it
-    if (signal) __hip_atomic_store(signal, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  b.job[b.count].first = blocks;
+  b.out = c.partials;
+  b.tag = c.wait_tag();
+  if (blocks) {
+    hipLaunchKernelGGL((reduce_partials<T, A>), dim3(blocks),
+        dim3(most > kBlock * 4 ? kReduceBlock : kBlock), 0, c.stream, b, init[0], init[1], init[2]);
+    OSH_HIP(hipGetLastError());
+    c.wait_partials(int(blocks));
+  }
+  for (int j = 0; j < b.count; ++j) {
+    out[j] = init[b.job[j].op];
+    for (unsigned k = b.job[j].first; k < b.job[j + 1].first; ++k) {
+      A v;
+      std::memcpy(&v, &c.partials[k].value, sizeof(A));
+      out[j] = combine<A>(b.job[j].op, out[j], v);
+    }
   }
 }
 
-// the reduction of a, waited for
-template <class T, int Op>
-T reduce(Ctx& c, DArray<T> const& a, T init) {
-  LO n = a.size();
-  if (n == 0) return init;
-  T* result = static_cast<T*>(c.pinned);
-  unsigned* signal = c.signal_word();
-  unsigned value = c.wait_tag();
-  LO nb = LO(nblocks(n, kBlock * 4));
-  if (nb > 1024) nb = 1024;
-  if (nb == 1) {
-    hipLaunchKernelGGL((reduce_blocks<T, Op>), dim3(1), dim3(kBlock), 0, c.stream, n, a.data(),
-        result, init, signal, value);
-  } else {
-    T* part = static_cast<T*>(c.partials);
-    hipLaunchKernelGGL((reduce_blocks<T, Op>), dim3(nb), dim3(kBlock), 0, c.stream, n, a.data(),
-        part, init, (unsigned*)nullptr, 0u);
-    OSH_HIP(hipGetLastError());
-    hipLaunchKernelGGL((reduce_blocks<T, Op>), dim3(1), dim3(kBlock), 0, c.stream, nb, part,
-        result, init, signal, value);
-  }
-  OSH_HIP(hipGetLastError());
-  c.wait_signalled();
-  return read_slot<T>(c, 0);
+constexpr Real kRealInit[3] = {1.79769313486231570815e+308, -1.79769313486231570815e+308, 0.0};
+constexpr LO kWholeInit[3] = {0x7fffffff, -0x7fffffff - 1, 0};
+
+template <class T, class A>
+A reduce_one(Ctx& c, DArray<T> const& a, int op, A const (&init)[3]) {
+  ReduceBatch<T> b{};
+  b.count = 1;
+  b.job[0] = {a.data(), a.size(), 1, op, 0u};
+  A out;
+  reduce<T, A>(c, b, init, &out);
+  return out;
 }
 
 }  // namespace
+
+void reduce_reals(Ctx& c, ReduceJob const* jobs, int njobs, Real* out) {
+  for (int at = 0; at < njobs; at += kMaxReduceJobs) {
+    ReduceBatch<Real> b{};
+    for (; b.count < kMaxReduceJobs && at + b.count < njobs; ++b.count) {
+      ReduceJob const& j = jobs[at + b.count];
+      b.job[b.count] = {j.in, j.n, j.stride, j.max ? kMax : kMin, 0u};
+    }
+    reduce<Real, Real>(c, b, kRealInit, out + at);
+  }
+}
 
 LOs offset_scan(Ctx& c, LOs const& counts, LO* total) {
   LOs out = offset_scan_t<LO, false>(c, counts, total ? total_slot(c, 0) : nullptr);
@@ -997,17 +1062,16 @@ Reals fill_real(Ctx& c, LO n, Real value) {
   return out;
 }
 
-I8 max_i8(Ctx& c, Bytes const& a) { return reduce<I8, kMax>(c, a, I8(-128)); }
-Real min_real(Ctx& c, Reals const& a) { return reduce<Real, kMin>(c, a, 1.79769313486231570815e+308); }
+I8 max_i8(Ctx& c, Bytes const& a) {
+  return a.size() ? I8(reduce_one<I8, LO>(c, a, kMax, kWholeInit)) : I8(-128);
+}
+Real min_real(Ctx& c, Reals const& a) { return reduce_one<Real, Real>(c, a, kMin, kRealInit); }
 Real min_real_wait(Ctx& c, Reals const& a) {
-  if (a.size() == 0) {
-    c.wait();
-    return 1.79769313486231570815e+308;
-  }
+  if (a.size() == 0) c.wait();
   return min_real(c, a);
 }
-Real max_real(Ctx& c, Reals const& a) { return reduce<Real, kMax>(c, a, -1.79769313486231570815e+308); }
-LO sum_lo(Ctx& c, LOs const& a) { return reduce<LO, kSum>(c, a, 0); }
+Real max_real(Ctx& c, Reals const& a) { return reduce_one<Real, Real>(c, a, kMax, kRealInit); }
+LO sum_lo(Ctx& c, LOs const& a) { return reduce_one<LO, LO>(c, a, kSum, kWholeInit); }
 
 namespace {
 

@@ -111,8 +111,13 @@ struct Ctx {
   static constexpr int kSlots = 16;
   void* pinned = nullptr;
   int* error_word() const { return reinterpret_cast<int*>(static_cast<char*>(pinned) + 8 * kSlots); }
-  // per-block partials of reductions
-  void* partials = nullptr;
+  // pinned: the workgroups' partial results of reductions, each with a tag
+  struct Partial {
+    unsigned long long value;
+    unsigned long long tag;
+  };
+  static constexpr int kPartials = 64 * 24;
+  Partial* partials = nullptr;
   // single-pass scans: tile status words (tagged with a per-scan epoch) and
   // the tile ticket counter, whose running total the host tracks
   void* scan_status = nullptr;
@@ -156,6 +161,8 @@ struct Ctx {
   // waits for the scan totals of the given slots (bits) that the last
   // offset_scans call since the last wait writes
   void wait_totals(unsigned slots);
+  // waits for the first n partials
+  void wait_partials(int n);
   // for a kernel that signals by itself, as its last store (a release at
   // system scope of wait_tag() into signal_word()): waits for that
   void wait_signalled();
@@ -441,6 +448,16 @@ LOs iota(Ctx& c, LO n, LO start = 0, LO stride = 1);
 LOs fill_lo(Ctx& c, LO n, LO value);
 Bytes fill_i8(Ctx& c, LO n, I8 value);
 Reals fill_real(Ctx& c, LO n, Real value);
+// minima and maxima of several arrays (entries 0, stride, ...) by one launch
+// and one wait a kMaxReduceJobs
+struct ReduceJob {
+  Real const* in;
+  LO n;
+  LO stride;
+  bool max;
+};
+constexpr int kMaxReduceJobs = 24;
+void reduce_reals(Ctx& c, ReduceJob const* jobs, int njobs, Real* out);
 I8 max_i8(Ctx& c, Bytes const& a);
 Real min_real(Ctx& c, Reals const& a);
 // the same, bringing everything kernels left in pinned words with it
