@@ -181,7 +181,15 @@ __global__ void __launch_bounds__(kBlock) rank_uses(UseJobs j) {
   if (a.marks && !a.marks[l]) return;
   LO b = a.a2ab[l], e = a.a2ab[l + 1];
   LO rank = 0;
-  for (LO k = b; k < e; ++k) rank += (a.ab2hl[k] < hl);
+  LO k = b;
+  for (; k + 4 <= e; k += 4) {
+    LO u[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) u[i] = a.ab2hl[k + i];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rank += (u[i] < hl);
+  }
+  for (; k < e; ++k) rank += (a.ab2hl[k] < hl);
   a.ab2b[b + rank] = hl / a.deg;
   a.codes[b + rank] = use_code(a, hl);
 }
