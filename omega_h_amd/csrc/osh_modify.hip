@@ -637,27 +637,55 @@ __global__ void dual_max_kernel(LO n, int nspe, LO const* es2s,
 constexpr int kCountedLayers = 16;
 constexpr int kUnlinkedWord = 3;  // the sets and the star sweeps use the others
 
+// the interior edges of an element, marked by the sweep that marks it
+struct EdgeMarks {
+  LO const* e2e;
+  I8 const* edim;
+  I8* marks;  // null: not asked for
+};
+
+template <int NSPE>
+__device__ __forceinline__ void mark_edges(LO e, EdgeMarks const& a) {
+  constexpr int nepe = NSPE == 4 ? 6 : 3;
+#pragma unroll
+  for (int i = 0; i < nepe; ++i) {
+    LO ed = a.e2e[std::size_t(e) * nepe + i];
+    if (a.edim[ed] == NSPE - 1) a.marks[ed] = 1;
+  }
+}
+
+template <int NSPE>
+__global__ void mark_interior_edges_kernel(LO n, I8 const* elem_marks, EdgeMarks edges) {
+  LO e = thread_index();
+  if (e < n && elem_marks[e]) mark_edges<NSPE>(e, edges);
+}
+
 template <int NSPE>
 __global__ void sliver_layer(LO n, int layer, int nlayers, LO const* es2s, Real const* q,
-    Real ceil, unsigned* counts, I8* marks) {
+    Real ceil, unsigned* counts, I8* marks, EdgeMarks edges) {
   LO e = thread_index();
   if (e >= n) return;
   LO sides[NSPE];
-#pragma unroll
-  for (int j = 0; j < NSPE; ++j) sides[j] = es2s[std::size_t(e) * NSPE + j];
   bool in = false;
-  if (layer == 0) {
-    in = q[e] < ceil;
-  } else {
+  if (layer == 0) in = q[e] < ceil;
+  if (layer != 0 || in) {
+#pragma unroll
+    for (int j = 0; j < NSPE; ++j) sides[j] = es2s[std::size_t(e) * NSPE + j];
+  }
+  if (layer != 0) {
     unsigned own = marks[e] != 0;
 #pragma unroll
     for (int j = 0; j < NSPE; ++j)
       in = in || ((counts[sides[j]] >> (2 * (layer - 1))) & 3u) > own;
   }
   marks[e] = in;
-  if (!in || layer == nlayers) return;
+  if (!in) return;
+  if (layer < nlayers) {
 #pragma unroll
-  for (int j = 0; j < NSPE; ++j) atomicAdd(&counts[sides[j]], 1u << (2 * layer));
+    for (int j = 0; j < NSPE; ++j) atomicAdd(&counts[sides[j]], 1u << (2 * layer));
+  } else if (edges.marks) {
+    mark_edges<NSPE>(e, edges);
+  }
 }
 
 // a later layer, pushed from the marked elements (the first one's output has
@@ -1100,15 +1128,17 @@ Bytes SliverLayers::mark(Real qual_ceil) {
     return marks;
   }
   LO const* es2s = m.down[m.dim].data();
+  EdgeMarks edges{nullptr, m.class_dim[1].data(), edge_marks_};
+  if (edge_marks_) edges.e2e = ask_down(c, m, m.dim, 1, nullptr).data();
   if (counts_.exists()) {
     unsigned* counts = reinterpret_cast<unsigned*>(counts_.data());
     for (int k = 0; k <= nlayers_; ++k) {
       if (m.dim == 3)
         OSH_LAUNCH(sliver_layer<4>, ne, c, k, nlayers_, es2s, q.data(), qual_ceil, counts,
-            marks.data());
+            marks.data(), edges);
       else
         OSH_LAUNCH(sliver_layer<3>, ne, c, k, nlayers_, es2s, q.data(), qual_ceil, counts,
-            marks.data());
+            marks.data(), edges);
     }
     return marks;
   }
@@ -1133,6 +1163,19 @@ Bytes SliverLayers::mark(Real qual_ceil) {
     marks = next[b];
   }
   return marks;
+}
+
+void SliverLayers::mark_interior_edges(Real qual_ceil, Bytes& edge_marks) {
+  Ctx& c = c_;
+  DMesh& m = m_;
+  edge_marks_ = edge_marks.data();
+  Bytes marks = mark(qual_ceil);
+  if (counts_.exists()) return;  // the last layer has marked them
+  EdgeMarks edges{ask_down(c, m, m.dim, 1, nullptr).data(), m.class_dim[1].data(), edge_marks_};
+  if (m.dim == 3)
+    OSH_LAUNCH(mark_interior_edges_kernel<4>, m.nents[3], c, marks.data(), edges);
+  else
+    OSH_LAUNCH(mark_interior_edges_kernel<3>, m.nents[2], c, marks.data(), edges);
 }
 
 void SliverLayers::settle() {

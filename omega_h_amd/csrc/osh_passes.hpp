@@ -167,6 +167,9 @@ class SliverLayers {
  public:
   SliverLayers(Ctx& c, DMesh& m, int nlayers, Fills& fills);
   Bytes mark(Real qual_ceil);
+  // marks (zero so far) of the marked elements' edges of class dimension dim:
+  // mark_by_class_dim of their edges
+  void mark_interior_edges(Real qual_ceil, Bytes& edge_marks);
   // after a find_indset that follows mark(): records what it has found out
   // about the mesh (DMesh::linked)
   void settle();
@@ -177,6 +180,7 @@ class SliverLayers {
   int nlayers_;
   LOs counts_;
   unsigned tag_ = 0;
+  I8* edge_marks_ = nullptr;
 };
 LOs degrees_of(Ctx& c, LOs const& a2ab, LOs const& rows);
 

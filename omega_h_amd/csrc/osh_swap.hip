@@ -631,17 +631,6 @@ __global__ void __launch_bounds__(kBlock) swap3d_local_down(int lanes, unsigned 
         tets, error);
 }
 
-// the interior edges (mark_by_class_dim) of the marked elements
-__global__ void mark_interior_edges(LO nelems, int nepe, LO const* elem2edges,
-    I8 const* elem_marks, int dim, I8 const* edim, I8* marks) {
-  LO t = thread_index();
-  if (t >= nelems || !elem_marks[t]) return;
-  for (int i = 0; i < nepe; ++i) {
-    LO e = elem2edges[t * nepe + i];
-    if (edim[e] == dim) marks[e] = 1;
-  }
-}
-
 // swap3d_topology (src/Omega_h_swap3d_topology.cpp:12-119): the key list, each
 // key's product offsets and representatives from the per-candidate scans, and
 // its new edges, faces and tets in template order; kRow threads per candidate
@@ -988,10 +977,7 @@ bool swap_edges_3d(Ctx& c, DMesh& m, AdaptOptions const& o, SwapCache* cache) {
     cache->q = Reals(c, ne);
   }
   fills.run();
-  Bytes elems = layers.mark(o.min_quality_desired);
-  LOs const& t2e = ask_down(c, m, 3, 1, nullptr);
-  OSH_LAUNCH(mark_interior_edges, nt, c, 6, t2e.data(), elems.data(), 3,
-      m.class_dim[1].data(), marks.data());
+  layers.mark_interior_edges(o.min_quality_desired, marks);
   Rings rings;
   build_rings(c, m, marks, ring_counts, rings);
   LO ncands = rings.cands.size();
@@ -1091,10 +1077,8 @@ bool swap_edges_2d(Ctx& c, DMesh& m, AdaptOptions const& o) {
   prepare_keys(m, 1, 1, 2, fills, km);
   LOs side_zeros = fills.ints(m.nents[0], 0);
   fills.run();
-  Bytes elems = layers.mark(o.min_quality_desired);
+  layers.mark_interior_edges(o.min_quality_desired, cand);
   Reals quals(c, ne);  // read where an edge is kept
-  OSH_LAUNCH(mark_interior_edges, m.nents[2], c, 3, m.down[2].data(), elems.data(), 2,
-      m.class_dim[1].data(), cand.data());
   LOs cands = collect_marked(c, cand);
   if (cands.size() == 0) return false;
   int md = (m.metric_ncomps == 1) ? 1 : 2;
