@@ -92,9 +92,8 @@ __device__ __forceinline__ int cell_job(CellSweep const& a, LO* c) {
   return w;
 }
 
-// The product builders below use kLanes threads per key.
-constexpr int kLanes = 8;
-constexpr int kMaxSideLanes = 32;
+constexpr int kLanes = 8;          // threads a key in the product builders below
+constexpr int kMaxSideLanes = 32;  // an edge's two sides share a wave
 
 // the vertices' metric determinants, which every quality around a vertex
 // needs (24 times in a tet mesh)
@@ -163,8 +162,7 @@ __global__ void __launch_bounds__(kBlock) coarsen_quality_lanes(LO nt, int lshif
   bool rejected = false;
   double const* pp[D + 1];
   double const* ms[D + 1];
-  auto points = [&](LO vc) {
-    LO cv[D + 1];
+  auto points = [&](LO vc, LO (&cv)[D + 1]) {
     if (!moved_cell<D>(a.cv2v, a.v2c_ab2b[vc], code_which_down(a.v2c_codes[vc]), v_onto, cv))
       return false;
     for (int k = 0; k < D + 1; ++k) {
@@ -177,7 +175,8 @@ __global__ void __launch_bounds__(kBlock) coarsen_quality_lanes(LO nt, int lshif
     float minq = 1.0f;
     bool unclear = false;
     for (LO vc = row + lane; vc < end; vc += lanes) {
-      if (!points(vc)) continue;
+      LO cv[D + 1];
+      if (!points(vc, cv)) continue;
       float q = f32::element_quality<D, M>(pp, ms, &unclear);
       minq = (q < minq) ? q : minq;
     }
@@ -191,9 +190,10 @@ __global__ void __launch_bounds__(kBlock) coarsen_quality_lanes(LO nt, int lshif
   }
   double minq = 1.0;
   for (LO vc = row + lane; vc < end; vc += lanes) {
-    if (!points(vc)) continue;
+    LO cv[D + 1];
+    if (!points(vc, cv)) continue;
     double dets[D + 1];
-    for (int k = 0; k < D + 1; ++k) dets[k] = a.dets[(ms[k] - a.metric) / nc];
+    for (int k = 0; k < D + 1; ++k) dets[k] = a.dets[cv[k]];
     minq = math::min2(minq, element_quality<D, M>(pp, ms, dets));
   }
   for (int d = lanes / 2; d > 0; d >>= 1) minq = math::min2(minq, __shfl_xor(minq, d, 64));
@@ -1419,7 +1419,6 @@ void coarsen_qualities(Ctx& c, DMesh& m, LO ncands, LO const* cands, I8 const* c
   Reals dets = metric_dets(c, m);
   SideQualities sq{cands, m.down[1].data(), cv2v.data(), v2c.a2ab.data(), v2c.ab2b.data(),
       v2c.codes.data(), m.coords.data(), m.metric.data(), dets.data(), qmin, codes.data(), out};
-  // an edge's two sides share a wave
   int lanes = c.tuning.coarsen_lanes < kMaxSideLanes ? c.tuning.coarsen_lanes : kMaxSideLanes;
   lanes = fit_lanes(ncands * 2, lanes);
   int lshift = lanes_shift(lanes);

@@ -277,7 +277,7 @@ Reals refine_qualities(Ctx& c, DMesh& m, LOs const& cands, Adj const& e2c,
   Reals mm(c, n * nc);
   mident_metrics(c, m, n, cands.data(), mm.data());
   LOs const& cv2v = verts_of(c, m, dim);
-  // lanes share a candidate's children, as the coarsen sweeps share a side's
+  // lanes share a candidate's children
   int lanes = fit_lanes(n, c.tuning.coarsen_lanes);
   int lshift = lanes_shift(lanes);
 #define OSH_RQ(D, M)                                                                    \
