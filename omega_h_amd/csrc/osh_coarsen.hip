@@ -13,6 +13,7 @@
 //   mark_dead_ents / find_coarsen_domains / coarsen_topology
 //                                    src/Omega_h_coarsen_topology.cpp:15-122
 //   transfer_coarsen                 src/Omega_h_transfer.cpp:585-619
+#include <algorithm>
 #include <cstdio>
 
 #include "osh_math.hpp"
@@ -253,7 +254,8 @@ struct StarSweep {
   I8 const* codes;
   bool sides_only;  // stop after the overshoot check, with the verdicts in `sides`
   bool checked;     // the codes are those of such a sweep
-  unsigned* word;   // receives the tag where a star is large
+  I8* large;        // by listed vertex: whether its star does not fit
+  unsigned* word;   // receives the tag where one does not (null: not wanted)
   unsigned tag;
   I8* sides;        // by (edge, direction)
   I8* vcand;        // zero on entry
@@ -262,20 +264,18 @@ struct StarSweep {
   LO* star;
 };
 
-// a star in LDS, shared by the WAVES waves that work on it
-template <int D, int M, int WAVES>
+// a wave's star in LDS
+template <int D, int M>
 struct StarData {
   static constexpr int nc = (M == 1) ? 1 : (M == 2 ? 3 : 6);
-  static constexpr int kThreads = WAVES * 64;
-  static constexpr int kEdges = kThreads - 1;  // at most a thread each; a byte holds a position
-  static constexpr int kCells = WAVES * 128;
+  static constexpr int kThreads = 64;
+  static constexpr int kEdges = kThreads - 1;  // at most a lane each; kSelf names the last one
+  static constexpr int kCells = 128;
   double coords[kThreads * D];
   double metric[kThreads * nc];
   double dets[kThreads];
   double lens[kThreads];
   unsigned long long minq[kThreads];
-  double least[WAVES];
-  int counts[WAVES];
   LO verts[kThreads];
   unsigned cells[kCells];  // positions of a cell's vertices, a byte each; kSelf: the vertex
   unsigned char list[kThreads];
@@ -285,32 +285,18 @@ struct StarData {
   I8 unsure[kThreads];
 
   __device__ __forceinline__ static void sync() {
-    if constexpr (WAVES > 1) {
-      __syncthreads();
-    } else {
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
-  // lists the sides whose thread says so, in order; how many
+  // lists the sides whose lane says so, in order; how many
   __device__ __forceinline__ int list_sides(bool in, int t) {
     unsigned long long b = __ballot(in);
     sync();
-    if (WAVES > 1 && t % 64 == 0) counts[t / 64] = __popcll(b);
-    if (WAVES > 1) sync();
-    int before = 0, total = __popcll(b);
-    if constexpr (WAVES > 1) {
-      total = 0;
-      for (int w = 0; w < WAVES; ++w) {
-        before += w < t / 64 ? counts[w] : 0;
-        total += counts[w];
-      }
-    }
-    if (in) list[before + __popcll(b & ((1ull << (t % 64)) - 1ull))] = static_cast<unsigned char>(t);
+    if (in) list[__popcll(b & ((1ull << t) - 1ull))] = static_cast<unsigned char>(t);
     sync();
-    return total;
+    return __popcll(b);
   }
-  // op(target, k) for the listed targets and k < n, over the threads
+  // op(target, k) for the listed targets and k < n, over the lanes
   template <class Op>
   __device__ __forceinline__ void for_pairs(int nlist, int n, int t, Op const& op) const {
     int at = t / n, k = t % n, step = kThreads / n, rest = kThreads % n;
@@ -341,15 +327,8 @@ struct StarData {
       if (first < n) nlist = list_sides(open && !veto[t], t);
     }
   }
-  __device__ __forceinline__ double min_of(double x, int t) {
+  __device__ __forceinline__ static double min_of(double x) {
     for (int d = 32; d > 0; d >>= 1) x = math::min2(x, __shfl_xor(x, d, 64));
-    if constexpr (WAVES > 1) {
-      sync();
-      if (t % 64 == 0) least[t / 64] = x;
-      sync();
-      x = least[0];
-      for (int w = 1; w < WAVES; ++w) x = math::min2(x, least[w]);
-    }
     return x;
   }
 };
@@ -379,10 +358,10 @@ struct Rail {
   }
 };
 
-template <int D, int M, bool MIXED, int WAVES>
+template <int D, int M, bool MIXED>
 __device__ __forceinline__ void small_star(StarSweep const& a, LO row, int nedges, LO crow,
-    int ncells, int t, StarData<D, M, WAVES>& s, Rail& rail) {
-  using S = StarData<D, M, WAVES>;
+    int ncells, int t, StarData<D, M>& s, Rail& rail) {
+  using S = StarData<D, M>;
   constexpr int nc = S::nc;
   LO e = -1;
   int eev = 0;
@@ -490,7 +469,7 @@ __device__ __forceinline__ void small_star(StarSweep const& a, LO row, int nedge
   }
   nopen = s.list_sides(open, t);
   if (nopen == 0) return;
-  if (a.old_quals) vold = s.min_of(vold, t);
+  if (a.old_quals) vold = s.min_of(vold);
   // the positions of cell i's vertices with its vertex moved onto target w;
   // false if it dies
   auto moved = [&](int w, int i, int (&at)[D + 1]) {
@@ -569,24 +548,42 @@ __device__ __forceinline__ void small_star(StarSweep const& a, LO row, int nedge
   if (nkept) rail.edge = a.e_ab2b[row + rail.edge];
 }
 
-// a star of any size: one side after another, from memory
+// The stars that do not fit a wave's LDS, of any size: their sides (in row order,
+// after those of the listed stars before) a wave each, from memory, and then the
+// rail of each star from the sides kept.  A few such stars among thousands are
+// the usual case, and their sides are all the parallelism there is: a pass over
+// a fan of 600 edges takes 0.52 ms in 2D and 0.36 in 3D, 8.5 and 12.8 when one
+// wave took a star's sides one after another.  With 129 edges it takes 0.27 and
+// 0.29, against 0.38 and 0.48 with a workgroup and its LDS a star; a thousand stars of
+// 100 edges are the one case seen where that form was faster (0.70 against 0.86).
+struct LargeStars {
+  LO nstars;
+  LO nsides;
+  LO const* stars;    // positions in StarSweep::verts
+  LO const* offsets;  // by star: its first side
+  I8* kept;           // by side
+  Real* quals;        // the minimum quality where kept
+};
+
 template <int D, int M, bool MIXED>
-__device__ __forceinline__ void large_star(StarSweep const& a, LO row, LO end, LO crow, LO cend,
-    int lane, Rail& rail) {
-  constexpr int nc = StarData<D, M, 1>::nc;
-  if (!a.sides_only)
-    for (LO ve = row + lane; ve < end; ve += 64)
-      a.star[ve] = a.ev2v[a.e_ab2b[ve] * 2 + 1 - code_which_down(a.e_codes[ve])];
-  double vold = 1.79769313486231570815e+308;
-  if (a.old_quals && !a.sides_only) {
-    for (LO vc = crow + lane; vc < cend; vc += 64)
-      vold = math::min2(vold, a.old_quals[a.c_ab2b[vc]]);
-    for (int d = 32; d > 0; d >>= 1) vold = math::min2(vold, __shfl_xor(vold, d, 64));
-  }
-  for (LO vw = row; vw < end; ++vw) {
+__global__ void __launch_bounds__(kBlock) large_star_sides(StarSweep a, LargeStars g) {
+  constexpr int nc = StarData<D, M>::nc;
+  int lane = int(threadIdx.x) % 64;
+  LO step = LO(gridDim.x) * (kBlock / 64);
+  for (LO side = LO(blockIdx.x) * (kBlock / 64) + LO(threadIdx.x) / 64; side < g.nsides;
+       side += step) {
+    LO star = row_of(side, g.nstars, g.offsets);
+    LO v = a.verts[g.stars[star]];
+    LO row = a.e_a2ab[v], end = a.e_a2ab[v + 1];
+    LO crow = a.c_a2ab[v], cend = a.c_a2ab[v + 1];
+    LO vw = row + (side - g.offsets[star]);
     LO e = a.e_ab2b[vw];
     int eev = code_which_down(a.e_codes[vw]);
     LO onto = a.ev2v[e * 2 + 1 - eev];
+    if (!a.sides_only && lane == 0) {
+      a.star[vw] = onto;
+      g.kept[side] = 0;
+    }
     bool open = collapses(a.codes[e], eev);
     if (open && !a.checked) {
       bool veto = false;
@@ -659,53 +656,84 @@ __device__ __forceinline__ void large_star(StarSweep const& a, LO row, LO end, L
       bool unclear = false;
       for (LO vc = crow + lane; vc < cend; vc += 64)
         if (moved(vc)) least = math::min2(least, f32::element_quality<D, M>(pp, ms, &unclear));
-      for (int d = 32; d > 0; d >>= 1) least = math::min2(least, __shfl_xor(least, d, 64));
+      least = StarData<D, M>::min_of(least);
       if (!__any(unclear) && least < a.qmin * (1.0 - double(f32::kScreenBand))) continue;
     }
+    double vold = 1.79769313486231570815e+308;
     double minq = 1.0;
-    for (LO vc = crow + lane; vc < cend; vc += 64)
-      if (moved(vc)) {
-        double dets[D + 1];
+    for (LO vc = crow + lane; vc < cend; vc += 64) {
+      if (a.old_quals) vold = math::min2(vold, a.old_quals[a.c_ab2b[vc]]);
+      if (!moved(vc)) continue;
+      double dets[D + 1];
 #pragma unroll
-        for (int k = 0; k < D + 1; ++k) dets[k] = M == 1 ? ms[k][0] : det<M>(get_symm<M>(ms[k]));
-        minq = math::min2(minq, element_quality<D, M>(pp, ms, dets));
-      }
-    for (int d = 32; d > 0; d >>= 1) minq = math::min2(minq, __shfl_xor(minq, d, 64));
-    if (minq >= a.qmin && (!a.old_quals || minq > vold)) rail.visit(e, a.lengths[e], minq);
+      for (int k = 0; k < D + 1; ++k) dets[k] = M == 1 ? ms[k][0] : det<M>(get_symm<M>(ms[k]));
+      minq = math::min2(minq, element_quality<D, M>(pp, ms, dets));
+    }
+    vold = StarData<D, M>::min_of(vold);
+    minq = StarData<D, M>::min_of(minq);
+    if (lane == 0 && minq >= a.qmin && (!a.old_quals || minq > vold)) {
+      g.kept[side] = 1;
+      g.quals[side] = minq;
+    }
   }
 }
 
-// WAVES 1: a wave a star, four stars a workgroup; 4: a workgroup a star, for the
-// stars too large for that; 0: a wave a star of any size, for those that are too
-// large for a workgroup.  `rest`: only the stars that the forms before do not
-// take; stars that do not fit are told by `word`.  One wave a star is the
-// faster form also for few stars (2400: 28 us against 33 with four), since it
-// drops vetoed sides sooner.
-template <int D, int M, bool MIXED, int WAVES>
-__global__ void __launch_bounds__(kBlock, WAVES ? 5 : 1) collapse_stars(StarSweep a, bool rest) {
-  using S = StarData<D, M, (WAVES ? WAVES : 1)>;
-  using Less = StarData<D, M, (WAVES ? 1 : 4)>;
-  constexpr int kStars = kBlock / S::kThreads;
-  int star = int(threadIdx.x) / S::kThreads, t = int(threadIdx.x) % S::kThreads;
+__global__ void large_star_degrees(LO n, LO const* stars, LO const* verts, LO const* a2ab,
+    LO* degrees) {
+  LO i = thread_index();
+  if (i >= n) return;
+  LO v = verts[stars[i]];
+  degrees[i] = a2ab[v + 1] - a2ab[v];
+}
+
+// a wave a star: the kept sides in row order
+__global__ void __launch_bounds__(kBlock) large_star_rails(StarSweep a, LargeStars g) {
+  LO star = LO(blockIdx.x) * (kBlock / 64) + LO(threadIdx.x) / 64;
+  int lane = int(threadIdx.x) % 64;
+  if (star >= g.nstars) return;
+  LO v = a.verts[g.stars[star]];
+  LO row = a.e_a2ab[v], n = a.e_a2ab[v + 1] - row;
+  LO first = g.offsets[star];
+  Rail rail;
+  for (LO base = 0; base < n; base += 64) {
+    LO j = base + lane;
+    bool kept = j < n && g.kept[first + j];
+    LO e = kept ? a.e_ab2b[row + j] : -1;
+    double len = kept ? a.lengths[e] : 0.0;
+    double q = kept ? g.quals[first + j] : 0.0;
+    for (unsigned long long b = __ballot(kept); b; b &= b - 1) {
+      int k = __ffsll(static_cast<long long>(b)) - 1;
+      rail.visit(__shfl(e, k, 64), __shfl(len, k, 64), __shfl(q, k, 64));
+    }
+  }
+  if (lane != 0 || rail.edge < 0) return;
+  a.vcand[v] = 1;
+  a.vqual[v] = rail.qual;
+  a.vrail[v] = rail.edge;
+}
+
+// a wave a star, four stars a workgroup; a star that does not fit is told in
+// `large` and by `word`, and left to the sweep above
+template <int D, int M, bool MIXED>
+__global__ void __launch_bounds__(kBlock, 5) collapse_stars(StarSweep a) {
+  constexpr int kStars = kBlock / 64;
+  using S = StarData<D, M>;
+  __shared__ S data[kStars];
+  int star = int(threadIdx.x) / 64, t = int(threadIdx.x) % 64;
   std::int64_t i = std::int64_t(blockIdx.x) * kStars + star;
   if (i >= a.nverts) return;
   LO v = a.verts[i];
   LO row = a.e_a2ab[v], end = a.e_a2ab[v + 1];
   LO crow = a.c_a2ab[v], cend = a.c_a2ab[v + 1];
-  if (rest && end - row <= Less::kEdges && cend - crow <= Less::kCells) return;
-  Rail rail;
-  if constexpr (WAVES == 0) {
-    large_star<D, M, MIXED>(a, row, end, crow, cend, t, rail);
-  } else {
-    __shared__ S data[kStars];
-    if (end - row > S::kEdges || cend - crow > S::kCells) {
-      if (t == 0)
-        __hip_atomic_store(a.word, a.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      return;
-    }
-    small_star<D, M, MIXED, WAVES>(a, row, int(end - row), crow, int(cend - crow), t, data[star],
-        rail);
+  bool fits = end - row <= S::kEdges && cend - crow <= S::kCells;
+  if (t == 0) a.large[i] = fits ? 0 : 1;
+  if (!fits) {
+    if (t == 0 && a.word)
+      __hip_atomic_store(a.word, a.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return;
   }
+  Rail rail;
+  small_star<D, M, MIXED>(a, row, int(end - row), crow, int(cend - crow), t, data[star], rail);
   if (a.sides_only || t != 0 || rail.edge < 0) return;
   a.vcand[v] = 1;
   a.vqual[v] = rail.qual;
@@ -1140,25 +1168,42 @@ Reals metric_dets(Ctx& c, DMesh& m) {
       LAUNCH(2, 1, false);                  \
   } while (0)
 
-template <int WAVES>
-void launch_stars(Ctx& c, int dim, int md, bool mixed, StarSweep const& a, bool rest) {
-  int waves = WAVES ? WAVES : 1;
-  unsigned blocks = unsigned((std::int64_t(a.nverts) * 64 * waves + kBlock - 1) / kBlock);
-#define OSH_STARS(D, M, X)                                                                     \
-  hipLaunchKernelGGL((collapse_stars<D, M, X, WAVES>), dim3(blocks), dim3(kBlock), 0, c.stream, \
-      a, rest)
+void sweep_stars(Ctx& c, int dim, int md, bool mixed, StarSweep const& a) {
+  unsigned blocks = unsigned((std::int64_t(a.nverts) * 64 + kBlock - 1) / kBlock);
+#define OSH_STARS(D, M, X) \
+  hipLaunchKernelGGL((collapse_stars<D, M, X>), dim3(blocks), dim3(kBlock), 0, c.stream, a)
   OSH_BY_FORM(OSH_STARS, dim, md, mixed);
 #undef OSH_STARS
   OSH_HIP(hipGetLastError());
 }
 
-// the stars that fit a wave, the others being told by the sweep's word
-void sweep_stars(Ctx& c, int dim, int md, bool mixed, StarSweep const& a) {
-  launch_stars<1>(c, dim, md, mixed, a, false);
-}
-void sweep_large_stars(Ctx& c, int dim, int md, bool mixed, StarSweep const& a) {
-  launch_stars<4>(c, dim, md, mixed, a, true);
-  launch_stars<0>(c, dim, md, mixed, a, true);
+// the stars that the sweep has told as large
+void sweep_large_stars(Ctx& c, int dim, int md, bool mixed, StarSweep const& a,
+    LOs const& stars) {
+  LO n = stars.size();
+  if (n == 0) return;
+  LOs degrees(c, n);
+  OSH_LAUNCH(large_star_degrees, n, c, stars.data(), a.verts, a.e_a2ab, degrees.data());
+  LargeStars g{};
+  LOs offsets = offset_scan(c, degrees, &g.nsides);
+  Bytes kept(c, g.nsides);
+  Reals quals(c, g.nsides);
+  g.nstars = n;
+  g.stars = stars.data();
+  g.offsets = offsets.data();
+  g.kept = kept.data();
+  g.quals = quals.data();
+  // more waves than the device holds at a time take several sides each
+  unsigned blocks = std::min(unsigned((std::int64_t(g.nsides) * 64 + kBlock - 1) / kBlock), 1u << 16);
+#define OSH_SIDES(D, M, X) \
+  hipLaunchKernelGGL((large_star_sides<D, M, X>), dim3(blocks), dim3(kBlock), 0, c.stream, a, g)
+  OSH_BY_FORM(OSH_SIDES, dim, md, mixed);
+#undef OSH_SIDES
+  OSH_HIP(hipGetLastError());
+  if (a.sides_only) return;
+  hipLaunchKernelGGL(large_star_rails, dim3(nblocks(n, kBlock / 64)), dim3(kBlock), 0, c.stream, a,
+      g);
+  OSH_HIP(hipGetLastError());
 }
 
 // Up to this many cells the collapsing vertices' rows of all dimensions are
@@ -1267,8 +1312,10 @@ bool coarsen_verts(Ctx& c, DMesh& m, AdaptOptions const& o, CoarsenArrays& vm,
   sw.vrail = vrail.data();
   sw.star = star.ab2b.data();
   bool mixed = o.precision == 1;
-  sw.word = c.words + kLargeStarWord;
-  sw.tag = c.wait_tag();
+  Bytes large(c, verts.size());
+  sw.large = large.data();
+  bool any;
+  Bytes keys;
   if (o.should_prevent_coarsen_flip) {
     // the flip check looks at the edges that the overshoot check leaves
     LOs cands = collect_marked(c, codes);
@@ -1276,21 +1323,29 @@ bool coarsen_verts(Ctx& c, DMesh& m, AdaptOptions const& o, CoarsenArrays& vm,
     sw.sides_only = true;
     sw.sides = sides.data();
     sweep_stars(c, dim, md, mixed, sw);
-    sweep_large_stars(c, dim, md, mixed, sw);
+    LOs stars = collect_marked(c, large);
+    sweep_large_stars(c, dim, md, mixed, sw, stars);
     OSH_LAUNCH(drop_sides, cands.size(), c, cands.data(), sides.data(), codes.data());
     prevent_coarsen_flip(c, m, cands, codes);
     sw.sides_only = false;
     sw.checked = true;
-  }
-  sweep_stars(c, dim, md, mixed, sw);
-  quality_range.end();
-  bool any;
-  // waits below bring the word along; a tag lasts until a sweep stores the next
-  unsigned tag = sw.tag;
-  Bytes keys = find_indset(c, m, 0, vqual, vm.cand, &any, nullptr, &star);
-  if (c.word_set(kLargeStarWord, tag)) {
-    sweep_large_stars(c, dim, md, mixed, sw);
+    sweep_stars(c, dim, md, mixed, sw);
+    sweep_large_stars(c, dim, md, mixed, sw, stars);
+    quality_range.end();
     keys = find_indset(c, m, 0, vqual, vm.cand, &any, nullptr, &star);
+  } else {
+    // few meshes have a large star: the first wait of the independent set brings
+    // the word along, and stops it where there is one
+    StopWord told{kLargeStarWord, c.wait_tag()};
+    sw.word = c.words + told.word;
+    sw.tag = told.tag;
+    sweep_stars(c, dim, md, mixed, sw);
+    quality_range.end();
+    keys = find_indset(c, m, 0, vqual, vm.cand, &any, nullptr, &star, &told);
+    if (c.word_set(told.word, told.tag)) {
+      sweep_large_stars(c, dim, md, mixed, sw, collect_marked(c, large));
+      keys = find_indset(c, m, 0, vqual, vm.cand, &any, nullptr, &star);
+    }
   }
   if (layers) layers->settle();
   if (!any) return false;

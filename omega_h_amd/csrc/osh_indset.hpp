@@ -5,7 +5,7 @@
 
 #include <utility>
 
-#include "osh_runtime.hpp"
+#include "osh_passes.hpp"
 
 namespace osh {
 
@@ -57,7 +57,7 @@ __device__ __forceinline__ void tell_round(I8 before, I8 after, IndsetWords w) {
 // launches one; the first reads `cands` (nonzero: a candidate), later ones the
 // states of the round before, which alternate between a and b.  Returns the
 // final states: 1 in the set, 0 not.  *any_cands tells whether there was a
-// candidate.
+// candidate.  `stop` as in find_indset.
 //
 // Rounds leave decided nodes as they are and take no node from the set, so
 // extra rounds after convergence change nothing: two rounds run before each of
@@ -66,7 +66,7 @@ __device__ __forceinline__ void tell_round(I8 before, I8 after, IndsetWords w) {
 // rounds and would otherwise spend a wait every two).
 template <class Round>
 Bytes indset_rounds(Ctx& c, LO n, Bytes const& cands, Bytes a, Bytes b, bool* any_cands,
-    Round const& round_of) {
+    Round const& round_of, StopWord const* stop = nullptr) {
   for (LO round = 0;;) {
     OSH_CHECK(round <= n + 1, "independent set does not converge");
     int batch = round < 8 ? 2 : (round < 16 ? 4 : (round < 32 ? 8 : 16));
@@ -79,6 +79,7 @@ Bytes indset_rounds(Ctx& c, LO n, Bytes const& cands, Bytes a, Bytes b, bool* an
     }
     c.wait();
     if (any_cands && round == 2) *any_cands = c.word_set(kCandWord, tag);
+    if (stop && c.word_set(stop->word, stop->tag)) return a;
     if (!c.word_set(kUndecidedWord, tag)) return a;
   }
 }

@@ -1053,7 +1053,7 @@ void transfer_pointwise(Ctx& c, DMesh& old, DMesh& nw, ModOut const& mo, int key
 }
 
 Bytes find_indset(Ctx& c, DMesh& m, int d, Reals const& quality, Bytes const& cands,
-    bool* any_cands, Adj const* edge_elems, Adj const* star) {
+    bool* any_cands, Adj const* edge_elems, Adj const* star, StopWord const* stop) {
   Range range(c, "find_indset");
   LO n = m.nents[d];
   if (d == m.dim) {  // src/Omega_h_indset.cpp:29
@@ -1092,7 +1092,8 @@ Bytes find_indset(Ctx& c, DMesh& m, int d, Reals const& quality, Bytes const& ca
         else
           OSH_LAUNCH(indset_iteration_edges<3>, n, c, e2c->a2ab.data(), e2c->ab2b.data(), c2e,
               quality.data(), in, out, dom.data(), w);
-      });
+      },
+      stop);
 }
 
 Bytes mark_down(Ctx& c, DMesh& m, int high, int low, Bytes const& marks) {

@@ -157,9 +157,16 @@ void conserve_correct(Ctx& c, DMesh& m, int max_sweeps);
 // *any_cands (when given) tells whether any entity was a candidate; for
 // edges, `edge_elems` (when given) is an edge -> element adjacency holding at
 // least the rows of the candidate edges; for vertices, `star` (when given) is
-// the vertex star holding at least the rows of the candidates
+// the vertex star holding at least the rows of the candidates.  With `stop`, a
+// word (Ctx::words) that earlier kernels may have set to the tag: the rounds end
+// at the first wait that brings it, and the set is of no use then
+struct StopWord {
+  int word;
+  unsigned tag;
+};
 Bytes find_indset(Ctx& c, DMesh& m, int d, Reals const& quality, Bytes const& cands,
-    bool* any_cands = nullptr, Adj const* edge_elems = nullptr, Adj const* star = nullptr);
+    bool* any_cands = nullptr, Adj const* edge_elems = nullptr, Adj const* star = nullptr,
+    StopWord const* stop = nullptr);
 Bytes mark_down(Ctx& c, DMesh& m, int high, int low, Bytes const& marks);
 // mark_sliver_layers: the arrays that start out constant go into `fills`, which
 // has to run before mark()

@@ -1,9 +1,15 @@
 """Coarsening around vertices with many edges on the GPU against the oracle, bit
-for bit: fans whose hub has just as many edges as a wave or a workgroup takes,
-one more, and more than both, in 2D (a disk) and 3D (tets around an axis), with
-every hub and rim vertex free to collapse by size."""
+for bit: hubs with just as many edges or cells as a wave takes, one more, and
+many more, in 2D (a disk) and 3D (tets around an axis, a ball around a point).
+The fans let every hub and rim vertex collapse by size; the disks and balls
+with a drawn metric and classification have sides vetoed by length, by quality
+and by exposure, with and without the flip check and the FP32 screens."""
+import statistics
+import time
+
 import numpy as np
 import pytest
+from scipy.spatial import ConvexHull
 
 import oracle_lib as O
 
@@ -72,3 +78,99 @@ def test_large_stars_match_oracle(ctx, dim, n, improve):
     assert did[0] and did[1]
     assert [g.nents(d) for d in range(dim + 1)] == [o.nents(d) for d in range(dim + 1)]
     assert g.digests() == o.digests()
+
+
+def ball(n, rng):
+    """tets from a hub to n points on a sphere (n edges, 2 n - 4 cells), and a
+    shell of prisms around them, so that the sphere's points are interior too"""
+    k = np.arange(n) + 0.5
+    z = 1 - 2 * k / n
+    phi = np.pi * (1 + 5 ** 0.5) * k
+    p = np.stack([np.sqrt(1 - z * z) * np.cos(phi), np.sqrt(1 - z * z) * np.sin(phi), z], axis=1)
+    p += rng.uniform(-0.1, 0.1, p.shape) / np.sqrt(n)
+    p /= np.linalg.norm(p, axis=1)[:, None]
+    tris = np.sort(ConvexHull(p).simplices, axis=1)
+    x = np.concatenate([[[0.0, 0.0, 0.0]], p * rng.uniform(0.8, 1.2, (n, 1)), 2 * p])
+    a, b, c = (1 + tris).T
+    # sorted corners: neighbouring prisms cut their common side along one diagonal
+    tets = np.concatenate([np.stack([0 * a, a, b, c], axis=1), np.stack([a, b, c, c + n], axis=1),
+                           np.stack([a, b, b + n, c + n], axis=1),
+                           np.stack([a, a + n, b + n, c + n], axis=1)])
+    q = x[tets]
+    vol = np.linalg.det(q[:, 1:] - q[:, :1])
+    tets[vol < 0] = tets[vol < 0][:, [1, 0, 2, 3]]
+    return tets, x
+
+
+def drawn_metric(dim, n, rng, ratio):
+    """rotated metrics with eigen-lengths log-uniform within `ratio`"""
+    q, _ = np.linalg.qr(rng.normal(size=(n, dim, dim)))
+    h = 2.0 * ratio ** rng.uniform(-1, 0, (n, dim))
+    m = np.einsum("nij,nj,nkj->nik", q, 1 / h ** 2, q)
+    if dim == 2:
+        return np.stack([m[:, 0, 0], m[:, 1, 1], m[:, 0, 1]], axis=1).ravel()
+    return np.stack([m[:, 0, 0], m[:, 1, 1], m[:, 2, 2], m[:, 0, 1], m[:, 1, 2], m[:, 0, 2]],
+                    axis=1).ravel()
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("flip", [False, True])
+@pytest.mark.parametrize("aniso", [False, True])
+@pytest.mark.parametrize("dim,n", [(2, 63), (2, 64), (2, 255), (2, 256), (2, 600), (3, 63),
+                                   (3, 64), (3, 66), (3, 67), (3, 255), (3, 256), (3, 600)])
+def test_large_stars_with_vetoes_match_oracle(ctx, dim, n, aniso, flip, mixed):
+    rng = np.random.default_rng(1000 * n + 10 * dim + aniso)
+    elems, x = fan(2, n) if dim == 2 else ball(n, rng)
+    if dim == 2:
+        x = x * rng.uniform(0.9, 1.1, (len(x), 1))
+    g = A.Mesh.from_elems(ctx, dim, elems.astype(np.int32).ravel(), len(x))
+    g.set_coords(np.ascontiguousarray(x.ravel()))
+    if aniso:
+        g.set_metric(drawn_metric(dim, len(x), rng, 3.0), dim * (dim + 1) // 2)
+    else:
+        g.set_metric(1 / (2.0 * 3.0 ** rng.uniform(-1, 0, len(x))) ** 2, 1)
+    classify(g, dim)
+    # some inner sides with all around them belong to another model face (the hub
+    # does not): their cells' collapses are exposed
+    ids, dims = g.classification(dim - 1)
+    inner = np.nonzero(dims == dim)[0]
+    sides = g.verts(dim - 1).reshape(-1, dim)
+    pick = rng.choice(inner, size=max(1, n // 20), replace=False)
+    dims[pick] = dim - 1
+    g.set_class(dim - 1, ids, dims)
+    print(f"star {dim}D n={n} aniso={aniso} flip={flip} mixed={mixed}", flush=True)
+    for improve in (False, True):
+        a, o = g.copy(), O.Mesh.copy_of(g)
+        did = []
+        for m, opts in ((o, O.default_opts(dim)), (a, ctx.default_opts(dim))):
+            opts.verbosity = 0
+            opts.min_quality_allowed = 0.05
+            opts.min_quality_desired = 0.9
+            opts.should_prevent_coarsen_flip = int(flip)
+            if m is a:
+                opts.precision = int(mixed)
+            did.append(bool(m.coarsen_slivers(opts) if improve else m.coarsen_by_size(opts)))
+        assert did[0] == did[1]
+        assert [a.nents(d) for d in range(dim + 1)] == [o.nents(d) for d in range(dim + 1)]
+        assert a.digests() == o.digests()
+
+
+def test_large_star_takes_its_sides_side_by_side(ctx):
+    """A hub of 3000 edges: 196 ms when one wave took its sides one after another,
+    1.8 ms with a wave each; the bound lies far from both."""
+    elems, x = fan(2, 3000)
+    g = A.Mesh.from_elems(ctx, 2, elems.astype(np.int32).ravel(), len(x))
+    g.set_coords(np.ascontiguousarray(x.ravel()))
+    g.set_metric(np.full(len(x), 1.0 / 6.0 ** 2), 1)
+    classify(g, 2)
+    opts = ctx.default_opts(2)
+    opts.verbosity = 0
+    opts.min_quality_allowed = 1e-3
+    times = []
+    for _ in range(4):
+        m = g.copy()
+        ctx.synchronize()
+        t0 = time.perf_counter()
+        assert m.coarsen_by_size(opts)
+        times.append(time.perf_counter() - t0)
+    assert statistics.median(times[1:]) < 0.04
