@@ -194,14 +194,14 @@ __global__ void mean_exps_kernel(LO nv, Real const* sums, LO const* ns, Real* ou
   if (bad) *error = kDegenerateEigen;
 }
 
-Reals limit_gradation_once(Ctx& c, DMesh& m, Reals const& values, Real max_rate, Real tol,
-    int word) {
+// one sweep over the vertex star; c.words[word] receives the tag when some value
+// moved by more than tol
+Reals limit_gradation_once(Ctx& c, DMesh& m, Adj const& star, Reals const& values,
+    Real max_rate, Real tol, int word, unsigned tag) {
   LO nv = m.nents[0];
-  Adj const& star = ask_star(c, m, 0);
   Reals out(c, values.size());
   int md = (m.metric_ncomps == 1) ? 1 : m.dim;
   unsigned* w = c.words + word;
-  unsigned tag = c.wait_tag();
 #define OSH_LG(S, M)                                                                       \
   OSH_LAUNCH((limit_gradation_kernel<S, M>), nv, c, star.a2ab.data(), star.ab2b.data(),    \
       m.coords.data(), values.data(), max_rate, tol, out.data(), w, tag, c.error_word())
@@ -227,6 +227,7 @@ int limit_metric_gradation(Ctx& c, DMesh& m, Real max_rate, Real tol) {
   // with a word of its own, and the first quiet one's values are the result,
   // whatever the next made of them.
   int batch = 1;
+  Adj const star = ask_star(c, m, 0);  // before the tags: building it may wait
   Reals values2 = m.metric;
   int steps = 0;
   for (;; batch = m.metric_ncomps == 1 ? 2 : 1) {
@@ -234,7 +235,8 @@ int limit_metric_gradation(Ctx& c, DMesh& m, Real max_rate, Real tol) {
     Reals made[2];
     unsigned tag = c.wait_tag();
     for (int k = 0; k < batch; ++k)
-      made[k] = limit_gradation_once(c, m, k ? made[k - 1] : values2, max_rate, tol, k);
+      made[k] =
+          limit_gradation_once(c, m, star, k ? made[k - 1] : values2, max_rate, tol, k, tag);
     c.wait();
     bool close = false;
     for (int k = 0; k < batch && !close; ++k) {
