@@ -121,6 +121,13 @@ __global__ void element_implied_kernel(LO ne, LO const* ev2v, Real const* coords
   for (int k = 0; k < nc; ++k) e2m[std::size_t(e) * nc + k] = x[k] * scalar;
 }
 
+// an array counts these, not their components, which would not fit an array's
+// size from 239 M tets on
+template <int M>
+struct FullMatrix {
+  Real m[M * M];
+};
+
 // project_metrics, src/Omega_h_metric.cpp:221-245: log-Euclidean average of
 // the metrics of a vertex's elements (average_metric_contrib/_finish with
 // degenerate metrics skipped, src/Omega_h_metric.hpp:125-139).  Each element's
@@ -273,17 +280,17 @@ Reals project_metric_array(Ctx& c, DMesh& m, int mdim, Reals const& e2m) {
   int nc = (mdim * (mdim + 1)) / 2;
   LO nv = m.nents[0], ne = m.nents[m.dim];
   Reals out(c, nv * nc);
-  DArray<Real> logs(c, ne * mdim * mdim);
   Bytes counts(c, ne);
-  Reals sums(c, nv * mdim * mdim);
   LOs ns(c, nv);
 #define OSH_PM(M, LANES)                                                                     \
   do {                                                                                       \
-    OSH_LAUNCH(metric_logs_kernel<M>, ne, c, e2m.data(), logs.data(), counts.data(),           \
-        c.error_word());                                                                     \
+    DArray<FullMatrix<M>> logs(c, ne), sums(c, nv);                                            \
+    Real* l = reinterpret_cast<Real*>(logs.data());                                            \
+    Real* s = reinterpret_cast<Real*>(sums.data());                                            \
+    OSH_LAUNCH(metric_logs_kernel<M>, ne, c, e2m.data(), l, counts.data(), c.error_word());     \
     OSH_LAUNCH64(sum_logs_kernel<M>, std::int64_t(nv) * LANES, c, v2e.a2ab.data(),             \
-        v2e.ab2b.data(), logs.data(), counts.data(), sums.data(), ns.data());                 \
-    OSH_LAUNCH(mean_exps_kernel<M>, nv, c, sums.data(), ns.data(), out.data(),                 \
+        v2e.ab2b.data(), static_cast<Real const*>(l), counts.data(), s, ns.data());             \
+    OSH_LAUNCH(mean_exps_kernel<M>, nv, c, static_cast<Real const*>(s), ns.data(), out.data(),  \
         c.error_word());                                                                     \
   } while (0)
   if (mdim == 3)
