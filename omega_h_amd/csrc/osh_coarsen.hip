@@ -756,17 +756,6 @@ __global__ void scatter_codes(LO n, LO const* cands, I8 const* cand_codes, I8* c
   if (i < n) codes[cands[i]] = cand_codes[i];
 }
 
-// the vertices that would collapse along some candidate edge
-__global__ void mark_collapsing_verts(LO ncands, LO const* cands, LO const* ev2v,
-    I8 const* codes, I8* vmarks) {
-  LO i = thread_index();
-  if (i >= ncands) return;
-  LO e = cands[i];
-  I8 code = codes[e];
-  for (int col = 0; col < 2; ++col)
-    if (collapses(code, col)) vmarks[ev2v[e * 2 + col]] = 1;
-}
-
 // mark_dead_ents (src/Omega_h_coarsen_topology.cpp:15-60): the rails die,
 // and so do the cells around a rail and each such cell's side opposite the
 // target vertex; rail_col[e] is the collapsing end of rail e (-1 elsewhere),

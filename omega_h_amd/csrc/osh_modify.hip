@@ -710,22 +710,7 @@ __global__ void push_layer_kernel(LO n, LO const* es2s, unsigned long long const
   }
 }
 
-__global__ void degrees_kernel(LO n, LO const* a2ab, LO const* rows, LO* out) {
-  LO i = thread_index();
-  if (i >= n) return;
-  LO r = rows ? rows[i] : i;
-  out[i] = a2ab[r + 1] - a2ab[r];
-}
-
 }  // namespace
-
-LOs degrees_of(Ctx& c, LOs const& a2ab, LOs const& rows) {
-  LO n = rows.exists() ? rows.size() : a2ab.size() - 1;
-  LOs out(c, n);
-  OSH_LAUNCH(degrees_kernel, n, c, a2ab.data(), rows.exists() ? rows.data() : (LO const*)nullptr,
-      out.data());
-  return out;
-}
 
 void prepare_keys(DMesh const& old, int key_dim, int d0, int d1, Fills& fills, KeyedMods& out) {
   for (int d = d0; d <= d1; ++d) {

@@ -189,7 +189,6 @@ class SliverLayers {
   unsigned tag_ = 0;
   I8* edge_marks_ = nullptr;
 };
-LOs degrees_of(Ctx& c, LOs const& a2ab, LOs const& rows);
 
 bool refine_by_size(Ctx& c, DMesh& m, AdaptOptions const& o);
 bool coarsen_by_size(Ctx& c, DMesh& m, AdaptOptions const& o);

@@ -380,8 +380,7 @@ __device__ __forceinline__ void put_total(unsigned long long* slot, unsigned tag
 
 __device__ __forceinline__ LO scan_input(void const* in, int kind, LO i) {
   if (kind == kScanLO) return static_cast<LO const*>(in)[i];
-  I8 x = static_cast<I8 const*>(in)[i];
-  return kind == kScanBytes ? LO(x) : LO(x != 0);
+  return LO(static_cast<I8 const*>(in)[i] != 0);
 }
 
 // without tickets (every job one tile) a workgroup's tile is its index
@@ -502,11 +501,10 @@ __device__ __forceinline__ void load_four(void const* in, int kind, LO i, LO n, 
       v[3] = q.w;
     } else {
       char4 q = *reinterpret_cast<char4 const*>(static_cast<I8 const*>(in) + i);
-      bool b = kind == kScanBytes;
-      v[0] = b ? LO(q.x) : LO(q.x != 0);
-      v[1] = b ? LO(q.y) : LO(q.y != 0);
-      v[2] = b ? LO(q.z) : LO(q.z != 0);
-      v[3] = b ? LO(q.w) : LO(q.w != 0);
+      v[0] = LO(q.x != 0);
+      v[1] = LO(q.y != 0);
+      v[2] = LO(q.z != 0);
+      v[3] = LO(q.w != 0);
     }
   } else {
 #pragma unroll
@@ -842,28 +840,17 @@ void offset_scans_noalloc(Ctx& c, ScanJob const* jobs, int njobs) {
 
 namespace {
 
-// the grand total lands in *total_out (device-visible) when given
-template <class T, bool NONZERO>
-LOs offset_scan_t(Ctx& c, DArray<T> const& counts, unsigned long long* total_out) {
-  LOs out(c, counts.size() + 1);
-  ScanJob job{counts.data(), sizeof(T) == 1 ? (NONZERO ? kScanNonzero : kScanBytes) : kScanLO,
-      counts.size(), out.data(), total_out};
-  offset_scans(c, &job, 1);
-  return out;
-}
-
 __global__ void iota_kernel(LO n, LO* out, LO start, LO stride) {
   LO i = thread_index();
   if (i < n) out[i] = start + i * stride;
 }
 
-enum ReduceOp { kMin, kMax, kSum };
+enum ReduceOp { kMin, kMax };
 
 template <class T>
 __host__ __device__ __forceinline__ T combine(int op, T a, T b) {
   if (op == kMin) return (b < a) ? b : a;
-  if (op == kMax) return (a < b) ? b : a;
-  return a + b;
+  return (a < b) ? b : a;
 }
 
 // Reductions: each job's workgroups write their partial results to pinned
@@ -898,13 +885,13 @@ static_assert(Ctx::kPartials >= kMaxReduceJobs, "a partial for each job");
 
 template <class T, class A>
 __global__ void __launch_bounds__(kReduceBlock) reduce_partials(ReduceBatch<T> b, A init_min,
-    A init_max, A init_sum) {
+    A init_max) {
   __shared__ A part[kReduceBlock / kWave];
   int w = 0;
   while (w + 1 < b.count && blockIdx.x >= b.job[w + 1].first) ++w;
   typename ReduceBatch<T>::Job a = b.job[w];
   unsigned block = blockIdx.x - a.first, blocks = b.job[w + 1].first - a.first;
-  A acc = a.op == kMin ? init_min : (a.op == kMax ? init_max : init_sum);
+  A acc = a.op == kMin ? init_min : init_max;
   std::int64_t step = std::int64_t(blocks) * blockDim.x;
 #pragma unroll 4
   for (std::int64_t i = std::int64_t(block) * blockDim.x + threadIdx.x; i < a.n; i += step)
@@ -924,7 +911,7 @@ __global__ void __launch_bounds__(kReduceBlock) reduce_partials(ReduceBatch<T> b
 // the reductions of up to kMaxReduceJobs jobs, waited for; an empty one gives
 // its init
 template <class T, class A>
-void reduce(Ctx& c, ReduceBatch<T>& b, A const (&init)[3], A* out) {
+void reduce(Ctx& c, ReduceBatch<T>& b, A const (&init)[2], A* out) {
   unsigned blocks = 0, share = unsigned(Ctx::kPartials / b.count);
   LO most = 0;
   for (int j = 0; j < b.count; ++j) {
@@ -939,7 +926,7 @@ void reduce(Ctx& c, ReduceBatch<T>& b, A const (&init)[3], A* out) {
   b.tag = c.wait_tag();
   if (blocks) {
     hipLaunchKernelGGL((reduce_partials<T, A>), dim3(blocks),
-        dim3(most > kBlock * 4 ? kReduceBlock : kBlock), 0, c.stream, b, init[0], init[1], init[2]);
+        dim3(most > kBlock * 4 ? kReduceBlock : kBlock), 0, c.stream, b, init[0], init[1]);
     OSH_HIP(hipGetLastError());
     c.wait_partials(int(blocks));
   }
@@ -953,11 +940,11 @@ void reduce(Ctx& c, ReduceBatch<T>& b, A const (&init)[3], A* out) {
   }
 }
 
-constexpr Real kRealInit[3] = {1.79769313486231570815e+308, -1.79769313486231570815e+308, 0.0};
-constexpr LO kWholeInit[3] = {0x7fffffff, -0x7fffffff - 1, 0};
+constexpr Real kRealInit[2] = {1.79769313486231570815e+308, -1.79769313486231570815e+308};
+constexpr LO kWholeInit[2] = {0x7fffffff, -0x7fffffff - 1};
 
 template <class T, class A>
-A reduce_one(Ctx& c, DArray<T> const& a, int op, A const (&init)[3]) {
+A reduce_one(Ctx& c, DArray<T> const& a, int op, A const (&init)[2]) {
   ReduceBatch<T> b{};
   b.count = 1;
   b.job[0] = {a.data(), a.size(), 1, op, 0u};
@@ -980,12 +967,10 @@ void reduce_reals(Ctx& c, ReduceJob const* jobs, int njobs, Real* out) {
 }
 
 LOs offset_scan(Ctx& c, LOs const& counts, LO* total) {
-  LOs out = offset_scan_t<LO, false>(c, counts, total ? total_slot(c, 0) : nullptr);
-  if (total) *total = scan_total(c, 0);
-  return out;
-}
-LOs offset_scan_bytes(Ctx& c, Bytes const& counts, LO* total) {
-  LOs out = offset_scan_t<I8, false>(c, counts, total ? total_slot(c, 0) : nullptr);
+  LOs out(c, counts.size() + 1);
+  ScanJob job{counts.data(), kScanLO, counts.size(), out.data(),
+      total ? total_slot(c, 0) : nullptr};
+  offset_scans(c, &job, 1);
   if (total) *total = scan_total(c, 0);
   return out;
 }
@@ -1097,7 +1082,6 @@ Real min_real_wait(Ctx& c, Reals const& a) {
   return min_real(c, a);
 }
 Real max_real(Ctx& c, Reals const& a) { return reduce_one<Real, Real>(c, a, kMax, kRealInit); }
-LO sum_lo(Ctx& c, LOs const& a) { return reduce_one<LO, LO>(c, a, kSum, kWholeInit); }
 
 namespace {
 
@@ -1341,7 +1325,7 @@ LOs sort_by_keys(Ctx& c, DArray<I64> const& keys, int width) {
         packed.data());
     radix_sort_pairs(c, packed, perm, packed_tmp, perm_tmp, group_differ[0]);
     int* ties = slot_ptr<int>(c, 0);
-    *ties = 0;  // the stream is idle here: the bits were read back
+    *ties = 0;  // nothing queued so far writes slot 0
     OSH_LAUNCH(find_ties, n, c, packed.data(), ties);
     if (pinned_value<int>(c) == 0) return perm;
     perm = iota(c, n);

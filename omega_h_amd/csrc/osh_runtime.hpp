@@ -303,20 +303,6 @@ inline LO scan_total(Ctx& c, int slot) {
 // what a raised kReflectDownNoMatch says
 constexpr char const* kNoMatchMessage = "reflect_down: entity without a unique match";
 
-template <class T>
-inline T get_value(Ctx& c, T const* dptr) {
-  OSH_HIP(hipMemcpyAsync(c.pinned, dptr, sizeof(T), hipMemcpyDeviceToHost, c.stream));
-  c.sync();
-  T v;
-  std::memcpy(&v, c.pinned, sizeof(T));
-  return v;
-}
-
-template <class T>
-inline T last(Ctx& c, DArray<T> const& a) {
-  return get_value(c, a.data() + a.size() - 1);
-}
-
 constexpr int kBlock = 256;
 
 inline unsigned nblocks(LO n, int block = kBlock) {
@@ -381,9 +367,9 @@ __device__ __forceinline__ LO row_of(LO p, LO nrows, LO const* offsets) {
 }
 
 // ---- primitives (osh_prims.hip) ----
-// exclusive scans (n + 1 outputs, out[0] = 0) of LO values, I8 values or I8
-// nonzero flags; several share one launch through offset_scans
-enum ScanKind { kScanLO = 0, kScanBytes = 1, kScanNonzero = 2 };
+// exclusive scans (n + 1 outputs, out[0] = 0) of LO values or I8 nonzero flags;
+// several share one launch through offset_scans
+enum ScanKind { kScanLO = 0, kScanNonzero = 1 };
 constexpr int kMaxScanJobs = 12;
 struct ScanJob {
   void const* in;
@@ -404,7 +390,6 @@ void noalloc_setup(int device);
 void offset_scans_noalloc(Ctx& c, ScanJob const* jobs, int njobs);
 // n+1 exclusive offsets; with `total`, also the sum (read back after a sync)
 LOs offset_scan(Ctx& c, LOs const& counts, LO* total = nullptr);
-LOs offset_scan_bytes(Ctx& c, Bytes const& counts, LO* total = nullptr);
 LOs collect_marked(Ctx& c, Bytes const& marks);       // indices of nonzero
 // the same, also returning the n+1 offsets of the nonzero marks
 LOs collect_marked(Ctx& c, Bytes const& marks, LOs* offsets_out);
@@ -464,7 +449,6 @@ Real min_real(Ctx& c, Reals const& a);
 // (Ctx::wait)
 Real min_real_wait(Ctx& c, Reals const& a);
 Real max_real(Ctx& c, Reals const& a);
-LO sum_lo(Ctx& c, LOs const& a);
 // stable sort of n tuples of `width` int64 keys; returns the permutation
 LOs sort_by_keys(Ctx& c, DArray<I64> const& keys, int width);
 
