@@ -628,7 +628,8 @@ static int pass(osh_mesh* mesh, const osh_adapt_opts* opts, int* did, int kind) 
       r = osh::swap_edges(c, mesh->m, o);
     else
       r = osh::coarsen_slivers(c, mesh->m, o);
-    c.sync();
+    // a pass that changed nothing has waited for all that it looked at
+    if (r) c.sync();
     if (did) *did = r ? 1 : 0;
   });
 }
