@@ -94,12 +94,13 @@ int osh_copy(osh_ctx* ctx, void* dst, const void* src, long long bytes);
 int osh_device_fill(osh_ctx* ctx, void* dst, long long n, int item_bytes, const void* value);
 /* *out = 1 when p is device memory */
 int osh_pointer_is_device(const void* p, int* out);
-/* the context's lane counts (no counterpart in the reference): "coarsen_lanes",
- * "side_lanes", "choose_lanes" and "first_lanes", each a power of two from 1
- * to 64, the threads that share one collapse side, one swap product side,
- * one swap candidate and one edge of the first independent-set round.  They
- * change no result, only speed; omega_h_amd/autotune.py picks them for a
- * workload. */
+/* the context's lane counts (no counterpart in the reference), each a power of
+ * two from 1 to 64: "coarsen_lanes", the threads that share one refine
+ * candidate, or one collapse side of osh_coarsen_qualities (at most 32 there);
+ * "side_lanes", one swap product side; "choose_lanes", a quarter of the threads
+ * that share one swap candidate, which are at least 8 and at most 64; and
+ * "first_lanes", one edge of the first independent-set round.  They change no
+ * result, only speed; omega_h_amd/autotune.py picks them for a workload. */
 int osh_ctx_set_tuning(osh_ctx* ctx, const char* name, int value);
 int osh_ctx_get_tuning(osh_ctx* ctx, const char* name, int* out);
 

@@ -4,8 +4,9 @@
     python -m omega_h_amd.autotune --workload batch --boxes 64
 
 Coordinate descent over a context's lane counts (Context.TUNING: the threads
-that share one collapse side, one swap product side, one swap candidate and
-one edge of the first independent-set round).  A setting is timed as the
+that share one refine candidate, one swap product side, a quarter of those that
+share one swap candidate, and those that share one edge of the first
+independent-set round).  A setting is timed as the
 median wall time of --reps adapt() calls, each on a fresh copy of the
 workload's input mesh made before the clock starts, and must leave the same
 mesh as the defaults (the four digests of vertex lists and classification,
@@ -30,7 +31,8 @@ TUNING_DIR = os.path.join(HERE, "tuning")
 CHOICES = {
     "coarsen_lanes": [2, 4, 8, 16, 32],
     "side_lanes": [4, 8, 16, 32, 64],
-    "choose_lanes": [2, 4, 8, 16, 32],
+    # four times as many threads, from 8 to 64: 1 is as 2, and 32 as 16
+    "choose_lanes": [2, 4, 8, 16],
     "first_lanes": [2, 4, 8, 16, 32],
 }
 

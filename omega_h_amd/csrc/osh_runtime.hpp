@@ -83,9 +83,9 @@ class Pool {
 // is spread over the device; omega_h_amd/autotune.py picks them for a
 // workload by timing adapt() and checking that the mesh stays the same.
 struct Tuning {
-  int coarsen_lanes = 8;  // threads per refine candidate; per side in coarsen_qualities
+  int coarsen_lanes = 8;  // threads per refine candidate; per side in coarsen_qualities (to 32)
   int side_lanes = 16;    // threads per swap product side searched for its match
-  int choose_lanes = 8;   // a quarter of the threads evaluating a swap candidate
+  int choose_lanes = 8;   // a quarter of the threads (8 to 64) evaluating a swap candidate
   int first_lanes = 8;    // threads per edge in the first independent-set round
 };
 
