@@ -10,8 +10,8 @@ A step is one adapt() of a fresh copy of that input mesh (the copies are made
 before the timed region; the mesh lives in HBM the whole time).  `value` is
 the adapt() throughput in the per-pass sense of the metric: the elements that
 entered every pass that rebuilt the mesh, divided by the summed wall time of
-those passes (each pass timed on the host clock with the stream drained at
-both ends), in millions per second.  `ms_per_step` is the wall time of a
+those passes (each timed on the host clock from when the pass before has been
+waited for to the wait for its own last kernel), in millions per second.  `ms_per_step` is the wall time of a
 whole adapt() call, including the calls that changed nothing.
 
 `mixed` times the same steps with the mixed-precision form (FP32 cavity
@@ -23,10 +23,10 @@ The `roofline` object covers the adapt's most expensive kernel, the
 coarsen quality sweep (coarsen_quality_lanes, through osh_coarsen_qualities)
 over every edge of the input shorter than 1/sqrt(2), both collapse
 directions, timed with HIP events on the library's own stream.  It is bound
-by FP64 arithmetic: achieved = 222 FP64 operations per cavity element
-evaluated (element_quality<3,3>: four 3x3 determinants, the volume, six
-metric products and the mean-ratio formula) times the elements evaluated,
-over the launch time, against MI355X's 78.6 TFLOP/s.  Divisions and cube
+by the issue of vector instructions: achieved = 166 FP64 operations per cavity
+element evaluated (element_quality<3,3> with the vertices' determinants in hand:
+the volume, six metric products and the mean-ratio formula) times the elements
+evaluated, over the launch time, against MI355X's 78.6 TFLOP/s.  Divisions and cube
 roots execute as instruction sequences, so the FP64 pipe's occupancy is
 larger than that fraction: `fp64_issue_frac` divides the kernel's FP64 wave
 instructions (counted by rocprofv3, profiles/) by what the pipe issues in the
@@ -59,11 +59,12 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0
 FP64_PEAK_TFLOPS = 78.6
 # FP64 operations (add, sub, mul, div, sqrt, cbrt: one each) of one
-# element_quality<3,3> (maxdet_metric + metric_element_quality): 4 x 14 for
-# the vertex metrics' determinants, 9 + 15 for the basis and volume, 2 for the
-# size, 9 for the other edge vectors, 6 x 20 + 6 + 1 for the mean squared
-# metric length, 5 for the mean ratio
-FLOPS_PER_QUALITY = 222
+# element_quality<3,3> with the vertices' determinants in hand
+# (metric_element_quality; the sweep takes each determinant once a vertex, 14
+# operations for some 240 qualities): 9 + 15 for the basis and volume, 2 for the
+# size, 9 for the other edge vectors, 6 x 20 + 6 + 1 for the mean squared metric
+# length, 4 for the mean ratio
+FLOPS_PER_QUALITY = 166
 PASS_NAMES = ("refine_by_size", "coarsen_by_size", "swap_edges", "coarsen_slivers")
 
 
