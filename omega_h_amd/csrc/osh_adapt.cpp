@@ -3,8 +3,9 @@
 //   adapt / pre_adapt / satisfy_lengths / satisfy_quality
 //   src/Omega_h_adapt.cpp:110-288
 // A pass is one refine_by_size, coarsen_by_size, swap_edges or
-// coarsen_slivers call that rebuilt the mesh; each is timed on the host
-// clock with the stream drained at both ends.
+// coarsen_slivers call that rebuilt the mesh; each is timed on the host clock
+// up to the wait for its last kernel, and begins when the one before has
+// been waited for.
 #include <chrono>
 #include <cstdio>
 #include <functional>
@@ -114,15 +115,15 @@ std::vector<int> below_quality(Ctx& c, std::vector<DMesh>& meshes, std::vector<i
   return low;
 }
 
-// *qmin (when given) receives the minimum element quality after a pass that
-// changed the mesh, whose reduction is also the pass's closing wait; one that
-// did not has waited for what it looked at
 // the most passes one adapt() records: a guard on the log, far above real
 // runs (the reference's loops have no limit; one 1.3M-tet box of the serving
 // workload under a constant anisotropic metric takes 4,639 swap and 283
 // sliver passes before it stops, unable to reach the quality goal)
 constexpr std::size_t kMaxLoggedPasses = std::size_t(1) << 22;
 
+// *qmin (when given) receives the minimum element quality after a pass that
+// changed the mesh, whose reduction is also the pass's closing wait; one that
+// did not has waited for what it looked at
 bool run_pass(Ctx& c, DMesh& m, AdaptOptions const& o, int kind,
     std::vector<PassRecord>* log, Real* qmin, PassHook const* hook,
     SwapCache* cache = nullptr) {

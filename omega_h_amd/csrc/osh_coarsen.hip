@@ -94,7 +94,7 @@ __device__ __forceinline__ int cell_job(CellSweep const& a, LO* c) {
 }
 
 constexpr int kLanes = 8;          // threads a key in the product builders below
-constexpr int kMaxSideLanes = 32;  // an edge's two sides share a wave
+constexpr int kMaxSideLanes = 32;  // a side's lanes are a 64-bit mask's, shifted into place
 
 // the vertices' metric determinants, which every quality around a vertex
 // needs (24 times in a tet mesh)
@@ -213,8 +213,9 @@ __global__ void __launch_bounds__(kBlock) coarsen_quality_lanes(LO nt, int lshif
 //    the one of higher quality among equally long ones, the first of those;
 //  - the vertex star (verts_across_edges, src/Omega_h_adj.cpp:512-530).
 //
-// Bound by FP64 issue (81 % of the cycles issue vector instructions): some 100
-// operations a new edge, 166 a quality, with their correctly rounded divisions.
+// Bound by the issue of vector instructions (all SIMD cycles of a large launch issue
+// one, 45 % of them FP64): some 100 operations a new edge, 166 a quality, with
+// their correctly rounded divisions.
 // A star's vertices are neighbors of all its sides, so they are brought to LDS
 // once, and the (target, edge) and (target, cell) pairs of the sides still open
 // are dealt out to the lanes together, a few edges or cells of each side at a

@@ -181,8 +181,9 @@ __global__ void mident_pairs_kernel(LO nt, LO const* edges, LO const* ev2v, Real
 }
 
 // up to this many edges the pairs of lanes fill places that would be empty: a
-// chain of two eigenvalue problems instead of three (11.6 against 16.5 us for
-// 100 edges)
+// chain of two eigenvalue problems instead of three: 7.4 against 12.7 us for 100
+// edges, 18.5 against 23.2 at the line.  Beyond it each exponential is still
+// taken twice and the lead shrinks (24.9 against 25.7 at 32,000)
 constexpr LO kPairEdges = 16384;
 
 // real_simplex_size (src/Omega_h_shape.hpp:77-100,166-170) of each element
